@@ -1,8 +1,10 @@
 // Matrix products C[M, N] = A[M, K] * W[N, K]^T (both operands K-contiguous, the layout of
 // activations and of nn.Linear weights; model/qwen/qwen_kv_paged.py:140-143, 224).
 //
+//  gemm_f32_mfma_kernel  a float32 operand (or two), K a multiple of four: the float32 matrix
+//                        instruction, nothing rounded below 32 bits.
 //  gemm_generic_kernel   any sizes and any mix of float32 / bfloat16 operands; plain FMA in
-//                        float32, K summed in order. This is the true 32-bit path.
+//                        float32, K summed in order.
 //  gemm_bf16_mfma_kernel bfloat16 operands, 128x128x64 tiles through LDS, 16x16x32 MFMA with
 //                        float32 accumulators. The library's product is faster for many rows
 //                        and is what the engine uses there; this kernel stays as the
@@ -98,6 +100,223 @@ SOC_EXPORT int soc_gemm_generic(const void* A, const void* W, void* C, int M, in
         case 7: return launch_generic<bf16, bf16, bf16>(A, W, C, M, N, K, stream);
     }
     return (int)hipErrorInvalidValue;
+}
+
+// ---------------------------------------------------------------------------------------------
+// Products with a float32 operand, on the matrix cores: v_mfma_f32_16x16x4_f32 multiplies and adds
+// in float32, so nothing is rounded that the FMA kernel above does not round (a bfloat16 operand
+// beside a float32 one is widened on its way into LDS, which is exact); only the order of the sums
+// differs. A wave owns NT x MT tiles of 16 x 16, four waves side by side along N (or two by two for
+// many rows) share a slab of 32 k of both operands in LDS, and the next slab is on its way into
+// registers meanwhile. The weight is the first operand, so a lane ends up with four consecutive
+// outputs of one row. A lane's four k of a 16-byte LDS read go to four products, so k is summed in
+// groups of four with a stride of four between a product's terms.
+// K may be cut over workgroups (float32 partial sums [S][M][N], added in order by the consumer or
+// by sum_parts_kernel below): few rows or a narrow output leave compute units idle otherwise.
+//
+// Measured, us cold (FMA kernel -> this one; what its bytes and its operations at 157 TFLOP/s take): 131 rows x 2,560 ->
+// 6,144 3,626 -> 64 (12, 26); 131 x 2,560 -> 19,456 686 -> 159 (38, 83); 131 x 9,728 -> 2,560 1,330 -> 86 (19, 42);
+// 3 x 2,560 -> 151,936 1,326 -> 339 (299, 15); 2,048 x 2,560 -> 6,144 1,886 -> 532 (12, 410). The error against 64
+// bits is the FMA kernel's or less (9.1e-7 -> 3.8e-7 to 9.1e-7 at K = 2,560: a part of K has a shorter chain).
+// Bound by the matrix cores and the padding of rows to 16 from a hundred rows on, by memory below.
+constexpr int FK = 32, FSTRIDE = FK + 4;         // k of a slab; floats from one LDS row to the next
+
+// four consecutive elements of a row, zeros outside the matrix (K is a multiple of four)
+template <typename T> __device__ __forceinline__ float4 f32_quad(const T* __restrict__ p, int row, int rows, int k, int k_end, int K) {
+    float x[4] = {0.f, 0.f, 0.f, 0.f};
+    if (row < rows && k < k_end) VecLoad<T, 4>::load(p + (size_t)row * K + k, x);
+    return make_float4(x[0], x[1], x[2], x[3]);
+}
+
+template <typename TA, typename TW, int MT, int NT, int WM>
+__global__ void __launch_bounds__(256)
+gemm_f32_mfma_kernel(const TA* __restrict__ A, const TW* __restrict__ W, float* __restrict__ C, bf16* __restrict__ Cb,
+                     int M, int N, int K, int m_blocks, int n_blocks, int k_part) {
+    constexpr int WN = 4 / WM, BMF = 16 * MT * WM, BNF = 16 * NT * WN;
+    constexpr int QA = (BMF * FK / 4 + 255) / 256, QW = BNF * FK / 4 / 256;    // 16-byte pieces per thread and slab
+    __shared__ __align__(16) float As[2][BMF][FSTRIDE];
+    __shared__ __align__(16) float Ws[2][BNF][FSTRIDE];
+    // Workgroups go round-robin over the eight XCDs: the row blocks of one run of weights follow each other on one
+    // XCD, so the weights come from memory once and then from its L2.
+    const int xcd = blockIdx.x % 8, idx = blockIdx.x / 8;
+    const int nb = idx / m_blocks * 8 + xcd, mb = idx % m_blocks;
+    if (nb >= n_blocks) return;
+    const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64, r = lane % 16, g = lane / 16;
+    const int wm = wave / WN, wn = wave % WN;
+    const int m0 = mb * BMF, n0 = nb * BNF;
+    const int k_lo = blockIdx.y * k_part, k_hi = min(K, k_lo + k_part);
+
+    f32x4 acc[NT][MT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int i = 0; i < MT; ++i) acc[j][i] = (f32x4){0.f, 0.f, 0.f, 0.f};
+
+    float4 a[QA], w[QW];
+    auto load = [&](int k0) {
+#pragma unroll
+        for (int q = 0; q < QW; ++q) {
+            const int piece = q * 256 + tid;
+            w[q] = f32_quad(W, n0 + piece / 8, N, k0 + piece % 8 * 4, k_hi, K);
+        }
+#pragma unroll
+        for (int q = 0; q < QA; ++q) {
+            const int piece = q * 256 + tid;
+            if (BMF * FK / 4 % 256 == 0 || piece < BMF * FK / 4) a[q] = f32_quad(A, m0 + piece / 8, M, k0 + piece % 8 * 4, k_hi, K);
+        }
+    };
+    auto store = [&](int b) {
+#pragma unroll
+        for (int q = 0; q < QW; ++q) {
+            const int piece = q * 256 + tid;
+            *reinterpret_cast<float4*>(&Ws[b][piece / 8][piece % 8 * 4]) = w[q];
+        }
+#pragma unroll
+        for (int q = 0; q < QA; ++q) {
+            const int piece = q * 256 + tid;
+            if (BMF * FK / 4 % 256 == 0 || piece < BMF * FK / 4) *reinterpret_cast<float4*>(&As[b][piece / 8][piece % 8 * 4]) = a[q];
+        }
+    };
+    load(k_lo);
+    store(0);
+    __syncthreads();
+    int b = 0;
+    for (int k0 = k_lo; k0 < k_hi; k0 += FK, b ^= 1) {
+        const bool more = k0 + FK < k_hi;
+        if (more) load(k0 + FK);
+#pragma unroll
+        for (int s = 0; s < FK; s += 16) {
+            float4 x[MT], y[NT];
+#pragma unroll
+            for (int i = 0; i < MT; ++i) x[i] = *reinterpret_cast<const float4*>(&As[b][(wm * MT + i) * 16 + r][s + 4 * g]);
+#pragma unroll
+            for (int j = 0; j < NT; ++j) y[j] = *reinterpret_cast<const float4*>(&Ws[b][(wn * NT + j) * 16 + r][s + 4 * g]);
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+#pragma unroll
+                for (int i = 0; i < MT; ++i) {
+                    acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(y[j].x, x[i].x, acc[j][i], 0, 0, 0);
+                    acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(y[j].y, x[i].y, acc[j][i], 0, 0, 0);
+                    acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(y[j].z, x[i].z, acc[j][i], 0, 0, 0);
+                    acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(y[j].w, x[i].w, acc[j][i], 0, 0, 0);
+                }
+        }
+        if (more) store(b ^ 1);          // the buffer that the slab before this one was read from: all are past it
+        __syncthreads();
+    }
+    if (C) C += (size_t)blockIdx.y * M * N;
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+        const int m = m0 + (wm * MT + i) * 16 + r;
+        if (m >= M) continue;
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            const int n = n0 + (wn * NT + j) * 16 + 4 * g;
+            const size_t at = (size_t)m * N + n;
+            if (n + 4 <= N && N % 4 == 0) {
+                if (C) *reinterpret_cast<float4*>(C + at) = make_float4(acc[j][i][0], acc[j][i][1], acc[j][i][2], acc[j][i][3]);
+                else *reinterpret_cast<uint2*>(Cb + at) = make_uint2(pack_bf16x2(acc[j][i][0], acc[j][i][1]), pack_bf16x2(acc[j][i][2], acc[j][i][3]));
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (n + e < N) {
+                        if (C) C[at + e] = acc[j][i][e];
+                        else Cb[at + e] = from_float<bf16>(acc[j][i][e]);
+                    }
+            }
+        }
+    }
+}
+
+// out[i] = the sum of parts[s][i] over s, in order; n is a multiple of four.
+template <typename TC>
+__global__ void __launch_bounds__(256)
+sum_parts_kernel(const float* __restrict__ parts, TC* __restrict__ out, size_t n, int S) {
+    const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    if (i >= n) return;
+    float4 t = *reinterpret_cast<const float4*>(parts + i);
+    for (int s = 1; s < S; ++s) {
+        const float4 v = *reinterpret_cast<const float4*>(parts + (size_t)s * n + i);
+        t.x += v.x; t.y += v.y; t.z += v.z; t.w += v.w;
+    }
+    if constexpr (sizeof(TC) == 4) *reinterpret_cast<float4*>(out + i) = t;
+    else *reinterpret_cast<uint2*>(out + i) = make_uint2(pack_bf16x2(t.x, t.y), pack_bf16x2(t.z, t.w));
+}
+
+// Form of such a product, the cheapest by a count of cycles whose constants were fitted to a sweep of all forms over the
+// shapes above (the choice is within 10 % of the sweep's best at each): `tiles` of 16 rows per wave (1 to 4, four waves along N; 5: 128 x 128 by two times two
+// waves) and how many workgroups share K.
+SOC_EXPORT int soc_gemm_f32_plan(int M, int N, int K, int partial_ok, int* tiles, int* splits) {
+    if (M < 1 || N < 1 || K < 4 || K % 4) return 0;
+    double best = 0.0;
+    *tiles = 0;
+    for (int t = 1; t <= 5; ++t) {
+        const int bm = t == 5 ? 128 : 16 * t, bn = t == 5 ? 128 : 64, per_wave = t == 5 ? 16 : t;
+        const double blocks = (double)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+        for (int s = 1; s <= 16; ++s) {
+            const int part = ((K + s - 1) / s + FK - 1) / FK * FK;
+            if (s > 1 && (part < 256 || (long)part * (s - 1) >= K || N % 4)) continue;
+            // Cycles per k: a wave alone waits for its slabs (65 per k measured: 76 us for one row of 2,560 x 6,144 uncut,
+            // 31 us in eight parts); waves that share a SIMD hide that and take 8 per tile of 16 x 16, 1.2 times that
+            // with the LDS reads and barriers beside them, and 4 for the slab. Whole workgroups per compute unit count while there are few.
+            const double per_cu = blocks * s / 256.0;
+            const double rounds = per_cu < 8.0 ? (double)(long)(per_cu + 0.999) : per_cu;
+            const double per_k = (9.6 * per_wave + 4.0) * rounds;
+            double us = (part * (per_k < 65.0 ? 65.0 : per_k) + 4000.0) / 2400.0;
+            // the weights come from memory once, and what is split is written and read again
+            const double stream = (double)N * K * 4 / 4.5e6;
+            if (us < stream) us = stream;
+            if (s > 1) us += (double)s * M * N * 4 * 2 / 4e6 + (partial_ok ? 0.0 : 4.0);
+            if (*tiles == 0 || us < best) { best = us; *tiles = t; *splits = s; }
+        }
+    }
+    return *tiles != 0;
+}
+
+template <typename TA, typename TW>
+static int launch_f32_mfma(const void* A, const void* W, float* C, bf16* Cb, int M, int N, int K, int tiles, int splits, hipStream_t s) {
+    const int bm = tiles == 5 ? 128 : 16 * tiles, bn = tiles == 5 ? 128 : 64;
+    const int mb = (M + bm - 1) / bm, nb = (N + bn - 1) / bn;
+    const int part = ((K + splits - 1) / splits + FK - 1) / FK * FK;
+    const long blocks = (long)((nb + 7) / 8) * 8 * mb;
+    if (blocks > 0x7fffffffL || (long)part * (splits - 1) >= K) return (int)hipErrorInvalidValue;
+    const dim3 grid((unsigned)blocks, splits);
+#define SOC_F32(MT_, NT_, WM_) \
+    hipLaunchKernelGGL((gemm_f32_mfma_kernel<TA, TW, MT_, NT_, WM_>), grid, dim3(256), 0, s, (const TA*)A, (const TW*)W, C, Cb, M, N, K, mb, nb, part)
+    switch (tiles) {
+        case 1: SOC_F32(1, 1, 1); break;
+        case 2: SOC_F32(2, 1, 1); break;
+        case 3: SOC_F32(3, 1, 1); break;
+        case 4: SOC_F32(4, 1, 1); break;
+        case 5: SOC_F32(4, 4, 2); break;
+        default: return (int)hipErrorInvalidValue;
+    }
+#undef SOC_F32
+    return soc_last_error();
+}
+
+// C [M, N] = A W^T with a float32 operand: dtypes 0 float32, 1 bfloat16, not both operands bfloat16. With splits > 1,
+// parts [splits][M][N] is written; C then receives their sum unless it is null (the consumer adds them). K is a
+// multiple of four and N too where K is split; A and W are aligned to four of their elements, C and parts to 16 bytes.
+SOC_EXPORT int soc_gemm_f32_mfma(const void* A, const void* W, void* C, float* parts, int M, int N, int K, int a_dtype,
+                                 int w_dtype, int c_dtype, int tiles, int splits, hipStream_t stream) {
+    if (M <= 0 || N <= 0) return 0;
+    if (K < 4 || K % 4 || splits < 1 || splits > 64 || (splits > 1 && (!parts || N % 4)) || (splits == 1 && !C)) return (int)hipErrorInvalidValue;
+    if (((uintptr_t)A % (a_dtype ? 8 : 16)) || ((uintptr_t)W % (w_dtype ? 8 : 16)) || ((uintptr_t)C % 16) || ((uintptr_t)parts % 16))
+        return (int)hipErrorInvalidValue;
+    float* out = splits > 1 ? parts : c_dtype == 0 ? (float*)C : nullptr;
+    bf16* out_b = out ? nullptr : (bf16*)C;
+    int err;
+    if (a_dtype == 0 && w_dtype == 0) err = launch_f32_mfma<float, float>(A, W, out, out_b, M, N, K, tiles, splits, stream);
+    else if (a_dtype == 0 && w_dtype == 1) err = launch_f32_mfma<float, bf16>(A, W, out, out_b, M, N, K, tiles, splits, stream);
+    else if (a_dtype == 1 && w_dtype == 0) err = launch_f32_mfma<bf16, float>(A, W, out, out_b, M, N, K, tiles, splits, stream);
+    else return (int)hipErrorInvalidValue;
+    if (err || splits == 1 || !C) return err;
+    const size_t n = (size_t)M * N;
+    const dim3 grid((unsigned)((n / 4 + 255) / 256));
+    if (c_dtype == 0) hipLaunchKernelGGL((sum_parts_kernel<float>), grid, dim3(256), 0, stream, parts, (float*)C, n, splits);
+    else hipLaunchKernelGGL((sum_parts_kernel<bf16>), grid, dim3(256), 0, stream, parts, (bf16*)C, n, splits);
+    return soc_last_error();
 }
 
 // ---------------------------------------------------------------------------------------------

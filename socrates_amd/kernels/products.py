@@ -409,8 +409,8 @@ class Products:
         return "library" if times[0] < 0.97 * times[1] else "own"
 
     def linear(self, x, w, out_dtype=None, allow_partial=False, row_tiles=0, n_waves=0, k_splits=0):
-        """x [M, K] times w [N, K] transposed. float32 operands (either) take the plain
-        float32 kernel. bfloat16 pairs: up to 16 rows the skinny MFMA kernel (it streams
+        """x [M, K] times w [N, K] transposed. float32 operands (either) take the
+        float32 kernels. bfloat16 pairs: up to 16 rows the skinny MFMA kernel (it streams
         the weights faster than the library does there); more rows the library product,
         or this package's tiled MFMA kernel if ``library_gemm`` is off. ``allow_partial``: the consumer
         (the residual-add + norm kernel) accepts float32 split-K partial sums [S, M, N]; the
@@ -533,6 +533,10 @@ class Products:
             if out_dtype == torch.bfloat16:
                 return torch.mm(x, w.t())
             return torch.mm(x, w.t(), out_dtype=out_dtype)
+        if not both_bf16:
+            out = self._linear_f32(x, w, out_dtype, allow_partial)
+            if out is not None:
+                return out
         out = torch.empty((M, N), dtype=out_dtype, device=self.device)
         args = (_ptr(x), _ptr(w), _ptr(out), c_int(M), c_int(N), c_int(K))
         if both_bf16 and K % 8 == 0 and K >= 8:
@@ -542,6 +546,27 @@ class Products:
                                               c_int(_DTYPE_CODE[out_dtype]), self._stream())
         _check(err, f"linear [{M}x{K}] x [{N}x{K}]^T")
         return out
+
+    def _linear_f32(self, x, w, out_dtype, allow_partial, tiles=0, splits=0):
+        """A product with a float32 operand on the matrix cores, in float32 throughout; None where
+        that kernel does not apply (K no multiple of four, an operand that is not aligned to four
+        of its elements: the FMA kernel takes those). ``tiles``, ``splits``: its form, override."""
+        (M, K), N = x.shape, w.shape[0]
+        if K % 4 or any(t.data_ptr() % (4 * t.element_size()) for t in (x, w)):
+            return None
+        t, s = c_int(0), c_int(0)
+        if not self._gemm.soc_gemm_f32_plan(c_int(M), c_int(N), c_int(K), c_int(1 if allow_partial else 0),
+                                            ctypes.byref(t), ctypes.byref(s)):
+            return None
+        tiles, splits = tiles or t.value, splits or s.value
+        parts = torch.empty((splits, M, N), dtype=torch.float32, device=self.device) if splits > 1 else None
+        out = None if allow_partial and splits > 1 else torch.empty((M, N), dtype=out_dtype, device=self.device)
+        self.forms[f"float32:{tiles}"] += 1
+        _check(self._gemm.soc_gemm_f32_mfma(_ptr(x), _ptr(w), _ptr(out), _ptr(parts), c_int(M), c_int(N), c_int(K),
+                                            c_int(_DTYPE_CODE[x.dtype]), c_int(_DTYPE_CODE[w.dtype]),
+                                            c_int(_DTYPE_CODE[out_dtype]), c_int(tiles), c_int(splits), self._stream()),
+               f"linear [{M}x{K}] x [{N}x{K}]^T")
+        return parts if out is None else out
 
     def settle(self, owed):
         """The normed rows themselves, bfloat16 [M, dim], of rows still owed their norm's factor."""

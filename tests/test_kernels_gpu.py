@@ -531,6 +531,38 @@ def test_weights_by_tile_give_the_same_bits(kernel_sets, M, d, K):
         hip.forget_packed()
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 64, 4), (3, 1000, 132), (16, 61, 260), (17, 128, 516), (49, 130, 1028),
+                                   (131, 192, 2564), (129, 257, 96)])
+@pytest.mark.parametrize("a,w", [(torch.float32, torch.float32), (torch.bfloat16, torch.float32), (torch.float32, torch.bfloat16)])
+def test_float32_products_on_the_matrix_cores(kernel_sets, M, N, K, a, w):
+    """Every form (rows per wave, parts of K), both results and partial sums. A float32 sum of K products is at most
+    K rounding steps of 2^-24 of the sum of their sizes off, in whatever order."""
+    hip, _ = kernel_sets[torch.float32]
+    x, weight = rnd((M, K), a, 31), rnd((N, K), w, 32)
+    want = x.double() @ weight.double().T
+    bound = (K + 16) * 2.0 ** -24 * (x.double().abs() @ weight.double().abs().T) + 1e-30
+    for tiles in (1, 2, 3, 4, 5):
+        for splits in (1, 2, 3):
+            part = -(-(-(-K // splits)) // 32) * 32
+            if splits > 1 and (part * (splits - 1) >= K or N % 4):
+                continue
+            got = hip._linear_f32(x, weight, torch.float32, False, tiles, splits)
+            assert ((got.double() - want).abs() <= bound).all(), (tiles, splits)
+            parts = hip._linear_f32(x, weight, torch.float32, True, tiles, splits)
+            assert tuple(parts.shape) == ((splits, M, N) if splits > 1 else (M, N))
+            assert torch.equal(parts if splits == 1 else sum(parts[1:], parts[0]), got)
+            rounded = hip._linear_f32(x, weight, torch.bfloat16, False, tiles, splits)
+            assert torch.equal(rounded, got.bfloat16())
+    hip.forms.clear()
+    close(hip.linear(x, weight, out_dtype=torch.float32), want, torch.float32, atol=float(bound.max()))
+    assert sum(hip.forms.values()) == 1
+    # an operand that starts in the middle of four, or a K that is no multiple of four: the FMA kernel
+    hip.forms.clear()
+    shifted = torch.empty(M * K + 1, dtype=a, device=DEV)[1:].view(M, K).copy_(x)
+    close(hip.linear(shifted, weight, out_dtype=torch.float32), want, torch.float32, atol=float(bound.max()))
+    assert not hip.forms
+
+
 def test_linear_float32_is_not_reduced_precision(kernel_sets):
     """Values that bfloat16 or a 19-bit matrix mode would round away survive."""
     hip, _ = kernel_sets[torch.float32]
