@@ -574,6 +574,23 @@ static void launch_linear_attention(const void* x, int ld, int col_q, int col_k,
 #undef SOC_LA_LAUNCH
 }
 
+// prep [n_tokens, 2 or 3, HD] as linear_prepare_kernel says.
+SOC_EXPORT int soc_linear_prepare(const void* x, int ld, int col_q, int col_k, float q_scale, int act, const float* z, const float* z_bias,
+                                  float tau, int HD, float* prep, int n_tokens, int dtype, hipStream_t stream) {
+    if (n_tokens <= 0 || HD <= 0) return 0;
+    if (z && (!z_bias || !(tau > 0.f))) return (int)hipErrorInvalidValue;
+    const float inv_tau = z ? 1.f / tau : 0.f;
+    const size_t total = (size_t)n_tokens * HD;
+    const int blocks = (int)((total + 255) / 256 < 16384 ? (total + 255) / 256 : 16384);
+    if (dtype == 0)
+        hipLaunchKernelGGL(linear_prepare_kernel<float>, dim3(blocks), dim3(256), 0, stream, (const float*)x, ld, col_q, col_k,
+                           q_scale, act, z, z_bias, inv_tau, HD, total, prep);
+    else
+        hipLaunchKernelGGL(linear_prepare_kernel<bf16>, dim3(blocks), dim3(256), 0, stream, (const bf16*)x, ld, col_q, col_k,
+                           q_scale, act, z, z_bias, inv_tau, HD, total, prep);
+    return soc_last_error();
+}
+
 SOC_EXPORT int soc_linear_attention(const void* x, int ld, int col_q, int col_k, int col_v, float q_scale, int act,
                                     const float* decays, const float* z, const float* z_bias, float tau, int H, int D, int Dv,
                                     float* state, long long stride, int offset, const int* seq_qstart, const int* seq_rows,
@@ -587,14 +604,8 @@ SOC_EXPORT int soc_linear_attention(const void* x, int ld, int col_q, int col_k,
     const float inv_tau = z ? 1.f / tau : 0.f;
     if (prep && !prepared) {                                            // scratch [n_tokens, 2 or 3, H * D]
         if (n_tokens <= 0) return (int)hipErrorInvalidValue;
-        const size_t total = (size_t)n_tokens * H * D;
-        const int blocks = (int)((total + 255) / 256 < 16384 ? (total + 255) / 256 : 16384);
-        if (dtype == 0)
-            hipLaunchKernelGGL(linear_prepare_kernel<float>, dim3(blocks), dim3(256), 0, stream, (const float*)x, ld, col_q, col_k,
-                               q_scale, act, z, z_bias, inv_tau, H * D, total, prep);
-        else
-            hipLaunchKernelGGL(linear_prepare_kernel<bf16>, dim3(blocks), dim3(256), 0, stream, (const bf16*)x, ld, col_q, col_k,
-                               q_scale, act, z, z_bias, inv_tau, H * D, total, prep);
+        const int err = soc_linear_prepare(x, ld, col_q, col_k, q_scale, act, z, z_bias, tau, H * D, prep, n_tokens, dtype, stream);
+        if (err) return err;
     }
 #define SOC_LA_F32(DK) launch_linear_attention<float, DK>(x, ld, col_q, col_k, col_v, q_scale, act, decays, z, z_bias, inv_tau, H, D, Dv, state, stride, offset, seq_qstart, seq_rows, prep, prepared, ones, out, n_seqs, cw, stream)
 #define SOC_LA_BF16(DK) launch_linear_attention<bf16, DK>(x, ld, col_q, col_k, col_v, q_scale, act, decays, z, z_bias, inv_tau, H, D, Dv, state, stride, offset, seq_qstart, seq_rows, prep, prepared, ones, out, n_seqs, cw, stream)

@@ -301,6 +301,22 @@ static void launch_retention(const void* x, int ld, int col_q, int col_k, int co
 #undef SOC_RET_LAUNCH
 }
 
+// turned [n_tokens, 2, H * D] float32: q and k of every token turned by its position, k times k_scale.
+SOC_EXPORT int soc_retention_turn(const void* x, int ld, int col_q, int col_k, const int* positions, const float* inv_freq, int half,
+                                  float k_scale, int H, int D, float* turned, int n_tokens, int dtype, hipStream_t stream) {
+    if (n_tokens <= 0 || H <= 0) return 0;
+    if (D < 1 || half < 0 || 2 * half > D || (half && !inv_freq)) return (int)hipErrorInvalidValue;
+    const size_t total = (size_t)n_tokens * H * (D - half);
+    const int blocks = (int)((total + 255) / 256 < 16384 ? (total + 255) / 256 : 16384);
+    if (dtype == 0)
+        hipLaunchKernelGGL(retention_turn_kernel<float>, dim3(blocks), dim3(256), 0, stream, (const float*)x, ld, col_q, col_k,
+                           positions, inv_freq, half, k_scale, H, D, total, turned);
+    else
+        hipLaunchKernelGGL(retention_turn_kernel<bf16>, dim3(blocks), dim3(256), 0, stream, (const bf16*)x, ld, col_q, col_k,
+                           positions, inv_freq, half, k_scale, H, D, total, turned);
+    return soc_last_error();
+}
+
 SOC_EXPORT int soc_retention(const void* x, int ld, int col_q, int col_k, int col_v, const int* positions, const float* inv_freq,
                              int half, float k_scale, const float* decays, int H, int D, int Dv, float* state, long long stride,
                              int offset, const int* seq_qstart, const int* seq_rows, float* turned, int n_tokens, float* out,
@@ -308,14 +324,8 @@ SOC_EXPORT int soc_retention(const void* x, int ld, int col_q, int col_k, int co
     if (n_seqs <= 0 || H <= 0) return 0;
     if (D < 1 || D > 256 || Dv < 1 || n_seqs > 65535 || 2 * half > D) return (int)hipErrorInvalidValue;
     if (turned) {                                          // scratch [n_tokens, 2, H * D]: turn q and k ahead of the walk
-        const size_t total = (size_t)n_tokens * H * (D - half);
-        const int blocks = (int)((total + 255) / 256 < 16384 ? (total + 255) / 256 : 16384);
-        if (dtype == 0)
-            hipLaunchKernelGGL(retention_turn_kernel<float>, dim3(blocks), dim3(256), 0, stream, (const float*)x, ld, col_q, col_k,
-                               positions, inv_freq, half, k_scale, H, D, total, turned);
-        else
-            hipLaunchKernelGGL(retention_turn_kernel<bf16>, dim3(blocks), dim3(256), 0, stream, (const bf16*)x, ld, col_q, col_k,
-                               positions, inv_freq, half, k_scale, H, D, total, turned);
+        const int err = soc_retention_turn(x, ld, col_q, col_k, positions, inv_freq, half, k_scale, H, D, turned, n_tokens, dtype, stream);
+        if (err) return err;
     }
     const int cw = columns_per_workgroup(H, Dv, n_seqs, max_q_len);
 #define SOC_RET_F32(DK) launch_retention<float, DK>(x, ld, col_q, col_k, col_v, positions, inv_freq, half, k_scale, decays, H, D, Dv, state, stride, offset, seq_qstart, seq_rows, turned, out, n_seqs, cw, stream)

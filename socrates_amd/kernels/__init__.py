@@ -14,7 +14,8 @@ arithmetic of key splits,
 ``mixers.py`` the mixers with a state per row, attention over a cached latent and blocks with norms
 on both sides of a branch, ``hybrid.py`` attention whose keys and values differ in size, retention, routed
 experts and a per-token side input, ``memory.py`` a matrix memory with exponential gates and the two maps of
-differential attention, ``delta.py`` the gated delta rule, ``streams.py`` several copies of the residual stream,
+differential attention, ``delta.py`` the gated delta rule, ``streams.py`` several copies of the residual stream, ``scan.py`` the
+recurrences with a matrix state in chunks of a prompt portion,
 ``common.py`` what they share, ``build.py`` the compiler and loader.
 """
 
@@ -37,13 +38,14 @@ from .common import (_ATTENTION_SIGNATURES, _ATTENTION_UP_TO_256, _DTYPE_CODE, _
                      NormOwed, RowsByTile, _check, _declare, _ptr)
 from .planning import MAX_KEY_SPLITS, plan_key_splits
 from .products import Products
+from .scan import Scan
 from .streams import Streams
 
 __all__ = ["HipKernels", "KernelBuildError", "KernelError", "MAX_KEY_SPLITS", "NormOwed", "RowsByTile", "build_all",
            "compile_library", "load_library", "plan_key_splits"]
 
 
-class HipKernels(Products, Attention, Latent, Mixers, Hybrid, Composite, Memory, Streams, Delta):
+class HipKernels(Products, Attention, Latent, Mixers, Hybrid, Composite, Memory, Streams, Delta, Scan):
     def __init__(self, dtype=torch.bfloat16, device="cuda:0"):
         if dtype not in _DTYPE_CODE:
             raise ValueError(f"compute dtype must be float32 or bfloat16, not {dtype}")

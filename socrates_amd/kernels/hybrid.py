@@ -5,7 +5,7 @@ a model first asks for one of them."""
 
 from __future__ import annotations
 
-from ctypes import c_float, c_int, c_longlong
+from ctypes import c_float, c_int, c_longlong, c_void_p
 
 import torch
 
@@ -17,6 +17,7 @@ EXPERT_TILE = 16         # places of one expert that a workgroup of the products
 # ... or, in bfloat16, (tokens per expert on average from which, places). Tiles of 256 places were measured and lost
 # (a prompt of 2,048 tokens at 4B-sized layers, 256 tokens per expert on average: 20.5 against 17.6 ms).
 EXPERT_TILES_MANY = ((48, 128),)
+from .scan import HEAD
 
 
 class ExpertRuns:
@@ -139,8 +140,17 @@ class Hybrid:
         # a step with a portion of some length: q and k are turned once, ahead of the walk (each of a head's
         # workgroups would turn them again); single tokens and short portions are turned where they are staged
         turned = None
-        if half and ctx.max_q_len >= self.retention_turn_ahead:
+        chunks = self._in_chunks(ctx, D)
+        if chunks or half and ctx.max_q_len >= self.retention_turn_ahead:
             turned = torch.empty((N, 2, H * D), dtype=torch.float32, device=self.device)
+        if chunks:
+            _check(self._hybrid().soc_retention_turn(
+                _ptr(x), c_int(ld), c_int(col_q), c_int(col_k), _ptr(ctx.positions), _ptr(inv_freq if half else None), c_int(half),
+                c_float(k_scale), c_int(H), c_int(D), _ptr(turned), c_int(N), c_int(self.code), self._stream()), "retention_turn")
+            ahead = [turned.data_ptr(), turned.data_ptr() + 4 * H * D]
+            return self._scan(HEAD, c_void_p(ahead[0]), 2 * H * D, D, c_void_p(ahead[1]), 2 * H * D, D,
+                              c_void_p(x.data_ptr() + col_v * x.element_size()), ld, Dv, _ptr(decays), H, D, Dv, state, stride, offset,
+                              ctx, N, out)
         _check(self._hybrid().soc_retention(
             _ptr(x), c_int(ld), c_int(col_q), c_int(col_k), c_int(col_v), _ptr(ctx.positions), _ptr(inv_freq if half else None),
             c_int(half), c_float(k_scale), _ptr(decays), c_int(H), c_int(D), c_int(Dv), _ptr(state), stride, c_int(offset),

@@ -4,13 +4,14 @@ and loaded when a model first asks for one of them."""
 
 from __future__ import annotations
 
-from ctypes import c_float, c_int, c_longlong
+from ctypes import c_float, c_int, c_longlong, c_void_p
 
 import torch
 
 from .build import load_library
 from .common import _DTYPE_CODE, _MIXER_SIGNATURES, KernelError, _check, _declare, _ptr
 from .hybrid import ExpertSums
+from .scan import BONUS, STEP
 
 
 class Mixers:
@@ -160,6 +161,10 @@ class Mixers:
         self._want(gain, "gain", torch.float32, (C,))
         stride = self._state(state, offset, H * D * D, ctx)
         raw = torch.empty((N, C), dtype=torch.float32, device=self.device)
+        if self._in_chunks(ctx, D):
+            self._scan(BONUS, _ptr(r), C, D, _ptr(k), C, D, _ptr(v), C, D, _ptr(decay), H, D, D, state, stride, offset, ctx, N, raw,
+                       q_f32=False, lda=C, params=[_ptr(bonus)])
+            return self.gated_group_norm(raw, g, gain, H, eps, gate_first=False)
         _check(self._mixers().soc_wkv(_ptr(r), _ptr(k), _ptr(v), _ptr(decay), _ptr(bonus), c_int(H), c_int(D), _ptr(state),
                                       stride, c_int(offset), _ptr(ctx.seq_qstart), _ptr(ctx.seq_rows), _ptr(raw),
                                       c_int(ctx.n_seqs), c_int(ctx.max_q_len), c_int(self.code), self._stream()), "wkv")
@@ -197,6 +202,11 @@ class Mixers:
             raise KernelError(f"ssd: {H} heads in {G} groups, state {Ns}, head size {P}")
         stride = self._state(state, offset, H * Ns * P, ctx)
         out = torch.empty((N, H * P), dtype=torch.float32, device=self.device)
+        if self._in_chunks(ctx, Ns):
+            ld, item = H * P + 2 * G * Ns, xbc.element_size()
+            b, c = (c_void_p(xbc.data_ptr() + (H * P + i * G * Ns) * item) for i in range(2))
+            return self._scan(STEP, c, ld, Ns, b, ld, Ns, _ptr(xbc), ld, P, _ptr(dt), H, Ns, P, state, stride, offset, ctx, N, out,
+                              group=H // G, q_f32=False, params=[_ptr(dt_bias), _ptr(a_log), _ptr(skip)])
         _check(self._mixers().soc_ssd(_ptr(xbc), _ptr(dt), _ptr(dt_bias), _ptr(a_log), _ptr(skip), c_int(H), c_int(P), c_int(Ns),
                                       c_int(G), _ptr(state), stride, c_int(offset), _ptr(ctx.seq_qstart), _ptr(ctx.seq_rows),
                                       _ptr(out), c_int(ctx.n_seqs), c_int(ctx.max_q_len), c_int(self.code), self._stream()), "ssd")

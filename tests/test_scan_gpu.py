@@ -1,0 +1,182 @@
+"""The recurrences with a matrix state taken 64 tokens at a time, against float64 token by token and against the
+walk: portions around whole chunks and runs of 16 tokens, sizes that are no multiple of a tile, decays of one, of
+almost nothing and of zero, states that are not zero, and the chunks taken in several rounds."""
+
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+DTYPES = {"float32": torch.float32, "bfloat16": torch.bfloat16}
+
+
+@pytest.fixture(scope="module")
+def kernel_sets():
+    from socrates_amd.kernels import HipKernels
+    return {n: HipKernels(dt, DEV) for n, dt in DTYPES.items()}
+
+
+def step_of(lengths):
+    starts = torch.tensor([0] + lengths).cumsum(0)
+    return SimpleNamespace(n_seqs=len(lengths), max_q_len=max(lengths), n_tokens=int(starts[-1]), seq_qstart=starts.int().to(DEV),
+                           seq_rows=torch.arange(len(lengths)).flip(0).int().to(DEV), positions=torch.arange(int(starts[-1])).int().to(DEV))
+
+
+def rnd(shape, dtype, seed, scale=1.0):
+    return (torch.randn(shape, generator=torch.Generator().manual_seed(seed)) * scale).to(dtype).to(DEV)
+
+
+def decays_of(shape, seed):
+    """Most between 0.3 and 1; some 1, some 1e-30, some 0."""
+    g = torch.Generator().manual_seed(seed)
+    a = torch.rand(shape, generator=g) * 0.7 + 0.3
+    for share, value in ((0.2, 1.0), (0.01, 1e-30), (0.01, 0.0)):
+        a[torch.rand(shape, generator=g) < share] = value
+    return a.to(DEV)
+
+
+def walk64(ctx, q, k, v, a, S, bonus=None, take=None, skip=None):
+    """q, k, a [N, H, D], v [N, H, Dv], S [rows, H, D, Dv], all float64; S is moved on in place."""
+    out = torch.empty_like(v)
+    starts, rows = ctx.seq_qstart.tolist(), ctx.seq_rows.tolist()
+    for i, row in enumerate(rows):
+        for n in range(starts[i], starts[i + 1]):
+            add = k[n][:, :, None] * v[n][:, None]
+            if bonus is None:
+                S[row] = a[n][:, :, None] * S[row] + add
+                out[n] = (q[n][:, None] @ S[row])[:, 0]
+            else:
+                out[n] = (q[n][:, None] @ (S[row] + bonus[:, :, None] * add))[:, 0]
+                S[row] = a[n][:, :, None] * S[row] + add
+    return out if skip is None else out + skip[:, None] * v
+
+
+LENGTHS = [[64, 63, 1], [65, 16, 17, 200], [129], [256, 5], [7]]
+
+
+def check(ops, call, want, S0, S1):
+    """In chunks as close to float64 as the walk, or within a few roundings of the sums; the same in rounds."""
+    got = {}
+    for name, settings in (("walk", dict(scan_from=0)), ("chunks", dict(scan_from=1)), ("rounds", dict(scan_from=1, scan_scratch=1))):
+        for s, v in settings.items():
+            setattr(ops, s, v)
+        try:
+            state = S0.clone()
+            ops.forms.clear()
+            got[name] = (call(state), state)
+            assert ops.forms["scan"] == (name != "walk")
+        finally:
+            for s in settings:
+                delattr(ops, s)
+    for i, exact in enumerate((want, S1)):
+        def off(name):
+            return float((got[name][i].double().reshape(exact.shape) - exact).norm() / exact.norm())
+        assert off("chunks") <= 1.5 * off("walk") + 2e-7, (off("chunks"), off("walk"))
+        assert torch.equal(got["chunks"][i], got["rounds"][i])
+
+
+@pytest.mark.parametrize("dtype", list(DTYPES))
+@pytest.mark.parametrize("lengths", LENGTHS)
+@pytest.mark.parametrize("H,D,Dv", [(2, 64, 64), (1, 128, 256), (3, 20, 33), (1, 100, 65)])
+@pytest.mark.parametrize("kind", ["head", "channel", "prepared"])
+def test_linear_attention_in_chunks(kernel_sets, dtype, lengths, H, D, Dv, kind):
+    ops, dt, ctx = kernel_sets[dtype], DTYPES[dtype], step_of(lengths)
+    N = ctx.n_tokens
+    x = rnd((N, 5 + 2 * H * D + H * Dv), dt, 1, 0.5)
+    cols = (5, 5 + H * D, 5 + 2 * H * D)
+    q, k = (x[:, c:c + H * D].double().view(N, H, D) for c in cols[:2])
+    v = x[:, cols[2]:cols[2] + H * Dv].double().view(N, H, Dv)
+    S0 = rnd((len(lengths), 3 + H * D * Dv), torch.float32, 2)
+    S = S0[:, 3:].double().view(-1, H, D, Dv).clone()
+    if kind == "head":
+        decays = decays_of((H,), 5)
+        silu = torch.nn.functional.silu
+        want = walk64(ctx, silu(q) * 0.3, silu(k), silu(v), decays.double()[None, :, None].expand(N, H, D), S)
+        args, more = (0.3, True, decays, None, None, 1.0), {}
+    elif kind == "channel":
+        z, zb = rnd((N, H * D), torch.float32, 3, 8.0), rnd((H * D,), torch.float32, 4)
+        a = torch.exp(torch.nn.functional.logsigmoid(z.double() + zb.double()) / 4.0).view(N, H, D)
+        want = walk64(ctx, q * 0.3, k, v, a, S)
+        args, more = (0.3, False, None, z, zb, 4.0), {}
+    else:
+        a = decays_of((N, H, D), 6)
+        prepared = torch.stack([q.float(), k.float(), a], 1).view(N, 3, H * D).contiguous()
+        ones = 1
+        v = torch.cat([x[:, cols[2]:cols[2] + H * (Dv - 1)].double().view(N, H, Dv - 1), torch.ones(N, H, 1, dtype=torch.float64, device=DEV)], -1)
+        want = walk64(ctx, q, k, v, a.double(), S)
+        args, more = (1.0, False, None, None, None, 1.0), dict(prepared=prepared, ones=ones)
+
+    def call(state):
+        return ops.linear_attention(x, cols, H, D, Dv, *args, state, 3, ctx, **more)
+    check(ops, call, want.reshape(N, -1), S0, torch.cat([S0[:, :3].double(), S.reshape(len(lengths), -1)], 1))
+
+
+@pytest.mark.parametrize("dtype", list(DTYPES))
+@pytest.mark.parametrize("lengths", LENGTHS)
+@pytest.mark.parametrize("H,D", [(3, 64), (1, 128), (2, 36)])
+def test_bonus_recurrence_in_chunks(kernel_sets, dtype, lengths, H, D):
+    ops, dt, ctx = kernel_sets[dtype], DTYPES[dtype], step_of(lengths)
+    N, C = ctx.n_tokens, H * D
+    r, k, v = (rnd((N, C), dt, i, 0.5) for i in range(3))
+    decay, bonus = decays_of((N, C), 7), rnd((H, D), torch.float32, 8)
+    S0 = rnd((len(lengths), C * D), torch.float32, 9)
+    S = S0.double().view(-1, H, D, D).clone()
+    want = walk64(ctx, *(t.double().view(N, H, D) for t in (r, k, v, decay)), S, bonus=bonus.double())
+    kept = ops.gated_group_norm
+    ops.gated_group_norm = lambda raw, *a, **kw: raw           # the recurrence alone
+    try:
+        check(ops, lambda state: ops.wkv(r, k, v, decay, v, bonus, bonus.view(-1), 1e-5, H, state, 0, ctx), want.reshape(N, C), S0,
+              S.reshape(len(lengths), -1))
+    finally:
+        ops.gated_group_norm = kept
+
+
+@pytest.mark.parametrize("dtype", list(DTYPES))
+@pytest.mark.parametrize("lengths", LENGTHS)
+@pytest.mark.parametrize("H,P,Ns,G", [(4, 64, 128, 1), (2, 33, 20, 2), (6, 24, 64, 3)])
+def test_step_size_recurrence_in_chunks(kernel_sets, dtype, lengths, H, P, Ns, G):
+    ops, dt, ctx = kernel_sets[dtype], DTYPES[dtype], step_of(lengths)
+    N = ctx.n_tokens
+    xbc, raw = rnd((N, H * P + 2 * G * Ns), dt, 1, 0.5), rnd((N, H), torch.float32, 2, 2.0)
+    bias, a_log, skip = rnd((H,), torch.float32, 3), rnd((H,), torch.float32, 4), rnd((H,), torch.float32, 5)
+    step = torch.nn.functional.softplus(raw.double() + bias.double(), threshold=1e9)
+    decay = torch.exp(-torch.exp(a_log.double()) * step)[..., None].expand(N, H, Ns)
+    x = xbc[:, :H * P].double().view(N, H, P)
+    B, C = (xbc[:, H * P + i * G * Ns:H * P + (i + 1) * G * Ns].double().view(N, G, Ns).repeat_interleave(H // G, 1) for i in range(2))
+    S0 = rnd((len(lengths), H * Ns * P), torch.float32, 6)
+    S = S0.double().view(-1, H, Ns, P).clone()
+    want = walk64(ctx, C, B * step[..., None], x, decay, S, skip=skip.double())
+    check(ops, lambda state: ops.ssd(xbc, raw, bias, a_log, skip, H, P, Ns, G, state, 0, ctx), want.reshape(N, -1), S0,
+          S.reshape(len(lengths), -1))
+
+
+@pytest.mark.parametrize("dtype", list(DTYPES))
+@pytest.mark.parametrize("H,D,Dv,rot", [(2, 128, 128, 128), (3, 20, 28, 12), (1, 48, 80, 0)])
+def test_retention_in_chunks(kernel_sets, dtype, H, D, Dv, rot):
+    ops, dt, ctx = kernel_sets[dtype], DTYPES[dtype], step_of([65, 16, 17, 200])
+    N = ctx.n_tokens
+    x = rnd((N, 2 * H * D + H * Dv), dt, 1, 0.5)
+    inv_freq = (1e4 ** (-torch.arange(rot // 2).double() * 2 / max(rot, 1))).float().to(DEV) if rot else None
+    decays = torch.tensor([0.9, 1.0, 0.0][:H], device=DEV)
+    S0 = rnd((4, H * D * Dv), torch.float32, 2)
+    S = S0.double().view(-1, H, D, Dv).clone()
+    q, k = (x[:, i * H * D:(i + 1) * H * D].double().view(N, H, D) for i in range(2))
+    if rot:
+        angle = (ctx.positions.float()[:, None] * inv_freq[None]).double()[:, None]          # the angle itself is float32
+        def turn(t):
+            a, b = t[..., :rot // 2], t[..., rot // 2:rot]
+            return torch.cat([a * angle.cos() - b * angle.sin(), b * angle.cos() + a * angle.sin(), t[..., rot:]], -1)
+        q, k = turn(q), turn(k)
+    v = x[:, 2 * H * D:].double().view(N, H, Dv)
+    want = walk64(ctx, q, k * D ** -0.5, v, decays.double()[None, :, None].expand(N, H, D), S)
+    check(ops, lambda state: ops.retention(x, (0, H * D, 2 * H * D), H, D, Dv, inv_freq, rot, D ** -0.5, decays, state, 0, ctx),
+          want.reshape(N, -1), S0, S.reshape(4, -1))
+
+
+def test_from_which_portion_on(kernel_sets):
+    ops = kernel_sets["float32"]
+    assert [ops._in_chunks(SimpleNamespace(max_q_len=n), D) for n, D in ((1, 64), (127, 64), (128, 64), (4000, 128), (4000, 129))] == [
+        False, False, True, True, False]
