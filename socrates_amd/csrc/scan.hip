@@ -17,15 +17,21 @@
 // chunk's queries, keys and decays of 128 channels do not fit LDS.
 //
 // Measured for 2,048 tokens of one prompt, us, the walk -> these kernels with what prepares them: retention (20 heads of
-// 128 x 128) 908 -> 110 (chunks 48, states 17, apply 30), gated linear attention (10 of 128 x 256) 1,032 -> 136 (75, 17, 30),
-// wkv (40 of 64 x 64) 595 -> 100 with its norm (55, 10, 18), ssd (80 of 128 x 64) 1,166 -> 175 (101, 24, 58).
+// 128 x 128) 908 -> 108 (chunks 46, states 18, apply 31), gated linear attention (10 of 128 x 256) 1,030 -> 131 (67, 18, 29),
+// wkv (40 of 64 x 64) 595 -> 100 with its norm (53, 10, 16), ssd (80 of 128 x 64) 1,166 -> 168 (97, 24, 54); the gated
+// delta rule (20 of 128 x 128), 3,000 tokens, 700 -> 290 with its convolutions (127, states 93, 37). scan_chunks is
+// bound by its reads of LDS, a 4-byte read per operand and product where an operand lies across the tokens.
 #include "common.h"
+#include "recurrent.h"          // lds_barrier: loads and stores on their way are not waited for
 
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 constexpr int SCAN_C = 64;                 // tokens of a chunk
 constexpr int SCAN_AS = SCAN_C + 4;        // floats from one row of scores to the next in LDS
 constexpr int SCAN_VC = 32, SCAN_VS = SCAN_VC + 4;   // value columns at a time, floats from one row to the next
+
+// Waves of a workgroup that takes a chunk: 16 where LDS leaves room for one workgroup on a compute unit only.
+constexpr int scan_waves(int DK, bool one) { return DK == 128 && one ? 16 : 8; }
 
 // What the decays are, and which state an output sees.
 enum { SCAN_HEAD = 0,      // decays[h]; the state after the token
@@ -45,40 +51,104 @@ struct ScanArgs {
     float* state;
     long long stride;
     int offset;
-    // [N, H Dv]; per slot and head: addend, later state [D, Dv]; queries decayed to the chunk's start [64, DK] (a decay
+    // [N, H Dv]; per slot and head: addend, later state, in tiles; queries decayed to the chunk's start [64, DK] (a decay
     // per channel) or those decays [64]; the chunk's whole decay [DK]
     float *out, *adds, *queries, *factors;
 };
+
+// Addends and states lie in tiles of 16 channels x 16 columns as a lane of the matrix products has them, so that a
+// wave's store or load is 1 KB in one piece and no size needs a mask: [channel tile][column tile][lane][4], lane
+// (r, g) = (lane % 16, lane / 16) holding channels 4 g .. 4 g + 3 of one column. The columns of two neighbouring tiles
+// take turns by fours, so that the outputs of a lane of scan_apply are eight neighbours.
+__device__ __forceinline__ int scan_col(int p, int r) { return r / 4 * 8 + p * 4 + r % 4; }     // within 32 columns
+__host__ __device__ __forceinline__ int scan_tiles(int Dv) { return (Dv + 31) / 32 * 2; }
 
 // Scratch of a sequence's chunk: with one launch over all tokens the chunks lie one behind the other.
 __device__ __forceinline__ size_t scan_slot(const ScanArgs& a, int seq, int c) {
     return a.compact ? (size_t)(a.qstart[seq] / SCAN_C + seq + c) : (size_t)seq * a.count + c;
 }
 
-template <typename T> __device__ __forceinline__ float4 scan_quad(const T* __restrict__ p, int n, int vec) {
+// Four elements of a row of which the first n exist (n <= 0: none; then p is not read where vec). With vec the load
+// stands on its own, at an address that exists whatever n: a branch around it would make the wave wait for it there.
+template <typename T> __device__ __forceinline__ float4 scan_quad(const T* __restrict__ p, const T* __restrict__ any, int n, int vec) {
     float x[4] = {0.f, 0.f, 0.f, 0.f};
-    if (vec && n >= 4) VecLoad<T, 4>::load(p, x);
-    else
+    if (vec) {
+        VecLoad<T, 4>::load(n > 0 ? p : any, x);
+        return n > 0 ? make_float4(x[0], x[1], x[2], x[3]) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-            if (e < n) x[e] = to_float(p[e]);
+    for (int e = 0; e < 4; ++e)
+        if (e < n) x[e] = to_float(p[e]);
     return make_float4(x[0], x[1], x[2], x[3]);
 }
 
 __device__ __forceinline__ float4 mul4(float4 a, float4 b) { return make_float4(a.x * b.x, a.y * b.y, a.z * b.z, a.w * b.w); }
 __device__ __forceinline__ float4 mul4(float4 a, float b) { return make_float4(a.x * b, a.y * b, a.z * b, a.w * b); }
 
+__device__ __forceinline__ f32x4 mfma4(float a0, float a1, float a2, float a3, float4 b, f32x4 c) {
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, b.x, c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, b.y, c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a2, b.z, c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a3, b.w, c, 0, 0, 0);
+}
+// sum over k of 16 of col[k][m] row[n][k]: col points at [4 g][m of the lane] with ld floats between the k, row at [n of the lane][4 g]
+__device__ __forceinline__ f32x4 mfma_col_row(const float* col, int ld, const float* row, f32x4 c) {
+    return mfma4(col[0], col[ld], col[2 * ld], col[3 * ld], *reinterpret_cast<const float4*>(row), c);
+}
+
+// 32 columns of values (Vs [64][SCAN_VS]): out = X V of the chunk's tokens (X [64][SCAN_AS], lower triangle), and the
+// addend Z^T V to the state in tiles (Z [64][DK + 4]). NW waves, eight or more.
+template <int DK, int NW>
+__device__ __forceinline__ void scan_values(float* __restrict__ out, int H, int Dv, bool by4, int lo, int nt, int head, int col0, int tiles,
+                                            const float* Z, const float* Vs, const float* X, float* __restrict__ adds, int ch_tiles,
+                                            int wave, int r, int g) {
+    constexpr int LS = DK + 4, PER = NW * 16 / DK, TILES = 2 / PER;      // PER: waves that share 16 channels
+    if (NW == 8 || wave < 8) {
+        const int I = wave / 2, p = wave % 2;
+        f32x4 o = {0.f, 0.f, 0.f, 0.f};
+        for (int s = 0; s <= I; ++s)
+            o = mfma_col_row(Vs + (16 * s + 4 * g) * SCAN_VS + p * 16 + r, SCAN_VS, X + (I * 16 + r) * SCAN_AS + 16 * s + 4 * g, o);
+        const int t = I * 16 + r, col = col0 + p * 16 + 4 * g;
+        if (t < nt) {
+            float* to = out + ((size_t)(lo + t) * H + head) * Dv + col;
+            if (by4 && col + 4 <= Dv) *reinterpret_cast<float4*>(to) = make_float4(o[0], o[1], o[2], o[3]);
+            else
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (col + e < Dv) to[e] = o[e];
+        }
+    }
+    const int ct = wave / PER, p0 = wave % PER;      // 16 channels by both tiles of columns, or by one
+    f32x4 s[TILES];
+#pragma unroll
+    for (int p = 0; p < TILES; ++p) s[p] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int m = 0; m < SCAN_C; m += 16)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int t = m + 4 * g + e;
+            const float x = Z[t * LS + ct * 16 + r];
+#pragma unroll
+            for (int p = 0; p < TILES; ++p) s[p] = __builtin_amdgcn_mfma_f32_16x16x4f32(x, Vs[t * SCAN_VS + scan_col(p0 + p, r)], s[p], 0, 0, 0);
+        }
+    if (ct < ch_tiles) {
+#pragma unroll
+        for (int p = 0; p < TILES; ++p)
+            *reinterpret_cast<float4*>(adds + ((size_t)(ct * tiles + col0 / 16 + p0 + p) * 64 + 16 * g + r) * 4) = make_float4(s[p][0], s[p][1], s[p][2], s[p][3]);
+    }
+}
+
 template <int DK, int MODE, typename TQ, typename TV>
-__global__ void __launch_bounds__(512)
+__global__ void __launch_bounds__(64 * scan_waves(DK, MODE >= SCAN_CHANNEL))
 scan_chunks_kernel(ScanArgs a) {
     constexpr bool CH = MODE >= SCAN_CHANNEL;
-    constexpr int LS = DK + 4, Q4 = DK / 4;
+    constexpr int LS = DK + 4, Q4 = DK / 4, NW = scan_waves(DK, CH), NT = 64 * NW;
     constexpr bool V_IN_Q = SCAN_C * LS >= SCAN_C * (SCAN_AS + SCAN_VS);
     __shared__ __align__(16) float Qs[SCAN_C * LS];                  // later the scores, and behind them the values
     __shared__ __align__(16) float Ks[SCAN_C * LS];
     __shared__ __align__(16) float Ds[CH ? SCAN_C * LS : 4];
     __shared__ __align__(16) float Vx[V_IN_Q ? 4 : SCAN_C * SCAN_VS];
-    __shared__ __align__(16) float dg[CH ? 2 : 1][4][16][16];        // decays (CH: scores) inside a run of 16 tokens
+    __shared__ __align__(16) float dg[CH ? NW / 4 : 1][4][16][16];   // decays (CH: scores) inside a run of 16 tokens
     __shared__ __align__(16) float tot[4][CH ? DK : 1];              // a run's whole decay
     __shared__ float sa[SCAN_C], sdt[SCAN_C], pin[SCAN_C], sfx[SCAN_C];
     float* As = Qs;
@@ -108,24 +178,37 @@ scan_chunks_kernel(ScanArgs a) {
         }
         if (MODE == SCAN_STEP) skip = a.p3[head];
     }
-    const TQ* q = (const TQ*)a.q + (size_t)(head / a.group) * a.hq;
-    const TQ* k = (const TQ*)a.k + (size_t)(head / a.group) * a.hk;
+    const TQ* q = (const TQ*)a.q + (size_t)(head / a.group) * a.hq + (size_t)lo * a.ldq;
+    const TQ* k = (const TQ*)a.k + (size_t)(head / a.group) * a.hk + (size_t)lo * a.ldk;
+    const float* dec = CH ? a.decay + (size_t)lo * a.lda + head * a.D : nullptr;
+    constexpr int ROUNDS = SCAN_C * Q4 / NT;
+    float4 fq[ROUNDS], fk[ROUNDS], fd[CH ? ROUNDS : 1];
 #pragma unroll
-    for (int it = 0; it < SCAN_C * Q4 / 512; ++it) {
-        const int e = it * 512 + tid, t = e / Q4, i = e % Q4 * 4;
-        const int n = t < nt ? a.D - i : 0;
-        const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
-        *reinterpret_cast<float4*>(Qs + t * LS + i) = n > 0 ? scan_quad(q + (size_t)(lo + t) * a.ldq + i, n, a.vec) : zero;
-        *reinterpret_cast<float4*>(Ks + t * LS + i) = n > 0 ? scan_quad(k + (size_t)(lo + t) * a.ldk + i, n, a.vec) : zero;
-        if constexpr (CH)
-            *reinterpret_cast<float4*>(Ds + t * LS + i) =
-                n > 0 ? scan_quad(a.decay + (size_t)(lo + t) * a.lda + head * a.D + i, n, a.vec) : make_float4(1.f, 1.f, 1.f, 1.f);
+    for (int it = 0; it < ROUNDS; ++it) {            // all loads before the first use
+        const int e = it * NT + tid, t = e / Q4, i = e % Q4 * 4, n = t < nt ? a.D - i : 0;
+        fq[it] = scan_quad(q + (size_t)t * a.ldq + i, q, n, a.vec);
+        fk[it] = scan_quad(k + (size_t)t * a.ldk + i, k, n, a.vec);
+        if constexpr (CH) {
+            fd[it] = scan_quad(dec + (size_t)t * a.lda + i, dec, n, a.vec);
+            if (n < 1) fd[it].x = 1.f;
+            if (n < 2) fd[it].y = 1.f;
+            if (n < 3) fd[it].z = 1.f;
+            if (n < 4) fd[it].w = 1.f;
+        }
+    }
+#pragma unroll
+    for (int it = 0; it < ROUNDS; ++it) {
+        const int e = it * NT + tid, t = e / Q4, i = e % Q4 * 4;
+        *reinterpret_cast<float4*>(Qs + t * LS + i) = fq[it];
+        *reinterpret_cast<float4*>(Ks + t * LS + i) = fk[it];
+        if constexpr (CH) *reinterpret_cast<float4*>(Ds + t * LS + i) = fd[it];
     }
     __syncthreads();
 
     // -- scores: blocks of 16 x 16 (run I of queries, run J <= I of keys)
-    f32x4 sc[2];
-    int bi[2], bj[2];
+    constexpr int BLOCKS = CH ? 6 : 10, MINE = (BLOCKS + NW - 1) / NW;
+    f32x4 sc[MINE];
+    int bi[MINE], bj[MINE];
     if constexpr (!CH) {
         if (tid < SCAN_C) {                          // down a column of its run: decay from behind token j to token i
             const int I = tid / 16, j = tid % 16;
@@ -143,9 +226,9 @@ scan_chunks_kernel(ScanArgs a) {
             if (i % 16 == 15) tot[I][0] = p;
         }
     } else {
-        // inside a run pair by pair: wave (run, half of the channels), lane (query r, a quarter of the half's channels)
-        constexpr int CPL = DK / 8;
-        const int I = wave / 2, c0 = (wave % 2) * (DK / 2) + g * CPL;
+        // inside a run pair by pair: wave (run, share of the channels), lane (query r, a quarter of the share)
+        constexpr int PARTS = NW / 4, CPL = DK / 4 / PARTS;
+        const int I = wave / PARTS, c0 = (wave % PARTS) * (DK / PARTS) + g * CPL;
         float qv[CPL], w[CPL], u[MODE == SCAN_BONUS ? CPL : 1];
 #pragma unroll
         for (int i = 0; i < CPL; ++i) {
@@ -174,11 +257,11 @@ scan_chunks_kernel(ScanArgs a) {
                 }
             }
             s = sum_xor32(sum_xor16(j <= r ? s : 0.f));
-            if (g == 0) dg[wave % 2][I][r][j] = s;
+            if (g == 0) dg[wave % PARTS][I][r][j] = s;
         }
-        __syncthreads();
+        lds_barrier();
         // queries decayed back to their run's start, keys to its end, in place
-        for (int e = tid; e < 4 * DK; e += 512) {
+        for (int e = tid; e < 4 * DK; e += NT) {
             const int run = e / DK, ch = e % DK;
             float p = 1.f;
 #pragma unroll
@@ -196,12 +279,11 @@ scan_chunks_kernel(ScanArgs a) {
                 p *= Ds[at];
             }
         }
-        __syncthreads();
+        lds_barrier();
     }
-    constexpr int BLOCKS = CH ? 6 : 10;
 #pragma unroll
-    for (int x = 0; x < 2; ++x) {
-        const int b = wave + 8 * x;
+    for (int x = 0; x < MINE; ++x) {
+        const int b = wave + NW * x;
         bi[x] = -1;
         if (b >= BLOCKS) continue;
         int I, J;
@@ -222,13 +304,13 @@ scan_chunks_kernel(ScanArgs a) {
         }
         sc[x] = s;
     }
-    if constexpr (!CH) __syncthreads();             // the factors of the runs
+    if constexpr (!CH) lds_barrier();             // the factors of the runs
 
     // -- queries decayed back to the chunk's start, for scan_apply (one decay for all channels: that alone); the whole decay
     if constexpr (CH) {
 #pragma unroll
-        for (int it = 0; it < SCAN_C * Q4 / 512; ++it) {
-            const int e = it * 512 + tid, t = e / Q4, i = e % Q4 * 4, I = t / 16;
+        for (int it = 0; it < SCAN_C * Q4 / NT; ++it) {
+            const int e = it * NT + tid, t = e / Q4, i = e % Q4 * 4, I = t / 16;
             float4 x = *reinterpret_cast<const float4*>(Qs + t * LS + i);
             for (int run = 0; run < I; ++run) x = mul4(x, *reinterpret_cast<const float4*>(&tot[run][i]));
             *reinterpret_cast<float4*>(a.queries + (slot * SCAN_C + t) * DK + i) = x;
@@ -242,11 +324,11 @@ scan_chunks_kernel(ScanArgs a) {
         const int ch = CH ? tid : 0;
         a.factors[slot * DK + tid] = tot[0][ch] * tot[1][ch] * tot[2][ch] * tot[3][ch];
     }
-    __syncthreads();
+    lds_barrier();
 
     // -- the scores over the queries' place; keys decayed on to the chunk's end, in place
 #pragma unroll
-    for (int x = 0; x < 2; ++x) {
+    for (int x = 0; x < MINE; ++x) {
         if (bi[x] < 0) continue;
         const int I = bi[x], J = bj[x], i = I * 16 + r;
         float f[4] = {1.f, 1.f, 1.f, 1.f};
@@ -266,14 +348,17 @@ scan_chunks_kernel(ScanArgs a) {
         *reinterpret_cast<float4*>(As + i * SCAN_AS + J * 16 + 4 * g) = s;
     }
     if constexpr (CH) {
-        for (int e = tid; e < 4 * 16 * 16; e += 512) {
+        for (int e = tid; e < 4 * 16 * 16; e += NT) {
             const int I = e / 256, i = e / 16 % 16, j = e % 16;
-            As[(I * 16 + i) * SCAN_AS + I * 16 + j] = dg[0][I][i][j] + dg[1][I][i][j];
+            float x = dg[0][I][i][j];
+#pragma unroll
+            for (int part = 1; part < NW / 4; ++part) x += dg[part][I][i][j];
+            As[(I * 16 + i) * SCAN_AS + I * 16 + j] = x;
         }
     }
 #pragma unroll
-    for (int it = 0; it < SCAN_C * Q4 / 512; ++it) {
-        const int e = it * 512 + tid, t = e / Q4, i = e % Q4 * 4, I = t / 16;
+    for (int it = 0; it < SCAN_C * Q4 / NT; ++it) {
+        const int e = it * NT + tid, t = e / Q4, i = e % Q4 * 4, I = t / 16;
         float4 x = *reinterpret_cast<const float4*>(Ks + t * LS + i);
         if constexpr (CH) {
             for (int run = 3; run > I; --run) x = mul4(x, *reinterpret_cast<const float4*>(&tot[run][i]));
@@ -286,111 +371,72 @@ scan_chunks_kernel(ScanArgs a) {
     }
 
     // -- values, 32 columns at a time: the scores' share of the outputs, and the addend to the state
-    const TV* v = (const TV*)a.v + (size_t)head * a.hv;
+    const TV* v = (const TV*)a.v + (size_t)head * a.hv + (size_t)lo * a.ldv;
     const int vt = tid / 8, vc = tid % 8 * 4;
     auto fetch = [&](int col) {
-        float x[4] = {0.f, 0.f, 0.f, 0.f};
-        if (vt < nt) {
-            const TV* row = v + (size_t)(lo + vt) * a.ldv + col;
-            if (a.vec && col + 4 <= a.held) VecLoad<TV, 4>::load(row, x);
-            else
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (col + e < a.Dv) x[e] = col + e < a.held ? to_float(row[e]) : 1.f;
-            if (a.v_act)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) x[e] = x[e] / (1.f + expf(-x[e]));
+        float4 x = scan_quad(v + (size_t)vt * a.ldv + col, v, vt < nt ? a.held - col : 0, a.vec);      // (threads from 512 on: none)
+        if (a.held < a.Dv && vt < nt) {
+            if (col >= a.held) x.x = 1.f;
+            if (col + 1 >= a.held) x.y = 1.f;
+            if (col + 2 >= a.held) x.z = 1.f;
+            if (col + 3 >= a.held) x.w = 1.f;
         }
-        return make_float4(x[0], x[1], x[2], x[3]);
-    };
-    auto put = [&](float* p, int n, const f32x4& y, bool whole) {    // n columns are left
-        if (whole && n >= 4) *reinterpret_cast<float4*>(p) = make_float4(y[0], y[1], y[2], y[3]);
-        else
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                if (e < n) p[e] = y[e];
+        return x;
     };
     const bool by4 = a.Dv % 4 == 0;
+    const int tiles = scan_tiles(a.Dv);
+    float* adds = a.adds + slot * ((a.D + 15) / 16) * tiles * 256;
     float4 next = fetch(vc);
     for (int col0 = 0; col0 < a.Dv; col0 += SCAN_VC) {
-        __syncthreads();                            // the scores are there; the values before these have been read
-        *reinterpret_cast<float4*>(Vs + vt * SCAN_VS + vc) = next;
-        __syncthreads();
+        if (a.v_act) next = make_float4(next.x / (1.f + expf(-next.x)), next.y / (1.f + expf(-next.y)), next.z / (1.f + expf(-next.z)), next.w / (1.f + expf(-next.w)));
+        lds_barrier();                              // the scores are there; the values before these have been read
+        if (NT == 512 || tid < 512) *reinterpret_cast<float4*>(Vs + vt * SCAN_VS + vc) = next;
+        lds_barrier();
         if (col0 + SCAN_VC < a.Dv) next = fetch(col0 + SCAN_VC + vc);
-        {
-            const int I = wave / 2, p = wave % 2;
-            f32x4 o = {0.f, 0.f, 0.f, 0.f};
-            for (int s = 0; s <= I; ++s) {
-                const float4 x = *reinterpret_cast<const float4*>(As + (I * 16 + r) * SCAN_AS + 16 * s + 4 * g);
-                const float* y = Vs + (16 * s + 4 * g) * SCAN_VS + p * 16 + r;
-                o = __builtin_amdgcn_mfma_f32_16x16x4f32(y[0], x.x, o, 0, 0, 0);
-                o = __builtin_amdgcn_mfma_f32_16x16x4f32(y[SCAN_VS], x.y, o, 0, 0, 0);
-                o = __builtin_amdgcn_mfma_f32_16x16x4f32(y[2 * SCAN_VS], x.z, o, 0, 0, 0);
-                o = __builtin_amdgcn_mfma_f32_16x16x4f32(y[3 * SCAN_VS], x.w, o, 0, 0, 0);
-            }
-            const int t = I * 16 + r, col = col0 + p * 16 + 4 * g;
-            if (t < nt && col < a.Dv) put(a.out + ((size_t)(lo + t) * a.H + head) * a.Dv + col, a.Dv - col, o, by4);
-        }
-        {
-            // 16 channels by 32 columns a wave, or with 64 channels by 16
-            constexpr int TILES = DK / 64;
-            const int ct = DK == 128 ? wave : wave / 2, p0 = DK == 128 ? 0 : wave % 2;
-            f32x4 s[TILES];
-#pragma unroll
-            for (int p = 0; p < TILES; ++p) s[p] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int m = 0; m < SCAN_C; m += 16)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int t = m + 4 * g + e;
-                    const float x = Ks[t * LS + ct * 16 + r];
-#pragma unroll
-                    for (int p = 0; p < TILES; ++p)
-                        s[p] = __builtin_amdgcn_mfma_f32_16x16x4f32(Vs[t * SCAN_VS + (p0 + p) * 16 + r], x, s[p], 0, 0, 0);
-                }
-            const int ch = ct * 16 + r;
-#pragma unroll
-            for (int p = 0; p < TILES; ++p) {
-                const int col = col0 + (p0 + p) * 16 + 4 * g;
-                if (ch < a.D && col < a.Dv) put(a.adds + (slot * a.D + ch) * a.Dv + col, a.Dv - col, s[p], by4);
-            }
-        }
+        scan_values<DK, NW>(a.out, a.H, a.Dv, by4, lo, nt, head, col0, tiles, Ks, Vs, As, adds, (a.D + 15) / 16, wave, r, g);
     }
 }
 
 // In place: every chunk's addend becomes the state before that chunk, and the row's state moves on to the end of the
-// last one. A thread owns V elements of a head's state; the addends of eight chunks are on their way at a time.
-template <int V>
+// last one. A thread owns a lane's four elements of a tile; the addends of eight chunks are on their way at a time.
 __global__ void __launch_bounds__(256)
 scan_states_kernel(ScanArgs a, int dk) {
-    const int head = blockIdx.y, seq = blockIdx.z;
-    const int size = a.D * a.Dv, at = ((int)blockIdx.x * 256 + (int)threadIdx.x) * V;
+    const int head = blockIdx.y, seq = blockIdx.z, tiles = scan_tiles(a.Dv);
+    const int size = (a.D + 15) / 16 * tiles * 64, at = (int)blockIdx.x * 256 + (int)threadIdx.x;     // in pieces of four
     const int left = a.qstart[seq + 1] - a.qstart[seq] - a.first * SCAN_C;
     if (at >= size || left <= 0) return;
     const int n = min(a.count, (left + SCAN_C - 1) / SCAN_C);
-    float* S = a.state + (size_t)a.rows[seq] * a.stride + a.offset + (size_t)head * size + at;
+    const int lane = at % 64, ct = at / 64 % tiles, ch = at / 64 / tiles * 16 + lane / 16 * 4;
+    const int col = ct / 2 * 32 + scan_col(ct % 2, lane % 16);
+    float* S = a.state + (size_t)a.rows[seq] * a.stride + a.offset + (size_t)head * a.D * a.Dv + (size_t)ch * a.Dv + col;
     const size_t slot0 = scan_slot(a, seq, 0) * a.H + head;
-    float* add = a.adds + slot0 * size + at;
-    const float* f = a.factors + slot0 * dk + at / a.Dv;
+    float4* add = reinterpret_cast<float4*>(a.adds) + slot0 * size + at;
+    const float* f = a.factors + slot0 * dk + ch;
     const size_t step = (size_t)a.H * size, fstep = (size_t)a.H * dk;
-    float s[V], x[8][V], y[8];
-    VecLoad<float, V>::load(S, s);
-    for (int c = 0; c < n; c += 8) {
+    float s[4];
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
-            if (c + i < n) { VecLoad<float, V>::load(add + (c + i) * step, x[i]); y[i] = f[(c + i) * fstep]; }
+    for (int e = 0; e < 4; ++e) s[e] = col < a.Dv && ch + e < a.D ? S[(size_t)e * a.Dv] : 0.f;
+    for (int c = 0; c < n; c += 8) {
+        float4 x[8], y[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int cc = min(c + i, n - 1);
+            x[i] = add[cc * step];
+            y[i] = *reinterpret_cast<const float4*>(f + cc * fstep);
+        }
 #pragma unroll
         for (int i = 0; i < 8; ++i)
             if (c + i < n) {
-                float* p = add + (c + i) * step;
-                if constexpr (V == 4) *reinterpret_cast<float4*>(p) = make_float4(s[0], s[1], s[2], s[3]);
-                else p[0] = s[0];
-#pragma unroll
-                for (int e = 0; e < V; ++e) s[e] = fmaf(y[i], s[e], x[i][e]);
+                add[(c + i) * step] = make_float4(s[0], s[1], s[2], s[3]);
+                s[0] = fmaf(y[i].x, s[0], x[i].x);
+                s[1] = fmaf(y[i].y, s[1], x[i].y);
+                s[2] = fmaf(y[i].z, s[2], x[i].z);
+                s[3] = fmaf(y[i].w, s[3], x[i].w);
             }
     }
-    if constexpr (V == 4) *reinterpret_cast<float4*>(S) = make_float4(s[0], s[1], s[2], s[3]);
-    else S[0] = s[0];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        if (col < a.Dv && ch + e < a.D) S[(size_t)e * a.Dv] = s[e];
 }
 
 // out += queries S, 64 tokens by 32 CG columns a workgroup: CG waves side by side with 32 columns of S in registers,
@@ -409,19 +455,16 @@ scan_apply_kernel(ScanArgs a) {
     const int lane = tid % 64, wave = tid / 64, r = lane % 16, g = lane / 16;
     const size_t slot = scan_slot(a, seq, c) * a.H + head;
     const int col0 = (blockIdx.x % blocks) * 32 * CG + (wave % CG) * 32, row0 = (wave / CG) * 16 * CG;
-    const float* S = a.adds + slot * a.D * a.Dv + col0 + 2 * r;
-    const int n = a.Dv - col0 - 2 * r;
-    const bool by2 = a.Dv % 2 == 0;
-    float sx[DK / 4], sy[DK / 4];                    // columns 2 r and 2 r + 1 of channels 16 s + 4 g + e
+    // two tiles of 16 columns; channels 16 s + 4 g .. + 3 in piece s (tiles beyond the last channel's, columns beyond the
+    // last tile's: read at a place that exists, not used)
+    const int tiles = scan_tiles(a.Dv), ch_tiles = (a.D + 15) / 16;
+    const float4* S = reinterpret_cast<const float4*>(a.adds) + (slot * ch_tiles * tiles + min(col0 / 16, tiles - 2)) * 64 + lane;
+    float4 sx[DK / 16], sy[DK / 16];
 #pragma unroll
-    for (int i = 0; i < DK / 4; ++i) {
-        const int ch = i / 4 * 16 + 4 * g + i % 4;
-        sx[i] = sy[i] = 0.f;
-        if (ch < a.D && n > 0) {
-            const float* p = S + (size_t)ch * a.Dv;
-            if (by2) { const float2 t = *reinterpret_cast<const float2*>(p); sx[i] = t.x; sy[i] = t.y; }
-            else { sx[i] = p[0]; if (n > 1) sy[i] = p[1]; }
-        }
+    for (int i = 0; i < DK / 16; ++i) {
+        const float4* p = S + (size_t)min(i, ch_tiles - 1) * tiles * 64;
+        sx[i] = p[0];
+        sy[i] = p[64];
     }
 #pragma unroll
     for (int it = 0; it < SCAN_C * Q4 / 256; ++it) {
@@ -429,8 +472,8 @@ scan_apply_kernel(ScanArgs a) {
         float4 x;
         if constexpr (CH) x = *reinterpret_cast<const float4*>(a.queries + (slot * SCAN_C + t) * DK + i);
         else {
-            const TQ* q = (const TQ*)a.q + (size_t)(head / a.group) * a.hq + (size_t)(lo + t) * a.ldq + i;
-            x = t < nt && i < a.D ? mul4(scan_quad(q, a.D - i, a.vec), a.queries[slot * SCAN_C + t]) : make_float4(0.f, 0.f, 0.f, 0.f);
+            const TQ* q = (const TQ*)a.q + (size_t)(head / a.group) * a.hq + (size_t)lo * a.ldq;
+            x = mul4(scan_quad(q + (size_t)t * a.ldq + i, q, t < nt ? a.D - i : 0, a.vec), a.queries[slot * SCAN_C + t]);
         }
         *reinterpret_cast<float4*>(Qs + t * LS + i) = x;
     }
@@ -440,16 +483,13 @@ scan_apply_kernel(ScanArgs a) {
     for (int i = 0; i < CG; ++i) x[i] = y[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < DK / 16; ++s) {
-        float q[CG][4];
+        if (s >= ch_tiles) break;
 #pragma unroll
-        for (int i = 0; i < CG; ++i) VecLoad<float, 4>::load(Qs + (row0 + i * 16 + r) * LS + 16 * s + 4 * g, q[i]);
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-#pragma unroll
-            for (int i = 0; i < CG; ++i) {
-                x[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(sx[s * 4 + e], q[i][e], x[i], 0, 0, 0);
-                y[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(sy[s * 4 + e], q[i][e], y[i], 0, 0, 0);
-            }
+        for (int i = 0; i < CG; ++i) {
+            const float4 q = *reinterpret_cast<const float4*>(Qs + (row0 + i * 16 + r) * LS + 16 * s + 4 * g);
+            x[i] = mfma4(sx[s].x, sx[s].y, sx[s].z, sx[s].w, q, x[i]);
+            y[i] = mfma4(sy[s].x, sy[s].y, sy[s].z, sy[s].w, q, y[i]);
+        }
     }
     // a lane has columns col0 + 8 g .. + 7 of token row0 + 16 i + r
 #pragma unroll
@@ -459,24 +499,23 @@ scan_apply_kernel(ScanArgs a) {
         float* p = a.out + ((size_t)(lo + t) * a.H + head) * a.Dv + col;
         if (a.Dv % 4 == 0 && col + 8 <= a.Dv) {
             float4 u = *reinterpret_cast<const float4*>(p), w = *reinterpret_cast<const float4*>(p + 4);
-            u.x += x[i][0]; u.y += y[i][0]; u.z += x[i][1]; u.w += y[i][1];
-            w.x += x[i][2]; w.y += y[i][2]; w.z += x[i][3]; w.w += y[i][3];
+            u.x += x[i][0]; u.y += x[i][1]; u.z += x[i][2]; u.w += x[i][3];
+            w.x += y[i][0]; w.y += y[i][1]; w.z += y[i][2]; w.w += y[i][3];
             *reinterpret_cast<float4*>(p) = u;
             *reinterpret_cast<float4*>(p + 4) = w;
         } else {
 #pragma unroll
             for (int e = 0; e < 8; ++e)
-                if (col + e < a.Dv) p[e] += e % 2 ? y[i][e / 2] : x[i][e / 2];
+                if (col + e < a.Dv) p[e] += e < 4 ? x[i][e] : y[i][e - 4];
         }
     }
 }
 
 template <int DK, int MODE, typename TQ, typename TV>
-static void launch_scan(const ScanArgs& a, int n_seqs, bool vec_state, hipStream_t s) {
-    hipLaunchKernelGGL((scan_chunks_kernel<DK, MODE, TQ, TV>), dim3(a.H, a.count, n_seqs), dim3(512), 0, s, a);
-    const int size = a.D * a.Dv;
-    if (vec_state) hipLaunchKernelGGL((scan_states_kernel<4>), dim3((size / 4 + 255) / 256, a.H, n_seqs), dim3(256), 0, s, a, DK);
-    else hipLaunchKernelGGL((scan_states_kernel<1>), dim3((size + 255) / 256, a.H, n_seqs), dim3(256), 0, s, a, DK);
+static void launch_scan(const ScanArgs& a, int n_seqs, hipStream_t s) {
+    hipLaunchKernelGGL((scan_chunks_kernel<DK, MODE, TQ, TV>), dim3(a.H, a.count, n_seqs), dim3(64 * scan_waves(DK, MODE >= SCAN_CHANNEL)), 0, s, a);
+    const int pieces = (a.D + 15) / 16 * scan_tiles(a.Dv) * 64;
+    hipLaunchKernelGGL(scan_states_kernel, dim3((pieces + 255) / 256, a.H, n_seqs), dim3(256), 0, s, a, DK);
     constexpr bool CH = MODE >= SCAN_CHANNEL;
     if (a.Dv <= 32) hipLaunchKernelGGL((scan_apply_kernel<DK, 1, CH, TQ>), dim3(a.H, a.count, n_seqs), dim3(256), 0, s, a);
     else if (a.Dv <= 64) hipLaunchKernelGGL((scan_apply_kernel<DK, 2, CH, TQ>), dim3(a.H, a.count, n_seqs), dim3(256), 0, s, a);
@@ -502,16 +541,365 @@ SOC_EXPORT int soc_scan(int mode, const void* q, long long ldq, int hq, const vo
     a.first = first; a.count = count; a.compact = compact; a.qstart = seq_qstart; a.rows = seq_rows;
     a.state = state; a.stride = stride; a.offset = offset; a.out = out; a.adds = adds; a.queries = queries; a.factors = factors;
     const int qe = q_f32 || dtype == 0 ? 16 : 8, ve = dtype == 0 ? 16 : 8;       // bytes of four elements
-    a.vec = D % 4 == 0 && ldq % 4 == 0 && ldk % 4 == 0 && ldv % 4 == 0 && lda % 4 == 0 && hq % 4 == 0 && hk % 4 == 0 && hv % 4 == 0 &&
+    a.vec = D % 4 == 0 && a.held % 4 == 0 && ldq % 4 == 0 && ldk % 4 == 0 && ldv % 4 == 0 && lda % 4 == 0 && hq % 4 == 0 && hk % 4 == 0 && hv % 4 == 0 &&
             (uintptr_t)q % qe == 0 && (uintptr_t)k % qe == 0 && (uintptr_t)v % ve == 0 && (uintptr_t)decay % 16 == 0;
-    const bool vec_state = Dv % 4 == 0 && stride % 4 == 0 && offset % 4 == 0 && (uintptr_t)state % 16 == 0;
 #define SOC_SCAN(MODE_, TQ_, TV_) \
-    do { if (D <= 64) launch_scan<64, MODE_, TQ_, TV_>(a, n_seqs, vec_state, stream); else launch_scan<128, MODE_, TQ_, TV_>(a, n_seqs, vec_state, stream); } while (0)
+    do { if (D <= 64) launch_scan<64, MODE_, TQ_, TV_>(a, n_seqs, stream); else launch_scan<128, MODE_, TQ_, TV_>(a, n_seqs, stream); } while (0)
     if (mode == SCAN_HEAD && q_f32) { if (dtype == 0) SOC_SCAN(SCAN_HEAD, float, float); else SOC_SCAN(SCAN_HEAD, float, bf16); }
     else if (mode == SCAN_CHANNEL && q_f32) { if (dtype == 0) SOC_SCAN(SCAN_CHANNEL, float, float); else SOC_SCAN(SCAN_CHANNEL, float, bf16); }
     else if (mode == SCAN_STEP && !q_f32 && p1 && p2 && p3) { if (dtype == 0) SOC_SCAN(SCAN_STEP, float, float); else SOC_SCAN(SCAN_STEP, bf16, bf16); }
     else if (mode == SCAN_BONUS && !q_f32 && p1) { if (dtype == 0) SOC_SCAN(SCAN_BONUS, float, float); else SOC_SCAN(SCAN_BONUS, bf16, bf16); }
     else return (int)hipErrorInvalidValue;
 #undef SOC_SCAN
+    return soc_last_error();
+}
+
+// ---- the gated delta rule in chunks ---------------------------------------------------------------------------------
+// S <- g S; u = beta (v - S^T k); S <- S + k u^T; o = S^T q. With the chunk's start state S0, the decays D_ij from
+// behind token j to token i and the decay G_i from the start to i, the u of a chunk solve a triangular system,
+//   (I + M) U = diag(beta) (V - diag(G) K S0),   M_ij = beta_i D_ij k_i . k_j for j < i,
+// and with T = (I + M)^-1 (by blocks of 16), A_ij = D_ij q_i . k_j for j <= i, X = A T diag(beta) and
+// Z = diag(beta) T^T (keys decayed to the chunk's end):
+//   O  = X V + (queries decayed to the start - X diag(G) K) S0          the bracket goes where scan_apply reads it
+//   S' = (G_end I - Z^T diag(G) K) S0 + Z^T V                           the bracket is the chunk's transition
+// so everything but S0's share is the chunk's own, and what is left to do in order is one product per chunk.
+// gates float32 [N, H, 2] = (g, beta); the state of a row is [H, Dv, D].
+struct DeltaArgs {
+    const float *q, *k, *gates;
+    const void* v;
+    long long ldq, ldv;
+    int hq, hv, group, H, D, Dv, vec, first, count, compact;
+    const int* qstart;
+    const int* rows;
+    float* state;
+    long long stride;
+    int offset;
+    float *out, *adds, *queries, *moves;      // moves: per slot and head [DK, DK] in tiles
+};
+
+template <int DK, typename TV>
+__global__ void __launch_bounds__(64 * scan_waves(DK, true))
+delta_chunks_kernel(DeltaArgs a) {
+    constexpr int LS = DK + 4, Q4 = DK / 4, NW = scan_waves(DK, true), NT = 64 * NW;
+    __shared__ __align__(16) float Qs[SCAN_C * LS];                  // later Z
+    __shared__ __align__(16) float Ks[SCAN_C * LS];
+    __shared__ __align__(16) float As[SCAN_C * SCAN_AS], Ms[SCAN_C * SCAN_AS], Ts[SCAN_C * SCAN_AS];     // Ms later X
+    __shared__ __align__(16) float Vs[SCAN_C * SCAN_VS];
+    __shared__ __align__(16) float dg[4][16][16];
+    __shared__ float sa[SCAN_C], sb[SCAN_C], pin[SCAN_C], sfx[SCAN_C], from[SCAN_C], rest[SCAN_C], tot[4];
+    const int head = blockIdx.x, c = blockIdx.y, seq = blockIdx.z, tid = threadIdx.x;
+    const int lo = a.qstart[seq] + (a.first + c) * SCAN_C, hi = a.qstart[seq + 1];
+    if (lo >= hi) return;
+    const int nt = min(SCAN_C, hi - lo);
+    const int lane = tid % 64, wave = tid / 64, r = lane % 16, g = lane / 16;
+    const size_t slot = (a.compact ? (size_t)(a.qstart[seq] / SCAN_C + seq + c) : (size_t)seq * a.count + c) * a.H + head;
+
+    const float* q = a.q + (size_t)(head / a.group) * a.hq + (size_t)lo * a.ldq;
+    const float* k = a.k + (size_t)(head / a.group) * a.hq + (size_t)lo * a.ldq;
+    constexpr int ROUNDS = SCAN_C * Q4 / NT;
+    float4 fq[ROUNDS], fk[ROUNDS];
+#pragma unroll
+    for (int it = 0; it < ROUNDS; ++it) {            // (q and k are padded with zeros to DK; all loads before the first use)
+        const int e = it * NT + tid, t = e / Q4, i = e % Q4 * 4;
+        fq[it] = scan_quad(q + (size_t)t * a.ldq + i, q, t < nt ? 4 : 0, 1);
+        fk[it] = scan_quad(k + (size_t)t * a.ldq + i, k, t < nt ? 4 : 0, 1);
+    }
+    if (tid < SCAN_C) {
+        const float2 gb = reinterpret_cast<const float2*>(a.gates)[(size_t)(lo + min(tid, nt - 1)) * a.H + head];
+        sa[tid] = tid < nt ? gb.x : 1.f;
+        sb[tid] = tid < nt ? gb.y : 0.f;
+    }
+#pragma unroll
+    for (int it = 0; it < ROUNDS; ++it) {
+        const int e = it * NT + tid, t = e / Q4, i = e % Q4 * 4;
+        *reinterpret_cast<float4*>(Qs + t * LS + i) = fq[it];
+        *reinterpret_cast<float4*>(Ks + t * LS + i) = fk[it];
+    }
+    __syncthreads();
+    if (tid < SCAN_C) {
+        const int I = tid / 16, j = tid % 16;
+        float p = 1.f;
+        for (int i = 0; i < 16; ++i) {
+            if (i > j) p *= sa[I * 16 + i];
+            dg[I][i][j] = i >= j ? p : 0.f;
+        }
+        sfx[tid] = p;
+    } else if (tid < 2 * SCAN_C) {
+        const int i = tid - SCAN_C, I = i / 16;
+        float p = 1.f;
+        for (int t = I * 16; t <= i; ++t) p *= sa[t];
+        pin[i] = p;
+        if (i % 16 == 15) tot[I] = p;
+    }
+    // A and M: twenty blocks of 16 x 16
+    constexpr int MINE = (20 + NW - 1) / NW;
+    f32x4 sc[MINE];
+#pragma unroll
+    for (int x = 0; x < MINE; ++x) {
+        const int b = wave + NW * x, bb = b % 10;
+        if (b >= 20) continue;
+        const int I = bb < 1 ? 0 : bb < 3 ? 1 : bb < 6 ? 2 : 3, J = bb - I * (I + 1) / 2;
+        const float* rows = b < 10 ? Qs : Ks;
+        f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int m = 0; m < DK; m += 16) {
+            const float4 qf = *reinterpret_cast<const float4*>(rows + (I * 16 + r) * LS + m + 4 * g);
+            const float4 kf = *reinterpret_cast<const float4*>(Ks + (J * 16 + r) * LS + m + 4 * g);
+            s = mfma4(kf.x, kf.y, kf.z, kf.w, qf, s);
+        }
+        sc[x] = s;
+    }
+    lds_barrier();
+    if (tid < SCAN_C) {
+        float p = pin[tid], s = sfx[tid];
+        for (int run = 0; run < tid / 16; ++run) p *= tot[run];
+        for (int run = tid / 16 + 1; run < 4; ++run) s *= tot[run];
+        from[tid] = p;
+        rest[tid] = s;
+    }
+#pragma unroll
+    for (int x = 0; x < MINE; ++x) {
+        const int b = wave + NW * x, bb = b % 10;
+        if (b >= 20) continue;
+        const int I = bb < 1 ? 0 : bb < 3 ? 1 : bb < 6 ? 2 : 3, J = bb - I * (I + 1) / 2, i = I * 16 + r;
+        float f[4], p = pin[i];
+        for (int run = J + 1; run < I; ++run) p *= tot[run];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            f[e] = I == J ? dg[I][r][4 * g + e] : p * sfx[J * 16 + 4 * g + e];
+            if (b >= 10) f[e] = I == J && 4 * g + e >= r ? 0.f : f[e] * sb[i];
+        }
+        *reinterpret_cast<float4*>((b < 10 ? As : Ms) + i * SCAN_AS + J * 16 + 4 * g) =
+            make_float4(sc[x][0] * f[0], sc[x][1] * f[1], sc[x][2] * f[2], sc[x][3] * f[3]);
+    }
+    lds_barrier();
+    // T, the diagonal blocks by substitution, a thread per column
+    if (tid < SCAN_C) {
+        const int I = tid / 16, col = tid % 16;
+        const float* m = Ms + I * 16 * SCAN_AS + I * 16;
+        float x[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            float s = i == col ? 1.f : 0.f;
+#pragma unroll
+            for (int j = 0; j < i; ++j) s = fmaf(-m[i * SCAN_AS + j], x[j], s);
+            x[i] = s;
+            Ts[(I * 16 + i) * SCAN_AS + I * 16 + col] = s;
+        }
+    }
+    lds_barrier();
+    // below them T_IJ = -T_II sum_m M_Im T_mJ, one diagonal after the other
+    for (int d = 1; d < 4; ++d) {
+        if (wave < 4 - d) {
+            const int J = wave, I = wave + d;
+            float* mid = Vs + wave * 16 * 20;
+            f32x4 x = {0.f, 0.f, 0.f, 0.f};
+            for (int m = J; m < I; ++m)
+                x = mfma_col_row(Ts + (m * 16 + 4 * g) * SCAN_AS + J * 16 + r, SCAN_AS, Ms + (I * 16 + r) * SCAN_AS + m * 16 + 4 * g, x);
+            *reinterpret_cast<float4*>(mid + r * 20 + 4 * g) = make_float4(x[0], x[1], x[2], x[3]);
+            __builtin_amdgcn_wave_barrier();
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            x = (f32x4){0.f, 0.f, 0.f, 0.f};
+            x = mfma_col_row(mid + 4 * g * 20 + r, 20, Ts + (I * 16 + r) * SCAN_AS + I * 16 + 4 * g, x);
+            *reinterpret_cast<float4*>(Ts + (I * 16 + r) * SCAN_AS + J * 16 + 4 * g) = make_float4(-x[0], -x[1], -x[2], -x[3]);
+        }
+        lds_barrier();
+    }
+    // X = A T diag(beta), over M
+#pragma unroll
+    for (int x = 0; x < (10 + NW - 1) / NW; ++x) {
+        const int b = wave + NW * x;
+        if (b >= 10) continue;
+        const int I = b < 1 ? 0 : b < 3 ? 1 : b < 6 ? 2 : 3, J = b - I * (I + 1) / 2;
+        f32x4 s = {0.f, 0.f, 0.f, 0.f};
+        for (int m = J; m <= I; ++m)
+            s = mfma_col_row(Ts + (m * 16 + 4 * g) * SCAN_AS + J * 16 + r, SCAN_AS, As + (I * 16 + r) * SCAN_AS + m * 16 + 4 * g, s);
+        const float* be = sb + J * 16 + 4 * g;
+        *reinterpret_cast<float4*>(Ms + (I * 16 + r) * SCAN_AS + J * 16 + 4 * g) = make_float4(s[0] * be[0], s[1] * be[1], s[2] * be[2], s[3] * be[3]);
+    }
+    lds_barrier();
+    constexpr int PER = NW * 16 / DK;                // waves that share 16 channels: two
+    static_assert(PER == 2, "rows and columns are shared out by halves");
+    const int ct = wave / PER, part = wave % PER;
+    f32x4 z[4 / PER];
+    // queries decayed to the start - X diag(G) K; Z
+#pragma unroll
+    for (int y = 0; y < 4 / PER; ++y) {
+        const int I = 2 * y + part;
+        const int i = I * 16 + r;
+        const float4 q4 = *reinterpret_cast<const float4*>(Qs + i * LS + ct * 16 + 4 * g);
+        f32x4 o = {q4.x * from[i], q4.y * from[i], q4.z * from[i], q4.w * from[i]};
+        for (int s = 0; s <= I; ++s) {
+            const int j = 16 * s + 4 * g;
+            const float* col = Ks + j * LS + ct * 16 + r;
+            o = mfma4(-from[j] * col[0], -from[j + 1] * col[LS], -from[j + 2] * col[2 * LS], -from[j + 3] * col[3 * LS],
+                      *reinterpret_cast<const float4*>(Ms + i * SCAN_AS + j), o);
+        }
+        *reinterpret_cast<float4*>(a.queries + (slot * SCAN_C + i) * DK + ct * 16 + 4 * g) = make_float4(o[0], o[1], o[2], o[3]);
+        f32x4 w = {0.f, 0.f, 0.f, 0.f};
+        for (int s = I; s < 4; ++s) {                // row I * 16 + r of T^T
+            const int t = 16 * s + 4 * g;
+            const float* col = Ks + t * LS + ct * 16 + r;
+            const float* tt = Ts + t * SCAN_AS + I * 16 + r;
+            w = mfma4(rest[t] * col[0], rest[t + 1] * col[LS], rest[t + 2] * col[2 * LS], rest[t + 3] * col[3 * LS],
+                      make_float4(tt[0], tt[SCAN_AS], tt[2 * SCAN_AS], tt[3 * SCAN_AS]), w);
+        }
+        const float be = sb[i];
+        z[y] = (f32x4){w[0] * be, w[1] * be, w[2] * be, w[3] * be};
+    }
+    lds_barrier();
+#pragma unroll
+    for (int y = 0; y < 4 / PER; ++y) {
+        const int I = 2 * y + part;
+        *reinterpret_cast<float4*>(Qs + (I * 16 + r) * LS + ct * 16 + 4 * g) = make_float4(z[y][0], z[y][1], z[y][2], z[y][3]);
+    }
+    // the values' first columns are on their way while the transition is formed
+    const TV* v = (const TV*)a.v + (size_t)head * a.hv + (size_t)lo * a.ldv;
+    const int vt = tid / 8, vc = tid % 8 * 4;
+    auto fetch = [&](int col) { return scan_quad(v + (size_t)vt * a.ldv + col, v, vt < nt ? a.Dv - col : 0, a.vec); };
+    float4 next = fetch(vc);
+    lds_barrier();
+    const float whole = tot[0] * tot[1] * tot[2] * tot[3];
+#pragma unroll
+    for (int y0 = 0; y0 < DK / 16 / PER; y0 += 4 / PER) {
+        f32x4 s[4 / PER];
+#pragma unroll
+        for (int y = 0; y < 4 / PER; ++y) s[y] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int m = 0; m < SCAN_C; m += 16)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int t = m + 4 * g + e;
+                const float x = Qs[t * LS + ct * 16 + r], ge = from[t];
+#pragma unroll
+                for (int y = 0; y < 4 / PER; ++y) {
+                    const int c2 = ((y0 + y) * PER + part) * 16 + r;
+                    s[y] = __builtin_amdgcn_mfma_f32_16x16x4f32(Ks[t * LS + c2] * ge, x, s[y], 0, 0, 0);
+                }
+            }
+        const int row = ct * 16 + r;
+#pragma unroll
+        for (int y = 0; y < 4 / PER; ++y) {
+            const int c2 = ((y0 + y) * PER + part) * 16 + 4 * g;
+            float4 w = make_float4(-s[y][0], -s[y][1], -s[y][2], -s[y][3]);
+            if (row == c2) w.x += whole;
+            if (row == c2 + 1) w.y += whole;
+            if (row == c2 + 2) w.z += whole;
+            if (row == c2 + 3) w.w += whole;
+            *reinterpret_cast<float4*>(a.moves + slot * DK * DK + ((size_t)(ct * (DK / 16) + (y0 + y) * PER + part) * 64 + lane) * 4) = w;
+        }
+    }
+    const bool by4 = a.Dv % 4 == 0;
+    const int tiles = scan_tiles(a.Dv);
+    float* adds = a.adds + slot * ((a.D + 15) / 16) * tiles * 256;
+    for (int col0 = 0; col0 < a.Dv; col0 += SCAN_VC) {
+        lds_barrier();
+        if (NT == 512 || tid < 512) *reinterpret_cast<float4*>(Vs + vt * SCAN_VS + vc) = next;
+        lds_barrier();
+        if (col0 + SCAN_VC < a.Dv) next = fetch(col0 + SCAN_VC + vc);
+        scan_values<DK, NW>(a.out, a.H, a.Dv, by4, lo, nt, head, col0, tiles, Qs, Vs, Ms, adds, (a.D + 15) / 16, wave, r, g);
+    }
+}
+
+// The states in order: a workgroup owns 16 columns of a head's state, transposed in LDS; per chunk its old value goes
+// where the addend was (scan_apply reads it there) and S <- (transition) S + addend. The next chunk's transition and
+// addend are on their way meanwhile. Workgroups of one head follow each other on one XCD, whose L2 then serves
+// the transitions that they all read.
+template <int DK>
+__global__ void __launch_bounds__(256)
+delta_states_kernel(DeltaArgs a, int blocks) {
+    constexpr int LS = DK + 4, TILES = DK / 64;       // tiles of 16 channels per wave
+    __shared__ __align__(16) float St[2][16][LS];
+    const int b = blockIdx.x, head = b / (8 * blocks) * 8 + b % 8, cb = b / 8 % blocks, seq = blockIdx.y, tid = threadIdx.x;
+    if (head >= a.H) return;
+    const int left = a.qstart[seq + 1] - a.qstart[seq] - a.first * SCAN_C;
+    if (left <= 0) return;
+    const int n = min(a.count, (left + SCAN_C - 1) / SCAN_C);
+    const int lane = tid % 64, wave = tid / 64, r = lane % 16, g = lane / 16;
+    float* S = a.state + (size_t)a.rows[seq] * a.stride + a.offset + (size_t)head * a.Dv * a.D;
+    const size_t slot0 = (a.compact ? (size_t)(a.qstart[seq] / SCAN_C + seq) : (size_t)seq * a.count) * a.H + head;
+    for (int e = tid; e < 16 * DK; e += 256) {
+        const int cl = e / DK, ch = e % DK, col = cb / 2 * 32 + scan_col(cb % 2, cl);
+        St[0][cl][ch] = col < a.Dv && ch < a.D ? S[(size_t)col * a.D + ch] : 0.f;
+    }
+    const int tiles = scan_tiles(a.Dv), ch_tiles = (a.D + 15) / 16;
+    struct Next { float4 m[TILES][DK / 16], x[TILES]; } even, odd;
+    float4* adds = reinterpret_cast<float4*>(a.adds) + lane;
+    auto place = [&](int c, int t) { return (((slot0 + (size_t)c * a.H) * ch_tiles + min(wave * TILES + t, ch_tiles - 1)) * tiles + cb) * 64; };
+    auto fetch = [&](int c, Next& to) {
+        const float4* m = reinterpret_cast<const float4*>(a.moves) + (slot0 + (size_t)c * a.H) * (DK * DK / 4) + lane;
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+#pragma unroll
+            for (int s = 0; s < DK / 16; ++s) to.m[t][s] = m[((wave * TILES + t) * (DK / 16) + s) * 64];
+            to.x[t] = adds[place(c, t)];
+        }
+    };
+    fetch(0, even);
+    lds_barrier();
+    float4 old[TILES];
+#pragma unroll
+    for (int t = 0; t < TILES; ++t) old[t] = *reinterpret_cast<const float4*>(&St[0][r][(wave * TILES + t) * 16 + 4 * g]);
+    auto move = [&](int c, int from, Next& now, Next& then) {
+        if (c + 1 < n) fetch(c + 1, then);
+        f32x4 s[TILES];
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) s[t] = (f32x4){now.x[t].x, now.x[t].y, now.x[t].z, now.x[t].w};
+        float4 y[DK / 16];
+#pragma unroll
+        for (int k = 0; k < DK / 16; ++k) y[k] = *reinterpret_cast<const float4*>(&St[from][r][16 * k + 4 * g]);
+#pragma unroll
+        for (int k = 0; k < DK / 16; ++k)
+#pragma unroll
+            for (int t = 0; t < TILES; ++t) s[t] = mfma4(now.m[t][k].x, now.m[t][k].y, now.m[t][k].z, now.m[t][k].w, y[k], s[t]);
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+            if (wave * TILES + t < ch_tiles) adds[place(c, t)] = old[t];
+            old[t] = wave * TILES + t < ch_tiles ? make_float4(s[t][0], s[t][1], s[t][2], s[t][3]) : make_float4(0.f, 0.f, 0.f, 0.f);
+            *reinterpret_cast<float4*>(&St[from ^ 1][r][(wave * TILES + t) * 16 + 4 * g]) = old[t];
+        }
+        lds_barrier();
+    };
+    for (int c = 0; c < n; c += 2) {
+        move(c, 0, even, odd);
+        if (c + 1 < n) move(c + 1, 1, odd, even);
+    }
+    for (int e = tid; e < 16 * DK; e += 256) {
+        const int cl = e / DK, ch = e % DK, col = cb / 2 * 32 + scan_col(cb % 2, cl);
+        if (col < a.Dv && ch < a.D) S[(size_t)col * a.D + ch] = St[n % 2][cl][ch];
+    }
+}
+
+template <int DK>
+static void launch_delta(const DeltaArgs& a, int n_seqs, int dtype, hipStream_t s) {
+    if (dtype == 0) hipLaunchKernelGGL((delta_chunks_kernel<DK, float>), dim3(a.H, a.count, n_seqs), dim3(64 * scan_waves(DK, true)), 0, s, a);
+    else hipLaunchKernelGGL((delta_chunks_kernel<DK, bf16>), dim3(a.H, a.count, n_seqs), dim3(64 * scan_waves(DK, true)), 0, s, a);
+    const int blocks = scan_tiles(a.Dv);
+    hipLaunchKernelGGL((delta_states_kernel<DK>), dim3((a.H + 7) / 8 * 8 * blocks, n_seqs), dim3(256), 0, s, a, blocks);
+    ScanArgs b = {};
+    b.H = a.H; b.D = a.D; b.Dv = a.Dv; b.first = a.first; b.count = a.count; b.compact = a.compact; b.qstart = a.qstart;
+    b.out = a.out; b.adds = a.adds; b.queries = a.queries;
+    if (a.Dv <= 32) hipLaunchKernelGGL((scan_apply_kernel<DK, 1, true, float>), dim3(a.H, a.count, n_seqs), dim3(256), 0, s, b);
+    else if (a.Dv <= 64) hipLaunchKernelGGL((scan_apply_kernel<DK, 2, true, float>), dim3(a.H, a.count, n_seqs), dim3(256), 0, s, b);
+    else hipLaunchKernelGGL((scan_apply_kernel<DK, 4, true, float>), dim3(a.H * ((a.Dv + 127) / 128), a.count, n_seqs), dim3(256), 0, s, b);
+}
+
+// The gated delta rule over chunks first .. first + count - 1 of every sequence, from and into the rows' states. qk float32
+// [N, 2, G, Dp] as soc_delta_prepare leaves it, Dp 64 or 128; v [N, H Dv] in dtype. Scratch as for soc_scan, queries
+// [slots, H, 64, Dp], moves [slots, H, Dp, Dp].
+SOC_EXPORT int soc_delta_scan(const float* qk, const void* v, const float* gates, int G, int H, int D, int Dv, int Dp, float* state,
+                              long long stride, int offset, const int* seq_qstart, const int* seq_rows, int n_seqs, int first, int count,
+                              int compact, float* out, float* adds, float* queries, float* moves, int dtype, hipStream_t stream) {
+    if (n_seqs <= 0 || H <= 0 || count <= 0) return 0;
+    if (G < 1 || H % G || D < 1 || Dv < 1 || Dp != (D + 63) / 64 * 64 || Dp > 128 || n_seqs > 65535 || count > 65535 || first < 0 ||
+        (compact && first) || !adds || !queries || !moves)
+        return (int)hipErrorInvalidValue;
+    DeltaArgs a;
+    a.q = qk; a.k = qk + (size_t)G * Dp; a.gates = gates; a.v = v; a.ldq = 2ll * G * Dp; a.ldv = (long long)H * Dv;
+    a.hq = Dp; a.hv = Dv; a.group = H / G; a.H = H; a.D = D; a.Dv = Dv;
+    a.vec = Dv % 4 == 0 && (uintptr_t)v % (dtype == 0 ? 16 : 8) == 0;
+    a.first = first; a.count = count; a.compact = compact; a.qstart = seq_qstart; a.rows = seq_rows;
+    a.state = state; a.stride = stride; a.offset = offset; a.out = out; a.adds = adds; a.queries = queries; a.moves = moves;
+    if (Dp == 64) launch_delta<64>(a, n_seqs, dtype, stream); else launch_delta<128>(a, n_seqs, dtype, stream);
     return soc_last_error();
 }

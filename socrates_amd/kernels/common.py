@@ -108,6 +108,7 @@ _DELTA_SIGNATURES = {
 }
 _SCAN_SIGNATURES = {
     "soc_scan": [I, P, L, I, P, L, I, I, I, P, L, I, I, I, P, L, P, P, P, I, I, I, P, L, I, P, P, I, I, I, I, P, P, P, P, I, P],
+    "soc_delta_scan": [P, P, P, I, I, I, I, I, P, L, I, P, P, I, I, I, I, P, P, P, P, I, P],
 }
 _SAMPLING_SIGNATURES = {"soc_sample": [P, P, P, P, P, I, I, P], "soc_argmax": [P, P, P, I, I, I, P]}
 _ATTENTION_SIGNATURES = {

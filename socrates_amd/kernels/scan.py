@@ -15,11 +15,17 @@ CHUNK = 64
 HEAD, STEP, CHANNEL, BONUS = range(4)          # what the decays are: see csrc/scan.hip
 
 
+def _tiles(D, Dv):
+    """Elements of a head's state in tiles of 16 channels by 16 columns, an even number of them along the columns."""
+    return -(-D // 16) * 16 * -(-Dv // 32) * 32
+
+
 class Scan:
     # Tokens of a step's longest portion from which it is taken in chunks (0: never). Measured in us, walk -> chunks, at
     # the heads of a 4B-sized layer: 64 tokens: retention 34 -> 42, gated linear attention 34 -> 57, wkv 30 -> 48,
     # ssd 33 -> 32; 100 tokens: 46 -> 40, 48 -> 58, 39 -> 45, 48 -> 33; 300: 149 -> 60, 162 -> 72, 85 -> 44, 175 -> 63.
-    scan_from = 128
+    # The gated delta rule, whose chunk costs more and whose walk is faster: 200 tokens 62 -> 73, 300: 89 -> 75.
+    scan_from, delta_scan_from = 128, 256
     scan_scratch = 1 << 30           # bytes of scratch that one launch over all chunks may take; beyond, in rounds
 
     def _scan_lib(self):
@@ -29,11 +35,24 @@ class Scan:
             _declare(lib, _SCAN_SIGNATURES)
         return lib
 
-    def _in_chunks(self, ctx, D):
+    def _in_chunks(self, ctx, D, least=None):
         """Whether a step's recurrences with keys of ``D`` run in chunks: a portion of some length (single tokens and
         short portions walk: a chunk costs the same however few of its tokens there are) and a state whose
-        queries, keys and decays of a chunk fit LDS."""
-        return 0 < self.scan_from <= ctx.max_q_len and D <= 128
+        queries, keys and decays of a chunk fit LDS. ``least``: tokens, in place of ``scan_from``."""
+        return 0 < (self.scan_from if least is None else least) <= ctx.max_q_len and D <= 128
+
+    def _scan_scratch(self, ctx, N, sizes):
+        """(chunks of the longest portion, chunks of every sequence that one launch takes, whether those lie one behind the
+        other, scratch of ``sizes`` floats per chunk slot): all chunks at once where the scratch allows it, else rounds
+        over a few chunks of every sequence with the state in the row between them."""
+        chunks, per_slot = -(-ctx.max_q_len // CHUNK), 4 * sum(sizes)
+        slots, count = N // CHUNK + ctx.n_seqs, chunks
+        compact = slots * per_slot <= self.scan_scratch
+        if not compact:
+            count = max(1, min(chunks, self.scan_scratch // (ctx.n_seqs * per_slot)))
+            slots = ctx.n_seqs * count
+        # (each starts on 16 bytes)
+        return chunks, count, compact, [torch.empty(slots * n, dtype=torch.float32, device=self.device) for n in sizes]
 
     def _scan(self, mode, q, ldq, hq, k, ldk, hk, v, ldv, hv, decay, H, D, Dv, state, stride, offset, ctx, N, out, group=1, q_f32=True,
               v_act=False, ones=0, lda=0, params=()):
@@ -41,21 +60,7 @@ class Scan:
         the next, h* from one head to the next."""
         dk = 64 if D <= 64 else 128
         rows = CHUNK * dk if mode in (CHANNEL, BONUS) else CHUNK
-        per_slot = H * (D * Dv + rows + dk)
-        chunks = -(-ctx.max_q_len // CHUNK)
-        slots = N // CHUNK + ctx.n_seqs
-        compact = slots * per_slot * 4 <= self.scan_scratch
-        if not compact:
-            # rounds over a few chunks of every sequence, the state in the row between them
-            count = max(1, min(chunks, self.scan_scratch // (ctx.n_seqs * per_slot * 4)))
-            slots = ctx.n_seqs * count
-        else:
-            count = chunks
-        scratch = torch.empty(slots * per_slot, dtype=torch.float32, device=self.device)
-        adds, queries, factors = scratch.split([slots * H * D * Dv, slots * H * rows, slots * H * dk])
-        if D * Dv % 4:
-            # (what lies behind the addends is read by fours)
-            queries, factors = (torch.empty_like(t) for t in (queries, factors))
+        chunks, count, compact, (adds, queries, factors) = self._scan_scratch(ctx, N, [H * _tiles(D, Dv), H * rows, H * dk])
         p = list(params) + [None] * (3 - len(params))
         self.forms["scan"] += 1
         for first in range(0, chunks, count):
@@ -63,6 +68,17 @@ class Scan:
                 c_int(mode), q, c_longlong(ldq), c_int(hq), k, c_longlong(ldk), c_int(hk), c_int(group), c_int(1 if q_f32 else 0),
                 v, c_longlong(ldv), c_int(hv), c_int(1 if v_act else 0), c_int(ones), decay, c_longlong(lda), *p, c_int(H), c_int(D),
                 c_int(Dv), _ptr(state), stride, c_int(offset), _ptr(ctx.seq_qstart), _ptr(ctx.seq_rows), c_int(ctx.n_seqs),
-                c_int(first), c_int(min(count, chunks - first)) if compact else c_int(count), c_int(1 if compact else 0), _ptr(out),
+                c_int(first), c_int(count), c_int(1 if compact else 0), _ptr(out),
                 _ptr(adds), _ptr(queries), _ptr(factors), c_int(self.code), self._stream()), "scan")
+        return out
+
+    def _delta_scan(self, qk, v, gates, G, H, D, Dv, Dp, state, stride, offset, ctx, N, out):
+        """The gated delta rule in chunks, from what ``soc_delta_prepare`` leaves."""
+        chunks, count, compact, (adds, queries, moves) = self._scan_scratch(ctx, N, [H * _tiles(D, Dv), H * CHUNK * Dp, H * Dp * Dp])
+        self.forms["scan"] += 1
+        for first in range(0, chunks, count):
+            _check(self._scan_lib().soc_delta_scan(
+                _ptr(qk), _ptr(v), _ptr(gates), c_int(G), c_int(H), c_int(D), c_int(Dv), c_int(Dp), _ptr(state), stride, c_int(offset),
+                _ptr(ctx.seq_qstart), _ptr(ctx.seq_rows), c_int(ctx.n_seqs), c_int(first), c_int(count), c_int(1 if compact else 0),
+                _ptr(out), _ptr(adds), _ptr(queries), _ptr(moves), c_int(self.code), self._stream()), "delta_scan")
         return out
