@@ -501,8 +501,9 @@ SOC_EXPORT int soc_moe_route(const float* z, int ldz, const float* bias, const f
 // idx [M] (M = tokens x top): the expert of each (token, choice) pair. One workgroup counts the pairs of each
 // expert, lays the experts' runs one after the other (offsets [E + 1]), gives each pair its place (place [M]) and
 // each place its pair (pair_at [M]), and lists the tiles of TM places that the products walk: tiles [max_tiles, 2]
-// = (expert, first place), expert -1 behind the last tile. max_tiles >= M / TM + E. A pair whose expert is E or more (an
-// identity expert: nothing to compute) gets no place: -1.
+// = (expert, first place), expert -1 behind the last tile, and behind those the number of tiles. max_tiles >= M / TM + E.
+// Tiles hold TM places and an expert's last one the rest; with TM = 256 an expert's tiles hold nearly the same number. A
+// pair whose expert is E or more (an identity expert: nothing to compute) gets no place: -1.
 __global__ void __launch_bounds__(1024)
 moe_sort_kernel(const int* __restrict__ idx, int M, int E, int TM, int max_tiles, int* __restrict__ offsets,
                 int* __restrict__ place, int* __restrict__ pair_at, int* __restrict__ tiles) {
@@ -541,11 +542,14 @@ moe_sort_kernel(const int* __restrict__ idx, int M, int E, int TM, int max_tiles
                 if (tile0[mid] <= t) lo = mid; else hi = mid - 1;
             }
             e = lo;
-            first = start[e] + (t - tile0[e]) * TM;
+            // (256 places: an expert's places in as many tiles, of nearly equal size in blocks of 16)
+            const int n = tile0[e + 1] - tile0[e], rows = TM == 256 ? ((count[e] + n - 1) / n + 15) / 16 * 16 : TM;
+            first = start[e] + (t - tile0[e]) * rows;
         }
         tiles[2 * t] = e;
         tiles[2 * t + 1] = first;
     }
+    if (tid == 0) tiles[2 * max_tiles] = tile0[E];
 }
 
 SOC_EXPORT int soc_moe_sort(const int* idx, int M, int E, int TM, int max_tiles, int* offsets, int* place, int* pair_at,
@@ -765,22 +769,161 @@ grouped_mfma_kernel(const bf16* __restrict__ x, int ldx, const int* __restrict__
         }
 }
 
+// The same for many places per expert: up to 256 places x 256 weight rows by eight waves (2 x 4; blocks of 16 places take
+// turns between the two, 64 weight rows each), 64 k at a time in two LDS buffers that global_load_lds fills while the
+// other is multiplied: no registers, no LDS writes, one barrier per 64 k. A wave's products of 128 x 64 read LDS for
+// three quarters of their own time; at 64 x 64 a wave the reads take longer than the products. Such a load
+// puts a wave's 64 pieces of 16 bytes one behind the other, so rows cannot be padded apart: a row's eight pieces are
+// swapped among themselves instead, by a pattern over the rows that lets 16 rows of one k be read without bank
+// conflicts. The weights are the first operand: a lane ends up with four neighbouring outputs of one place.
+// An expert's places are cut into tiles of nearly equal size (moe_sort), because each tile reads the expert's weights
+// again. Workgroups go round-robin over the eight XCDs; each XCD gets a run of (tile, block of outputs) in order,
+// so that the tiles of an expert meet in one L2. Measured against the kernel above (tiles of 128) at 32 experts of 2,432
+// and a width of 2,560, us: 8,320 places gate / up 469 -> 388, down 285 -> 252; 12,000 places 550 -> 436 and 347 -> 265
+// (685 TFLOP/s; its weights alone take 166 us at a copy's rate). Bound by the LDS reads beside the products and,
+// with one workgroup per compute unit, by the last round of workgroups, which is seldom full. K is a multiple of 64; places and weight rows outside are read from
+// a row that exists and not written.
+template <int N> struct ga_blocks { static constexpr int value = N; };
+__device__ __forceinline__ int ga_swap(int row) { return (row >> 1) & 7; }
+
+__device__ __forceinline__ void ga_load(const bf16* from, uint16_t* lds) {
+    // (the wave's LDS address goes through m0; nothing comes back in registers)
+    const uint32_t to = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t*)lds;
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(__builtin_amdgcn_readfirstlane(to)), "v"(from) : "memory");
+}
+
+template <bool GLU, typename TO>
+__global__ void __launch_bounds__(512)
+grouped_wide_kernel(const bf16* __restrict__ x, int ldx, const int* __restrict__ pair_at, int top, const bf16* __restrict__ w,
+                    const int* __restrict__ offsets, const int* __restrict__ tiles, int max_tiles, int blocks, TO* __restrict__ out, int n_out,
+                    int K, int ff, float limit, float slope, float shift, int squared) {
+    constexpr int BM = 256, BN = 256, BK = 64, COLS = GLU ? BN / 2 : BN;
+    __shared__ __attribute__((aligned(1024))) uint16_t As[2][BM * BK], Ws[2][BN * BK];
+    const int n_tiles = tiles[2 * max_tiles], total = n_tiles * blocks, chunk = (total + 7) / 8;
+    const int item = (int)(blockIdx.x % 8) * chunk + (int)(blockIdx.x / 8);
+    if ((int)(blockIdx.x / 8) >= chunk || item >= total) return;
+    const int tile = item / blocks, o0 = item % blocks * COLS;
+    const int e = tiles[2 * tile], p0 = tiles[2 * tile + 1];
+    const int pend = tile + 1 < n_tiles && tiles[2 * tile + 2] == e ? tiles[2 * tile + 3] : offsets[e + 1];
+    const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64), li = lane % 16, g = lane / 16;
+    const int wm = wave / 4, wn = wave % 4;
+    const bf16* we = w + (size_t)e * (GLU ? 2 * ff : n_out) * K;
+    const bf16* a_src[4];                                    // a wave fills 32 rows of each, eight per load
+    const bf16* w_src[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int row = (wave * 4 + i) * 8 + lane / 8, piece = ((lane % 8) ^ ga_swap(row)) * 8, p = min(p0 + row, pend - 1);
+        a_src[i] = x + (size_t)(pair_at ? pair_at[p] / top : p) * ldx + piece;
+        int at;
+        if (GLU) at = min(o0 + row / 64 * 32 + row % 64 / 32 * 16 + row % 16, ff - 1) + (row / 16 % 2 ? ff : 0);     // gate and up tiles alternate
+        else at = min(o0 + row, n_out - 1);
+        w_src[i] = we + (size_t)at * K + piece;
+    }
+    const int rows = pend - p0, steps = K / BK;
+    auto issue = [&](int k0, int buf) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ga_load(w_src[i] + k0, &Ws[buf][(wave * 4 + i) * 512]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if ((wave * 4 + i) * 8 < rows) ga_load(a_src[i] + k0, &As[buf][(wave * 4 + i) * 512]);      // the same in all lanes
+    };
+    hyb_f32x4 acc[8][4];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] = (hyb_f32x4){0.f, 0.f, 0.f, 0.f};
+    issue(0, 0);
+    // NB: blocks of 16 places per wave (a branch per block would stand between every read and its products)
+    auto walk = [&](auto blocks_of_16) {
+        constexpr int NB = decltype(blocks_of_16)::value;
+        for (int s = 0; s < steps; ++s) {
+            // this step's pieces have landed, and every wave has read the other buffer
+            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            if (s + 1 < steps) issue((s + 1) * BK, (s + 1) % 2);
+            const uint16_t* a = As[s % 2];
+            const uint16_t* b = Ws[s % 2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                hyb_bf16x8 wf[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int row = wn * 64 + j * 16 + li;
+                    wf[j] = *reinterpret_cast<const hyb_bf16x8*>(&b[row * BK + ((4 * h + g) ^ ga_swap(row)) * 8]);
+                }
+#pragma unroll
+                for (int i = 0; i < NB; ++i) {
+                    const int row = (2 * i + wm) * 16 + li;
+                    const hyb_bf16x8 af = *reinterpret_cast<const hyb_bf16x8*>(&a[row * BK + ((4 * h + g) ^ ga_swap(row)) * 8]);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], af, acc[i][j], 0, 0, 0);
+                }
+            }
+        }
+    };
+    if (rows > 192) walk(ga_blocks<8>{});
+    else if (rows > 128) walk(ga_blocks<6>{});
+    else if (rows > 64) walk(ga_blocks<4>{});
+    else walk(ga_blocks<2>{});
+    // acc[i][j][r] belongs to place lane % 16 of block i and weight row 4 g + r of tile j
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const int p = p0 + (2 * i + wm) * 16 + li;
+        if (p >= pend) continue;
+        constexpr int STEP = GLU ? 2 : 1;
+#pragma unroll
+        for (int j = 0; j < 4; j += STEP) {
+            const int col = o0 + (GLU ? wn * 32 + j / 2 * 16 : wn * 64 + j * 16) + 4 * g;
+            float y[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                if constexpr (GLU) {
+                    const float gt = fminf(to_float(from_float<bf16>(acc[i][j][r])), limit);
+                    const float up = fminf(fmaxf(to_float(from_float<bf16>(acc[i][j + 1][r])), -limit), limit);
+                    y[r] = gt * hyb_sigmoid(slope * gt) * (up + shift);
+                } else {
+                    y[r] = acc[i][j][r];
+                    if (squared) { y[r] = fmaxf(y[r], 0.f); y[r] *= y[r]; }
+                }
+            }
+            TO* to = out + (size_t)p * n_out + col;
+            if (n_out % 4 == 0 && col + 4 <= n_out) {
+                if constexpr (sizeof(TO) == 4) *reinterpret_cast<float4*>(to) = make_float4(y[0], y[1], y[2], y[3]);
+                else *reinterpret_cast<uint2*>(to) = make_uint2(pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3]));
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (col + r < n_out) to[r] = from_float<TO>(y[r]);
+            }
+        }
+    }
+}
+
 // x [*, K]; w [E, 2 ff or n_out, K]; out [M, n_out] in the compute dtype (out_f32 0) or float32 (1). tile: the
 // places per tile that the sorting kernel was given: 16 (any dtype; bfloat16 with K and ldx multiples of 8 on the
-// matrix cores) or 128 (bfloat16 on the matrix cores only).
+// matrix cores), 128 or 256 (bfloat16 on the matrix cores only; 256: K a multiple of 64, x and w on 16 bytes).
 SOC_EXPORT int soc_grouped_linear(const void* x, int ldx, const int* pair_at, int top, const void* w, const int* offsets,
                                   const int* tiles, int max_tiles, int tile, void* out, int n_out, int K, int ff, float limit,
                                   float slope, float shift, int squared, int out_f32, int dtype, hipStream_t stream) {
     if (max_tiles <= 0 || n_out <= 0) return 0;
     if (K < 1 || max_tiles > 65535 || (ff > 0 && (ff != n_out || out_f32 || squared))) return (int)hipErrorInvalidValue;
     const bool mfma = dtype == 1 && K % 8 == 0 && ldx % 8 == 0;
-    if ((tile != 16 && tile != 128) || (tile > 16 && !mfma)) return (int)hipErrorInvalidValue;
+    if ((tile != 16 && tile != 128 && tile != 256) || (tile > 16 && !mfma)) return (int)hipErrorInvalidValue;
     if (mfma) {
 #define SOC_GM(WM, WN, MI, NI, GLU, TO)                                                                                          \
     hipLaunchKernelGGL((grouped_mfma_kernel<WM, WN, MI, NI, GLU, TO>), dim3((n_out + (GLU ? 63 : 127)) / (GLU ? 64 : 128), max_tiles), \
                        dim3(256), 0, stream, (const bf16*)x, ldx, pair_at, top, (const bf16*)w, offsets, tiles, (TO*)out, n_out, \
                        K, ff, limit, slope, shift, squared)
-        if (tile == 128) {
+#define SOC_GA(GLU, TO)                                                                                                          \
+    do {                                                                                                                         \
+        const int blocks = (n_out + (GLU ? 127 : 255)) / (GLU ? 128 : 256);                                                      \
+        hipLaunchKernelGGL((grouped_wide_kernel<GLU, TO>), dim3((blocks * max_tiles + 7) / 8 * 8), dim3(512), 0, stream, (const bf16*)x, ldx, \
+                           pair_at, top, (const bf16*)w, offsets, tiles, max_tiles, blocks, (TO*)out, n_out, K, ff, limit, slope, shift, squared); \
+    } while (0)
+        if (tile == 256) {
+            if (K % 64 || (uintptr_t)x % 16 || (uintptr_t)w % 16) return (int)hipErrorInvalidValue;
+            if (ff > 0) SOC_GA(true, bf16); else if (out_f32) SOC_GA(false, float); else SOC_GA(false, bf16);
+#undef SOC_GA
+        } else if (tile == 128) {
             if (ff > 0) SOC_GM(2, 2, 4, 4, true, bf16); else if (out_f32) SOC_GM(2, 2, 4, 4, false, float); else SOC_GM(2, 2, 4, 4, false, bf16);
         } else {
             if (ff > 0) SOC_GM(1, 4, 1, 2, true, bf16); else if (out_f32) SOC_GM(1, 4, 1, 2, false, float); else SOC_GM(1, 4, 1, 2, false, bf16);

@@ -14,9 +14,10 @@ from .common import _HYBRID_SIGNATURES, KernelError, _check, _declare, _ptr
 
 MAX_EXPERTS = 256        # what the routing and sorting kernels hold per token and per workgroup
 EXPERT_TILE = 16         # places of one expert that a workgroup of the products per expert takes ...
-# ... or, in bfloat16, (tokens per expert on average from which, places). Tiles of 256 places were measured and lost
-# (a prompt of 2,048 tokens at 4B-sized layers, 256 tokens per expert on average: 20.5 against 17.6 ms).
-EXPERT_TILES_MANY = ((48, 128),)
+# ... or, in bfloat16, (places per expert on average from which, places, what both sums' lengths are multiples of). Us for
+# the two products at 32 experts of 2,432 and a width of 2,560, tiles of 16 / 128 / 256 places: 19 places per expert
+# 395 / 389 / 404, 37: 506 / 401 / 413, 125: 1,068 / 451 / 459, 260: 2,156 / 754 / 640, 375: 3,067 / 897 / 701.
+EXPERT_TILES_MANY = ((160, 256, 64), (48, 128, 8))
 from .scan import HEAD
 
 
@@ -205,13 +206,14 @@ class Hybrid:
         self._want(idx, "experts", torch.int32)
         if not 1 <= E <= MAX_EXPERTS:
             raise KernelError(f"{E} experts (at most {MAX_EXPERTS})")
-        if tile not in (EXPERT_TILE,) + tuple(t for _, t in EXPERT_TILES_MANY):
+        if tile not in (EXPERT_TILE,) + tuple(t for _, t, _ in EXPERT_TILES_MANY):
             raise KernelError(f"tiles of {tile} places")
         M = N * top
         max_tiles = (M + tile - 1) // tile + min(E, M)
-        ints = torch.empty((2 * M + E + 1 + 2 * max_tiles,), dtype=torch.int32, device=self.device)
+        # (behind the tiles: how many of them there are)
+        ints = torch.empty((2 * M + E + 1 + 2 * max_tiles + 1,), dtype=torch.int32, device=self.device)
         place, pair_at, offsets = ints[:M], ints[M:2 * M], ints[2 * M:2 * M + E + 1]
-        tiles = ints[2 * M + E + 1:].view(max_tiles, 2)
+        tiles = ints[2 * M + E + 1:-1].view(max_tiles, 2)
         _check(self._hybrid().soc_moe_sort(_ptr(idx), c_int(M), c_int(E), c_int(tile), c_int(max_tiles), _ptr(offsets),
                                            _ptr(place), _ptr(pair_at), _ptr(tiles), self._stream()), "moe_sort")
         return ExpertRuns(place, pair_at, offsets, tiles, top, tile)
@@ -276,12 +278,14 @@ class Hybrid:
                                                   c_int(top), c_int(self.code), self._stream()), "moe_combine")
         return out
 
-    def _expert_tile(self, x, M, E, d, ff):
+    def _expert_tile(self, x, M, E, d, ff, *weights):
         """Places per tile of the products per expert."""
         # many tokens per expert, in bfloat16 with rows that start on 16 bytes: the larger tiles of the matrix cores
         # (a weight row then comes from memory once per 128 or 256 tokens of its expert)
-        if self.dtype == torch.bfloat16 and d % 8 == 0 and ff % 8 == 0 and x.stride(0) % 8 == 0:
-            return next((t for least, t in EXPERT_TILES_MANY if M >= least * E), EXPERT_TILE)
+        if self.dtype == torch.bfloat16 and x.stride(0) % 8 == 0:
+            aligned = all(t.data_ptr() % 16 == 0 for t in (x,) + weights)
+            return next((t for least, t, of in EXPERT_TILES_MANY
+                         if M >= least * E and d % of == 0 and ff % of == 0 and (t < 256 or aligned)), EXPERT_TILE)
         return EXPERT_TILE
 
     def moe_experts(self, x, idx, weight, w_gate_up, w_down, limit, slope, extra=None, shift=1.0, extra_gate=None, whole=True,
@@ -292,7 +296,7 @@ class Hybrid:
         experts, whose result is x. ``whole`` False (without an extra term): an ``ExpertSums``, the weighted sum left to
         the caller's own sum."""
         E, _, d = w_gate_up.shape
-        runs = self.moe_sort(idx, E, self._expert_tile(x, idx.numel(), E, d, w_down.shape[2]))
+        runs = self.moe_sort(idx, E, self._expert_tile(x, idx.numel(), E, d, w_down.shape[2], w_gate_up, w_down))
         act = self.grouped_linear(x, w_gate_up, runs, by_token=True, glu=(limit, slope, shift))
         y = self.grouped_linear(act, w_down, runs, by_token=False, out_dtype=torch.float32)
         through = x if identity else None
@@ -304,7 +308,7 @@ class Hybrid:
         """The same with experts Wd relu(Wu x)^2 (``w_up`` [E, ff, d], ``w_down`` [E, d, ff]). ``whole`` False (without
         an extra term): an ``ExpertSums``, the weighted sum left to ``branches_add``."""
         E, ff, d = w_up.shape
-        runs = self.moe_sort(idx, E, self._expert_tile(x, idx.numel(), E, d, ff))
+        runs = self.moe_sort(idx, E, self._expert_tile(x, idx.numel(), E, d, ff, w_up, w_down))
         act = self.grouped_linear(x, w_up, runs, by_token=True, squared=True)
         y = self.grouped_linear(act, w_down, runs, by_token=False, out_dtype=torch.float32)
         through = x if identity else None
