@@ -393,8 +393,14 @@ __device__ __forceinline__ void rescale_in_place(f32x4_t (&o)[RT_][DV_], const f
 // slices of a head hold both partners of every rotated pair, so nothing crosses lanes but the
 // sum of squares. The token's own key and value do not go through the cache: the wave whose
 // split holds the token's position adds them as one more tile from registers, and (for one
-// chunk of heads) stores them to the page for the steps to come. The work hides behind the
-// start of the walk (position -> table -> first keys), which it does not depend on.
+// chunk of heads) stores them to the page for the steps to come.
+// What bounds it up to some hundred keys per wave is a chain of trips to memory: position ->
+// table -> first keys, and the raw row -> queries. Everything of both is therefore on its way
+// before the first wait: the raw row, gains and rotation, then three tiles of keys and values,
+// and the norm, the rotation and the own key's tile run under the tiles' trip. With the row's
+// arithmetic before the lookups, and four bytes per access in the meeting of the splits, this
+// took, 32 query and 8 kv heads of 128 (us per launch): 1 row behind 700 keys 15.4, now 13.4;
+// 8 rows behind 2,048 keys 20.2, now 17.9; 3 rows behind 15,000 keys 37.9, now 33.5.
 struct FusedQkv {
     const bf16* qkv;            // [N, row_heads, D]: q heads, then (if the step writes the slot) k and v heads
     int row_heads;
@@ -418,6 +424,17 @@ struct SoftCap {
         return a * (1.f - 2.f * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(t * b) + 1.f));
     }
 };
+
+// Two floats at an address of a multiple of 8 bytes, past the caches of one XCD (agent scope).
+__device__ __forceinline__ void store_pair_agent(float* to, float a, float b) {
+    const unsigned long long both = (unsigned long long)__float_as_uint(b) << 32 | __float_as_uint(a);
+    __hip_atomic_store(reinterpret_cast<unsigned long long*>(to), both, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float2 load_pair_agent(const float* from) {
+    const unsigned long long both = __hip_atomic_load(reinterpret_cast<const unsigned long long*>(from),
+                                                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return make_float2(__uint_as_float((unsigned)both), __uint_as_float((unsigned)(both >> 32)));
+}
 
 template <int RT, bool TP, bool FUSED = false, bool CAP = false>
 __global__ void __launch_bounds__(256)
@@ -497,98 +514,40 @@ paged_attn_mfma_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k_po
         }
     }
     __shared__ float rope_cs[FUSED ? 4 : 1][FUSED ? D : 1];          // cos [0, D / 2), sin [D / 2, D) of the wave's token
+    __shared__ float gains[FUSED ? 4 : 1][FUSED ? 2 : 1][FUSED ? D : 1];     // the query heads' norm gain, the key's
     __shared__ uint4 new_kv[FUSED ? 4 : 1][FUSED ? 2 * (D / 8) : 1]; // the token's key (normed, rotated) and value, by 16-byte part
+    constexpr int PER_LANE = FUSED ? (D + SOC_WAVE - 1) / SOC_WAVE : 1;
+    uint4 qraw[FUSED ? QK_STEPS : 1], kraw[FUSED ? QK_STEPS : 1], vraw = make_uint4(0u, 0u, 0u, 0u);
+    float cs_in[PER_LANE], qg_in[PER_LANE], kg_in[PER_LANE];
     if constexpr (FUSED) {
+        // What the wave needs to make its queries and the token's own key, all of it on its way
+        // before the first key tiles and waited for behind them: the row's query head, the kv
+        // head's key, one part of its value (every wave loads; without k and v heads in the
+        // row, a query head stands in and is not used), both gains, and the token's cosines
+        // and sines, from the table (an accurate sincosf in each of a launch's thousands of
+        // waves would cost more vector time than the walk itself).
         const bf16* row_in = fz.qkv + (size_t)tok0 * fz.row_heads * D;
         const int g = chunk * 16 + (li & (Gp - 1));
-        const bool ok = row_pos[0] >= 0;
-        // raw slices first: the row's query head, the kv head's key, one part of its value
-        // (every wave loads; without k and v heads in the row, a query head stands in and is
-        // not used)
-        const size_t q_at = ((size_t)kvh * G + (ok ? g : 0)) * D;
+        const size_t q_at = ((size_t)kvh * G + (row_pos[0] >= 0 ? g : 0)) * D;
         const size_t k_at = own_key ? (size_t)(Hq + kvh) * D : q_at, v_at = own_key ? (size_t)(Hq + Hkv + kvh) * D : q_at;
-        uint4 qraw[QK_STEPS], kraw[QK_STEPS];
 #pragma unroll
         for (int kk = 0; kk < QK_STEPS; ++kk) {
             qraw[kk] = load_qk_slice(row_in + q_at, kk, kb);
             kraw[kk] = load_qk_slice(row_in + k_at, kk, kb);
         }
-        const uint4 vraw = *reinterpret_cast<const uint4*>(row_in + v_at + (lane % (D / 8)) * 8);
-        // the token's cosines and sines, from the table (an accurate sincosf in each of a
-        // launch's thousands of waves would cost more vector time than the walk itself)
+        vraw = *reinterpret_cast<const uint4*>(row_in + v_at + (lane % (D / 8)) * 8);
+        if (fz.q_gain) {
+#pragma unroll
+            for (int i = 0; i < PER_LANE; ++i) {
+                const int j = (lane + i * SOC_WAVE) % D;
+                qg_in[i] = fz.q_gain[j];
+                kg_in[i] = fz.k_gain[j];
+            }
+        }
         if (fz.rope_table) {
             const float* cs_row = fz.rope_table + (size_t)pos0 * D;
-            for (int j = lane; j < D; j += SOC_WAVE) rope_cs[wave][j] = cs_row[j];
-            __builtin_amdgcn_wave_barrier();
-        }
-        // norm and rotation of this lane's slices of one head: elements 32 kk + 8 kb + t; the
-        // partner of an element of the first half lies QK_STEPS / 2 slices on, in the same lane
-        auto norm_rope = [&](const uint4 (&raw)[QK_STEPS], const float* gain, uint4 (&res)[QK_STEPS]) {
-            float x[QK_STEPS][8];
-            float ss = 0.f;
 #pragma unroll
-            for (int kk = 0; kk < QK_STEPS; ++kk) {
-                const uint32_t w4[4] = {raw[kk].x, raw[kk].y, raw[kk].z, raw[kk].w};
-#pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    x[kk][2 * t] = __uint_as_float(w4[t] << 16);
-                    x[kk][2 * t + 1] = __uint_as_float(w4[t] & 0xffff0000u);
-                    ss += x[kk][2 * t] * x[kk][2 * t] + x[kk][2 * t + 1] * x[kk][2 * t + 1];
-                }
-            }
-            if (gain) {
-                ss = sum_xor32(sum_xor16(ss));
-                const float inv = 1.0f / sqrtf(ss / (float)D + fz.eps);
-#pragma unroll
-                for (int kk = 0; kk < QK_STEPS; ++kk) {
-                    float gn[8];
-                    VecLoad<float, 8>::load(gain + kk * 32 + kb * 8, gn);
-#pragma unroll
-                    for (int t = 0; t < 8; ++t) x[kk][t] = x[kk][t] * inv * gn[t];
-                }
-            }
-            if (fz.rope_table) {
-                constexpr int HK = QK_STEPS / 2;
-#pragma unroll
-                for (int kk = 0; kk < HK; ++kk)
-#pragma unroll
-                    for (int t = 0; t < 8; ++t) {
-                        const float cs = rope_cs[wave][kk * 32 + kb * 8 + t], sn = rope_cs[wave][D / 2 + kk * 32 + kb * 8 + t];
-                        const float a = x[kk][t], b = x[kk + HK][t];
-                        x[kk][t] = a * cs - b * sn;
-                        x[kk + HK][t] = b * cs + a * sn;
-                    }
-            }
-#pragma unroll
-            for (int kk = 0; kk < QK_STEPS; ++kk)
-                res[kk] = make_uint4(pack_bf16x2(x[kk][0], x[kk][1]), pack_bf16x2(x[kk][2], x[kk][3]),
-                                     pack_bf16x2(x[kk][4], x[kk][5]), pack_bf16x2(x[kk][6], x[kk][7]));
-        };
-        uint4 qn[QK_STEPS];
-        norm_rope(qraw, fz.q_gain, qn);
-#pragma unroll
-        for (int kk = 0; kk < QK_STEPS; ++kk) qf[0][kk] = ok ? qn[kk] : make_uint4(0u, 0u, 0u, 0u);
-        if (own_key && covers) {                              // uniform over the wave
-            uint4 kn[QK_STEPS];
-            norm_rope(kraw, fz.k_gain, kn);
-            if (li == 0) {
-#pragma unroll
-                for (int kk = 0; kk < QK_STEPS; ++kk) new_kv[wave][kk * 4 + kb] = kn[kk];
-            }
-            if (lane < D / 8) new_kv[wave][D / 8 + lane] = vraw;
-            if (chunk == 0) {
-                // to the page, for the steps to come (nothing of this launch reads it there)
-                const int page_i = bs_shift >= 0 ? pos0 >> bs_shift : pos0 / BS;
-                const size_t off = (size_t)table[page_i] * Hkv * BS * D + (size_t)kvh * BS * D +
-                                   (size_t)(pos0 - page_i * BS) * D;
-                if (li == 0) {
-#pragma unroll
-                    for (int kk = 0; kk < QK_STEPS; ++kk)
-                        *reinterpret_cast<uint4*>(fz.k_pool_w + off + kk * 32 + kb * 8) = kn[kk];
-                }
-                if (lane < D / 8) *reinterpret_cast<uint4*>(fz.v_pool_w + off + lane * 8) = vraw;
-            }
-            __builtin_amdgcn_wave_barrier();
+            for (int i = 0; i < PER_LANE; ++i) cs_in[i] = cs_row[(lane + i * SOC_WAVE) % D];
         }
     }
 
@@ -601,15 +560,6 @@ paged_attn_mfma_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k_po
         const int col = (int)(at - tok * width);
         return out + ((size_t)(col / 32) * out_tiled + tok) * 32 + col % 32;
     };
-    f32x4_t o[RT][DV];
-    float m[RT], l[RT];
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-        m[rt] = -INFINITY; l[rt] = 0.f;
-#pragma unroll
-        for (int j = 0; j < DV; ++j) o[rt][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-    }
-
     const float c2 = scale * 1.44269504088896340736f;   // scores to base 2
     const SoftCap capped(scale, softcap);
     const size_t page_stride = (size_t)Hkv * BS * D;
@@ -664,6 +614,117 @@ paged_attn_mfma_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k_po
             }
         }
     };
+
+    // Three tiles are in flight per wave (48 keys). Buffer b holds tiles b, b + 3, b + 6, ...
+    // of the wave's range; the page of a tile is looked up three tiles before its loads are
+    // issued.
+    KFrag kf0, kf1, kf2;
+    uint4 vr0[V_PER_LANE], vr1[V_PER_LANE], vr2[V_PER_LANE];
+    // Lookups first, then the tile loads: a wait for a lookup then leaves the loads in flight.
+    // Lookups may run past the end of the range (redirected); tile loads do not: the rounds
+    // of the main loop are those in which all three buffers have a tile to load, and what
+    // remains (at most five tiles, two of them still to load) follows without a loop.
+    const int k1 = klo + 16 < khi ? klo + 16 : klo, k2 = klo + 32 < khi ? klo + 32 : klo;
+    int pa = lookup(klo), pb = lookup(k1), pc = lookup(k2);
+    int pg0 = lookup(klo + 48), pg1 = lookup(klo + 64), pg2 = lookup(klo + 80);
+    fetch(klo, pa, kf0, vr0);
+    if constexpr (FUSED) {
+        // no branch around these loads, or the waits for the row's own loads, behind them,
+        // would take them in; a tile past the range is the first one once more
+        fetch(k1, pb, kf1, vr1);
+        fetch(k2, pc, kf2, vr2);
+    } else {
+        if (k1 != klo) fetch(k1, pb, kf1, vr1);
+        if (k2 != klo) fetch(k2, pc, kf2, vr2);
+    }
+    if constexpr (FUSED) {
+        const bool ok = row_pos[0] >= 0;
+        // (D not a multiple of 64: the lanes past it wrote what lane - D did)
+#pragma unroll
+        for (int i = 0; i < PER_LANE; ++i) {
+            const int j = (lane + i * SOC_WAVE) % D;
+            if (fz.rope_table) rope_cs[wave][j] = cs_in[i];
+            if (fz.q_gain) { gains[wave][0][j] = qg_in[i]; gains[wave][1][j] = kg_in[i]; }
+        }
+        __builtin_amdgcn_wave_barrier();
+        // norm and rotation of this lane's slices of one head: elements 32 kk + 8 kb + t; the
+        // partner of an element of the first half lies QK_STEPS / 2 slices on, in the same lane
+        auto norm_rope = [&](const uint4 (&raw)[QK_STEPS], const int which, uint4 (&res)[QK_STEPS]) {
+            float x[QK_STEPS][8];
+            float ss = 0.f;
+#pragma unroll
+            for (int kk = 0; kk < QK_STEPS; ++kk) {
+                const uint32_t w4[4] = {raw[kk].x, raw[kk].y, raw[kk].z, raw[kk].w};
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    x[kk][2 * t] = __uint_as_float(w4[t] << 16);
+                    x[kk][2 * t + 1] = __uint_as_float(w4[t] & 0xffff0000u);
+                    ss += x[kk][2 * t] * x[kk][2 * t] + x[kk][2 * t + 1] * x[kk][2 * t + 1];
+                }
+            }
+            if (fz.q_gain) {
+                ss = sum_xor32(sum_xor16(ss));
+                const float inv = 1.0f / sqrtf(ss / (float)D + fz.eps);
+#pragma unroll
+                for (int kk = 0; kk < QK_STEPS; ++kk) {
+#pragma unroll
+                    for (int t = 0; t < 8; ++t) x[kk][t] = x[kk][t] * inv * gains[wave][which][kk * 32 + kb * 8 + t];
+                }
+            }
+            if (fz.rope_table) {
+                constexpr int HK = QK_STEPS / 2;
+#pragma unroll
+                for (int kk = 0; kk < HK; ++kk)
+#pragma unroll
+                    for (int t = 0; t < 8; ++t) {
+                        const float cs = rope_cs[wave][kk * 32 + kb * 8 + t], sn = rope_cs[wave][D / 2 + kk * 32 + kb * 8 + t];
+                        const float a = x[kk][t], b = x[kk + HK][t];
+                        x[kk][t] = a * cs - b * sn;
+                        x[kk + HK][t] = b * cs + a * sn;
+                    }
+            }
+#pragma unroll
+            for (int kk = 0; kk < QK_STEPS; ++kk)
+                res[kk] = make_uint4(pack_bf16x2(x[kk][0], x[kk][1]), pack_bf16x2(x[kk][2], x[kk][3]),
+                                     pack_bf16x2(x[kk][4], x[kk][5]), pack_bf16x2(x[kk][6], x[kk][7]));
+        };
+        uint4 qn[QK_STEPS];
+        norm_rope(qraw, 0, qn);
+#pragma unroll
+        for (int kk = 0; kk < QK_STEPS; ++kk) qf[0][kk] = ok ? qn[kk] : make_uint4(0u, 0u, 0u, 0u);
+        if (own_key && covers) {                              // uniform over the wave
+            uint4 kn[QK_STEPS];
+            norm_rope(kraw, 1, kn);
+            if (li == 0) {
+#pragma unroll
+                for (int kk = 0; kk < QK_STEPS; ++kk) new_kv[wave][kk * 4 + kb] = kn[kk];
+            }
+            if (lane < D / 8) new_kv[wave][D / 8 + lane] = vraw;
+            if (chunk == 0) {
+                // to the page, for the steps to come (nothing of this launch reads it there)
+                const int page_i = bs_shift >= 0 ? pos0 >> bs_shift : pos0 / BS;
+                const size_t off = (size_t)table[page_i] * Hkv * BS * D + (size_t)kvh * BS * D +
+                                   (size_t)(pos0 - page_i * BS) * D;
+                if (li == 0) {
+#pragma unroll
+                    for (int kk = 0; kk < QK_STEPS; ++kk)
+                        *reinterpret_cast<uint4*>(fz.k_pool_w + off + kk * 32 + kb * 8) = kn[kk];
+                }
+                if (lane < D / 8) *reinterpret_cast<uint4*>(fz.v_pool_w + off + lane * 8) = vraw;
+            }
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+
+    f32x4_t o[RT][DV];
+    float m[RT], l[RT];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+        m[rt] = -INFINITY; l[rt] = 0.f;
+#pragma unroll
+        for (int j = 0; j < DV; ++j) o[rt][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    }
+
 
     // One tile: V to LDS, scores, online softmax, weighted values. MASKED: some key of the
     // tile is hidden from some row of the block (or lies outside the split).
@@ -776,20 +837,24 @@ paged_attn_mfma_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k_po
         weighted(pf, alpha, any_rescale);
     };
 
-    // Three tiles are in flight per wave (48 keys). Buffer b holds tiles b, b + 3, b + 6, ...
-    // of the wave's range; the page of a tile is looked up three tiles before its loads are
-    // issued.
-    KFrag kf0, kf1, kf2;
-    uint4 vr0[V_PER_LANE], vr1[V_PER_LANE], vr2[V_PER_LANE];
-    // Lookups first, then the tile loads: a wait for a lookup then leaves the loads in flight.
-    // Lookups may run past the end of the range (redirected); tile loads do not: the rounds
-    // of the main loop are those in which all three buffers have a tile to load, and what
-    // remains (at most five tiles, two of them still to load) follows without a loop.
-    int pa = lookup(klo), pb = lookup(klo + 16), pc = lookup(klo + 32);
-    int pg0 = lookup(klo + 48), pg1 = lookup(klo + 64), pg2 = lookup(klo + 80);
-    fetch(klo, pa, kf0, vr0);
-    if (klo + 16 < khi) fetch(klo + 16, pb, kf1, vr1);
-    if (klo + 32 < khi) fetch(klo + 32, pc, kf2, vr2);
+    if constexpr (FUSED) {
+        if (own_key && covers) {
+            // the token's own key and value, from where the prologue left them: one more tile
+            // whose first key is the only one there, first of all, while the others' keys and
+            // values are on their way
+            KFrag kfn;
+            uint4 vrn[V_PER_LANE];
+#pragma unroll
+            for (int kk = 0; kk < QK_STEPS; ++kk) kfn.v[kk] = new_kv[wave][kk * 4 + kb];
+#pragma unroll
+            for (int j = 0; j < V_PER_LANE; ++j) vrn[j] = new_kv[wave][D / 8 + (lane + 64 * j) % (D / 8)];
+            s16x4_t pf[RT];
+            float alpha[RT];
+            bool any_rescale;
+            scores(pos0, kfn, vrn, std::true_type{}, pf, alpha, any_rescale, pos0, pos0 + 1, pos0);
+            weighted(pf, alpha, any_rescale);
+        }
+    }
     int key0 = klo;
     for (; key0 + 80 < khi; key0 += 48) {
         tile(key0, kf0, vr0);
@@ -812,23 +877,6 @@ paged_attn_mfma_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k_po
         tile(key0 + 32, kf2, vr2);
     }
 
-    if constexpr (FUSED) {
-        if (own_key && covers) {
-            // the token's own key and value, from where the prologue left them: one more tile
-            // whose first key is the only one there
-            KFrag kfn;
-            uint4 vrn[V_PER_LANE];
-#pragma unroll
-            for (int kk = 0; kk < QK_STEPS; ++kk) kfn.v[kk] = new_kv[wave][kk * 4 + kb];
-#pragma unroll
-            for (int j = 0; j < V_PER_LANE; ++j) vrn[j] = new_kv[wave][D / 8 + (lane + 64 * j) % (D / 8)];
-            s16x4_t pf[RT];
-            float alpha[RT];
-            bool any_rescale;
-            scores(pos0, kfn, vrn, std::true_type{}, pf, alpha, any_rescale, pos0, pos0 + 1, pos0);
-            weighted(pf, alpha, any_rescale);
-        }
-    }
     // finish: the row sum is spread over the four lanes of the row's column
     float L[RT];
 #pragma unroll
@@ -894,15 +942,12 @@ paged_attn_mfma_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k_po
             } else {
                 // written through the caches (agent scope): another workgroup reads it below
                 float* dst = part_o + pi * D + j * 16 + 4 * kb;
-                __hip_atomic_store(dst, a.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(dst + 1, a.y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(dst + 2, a.z, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(dst + 3, a.w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                store_pair_agent(dst, a.x, a.y);
+                store_pair_agent(dst + 2, a.z, a.w);
             }
         }
         if (outer > 1 && wave == 0 && kb == 0) {
-            __hip_atomic_store(part_ml + pi * 2, M4, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(part_ml + pi * 2 + 1, L4, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            store_pair_agent(part_ml + pi * 2, M4, L4);
         }
     }
     if (outer == 1) return;
@@ -934,8 +979,8 @@ paged_attn_mfma_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k_po
         const size_t row = (size_t)(tok0 + tt) * Hq + (size_t)kvh * G + g;       // (token, head)
         const size_t p0 = (size_t)((long)row + shift * Hq) * outer;
         const int mine = lane < outer ? lane : 0;
-        const float ms_ = __hip_atomic_load(part_ml + (p0 + mine) * 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const float ls_ = __hip_atomic_load(part_ml + (p0 + mine) * 2 + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const float2 ml = load_pair_agent(part_ml + (p0 + mine) * 2);
+        const float ms_ = ml.x, ls_ = ml.y;
         float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
         float M = 0.f, Lt = 0.f, wl = 0.f;
         for (int s0 = 0; s0 < outer; s0 += ROUND * NG) {
@@ -944,10 +989,8 @@ paged_attn_mfma_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k_po
             for (int j = 0; j < ROUND; ++j) {
                 const int sp = s0 + sg + j * NG;
                 const float* src = part_o + (p0 + (sg < NG && sp < outer ? sp : 0)) * D + e4 * 4;
-                v[j].x = __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                v[j].y = __hip_atomic_load(src + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                v[j].z = __hip_atomic_load(src + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                v[j].w = __hip_atomic_load(src + 3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const float2 lo2 = load_pair_agent(src), hi2 = load_pair_agent(src + 2);
+                v[j] = make_float4(lo2.x, lo2.y, hi2.x, hi2.y);
             }
             if (s0 == 0) {
                 const float ms = lane < outer ? ms_ : -INFINITY;
