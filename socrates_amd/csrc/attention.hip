@@ -342,7 +342,10 @@ SOC_EXPORT int soc_paged_attention_tokens(const void* q, const void* k_pool, con
 constexpr bool QK_K32 = (D % 32 == 0);
 constexpr int QK_STEPS = QK_K32 ? D / 32 : D / 16;
 constexpr int DV = D / 16;                   // 16-wide blocks of the head dimension
-constexpr int V_STRIDE = D + 4;              // LDS row stride (elements): conflict-free transposed reads
+// LDS row stride (elements): 8 dwords, or an odd multiple of them, past a multiple of 64, so that the eight
+// rows that half a wave reads 32 bytes of each in a transposed read lie on all 64 banks once
+constexpr int V_STRIDE = D % 32 ? D : D + 16;
+typedef __attribute__((address_space(3))) s16x4_t lds_s16x4_t;
 constexpr int V_CHUNKS = 16 * D / 8;         // 16-byte chunks in a 16-key V tile
 constexpr int V_PER_LANE = (V_CHUNKS + 63) / 64;
 
@@ -392,15 +395,19 @@ __device__ __forceinline__ void rescale_in_place(f32x4_t (&o)[RT_][DV_], const f
 // rotation at the token's position, all in float32 with one rounding to bfloat16. A lane's
 // slices of a head hold both partners of every rotated pair, so nothing crosses lanes but the
 // sum of squares. The token's own key and value do not go through the cache: the wave whose
-// split holds the token's position adds them as one more tile from registers, and (for one
+// split holds the token's position puts them in their places of its last tile, and (for one
 // chunk of heads) stores them to the page for the steps to come.
 // What bounds it up to some hundred keys per wave is a chain of trips to memory: position ->
 // table -> first keys, and the raw row -> queries. Everything of both is therefore on its way
 // before the first wait: the raw row, gains and rotation, then three tiles of keys and values,
-// and the norm, the rotation and the own key's tile run under the tiles' trip. With the row's
-// arithmetic before the lookups, and four bytes per access in the meeting of the splits, this
-// took, 32 query and 8 kv heads of 128 (us per launch): 1 row behind 700 keys 15.4, now 13.4;
-// 8 rows behind 2,048 keys 20.2, now 17.9; 3 rows behind 15,000 keys 37.9, now 33.5.
+// and the norm and the rotation run under the tiles' trip, the key's in a spare column of the
+// queries' row tile (code of its own costs its first trip through the instruction cache: 0.7 us
+// for the workgroup that the others wait for). With the row's arithmetic before the lookups,
+// the own key as a tile of its own and four bytes per access in the meeting of the splits this
+// took, 32 query and 8 kv heads of 128 (us per launch): 1 row behind 700 keys 15.4, now 12.2;
+// 8 rows behind 2,048 keys 20.2, now 17.2; 3 rows behind 15,000 keys 37.9, now 33.5. One loop
+// for full rounds and the rest, with loads past the range redirected, is less code but reads
+// the redirected tiles: 0.3 us less for the first, 0.7, 0.9 and (64 rows behind 2,011 keys) 5 more.
 struct FusedQkv {
     const bf16* qkv;            // [N, row_heads, D]: q heads, then (if the step writes the slot) k and v heads
     int row_heads;
@@ -485,10 +492,12 @@ paged_attn_mfma_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k_po
     }
     const int split_lo = first_key + split * split_len;     // the split's first key
     int klo = split_lo;
-    // FUSED and writing: the token's own key is not read from the cache (it is not there yet)
+    // FUSED and writing: the token's own key and value do not come from the cache (they are not
+    // there yet); its tile is loaded like any other, and their places in it are filled when it
+    // is computed
     const bool own_key = FUSED && fz.write_kv;
     const bool covers = pos0 >= klo && pos0 < klo + split_len;      // this wave's split holds the token's position
-    int khi = min(klo + split_len, own_key ? pos0 : pos0 + ntok);
+    int khi = min(klo + split_len, pos0 + ntok);
     klo = max(klo, first_seen(pos0, window));
     const int kmin = klo;                                // first key any row of the block can see
     klo = klo & ~15;                                     // tiles are aligned to 16 keys
@@ -515,26 +524,28 @@ paged_attn_mfma_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k_po
     }
     __shared__ float rope_cs[FUSED ? 4 : 1][FUSED ? D : 1];          // cos [0, D / 2), sin [D / 2, D) of the wave's token
     __shared__ float gains[FUSED ? 4 : 1][FUSED ? 2 : 1][FUSED ? D : 1];     // the query heads' norm gain, the key's
-    __shared__ uint4 new_kv[FUSED ? 4 : 1][FUSED ? 2 * (D / 8) : 1]; // the token's key (normed, rotated) and value, by 16-byte part
+    __shared__ uint4 new_k[FUSED ? 4 : 1][FUSED ? D / 8 : 1];        // the token's key, normed and rotated, by 16-byte part
     constexpr int PER_LANE = FUSED ? (D + SOC_WAVE - 1) / SOC_WAVE : 1;
-    uint4 qraw[FUSED ? QK_STEPS : 1], kraw[FUSED ? QK_STEPS : 1], vraw = make_uint4(0u, 0u, 0u, 0u);
+    uint4 qraw[FUSED ? QK_STEPS : 1], vraw = make_uint4(0u, 0u, 0u, 0u);
+    // the column of the row tile that makes the key: a spare one next to the queries if there is one
+    const bool spare = Gp < 16;
+    const int k_col = spare ? Gp : 0;
     float cs_in[PER_LANE], qg_in[PER_LANE], kg_in[PER_LANE];
     if constexpr (FUSED) {
         // What the wave needs to make its queries and the token's own key, all of it on its way
-        // before the first key tiles and waited for behind them: the row's query head, the kv
-        // head's key, one part of its value (every wave loads; without k and v heads in the
-        // row, a query head stands in and is not used), both gains, and the token's cosines
-        // and sines, from the table (an accurate sincosf in each of a launch's thousands of
-        // waves would cost more vector time than the walk itself).
+        // before the first key tiles and waited for behind them: the row's query head (in a
+        // spare column the kv head's key), one part of the kv head's value (every wave loads;
+        // without k and v heads in the row, a query head stands in and is not used), both
+        // gains, and the token's cosines and sines, from the table (an accurate sincosf in
+        // each of a launch's thousands of waves would cost more vector time than the walk itself).
         const bf16* row_in = fz.qkv + (size_t)tok0 * fz.row_heads * D;
         const int g = chunk * 16 + (li & (Gp - 1));
-        const size_t q_at = ((size_t)kvh * G + (row_pos[0] >= 0 ? g : 0)) * D;
-        const size_t k_at = own_key ? (size_t)(Hq + kvh) * D : q_at, v_at = own_key ? (size_t)(Hq + Hkv + kvh) * D : q_at;
+        const size_t first_q = (size_t)kvh * G * D;
+        const size_t q_at = row_pos[0] >= 0 ? first_q + (size_t)g * D
+                            : own_key && spare && li == k_col ? (size_t)(Hq + kvh) * D : first_q;
+        const size_t v_at = own_key ? (size_t)(Hq + Hkv + kvh) * D : first_q;
 #pragma unroll
-        for (int kk = 0; kk < QK_STEPS; ++kk) {
-            qraw[kk] = load_qk_slice(row_in + q_at, kk, kb);
-            kraw[kk] = load_qk_slice(row_in + k_at, kk, kb);
-        }
+        for (int kk = 0; kk < QK_STEPS; ++kk) qraw[kk] = load_qk_slice(row_in + q_at, kk, kb);
         vraw = *reinterpret_cast<const uint4*>(row_in + v_at + (lane % (D / 8)) * 8);
         if (fz.q_gain) {
 #pragma unroll
@@ -589,7 +600,7 @@ paged_attn_mfma_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k_po
     // Global loads of one tile: this lane's K slices and its share of the V tile.
     auto fetch = [&](int key0, int page, KFrag& kf, uint4 (&vr)[V_PER_LANE]) {
         if constexpr (tile_in_page) {
-            const size_t tile_off = (size_t)page * page_stride + (size_t)((key0 & (BS - 1)) * D);
+            const size_t tile_off = (size_t)(unsigned)page * page_stride + (size_t)((key0 & (BS - 1)) * D);
             const bf16* krow = k_base + tile_off + li * D;
 #pragma unroll
             for (int kk = 0; kk < QK_STEPS; ++kk) kf.v[kk] = load_qk_slice(krow, kk, kb);
@@ -627,6 +638,7 @@ paged_attn_mfma_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k_po
     const int k1 = klo + 16 < khi ? klo + 16 : klo, k2 = klo + 32 < khi ? klo + 32 : klo;
     int pa = lookup(klo), pb = lookup(k1), pc = lookup(k2);
     int pg0 = lookup(klo + 48), pg1 = lookup(klo + 64), pg2 = lookup(klo + 80);
+    __builtin_amdgcn_sched_barrier(0);                      // no wait for one before all are on their way
     fetch(klo, pa, kf0, vr0);
     if constexpr (FUSED) {
         // no branch around these loads, or the waits for the row's own loads, behind them,
@@ -688,24 +700,31 @@ paged_attn_mfma_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k_po
                 res[kk] = make_uint4(pack_bf16x2(x[kk][0], x[kk][1]), pack_bf16x2(x[kk][2], x[kk][3]),
                                      pack_bf16x2(x[kk][4], x[kk][5]), pack_bf16x2(x[kk][6], x[kk][7]));
         };
-        uint4 qn[QK_STEPS];
-        norm_rope(qraw, 0, qn);
+        uint4 qn[QK_STEPS], kn[QK_STEPS];
+        norm_rope(qraw, own_key && spare && li == k_col ? 1 : 0, qn);
 #pragma unroll
-        for (int kk = 0; kk < QK_STEPS; ++kk) qf[0][kk] = ok ? qn[kk] : make_uint4(0u, 0u, 0u, 0u);
+        for (int kk = 0; kk < QK_STEPS; ++kk) {
+            kn[kk] = qn[kk];
+            qf[0][kk] = ok ? qn[kk] : make_uint4(0u, 0u, 0u, 0u);
+        }
         if (own_key && covers) {                              // uniform over the wave
-            uint4 kn[QK_STEPS];
-            norm_rope(kraw, 1, kn);
-            if (li == 0) {
+            if (!spare) {                                     // 16 query heads: the key in a pass of its own
+                const bf16* k_in = fz.qkv + ((size_t)tok0 * fz.row_heads + Hq + kvh) * D;
+                uint4 kraw[QK_STEPS];
 #pragma unroll
-                for (int kk = 0; kk < QK_STEPS; ++kk) new_kv[wave][kk * 4 + kb] = kn[kk];
+                for (int kk = 0; kk < QK_STEPS; ++kk) kraw[kk] = load_qk_slice(k_in, kk, kb);
+                norm_rope(kraw, 1, kn);
             }
-            if (lane < D / 8) new_kv[wave][D / 8 + lane] = vraw;
+            if (li == k_col) {
+#pragma unroll
+                for (int kk = 0; kk < QK_STEPS; ++kk) new_k[wave][kk * 4 + kb] = kn[kk];
+            }
             if (chunk == 0) {
-                // to the page, for the steps to come (nothing of this launch reads it there)
+                // to the page, for the steps to come (what this launch loads from there it replaces)
                 const int page_i = bs_shift >= 0 ? pos0 >> bs_shift : pos0 / BS;
                 const size_t off = (size_t)table[page_i] * Hkv * BS * D + (size_t)kvh * BS * D +
                                    (size_t)(pos0 - page_i * BS) * D;
-                if (li == 0) {
+                if (li == k_col) {
 #pragma unroll
                     for (int kk = 0; kk < QK_STEPS; ++kk)
                         *reinterpret_cast<uint4*>(fz.k_pool_w + off + kk * 32 + kb * 8) = kn[kk];
@@ -737,7 +756,7 @@ paged_attn_mfma_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k_po
     auto scores = [&](int key0, const KFrag& kf, const uint4 (&vr)[V_PER_LANE], auto masked_tag,
                       s16x4_t (&pf)[RT], float (&alpha)[RT], bool& any_rescale, int lo, int hi, int lo_seen) {
         constexpr bool MASKED = decltype(masked_tag)::value;
-        // V tile -> LDS, row-major with a padded stride (two 8-byte stores per chunk); keys
+        // V tile -> LDS, row-major with a padded stride; keys
         // that were not to be read become zeros here, now that their loads have landed
 #pragma unroll
         for (int j = 0; j < V_PER_LANE; ++j) {
@@ -749,9 +768,18 @@ paged_attn_mfma_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k_po
                     const int vkey = key0 + vk;
                     if (vkey < lo || vkey >= hi) t = make_uint4(0u, 0u, 0u, 0u);
                 }
-                uint2* dst = reinterpret_cast<uint2*>(&vl[vk * V_STRIDE + part * 8]);
-                dst[0] = make_uint2(t.x, t.y);
-                dst[1] = make_uint2(t.z, t.w);
+                *reinterpret_cast<uint4*>(&vl[vk * V_STRIDE + part * 8]) = t;
+            }
+        }
+        KFrag own_kf = kf;
+        if constexpr (FUSED && MASKED) {
+            // the token's own key and value, which are not in its page yet
+            if (own_key && pos0 >= key0 && pos0 < key0 + 16) {
+                if (lane < D / 8) *reinterpret_cast<uint4*>(&vl[(pos0 - key0) * V_STRIDE + lane * 8]) = vraw;
+                if (li == pos0 - key0) {
+#pragma unroll
+                    for (int kk = 0; kk < QK_STEPS; ++kk) own_kf.v[kk] = new_k[wave][kk * 4 + kb];
+                }
             }
         }
         __builtin_amdgcn_wave_barrier();
@@ -762,7 +790,7 @@ paged_attn_mfma_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k_po
             f32x4_t s = (f32x4_t){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int kk = 0; kk < QK_STEPS; ++kk)
-                s = qk_mfma(k_ok ? kf.v[kk] : make_uint4(0u, 0u, 0u, 0u), qf[rt][kk], s);
+                s = qk_mfma(k_ok ? own_kf.v[kk] : make_uint4(0u, 0u, 0u, 0u), qf[rt][kk], s);
             const int last_seen = min(row_pos[rt], hi - 1), first_key_seen = max(row_first[rt], lo_seen);
             float sv[4];
             float mx = -INFINITY;                           // of the raw scores: the scale is positive
@@ -807,12 +835,13 @@ paged_attn_mfma_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k_po
     };
     auto weighted = [&](const s16x4_t (&pf)[RT], const float (&alpha)[RT], bool any_rescale) {
         if (__any(any_rescale)) rescale_in_place(o, alpha);
-        // O^T += V^T P^T, one 16-wide block of d at a time; the V^T slice is shared by the row tiles
+        // O^T += V^T P^T, one 16-wide block of d at a time; the V^T slice is shared by the row tiles.
+        // A transposed read: 16 lanes name the 8-byte pieces of a block of 4 keys x 16 elements
+        // and each receives one element of the 4 keys (against four 2-byte reads a slice).
+        const uint16_t* vsrc = &vl[(4 * kb + li / 4) * V_STRIDE + (li % 4) * 4];
 #pragma unroll
         for (int j = 0; j < DV; ++j) {
-            const uint16_t* src = &vl[(4 * kb) * V_STRIDE + j * 16 + li];
-            const s16x4_t vt = (s16x4_t){(short)src[0], (short)src[V_STRIDE], (short)src[2 * V_STRIDE],
-                                         (short)src[3 * V_STRIDE]};
+            const s16x4_t vt = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)(vsrc + j * 16));
 #pragma unroll
             for (int rt = 0; rt < RT; ++rt)
                 o[rt][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(vt, pf[rt], o[rt][j], 0, 0, 0);
@@ -820,10 +849,12 @@ paged_attn_mfma_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k_po
         __builtin_amdgcn_wave_barrier();
     };
     // whole: every key of the tile lies in the split, at or before the block's first position
-    // and inside the window of its last one, so no score needs a mask
+    // and inside the window of its last one, so no score needs a mask, and it is not the one
+    // whose own key has to be filled in
+    const int last_whole = own_key ? pos0 - 1 : pos0;
     const int last_first = first_seen(pos0 + ntok - 1, window);
     auto tile = [&](int key0, const KFrag& kf, const uint4 (&vr)[V_PER_LANE]) {
-        const bool whole = key0 >= split_lo && key0 + 15 < khi && key0 + 15 <= pos0 &&
+        const bool whole = key0 >= split_lo && key0 + 15 < khi && key0 + 15 <= last_whole &&
                            key0 >= last_first;
         s16x4_t pf[RT];
         float alpha[RT];
@@ -837,24 +868,6 @@ paged_attn_mfma_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k_po
         weighted(pf, alpha, any_rescale);
     };
 
-    if constexpr (FUSED) {
-        if (own_key && covers) {
-            // the token's own key and value, from where the prologue left them: one more tile
-            // whose first key is the only one there, first of all, while the others' keys and
-            // values are on their way
-            KFrag kfn;
-            uint4 vrn[V_PER_LANE];
-#pragma unroll
-            for (int kk = 0; kk < QK_STEPS; ++kk) kfn.v[kk] = new_kv[wave][kk * 4 + kb];
-#pragma unroll
-            for (int j = 0; j < V_PER_LANE; ++j) vrn[j] = new_kv[wave][D / 8 + (lane + 64 * j) % (D / 8)];
-            s16x4_t pf[RT];
-            float alpha[RT];
-            bool any_rescale;
-            scores(pos0, kfn, vrn, std::true_type{}, pf, alpha, any_rescale, pos0, pos0 + 1, pos0);
-            weighted(pf, alpha, any_rescale);
-        }
-    }
     int key0 = klo;
     for (; key0 + 80 < khi; key0 += 48) {
         tile(key0, kf0, vr0);

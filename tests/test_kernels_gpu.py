@@ -735,6 +735,31 @@ def test_decode_attention_from_raw_qkv(kernel_sets, Hq, Hkv, D, bs, norm, rope):
     assert hip.decode_attention(qkv[:, :(Hq + 2 * Hkv) * 32], Hq, Hkv, 32, None, None, 1e-6, table32, slot_a, ctx, 0.2) is None
 
 
+@pytest.mark.parametrize("G", [3, 8, 15, 17])
+def test_decode_attention_makes_the_key_beside_the_queries(kernel_sets, G):
+    """The new key at every place of its tile, made in a spare column of the row tile (after 3 heads padded to 4, 8
+    heads, ...) or in a pass of its own (16 padded heads, two chunks of them), against the kernels one after the other."""
+    hip, _ = kernel_sets[torch.bfloat16]
+    Hkv, D, bs = 2, 64, 16
+    Hq = G * Hkv
+    lens = [n + 1 for n in range(40)] + [1000]
+    rows, pos = list(range(len(lens))), [n - 1 for n in lens]
+    gains = [(1 + 0.3 * torch.randn(D)).to(DEV) for _ in range(2)]
+    inv_freq = (1.0 / (10000.0 ** (torch.arange(0, D, 2).float() / D))).to(DEV)
+    table = hip.rope_table(inv_freq, 0, 1000)
+    qkv = rnd((len(lens), (Hq + 2 * Hkv) * D), torch.bfloat16, 64, 1.5)
+    ctx = ctx_for(rows, pos)
+    slots = [make_paged_case(lens, Hq, Hkv, D, bs, torch.bfloat16, seed=D + G)[0] for _ in range(2)]
+    hip.fuse_rope = False
+    q = hip.qk_norm_rope_write(qkv, Hq, Hkv, D, *gains, 1e-6, inv_freq, D, ctx.positions, ctx.token_rows, slots[0])
+    want = hip.paged_attention(q, slots[0], ctx, 0.2, None)
+    hip.fuse_rope = True
+    got = hip.decode_attention(qkv, Hq, Hkv, D, *gains, 1e-6, table, slots[1], ctx, 0.2, None, True)
+    close(got, want, torch.bfloat16)
+    assert torch.equal(slots[1].v, slots[0].v)
+    torch.testing.assert_close(slots[1].k.float(), slots[0].k.float(), atol=2e-2, rtol=1e-2)
+
+
 def plain_norm_rotate(x, gain, eps, positions, inv_freq):
     """Per-head RMSNorm (x / sqrt(mean(x^2) + eps) * gain) and the rotate-half rotation of
     x [N, H, D] in float32 on the CPU, rounded to bfloat16 once as a kernel's output is."""
