@@ -212,3 +212,29 @@ def test_head_project(kernel_sets, dtype, N, H, ldx, K, n_out):
     hip, ref = kernel_sets[dtype]
     x, w = rnd((N, H, ldx), dtype, 1), rnd((H, n_out, K), dtype, 2, 0.2)
     close(hip.head_project(x, w), ref.head_project(x, w), dtype, atol=5e-5 if dtype == torch.float32 else 3e-2)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("taps", [2, 3, 4])
+def test_causal_conv_silu_in_whole_chunks(kernel_sets, dtype, taps):
+    """Steps long enough for chunks of 32 tokens loaded whole: sequences that end on both sides of a chunk's edge,
+    or bring fewer tokens than the taps reach back."""
+    hip, ref = kernel_sets[dtype]
+    lengths = [1, 2, 3, 15, 31, 32, 33, 63, 64, 65, 70]
+    ctx, C, col = step_of(lengths, list(range(len(lengths)))), 300, 17
+    x = rnd((ctx.n_tokens, C + 40), dtype, 1)
+    w, b = rnd((C, taps), torch.float32, 2), rnd((C,), torch.float32, 3)
+    s1 = rnd((len(lengths), 5 + (taps - 1) * C), torch.float32, 4).to(dtype).float()
+    s2 = s1.clone()
+    close(hip.causal_conv_silu(x, col, C, w, b, s1, 5, ctx), ref.causal_conv_silu(x, col, C, w, b, s2, 5, ctx), dtype)
+    torch.testing.assert_close(s1, s2, atol=0, rtol=0)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("N,C", [(2040, 200), (2041, 200), (2047, 257), (1023, 257), (1018, 600)])
+def test_wkv_decay_eight_tokens_to_a_workgroup(kernel_sets, dtype, N, C):
+    """Around the number of workgroups from which eight tokens share one, with a last group that is not full. The
+    bound is the smaller test's: sums of 24 products in the same order."""
+    hip, ref = kernel_sets[dtype]
+    t, w2, w0 = rnd((N, 24), torch.float32, 1), rnd((24, C), dtype, 2, 0.3), rnd((C,), torch.float32, 3)
+    torch.testing.assert_close(hip.wkv_decay(t, w2, w0), ref.wkv_decay(t, w2, w0), atol=1e-5, rtol=1e-4)
