@@ -60,3 +60,26 @@ def test_which_tiles(ops):
     assert ops._expert_tile(x, 4000, 4, 128, 72, w) == 128 and ops._expert_tile(x, 4000, 4, 128, 66, w) == 16
     shifted = torch.empty(w.numel() + 1, dtype=w.dtype, device=DEV)[1:].view_as(w)
     assert ops._expert_tile(x, 4000, 4, 128, 64, shifted) == 128
+
+
+@pytest.mark.parametrize("top", [1, 2, 4, 8])
+@pytest.mark.parametrize("N,d", [(1, 4), (3, 1020), (5, 1024), (7, 1028), (2, 2562), (300, 2560)])
+@pytest.mark.parametrize("extra,skip", [(False, False), (True, False), (True, True)])
+def test_weighted_sums_of_experts(ops, top, N, d, extra, skip):
+    """Rows of whole and broken runs of four, one workgroup and several, with a shared expert behind a gate, and with
+    pairs that stand for the token itself. ``top`` + 1 roundings of float32 at sums of the sizes are the bound."""
+    from types import SimpleNamespace
+    g = torch.Generator().manual_seed(d + top)
+    place = torch.randperm(N * top, generator=g).int()
+    if skip:
+        place[::3] = -1
+    y, weight = torch.randn((N * top, d), generator=g), torch.rand((N, top), generator=g)
+    own, shared, gate = rnd((N, d), 5), rnd((N, d), 6), torch.randn((N, 3), generator=g)
+    got = ops.moe_combine(y.to(DEV), SimpleNamespace(place=place.to(DEV)), weight.to(DEV), shared if extra else None,
+                          gate.to(DEV)[:, 1] if extra else None, own if skip else None).double().cpu()
+    rows = torch.where(place[:, None] >= 0, y[place.clamp(min=0).long()].double(), own.cpu().double().repeat_interleave(top, 0))
+    terms = weight.double()[:, :, None] * rows.view(N, top, d)
+    if extra:
+        terms = torch.cat([terms, (gate[:, 1].double().sigmoid()[:, None] * shared.cpu().double())[:, None]], 1)
+    # (the gate's sigmoid in float32: a few roundings of it)
+    assert ((got - terms.sum(1)).abs() <= (top + 6) * 2.0 ** -24 * terms.abs().sum(1) + 1e-30).all()

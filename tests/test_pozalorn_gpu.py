@@ -485,3 +485,16 @@ def test_trace_runner_on_a_model_folder(tmp_path, folders):
             if rows:
                 got = torch.from_numpy(np.fromfile(out / f"{n}.f32", dtype="<f4").reshape(rows, cfg["vocab"]).copy())
                 compare(got, torch.cat([want[i][pos] for i, pos in here]), TOL[dtype], f"step {n} {dtype}")
+
+
+@pytest.mark.parametrize("dtype", list(DTYPES))
+@pytest.mark.parametrize("N,ff,ld", [(1, 8, 16), (3, 2056, 4112), (70, 72, 160), (5, 72, 150), (5, 76, 152)])
+def test_gelu_gate_in_runs_of_eight(kernel_sets, dtype, N, ff, ld):
+    """Rows in steps of eight elements and rows that are not, one workgroup and several, against float64."""
+    ops, dt = kernel_sets[dtype], DTYPES[dtype]
+    x = torch.randn((N, ld), generator=torch.Generator().manual_seed(ff)).to(dt).to(DEV)
+    g, u = x[:, :ff].double(), x[:, ff:2 * ff].double()
+    want = torch.nn.functional.gelu(g, approximate="tanh") * u
+    # 1 + tanh loses the low bits where tanh is near -1: steps of 2^-24 of g u, a few of them
+    slack = 8 * 2.0 ** -24 * (g * u).abs() + (2.0 ** -8 if dt == torch.bfloat16 else 0.0) * want.abs()
+    assert ((ops.glu_gelu(x, ff).double() - want).abs() <= slack + 1e-30).all()
