@@ -52,7 +52,7 @@ class Delta:
             c_float(q_scale), c_float(unit_eps), _ptr(z), _ptr(a_log), _ptr(dt_bias), _ptr(state), stride, c_int(conv_offset),
             _ptr(ctx.seq_qstart), _ptr(ctx.seq_rows), _ptr(qk), _ptr(v), _ptr(gates), c_int(ctx.n_seqs),
             c_int(max(1, ctx.max_q_len)), c_int(self.code), self._stream()), "delta_prepare")
-        if self._in_chunks(ctx, D, self.delta_scan_from):
+        if self._delta_in_chunks(ctx, N, D, H, Dv):
             return self._delta_scan(qk, v, gates, G, H, D, Dv, Dp, state, stride, offset, ctx, N, out)
         _check(lib.soc_delta_walk(
             _ptr(qk), _ptr(v), _ptr(gates), c_int(G), c_int(H), c_int(D), c_int(Dv), c_int(Dp), _ptr(state), stride, c_int(offset),

@@ -24,7 +24,8 @@ class Scan:
     # Tokens of a step's longest portion from which it is taken in chunks (0: never). Measured in us, walk -> chunks, at
     # the heads of a 4B-sized layer: 64 tokens: retention 34 -> 42, gated linear attention 34 -> 57, wkv 30 -> 48,
     # ssd 33 -> 32; 100 tokens: 46 -> 40, 48 -> 58, 39 -> 45, 48 -> 33; 300: 149 -> 60, 162 -> 72, 85 -> 44, 175 -> 63.
-    # The gated delta rule, whose chunk costs more and whose walk is faster: 200 tokens 62 -> 73, 300: 89 -> 75.
+    # The gated delta rule, whose chunk costs more and whose walk is faster: 200 tokens 62 -> 73, 256: 76 -> 68, 300: 89 -> 75.
+    # (For the others chunks stay ahead with several sequences: 5 of 200 tokens: 122 -> 77, 137 -> 80, 144 -> 71, 248 -> 117.)
     scan_from, delta_scan_from = 128, 256
     scan_scratch = 1 << 30           # bytes of scratch that one launch over all chunks may take; beyond, in rounds
 
@@ -40,6 +41,14 @@ class Scan:
         short portions walk: a chunk costs the same however few of its tokens there are) and a state whose
         queries, keys and decays of a chunk fit LDS. ``least``: tokens, in place of ``scan_from``."""
         return 0 < (self.scan_from if least is None else least) <= ctx.max_q_len and D <= 128
+
+    def _delta_in_chunks(self, ctx, N, D, H, Dv):
+        """Whether a step's gated delta rules run in chunks. The walk takes sequences side by side, its time goes with the
+        longest of them until their columns (16 to a workgroup) fill the chip; a chunk fills it alone, its time goes with
+        all tokens, behind a start worth 165 tokens of the walk. Measured in us, walk -> chunks, 20 heads of 128 x 128:
+        2 sequences of 300 tokens 96 -> 82, of 500 146 -> 128, of 1,000 271 -> 197; 3 of 300 101 -> 130, of 500
+        151 -> 151, of 1,000 280 -> 270; 5 of 300 139 -> 147, of 1,000 404 -> 455; 8 of 1,000 568 -> 682."""
+        return self._in_chunks(ctx, D, self.delta_scan_from) and N * H * -(-Dv // 16) < 600 * (ctx.max_q_len - 165)
 
     def _scan_scratch(self, ctx, N, sizes):
         """(chunks of the longest portion, chunks of every sequence that one launch takes, whether those lie one behind the

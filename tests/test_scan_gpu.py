@@ -226,4 +226,7 @@ def test_from_which_portion_on(kernel_sets):
     ops = kernel_sets["float32"]
     assert [ops._in_chunks(SimpleNamespace(max_q_len=n), D) for n, D in ((1, 64), (127, 64), (128, 64), (4000, 128), (4000, 129))] == [
         False, False, True, True, False]
-    assert [ops._in_chunks(SimpleNamespace(max_q_len=n), 64, ops.delta_scan_from) for n in (255, 256)] == [False, True]
+    delta = lambda lengths, D=128: ops._delta_in_chunks(SimpleNamespace(max_q_len=max(lengths)), sum(lengths), D, 20, 128)
+    assert [delta([n]) for n in (1, 255, 256, 3000)] == [False, False, True, True] and not delta([3000], 129)
+    assert [delta([n] * 2) for n in (256, 500, 1000)] == [False, True, True]             # side by side the walks cost little more
+    assert not delta([500] * 3) and delta([1000] * 3) and not delta([1000] * 5) and delta([2000] + [1] * 20)
