@@ -161,7 +161,7 @@ class Mixers:
         self._want(gain, "gain", torch.float32, (C,))
         stride = self._state(state, offset, H * D * D, ctx)
         raw = torch.empty((N, C), dtype=torch.float32, device=self.device)
-        if self._in_chunks(ctx, D):
+        if self._in_chunks(ctx, D, self.scan_from * 8 // 5):
             self._scan(BONUS, _ptr(r), C, D, _ptr(k), C, D, _ptr(v), C, D, _ptr(decay), H, D, D, state, stride, offset, ctx, N, raw,
                        q_f32=False, lda=C, params=[_ptr(bonus)])
             return self.gated_group_norm(raw, g, gain, H, eps, gate_first=False)
@@ -202,7 +202,7 @@ class Mixers:
             raise KernelError(f"ssd: {H} heads in {G} groups, state {Ns}, head size {P}")
         stride = self._state(state, offset, H * Ns * P, ctx)
         out = torch.empty((N, H * P), dtype=torch.float32, device=self.device)
-        if self._in_chunks(ctx, Ns):
+        if self._in_chunks(ctx, Ns, self.scan_from * 8 // 5):
             ld, item = H * P + 2 * G * Ns, xbc.element_size()
             b, c = (c_void_p(xbc.data_ptr() + (H * P + i * G * Ns) * item) for i in range(2))
             return self._scan(STEP, c, ld, Ns, b, ld, Ns, _ptr(xbc), ld, P, _ptr(dt), H, Ns, P, state, stride, offset, ctx, N, out,

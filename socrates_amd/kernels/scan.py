@@ -4,7 +4,7 @@ first asks for it."""
 
 from __future__ import annotations
 
-from ctypes import c_int, c_longlong
+from ctypes import c_int, c_longlong, c_void_p
 
 import torch
 
@@ -26,7 +26,11 @@ class Scan:
     # ssd 33 -> 32; 100 tokens: 46 -> 40, 48 -> 58, 39 -> 45, 48 -> 33; 300: 149 -> 60, 162 -> 72, 85 -> 44, 175 -> 63.
     # The gated delta rule, whose chunk costs more and whose walk is faster: 200 tokens 62 -> 73, 256: 76 -> 68, 300: 89 -> 75.
     # (For the others chunks stay ahead with several sequences: 5 of 200 tokens: 122 -> 77, 137 -> 80, 144 -> 71, 248 -> 117.)
-    scan_from, delta_scan_from = 128, 256
+    # A step of so few tokens is bound by the host's launches, of which chunks have two more per layer, so the line lies
+    # where whole steps gain (us, walk -> chunks, one prompt unless two are named): linear attention, 8 layers, 140 tokens
+    # 2,290 -> 2,360, 2 x 162 2,700 -> 2,470, 200 2,680 -> 2,390; retention, 6 layers, 140 3,140 -> 3,080; wkv and ssd, 6
+    # layers, 2 x 162 2,230 -> 2,310, 200 2,190 -> 2,260, 300 2,360 -> 2,290, 500 2,990 -> 2,370: from 8 / 5 as many.
+    scan_from, delta_scan_from = 160, 256
     scan_scratch = 1 << 30           # bytes of scratch that one launch over all chunks may take; beyond, in rounds
 
     def _scan_lib(self):
@@ -52,7 +56,7 @@ class Scan:
 
     def _scan_scratch(self, ctx, N, sizes):
         """(chunks of the longest portion, chunks of every sequence that one launch takes, whether those lie one behind the
-        other, scratch of ``sizes`` floats per chunk slot): all chunks at once where the scratch allows it, else rounds
+        other, the scratch of ``sizes`` floats per chunk slot, the addresses of its parts): all chunks at once where the scratch allows it, else rounds
         over a few chunks of every sequence with the state in the row between them."""
         chunks, per_slot = -(-ctx.max_q_len // CHUNK), 4 * sum(sizes)
         slots, count = N // CHUNK + ctx.n_seqs, chunks
@@ -60,8 +64,14 @@ class Scan:
         if not compact:
             count = max(1, min(chunks, self.scan_scratch // (ctx.n_seqs * per_slot)))
             slots = ctx.n_seqs * count
-        # (each starts on 16 bytes)
-        return chunks, count, compact, [torch.empty(slots * n, dtype=torch.float32, device=self.device) for n in sizes]
+        # one allocation, each part on 16 bytes
+        at, ends = 0, []
+        for n in sizes:
+            ends.append(at)
+            at += (slots * n + 3) & ~3
+        scratch = torch.empty(at, dtype=torch.float32, device=self.device)
+        base = scratch.data_ptr()
+        return chunks, count, compact, scratch, [c_void_p(base + 4 * e) for e in ends]
 
     def _scan(self, mode, q, ldq, hq, k, ldk, hk, v, ldv, hv, decay, H, D, Dv, state, stride, offset, ctx, N, out, group=1, q_f32=True,
               v_act=False, ones=0, lda=0, params=()):
@@ -69,7 +79,7 @@ class Scan:
         the next, h* from one head to the next."""
         dk = 64 if D <= 64 else 128
         rows = CHUNK * dk if mode in (CHANNEL, BONUS) else CHUNK
-        chunks, count, compact, (adds, queries, factors) = self._scan_scratch(ctx, N, [H * _tiles(D, Dv), H * rows, H * dk])
+        chunks, count, compact, scratch, parts = self._scan_scratch(ctx, N, [H * _tiles(D, Dv), H * rows, H * dk])
         p = list(params) + [None] * (3 - len(params))
         self.forms["scan"] += 1
         for first in range(0, chunks, count):
@@ -78,16 +88,16 @@ class Scan:
                 v, c_longlong(ldv), c_int(hv), c_int(1 if v_act else 0), c_int(ones), decay, c_longlong(lda), *p, c_int(H), c_int(D),
                 c_int(Dv), _ptr(state), stride, c_int(offset), _ptr(ctx.seq_qstart), _ptr(ctx.seq_rows), c_int(ctx.n_seqs),
                 c_int(first), c_int(count), c_int(1 if compact else 0), _ptr(out),
-                _ptr(adds), _ptr(queries), _ptr(factors), c_int(self.code), self._stream()), "scan")
+                *parts, c_int(self.code), self._stream()), "scan")
         return out
 
     def _delta_scan(self, qk, v, gates, G, H, D, Dv, Dp, state, stride, offset, ctx, N, out):
         """The gated delta rule in chunks, from what ``soc_delta_prepare`` leaves."""
-        chunks, count, compact, (adds, queries, moves) = self._scan_scratch(ctx, N, [H * _tiles(D, Dv), H * CHUNK * Dp, H * Dp * Dp])
+        chunks, count, compact, scratch, parts = self._scan_scratch(ctx, N, [H * _tiles(D, Dv), H * CHUNK * Dp, H * Dp * Dp])
         self.forms["scan"] += 1
         for first in range(0, chunks, count):
             _check(self._scan_lib().soc_delta_scan(
                 _ptr(qk), _ptr(v), _ptr(gates), c_int(G), c_int(H), c_int(D), c_int(Dv), c_int(Dp), _ptr(state), stride, c_int(offset),
                 _ptr(ctx.seq_qstart), _ptr(ctx.seq_rows), c_int(ctx.n_seqs), c_int(first), c_int(count), c_int(1 if compact else 0),
-                _ptr(out), _ptr(adds), _ptr(queries), _ptr(moves), c_int(self.code), self._stream()), "delta_scan")
+                _ptr(out), *parts, c_int(self.code), self._stream()), "delta_scan")
         return out

@@ -224,7 +224,7 @@ def test_delta_rule_in_chunks(kernel_sets, dtype, lengths, G, H, D, Dv, alike):
 
 def test_from_which_portion_on(kernel_sets):
     ops = kernel_sets["float32"]
-    assert [ops._in_chunks(SimpleNamespace(max_q_len=n), D) for n, D in ((1, 64), (127, 64), (128, 64), (4000, 128), (4000, 129))] == [
+    assert [ops._in_chunks(SimpleNamespace(max_q_len=n), D) for n, D in ((1, 64), (159, 64), (160, 64), (4000, 128), (4000, 129))] == [
         False, False, True, True, False]
     delta = lambda lengths, D=128: ops._delta_in_chunks(SimpleNamespace(max_q_len=max(lengths)), sum(lengths), D, 20, 128)
     assert [delta([n]) for n in (1, 255, 256, 3000)] == [False, False, True, True] and not delta([3000], 129)
