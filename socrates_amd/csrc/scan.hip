@@ -12,19 +12,29 @@
 // logarithm taken, so a decay of 0, or a product that underflows, gives what the walk gives. The decay is one number
 // per head, one per token and head, or one per token, head and key channel.
 //
+// No further off float64 than the walk: products of decays are formed in float64 and rounded once (a head's decay is the same
+// in every chunk, and so would its rounding be: its whole chunk's goes to scan_states in two parts), contractions are summed
+// in blocks, and the scores of the delta rule, whose chunk inverts a matrix of them, are float64 matrix instructions. Error of
+// results / states against the walk's, 2,048 tokens, 1e-7: retention 1.5 / 1.2 against 3.0 / 2.9, linear attention with
+// activations 1.1 / 0.9 against 1.6 / 3.0, with a decay per channel 11 / 15 against 12 / 15, wkv 1.4 / 1.1 against 2.5 / 2.5,
+// ssd 1.4 / 1.7 against 1.6 / 1.8, delta rule 0.8 to 4 / 0.7 to 7 against 0.8 to 9 / 0.6 to 16 (unlike to nearly repeating
+// keys). With one chain per sum and float32 throughout it was 11 / 11 for retention, 15 / 16 with activations, 1.9 to 10 / 2
+// to 14 for the delta rule, 2 to 9 times the walk's; the difference costs up to 5 % of the time.
+//
 // Bound by memory: per chunk and head the addend (D x Dv float32) is written, read, written as a state and read
 // again, the outputs written, read and written. 64 tokens: with 32 the addends weigh twice as much, with 128 a
 // chunk's queries, keys and decays of 128 channels do not fit LDS.
 //
 // Measured for 2,048 tokens of one prompt, us, the walk -> these kernels with what prepares them: retention (20 heads of
-// 128 x 128) 908 -> 108 (chunks 46, states 18, apply 31), gated linear attention (10 of 128 x 256) 1,030 -> 131 (67, 18, 29),
-// wkv (40 of 64 x 64) 595 -> 100 with its norm (53, 10, 16), ssd (80 of 128 x 64) 1,166 -> 168 (97, 24, 54); the gated
-// delta rule (20 of 128 x 128), 3,000 tokens, 700 -> 290 with its convolutions (127, states 93, 37). scan_chunks is
+// 128 x 128) 908 -> 109 (chunks 47, states 17, apply 30), gated linear attention (10 of 128 x 256) 1,030 -> 130 (66, 17, 28),
+// wkv (40 of 64 x 64) 595 -> 99 with its norm (52, 10, 17), ssd (80 of 128 x 64) 1,166 -> 168 (91, 22, 56); the gated
+// delta rule (20 of 128 x 128), 3,000 tokens, 700 -> 284 with its convolutions (2,048 tokens: chunks 104, states 65, apply 28). scan_chunks is
 // bound by its reads of LDS, a 4-byte read per operand and product where an operand lies across the tokens.
 #include "common.h"
 #include "recurrent.h"          // lds_barrier: loads and stores on their way are not waited for
 
 typedef __attribute__((ext_vector_type(4))) float f32x4;
+typedef __attribute__((ext_vector_type(4))) double f64x4;
 
 constexpr int SCAN_C = 64;                 // tokens of a chunk
 constexpr int SCAN_AS = SCAN_C + 4;        // floats from one row of scores to the next in LDS
@@ -91,6 +101,12 @@ __device__ __forceinline__ f32x4 mfma4(float a0, float a1, float a2, float a3, f
     c = __builtin_amdgcn_mfma_f32_16x16x4f32(a2, b.z, c, 0, 0, 0);
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a3, b.w, c, 0, 0, 0);
 }
+// f(I0) + .. + f(I0 + N - 1), pairwise: blocks of 16 of a contraction have sums of their own, because one chain of 64 or 128
+// additions into the same float32 sum is off by several times what the walk's short ones are.
+template <int N, int I0 = 0, typename F> __device__ __forceinline__ f32x4 sum_pairs(F f) {
+    if constexpr (N == 1) return f(I0);
+    else return sum_pairs<N / 2, I0>(f) + sum_pairs<N - N / 2, I0 + N / 2>(f);
+}
 // sum over k of 16 of col[k][m] row[n][k]: col points at [4 g][m of the lane] with ld floats between the k, row at [n of the lane][4 g]
 __device__ __forceinline__ f32x4 mfma_col_row(const float* col, int ld, const float* row, f32x4 c) {
     return mfma4(col[0], col[ld], col[2 * ld], col[3 * ld], *reinterpret_cast<const float4*>(row), c);
@@ -107,7 +123,7 @@ __device__ __forceinline__ void scan_values(float* __restrict__ out, int H, int 
         const int I = wave / 2, p = wave % 2;
         f32x4 o = {0.f, 0.f, 0.f, 0.f};
         for (int s = 0; s <= I; ++s)
-            o = mfma_col_row(Vs + (16 * s + 4 * g) * SCAN_VS + p * 16 + r, SCAN_VS, X + (I * 16 + r) * SCAN_AS + 16 * s + 4 * g, o);
+            o += mfma_col_row(Vs + (16 * s + 4 * g) * SCAN_VS + p * 16 + r, SCAN_VS, X + (I * 16 + r) * SCAN_AS + 16 * s + 4 * g, (f32x4){0.f, 0.f, 0.f, 0.f});
         const int t = I * 16 + r, col = col0 + p * 16 + 4 * g;
         if (t < nt) {
             float* to = out + ((size_t)(lo + t) * H + head) * Dv + col;
@@ -119,9 +135,11 @@ __device__ __forceinline__ void scan_values(float* __restrict__ out, int H, int 
         }
     }
     const int ct = wave / PER, p0 = wave % PER;      // 16 channels by both tiles of columns, or by one
-    f32x4 s[TILES];
+    f32x4 s[TILES][4];                               // (each sum from the first token on: under decays the terms grow along it)
 #pragma unroll
-    for (int p = 0; p < TILES; ++p) s[p] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    for (int p = 0; p < TILES; ++p)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[p][e] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int m = 0; m < SCAN_C; m += 16)
 #pragma unroll
@@ -129,12 +147,14 @@ __device__ __forceinline__ void scan_values(float* __restrict__ out, int H, int 
             const int t = m + 4 * g + e;
             const float x = Z[t * LS + ct * 16 + r];
 #pragma unroll
-            for (int p = 0; p < TILES; ++p) s[p] = __builtin_amdgcn_mfma_f32_16x16x4f32(x, Vs[t * SCAN_VS + scan_col(p0 + p, r)], s[p], 0, 0, 0);
+            for (int p = 0; p < TILES; ++p) s[p][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(x, Vs[t * SCAN_VS + scan_col(p0 + p, r)], s[p][e], 0, 0, 0);
         }
     if (ct < ch_tiles) {
 #pragma unroll
-        for (int p = 0; p < TILES; ++p)
-            *reinterpret_cast<float4*>(adds + ((size_t)(ct * tiles + col0 / 16 + p0 + p) * 64 + 16 * g + r) * 4) = make_float4(s[p][0], s[p][1], s[p][2], s[p][3]);
+        for (int p = 0; p < TILES; ++p) {
+            const f32x4 y = (s[p][0] + s[p][1]) + (s[p][2] + s[p][3]);
+            *reinterpret_cast<float4*>(adds + ((size_t)(ct * tiles + col0 / 16 + p0 + p) * 64 + 16 * g + r) * 4) = make_float4(y[0], y[1], y[2], y[3]);
+        }
     }
 }
 
@@ -151,6 +171,7 @@ scan_chunks_kernel(ScanArgs a) {
     __shared__ __align__(16) float dg[CH ? NW / 4 : 1][4][16][16];   // decays (CH: scores) inside a run of 16 tokens
     __shared__ __align__(16) float tot[4][CH ? DK : 1];              // a run's whole decay
     __shared__ float sa[SCAN_C], sdt[SCAN_C], pin[SCAN_C], sfx[SCAN_C];
+    __shared__ double run_decay[4];
     float* As = Qs;
     float* Vs = V_IN_Q ? Qs + SCAN_C * SCAN_AS : Vx;
 
@@ -212,18 +233,18 @@ scan_chunks_kernel(ScanArgs a) {
     if constexpr (!CH) {
         if (tid < SCAN_C) {                          // down a column of its run: decay from behind token j to token i
             const int I = tid / 16, j = tid % 16;
-            float p = sdt[tid];
+            double p = sdt[tid];
             for (int i = 0; i < 16; ++i) {
                 if (i > j) p *= sa[I * 16 + i];
-                dg[0][I][i][j] = i >= j ? p : 0.f;
+                dg[0][I][i][j] = i >= j ? (float)p : 0.f;
             }
-            sfx[tid] = p;
+            sfx[tid] = (float)p;
         } else if (tid < 2 * SCAN_C) {
             const int i = tid - SCAN_C, I = i / 16;
-            float p = 1.f;
+            double p = 1.0;
             for (int t = I * 16; t <= i; ++t) p *= sa[t];
-            pin[i] = p;
-            if (i % 16 == 15) tot[I][0] = p;
+            pin[i] = (float)p;
+            if (i % 16 == 15) { tot[I][0] = (float)p; run_decay[I] = p; }
         }
     } else {
         // inside a run pair by pair: wave (run, share of the channels), lane (query r, a quarter of the share)
@@ -263,19 +284,19 @@ scan_chunks_kernel(ScanArgs a) {
         // queries decayed back to their run's start, keys to its end, in place
         for (int e = tid; e < 4 * DK; e += NT) {
             const int run = e / DK, ch = e % DK;
-            float p = 1.f;
+            double p = 1.0;
 #pragma unroll
             for (int t = 0; t < 16; ++t) {
                 const int at = (run * 16 + t) * LS + ch;
-                if (MODE == SCAN_BONUS) { Qs[at] *= p; p *= Ds[at]; }
-                else { p *= Ds[at]; Qs[at] *= p; }
+                if (MODE == SCAN_BONUS) { Qs[at] = (float)(Qs[at] * p); p *= Ds[at]; }
+                else { p *= Ds[at]; Qs[at] = (float)(Qs[at] * p); }
             }
-            tot[run][ch] = p;
-            p = 1.f;
+            tot[run][ch] = (float)p;
+            p = 1.0;
 #pragma unroll
             for (int t = 15; t >= 0; --t) {
                 const int at = (run * 16 + t) * LS + ch;
-                Ks[at] *= p;
+                Ks[at] = (float)(Ks[at] * p);
                 p *= Ds[at];
             }
         }
@@ -290,19 +311,20 @@ scan_chunks_kernel(ScanArgs a) {
         if (CH) { I = b < 1 ? 1 : b < 3 ? 2 : 3; J = b - I * (I - 1) / 2; }
         else { I = b < 1 ? 0 : b < 3 ? 1 : b < 6 ? 2 : 3; J = b - I * (I + 1) / 2; }
         bi[x] = I; bj[x] = J;
-        f32x4 s = {0.f, 0.f, 0.f, 0.f};
+        float4 between[CH ? DK / 16 : 1];            // the whole runs' decays
+        if constexpr (CH) {
 #pragma unroll
-        for (int m = 0; m < DK; m += 16) {
-            float4 qf = *reinterpret_cast<const float4*>(Qs + (I * 16 + r) * LS + m + 4 * g);
-            const float4 kf = *reinterpret_cast<const float4*>(Ks + (J * 16 + r) * LS + m + 4 * g);
-            if constexpr (CH)
-                for (int run = J + 1; run < I; ++run) qf = mul4(qf, *reinterpret_cast<const float4*>(&tot[run][m + 4 * g]));
-            s = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.x, qf.x, s, 0, 0, 0);
-            s = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.y, qf.y, s, 0, 0, 0);
-            s = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.z, qf.z, s, 0, 0, 0);
-            s = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.w, qf.w, s, 0, 0, 0);
+            for (int m = 0; m < DK / 16; ++m) between[m] = make_float4(1.f, 1.f, 1.f, 1.f);
+            for (int run = J + 1; run < I; ++run)
+#pragma unroll
+                for (int m = 0; m < DK / 16; ++m) between[m] = mul4(between[m], *reinterpret_cast<const float4*>(&tot[run][16 * m + 4 * g]));
         }
-        sc[x] = s;
+        sc[x] = sum_pairs<DK / 16>([&](int m) {
+            float4 qf = *reinterpret_cast<const float4*>(Qs + (I * 16 + r) * LS + 16 * m + 4 * g);
+            const float4 kf = *reinterpret_cast<const float4*>(Ks + (J * 16 + r) * LS + 16 * m + 4 * g);
+            if constexpr (CH) qf = mul4(qf, between[m]);
+            return mfma4(kf.x, kf.y, kf.z, kf.w, qf, (f32x4){0.f, 0.f, 0.f, 0.f});
+        });
     }
     if constexpr (!CH) lds_barrier();             // the factors of the runs
 
@@ -320,9 +342,12 @@ scan_chunks_kernel(ScanArgs a) {
         for (int run = 0; run < tid / 16; ++run) p *= tot[run][0];
         a.queries[slot * SCAN_C + tid] = p;
     }
-    if (tid < DK) {
-        const int ch = CH ? tid : 0;
-        a.factors[slot * DK + tid] = tot[0][ch] * tot[1][ch] * tot[2][ch] * tot[3][ch];
+    if constexpr (CH) {
+        if (tid < DK) a.factors[slot * DK + tid] = tot[0][tid] * tot[1][tid] * tot[2][tid] * tot[3][tid];
+    } else if (tid == 0) {                           // in two parts: a head's decay is the same in every chunk, and so is its rounding
+        const double whole = run_decay[0] * run_decay[1] * run_decay[2] * run_decay[3];
+        a.factors[slot * DK] = (float)whole;
+        a.factors[slot * DK + 1] = (float)(whole - (double)(float)whole);
     }
     lds_barrier();
 
@@ -399,6 +424,8 @@ scan_chunks_kernel(ScanArgs a) {
 
 // In place: every chunk's addend becomes the state before that chunk, and the row's state moves on to the end of the
 // last one. A thread owns a lane's four elements of a tile; the addends of eight chunks are on their way at a time.
+// CH: a factor per channel; else one for all, in two parts.
+template <bool CH>
 __global__ void __launch_bounds__(256)
 scan_states_kernel(ScanArgs a, int dk) {
     const int head = blockIdx.y, seq = blockIdx.z, tiles = scan_tiles(a.Dv);
@@ -411,27 +438,36 @@ scan_states_kernel(ScanArgs a, int dk) {
     float* S = a.state + (size_t)a.rows[seq] * a.stride + a.offset + (size_t)head * a.D * a.Dv + (size_t)ch * a.Dv + col;
     const size_t slot0 = scan_slot(a, seq, 0) * a.H + head;
     float4* add = reinterpret_cast<float4*>(a.adds) + slot0 * size + at;
-    const float* f = a.factors + slot0 * dk + ch;
+    const float* f = a.factors + slot0 * dk + (CH ? ch : 0);
     const size_t step = (size_t)a.H * size, fstep = (size_t)a.H * dk;
     float s[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) s[e] = col < a.Dv && ch + e < a.D ? S[(size_t)e * a.Dv] : 0.f;
     for (int c = 0; c < n; c += 8) {
-        float4 x[8], y[8];
+        float4 x[8], y[CH ? 8 : 1];
+        float2 one[CH ? 1 : 8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const int cc = min(c + i, n - 1);
             x[i] = add[cc * step];
-            y[i] = *reinterpret_cast<const float4*>(f + cc * fstep);
+            if constexpr (CH) y[i] = *reinterpret_cast<const float4*>(f + cc * fstep);
+            else one[i] = *reinterpret_cast<const float2*>(f + cc * fstep);
         }
 #pragma unroll
         for (int i = 0; i < 8; ++i)
             if (c + i < n) {
                 add[(c + i) * step] = make_float4(s[0], s[1], s[2], s[3]);
-                s[0] = fmaf(y[i].x, s[0], x[i].x);
-                s[1] = fmaf(y[i].y, s[1], x[i].y);
-                s[2] = fmaf(y[i].z, s[2], x[i].z);
-                s[3] = fmaf(y[i].w, s[3], x[i].w);
+                if constexpr (CH) {
+                    s[0] = fmaf(y[i].x, s[0], x[i].x);
+                    s[1] = fmaf(y[i].y, s[1], x[i].y);
+                    s[2] = fmaf(y[i].z, s[2], x[i].z);
+                    s[3] = fmaf(y[i].w, s[3], x[i].w);
+                } else {
+                    s[0] = fmaf(one[i].x, s[0], fmaf(one[i].y, s[0], x[i].x));
+                    s[1] = fmaf(one[i].x, s[1], fmaf(one[i].y, s[1], x[i].y));
+                    s[2] = fmaf(one[i].x, s[2], fmaf(one[i].y, s[2], x[i].z));
+                    s[3] = fmaf(one[i].x, s[3], fmaf(one[i].y, s[3], x[i].w));
+                }
             }
     }
 #pragma unroll
@@ -455,8 +491,8 @@ scan_apply_kernel(ScanArgs a) {
     const int lane = tid % 64, wave = tid / 64, r = lane % 16, g = lane / 16;
     const size_t slot = scan_slot(a, seq, c) * a.H + head;
     const int col0 = (blockIdx.x % blocks) * 32 * CG + (wave % CG) * 32, row0 = (wave / CG) * 16 * CG;
-    // two tiles of 16 columns; channels 16 s + 4 g .. + 3 in piece s (tiles beyond the last channel's, columns beyond the
-    // last tile's: read at a place that exists, not used)
+    // two tiles of 16 columns; channels 16 s + 4 g .. + 3 in piece s (tiles beyond the last channel's: the last one, whose
+    // queries are zeros; columns beyond the last tile's: read at a place that exists, not used)
     const int tiles = scan_tiles(a.Dv), ch_tiles = (a.D + 15) / 16;
     const float4* S = reinterpret_cast<const float4*>(a.adds) + (slot * ch_tiles * tiles + min(col0 / 16, tiles - 2)) * 64 + lane;
     float4 sx[DK / 16], sy[DK / 16];
@@ -478,35 +514,46 @@ scan_apply_kernel(ScanArgs a) {
         *reinterpret_cast<float4*>(Qs + t * LS + i) = x;
     }
     __syncthreads();
-    f32x4 x[CG], y[CG];
-#pragma unroll
-    for (int i = 0; i < CG; ++i) x[i] = y[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s = 0; s < DK / 16; ++s) {
-        if (s >= ch_tiles) break;
-#pragma unroll
-        for (int i = 0; i < CG; ++i) {
-            const float4 q = *reinterpret_cast<const float4*>(Qs + (row0 + i * 16 + r) * LS + 16 * s + 4 * g);
-            x[i] = mfma4(sx[s].x, sx[s].y, sx[s].z, sx[s].w, q, x[i]);
-            y[i] = mfma4(sy[s].x, sy[s].y, sy[s].z, sy[s].w, q, y[i]);
-        }
-    }
-    // a lane has columns col0 + 8 g .. + 7 of token row0 + 16 i + r
-#pragma unroll
+    // a lane has columns col0 + 8 g .. + 7 of token row0 + 16 i + r; a column's sum in parts (see sum_pairs) of 16 channels, or,
+    // where the queries come undecayed and the walk's error is twice as large, 32 (fewer registers: 30 against 35 us)
+    constexpr int HALF = CH ? 4 : DK / 16;
+#pragma unroll 1
     for (int i = 0; i < CG; ++i) {
+        f32x4 xs, ys;
+#pragma unroll
+        for (int s0 = 0; s0 < DK / 16; s0 += HALF) {
+            f32x4 x[4], y[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] = y[e] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int s = s0; s < s0 + HALF; ++s) {
+                const float4 q = *reinterpret_cast<const float4*>(Qs + (row0 + i * 16 + r) * LS + 16 * s + 4 * g);
+                x[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(sx[s].x, q.x, x[0], 0, 0, 0);
+                y[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(sy[s].x, q.x, y[0], 0, 0, 0);
+                x[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(sx[s].y, q.y, x[1], 0, 0, 0);
+                y[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(sy[s].y, q.y, y[1], 0, 0, 0);
+                x[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(sx[s].z, q.z, x[2], 0, 0, 0);
+                y[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(sy[s].z, q.z, y[2], 0, 0, 0);
+                x[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(sx[s].w, q.w, x[3], 0, 0, 0);
+                y[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(sy[s].w, q.w, y[3], 0, 0, 0);
+            }
+            const f32x4 xh = (x[0] + x[1]) + (x[2] + x[3]), yh = (y[0] + y[1]) + (y[2] + y[3]);
+            xs = s0 ? xs + xh : xh;
+            ys = s0 ? ys + yh : yh;
+        }
         const int t = row0 + i * 16 + r, col = col0 + 8 * g;
         if (t >= nt || col >= a.Dv) continue;
         float* p = a.out + ((size_t)(lo + t) * a.H + head) * a.Dv + col;
         if (a.Dv % 4 == 0 && col + 8 <= a.Dv) {
             float4 u = *reinterpret_cast<const float4*>(p), w = *reinterpret_cast<const float4*>(p + 4);
-            u.x += x[i][0]; u.y += x[i][1]; u.z += x[i][2]; u.w += x[i][3];
-            w.x += y[i][0]; w.y += y[i][1]; w.z += y[i][2]; w.w += y[i][3];
+            u.x += xs[0]; u.y += xs[1]; u.z += xs[2]; u.w += xs[3];
+            w.x += ys[0]; w.y += ys[1]; w.z += ys[2]; w.w += ys[3];
             *reinterpret_cast<float4*>(p) = u;
             *reinterpret_cast<float4*>(p + 4) = w;
         } else {
 #pragma unroll
             for (int e = 0; e < 8; ++e)
-                if (col + e < a.Dv) p[e] += e < 4 ? x[i][e] : y[i][e - 4];
+                if (col + e < a.Dv) p[e] += e < 4 ? xs[e] : ys[e - 4];
         }
     }
 }
@@ -515,8 +562,8 @@ template <int DK, int MODE, typename TQ, typename TV>
 static void launch_scan(const ScanArgs& a, int n_seqs, hipStream_t s) {
     hipLaunchKernelGGL((scan_chunks_kernel<DK, MODE, TQ, TV>), dim3(a.H, a.count, n_seqs), dim3(64 * scan_waves(DK, MODE >= SCAN_CHANNEL)), 0, s, a);
     const int pieces = (a.D + 15) / 16 * scan_tiles(a.Dv) * 64;
-    hipLaunchKernelGGL(scan_states_kernel, dim3((pieces + 255) / 256, a.H, n_seqs), dim3(256), 0, s, a, DK);
     constexpr bool CH = MODE >= SCAN_CHANNEL;
+    hipLaunchKernelGGL(scan_states_kernel<CH>, dim3((pieces + 255) / 256, a.H, n_seqs), dim3(256), 0, s, a, DK);
     if (a.Dv <= 32) hipLaunchKernelGGL((scan_apply_kernel<DK, 1, CH, TQ>), dim3(a.H, a.count, n_seqs), dim3(256), 0, s, a);
     else if (a.Dv <= 64) hipLaunchKernelGGL((scan_apply_kernel<DK, 2, CH, TQ>), dim3(a.H, a.count, n_seqs), dim3(256), 0, s, a);
     else hipLaunchKernelGGL((scan_apply_kernel<DK, 4, CH, TQ>), dim3(a.H * ((a.Dv + 127) / 128), a.count, n_seqs), dim3(256), 0, s, a);
@@ -586,7 +633,8 @@ delta_chunks_kernel(DeltaArgs a) {
     __shared__ __align__(16) float As[SCAN_C * SCAN_AS], Ms[SCAN_C * SCAN_AS], Ts[SCAN_C * SCAN_AS];     // Ms later X
     __shared__ __align__(16) float Vs[SCAN_C * SCAN_VS];
     __shared__ __align__(16) float dg[4][16][16];
-    __shared__ float sa[SCAN_C], sb[SCAN_C], pin[SCAN_C], sfx[SCAN_C], from[SCAN_C], rest[SCAN_C], tot[4];
+    __shared__ float sa[SCAN_C], sb[SCAN_C], from[SCAN_C], rest[SCAN_C];
+    __shared__ double pin[SCAN_C], sfx[SCAN_C], tot[4];
     const int head = blockIdx.x, c = blockIdx.y, seq = blockIdx.z, tid = threadIdx.x;
     const int lo = a.qstart[seq] + (a.first + c) * SCAN_C, hi = a.qstart[seq + 1];
     if (lo >= hi) return;
@@ -618,59 +666,62 @@ delta_chunks_kernel(DeltaArgs a) {
     __syncthreads();
     if (tid < SCAN_C) {
         const int I = tid / 16, j = tid % 16;
-        float p = 1.f;
+        double p = 1.0;
         for (int i = 0; i < 16; ++i) {
             if (i > j) p *= sa[I * 16 + i];
-            dg[I][i][j] = i >= j ? p : 0.f;
+            dg[I][i][j] = i >= j ? (float)p : 0.f;
         }
         sfx[tid] = p;
     } else if (tid < 2 * SCAN_C) {
         const int i = tid - SCAN_C, I = i / 16;
-        float p = 1.f;
+        double p = 1.0;
         for (int t = I * 16; t <= i; ++t) p *= sa[t];
         pin[i] = p;
         if (i % 16 == 15) tot[I] = p;
     }
     // A and M: twenty blocks of 16 x 16
     constexpr int MINE = (20 + NW - 1) / NW;
-    f32x4 sc[MINE];
+    f64x4 sc[MINE];
 #pragma unroll
     for (int x = 0; x < MINE; ++x) {
         const int b = wave + NW * x, bb = b % 10;
         if (b >= 20) continue;
         const int I = bb < 1 ? 0 : bb < 3 ? 1 : bb < 6 ? 2 : 3, J = bb - I * (I + 1) / 2;
         const float* rows = b < 10 ? Qs : Ks;
-        f32x4 s = {0.f, 0.f, 0.f, 0.f};
+        f64x4 s = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
         for (int m = 0; m < DK; m += 16) {
             const float4 qf = *reinterpret_cast<const float4*>(rows + (I * 16 + r) * LS + m + 4 * g);
-            const float4 kf = *reinterpret_cast<const float4*>(Ks + (J * 16 + r) * LS + m + 4 * g);
-            s = mfma4(kf.x, kf.y, kf.z, kf.w, qf, s);
+            const float4 kf = *reinterpret_cast<const float4*>(Ks + (J * 16 + r % 4 * 4 + r / 4) * LS + m + 4 * g);
+            s = __builtin_amdgcn_mfma_f64_16x16x4f64((double)kf.x, (double)qf.x, s, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f64_16x16x4f64((double)kf.y, (double)qf.y, s, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f64_16x16x4f64((double)kf.z, (double)qf.z, s, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f64_16x16x4f64((double)kf.w, (double)qf.w, s, 0, 0, 0);
         }
         sc[x] = s;
     }
     lds_barrier();
     if (tid < SCAN_C) {
-        float p = pin[tid], s = sfx[tid];
+        double p = pin[tid], s = sfx[tid];
         for (int run = 0; run < tid / 16; ++run) p *= tot[run];
         for (int run = tid / 16 + 1; run < 4; ++run) s *= tot[run];
-        from[tid] = p;
-        rest[tid] = s;
+        from[tid] = (float)p;
+        rest[tid] = (float)s;
     }
 #pragma unroll
     for (int x = 0; x < MINE; ++x) {
         const int b = wave + NW * x, bb = b % 10;
         if (b >= 20) continue;
         const int I = bb < 1 ? 0 : bb < 3 ? 1 : bb < 6 ? 2 : 3, J = bb - I * (I + 1) / 2, i = I * 16 + r;
-        float f[4], p = pin[i];
+        double f[4], p = pin[i];
         for (int run = J + 1; run < I; ++run) p *= tot[run];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            f[e] = I == J ? dg[I][r][4 * g + e] : p * sfx[J * 16 + 4 * g + e];
-            if (b >= 10) f[e] = I == J && 4 * g + e >= r ? 0.f : f[e] * sb[i];
+            f[e] = I == J ? (double)dg[I][r][4 * g + e] : p * sfx[J * 16 + 4 * g + e];
+            if (b >= 10) f[e] = I == J && 4 * g + e >= r ? 0.0 : f[e] * sb[i];
         }
         *reinterpret_cast<float4*>((b < 10 ? As : Ms) + i * SCAN_AS + J * 16 + 4 * g) =
-            make_float4(sc[x][0] * f[0], sc[x][1] * f[1], sc[x][2] * f[2], sc[x][3] * f[3]);
+            make_float4((float)(sc[x][0] * f[0]), (float)(sc[x][1] * f[1]), (float)(sc[x][2] * f[2]), (float)(sc[x][3] * f[3]));
     }
     lds_barrier();
     // T, the diagonal blocks by substitution, a thread per column
@@ -732,8 +783,8 @@ delta_chunks_kernel(DeltaArgs a) {
         for (int s = 0; s <= I; ++s) {
             const int j = 16 * s + 4 * g;
             const float* col = Ks + j * LS + ct * 16 + r;
-            o = mfma4(-from[j] * col[0], -from[j + 1] * col[LS], -from[j + 2] * col[2 * LS], -from[j + 3] * col[3 * LS],
-                      *reinterpret_cast<const float4*>(Ms + i * SCAN_AS + j), o);
+            o += mfma4(-from[j] * col[0], -from[j + 1] * col[LS], -from[j + 2] * col[2 * LS], -from[j + 3] * col[3 * LS],
+                       *reinterpret_cast<const float4*>(Ms + i * SCAN_AS + j), (f32x4){0.f, 0.f, 0.f, 0.f});
         }
         *reinterpret_cast<float4*>(a.queries + (slot * SCAN_C + i) * DK + ct * 16 + 4 * g) = make_float4(o[0], o[1], o[2], o[3]);
         f32x4 w = {0.f, 0.f, 0.f, 0.f};
@@ -741,8 +792,8 @@ delta_chunks_kernel(DeltaArgs a) {
             const int t = 16 * s + 4 * g;
             const float* col = Ks + t * LS + ct * 16 + r;
             const float* tt = Ts + t * SCAN_AS + I * 16 + r;
-            w = mfma4(rest[t] * col[0], rest[t + 1] * col[LS], rest[t + 2] * col[2 * LS], rest[t + 3] * col[3 * LS],
-                      make_float4(tt[0], tt[SCAN_AS], tt[2 * SCAN_AS], tt[3 * SCAN_AS]), w);
+            w += mfma4(rest[t] * col[0], rest[t + 1] * col[LS], rest[t + 2] * col[2 * LS], rest[t + 3] * col[3 * LS],
+                       make_float4(tt[0], tt[SCAN_AS], tt[2 * SCAN_AS], tt[3 * SCAN_AS]), (f32x4){0.f, 0.f, 0.f, 0.f});
         }
         const float be = sb[i];
         z[y] = (f32x4){w[0] * be, w[1] * be, w[2] * be, w[3] * be};
@@ -759,7 +810,7 @@ delta_chunks_kernel(DeltaArgs a) {
     auto fetch = [&](int col) { return scan_quad(v + (size_t)vt * a.ldv + col, v, vt < nt ? a.Dv - col : 0, a.vec); };
     float4 next = fetch(vc);
     lds_barrier();
-    const float whole = tot[0] * tot[1] * tot[2] * tot[3];
+    const float whole = (float)(tot[0] * tot[1] * tot[2] * tot[3]);
 #pragma unroll
     for (int y0 = 0; y0 < DK / 16 / PER; y0 += 4 / PER) {
         f32x4 s[4 / PER];
@@ -842,16 +893,26 @@ delta_states_kernel(DeltaArgs a, int blocks) {
     for (int t = 0; t < TILES; ++t) old[t] = *reinterpret_cast<const float4*>(&St[0][r][(wave * TILES + t) * 16 + 4 * g]);
     auto move = [&](int c, int from, Next& now, Next& then) {
         if (c + 1 < n) fetch(c + 1, then);
-        f32x4 s[TILES];
+        f32x4 part[TILES][4], s[TILES];                 // (a sum in four parts: see sum_pairs)
 #pragma unroll
-        for (int t = 0; t < TILES; ++t) s[t] = (f32x4){now.x[t].x, now.x[t].y, now.x[t].z, now.x[t].w};
+        for (int t = 0; t < TILES; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) part[t][e] = (f32x4){0.f, 0.f, 0.f, 0.f};
         float4 y[DK / 16];
 #pragma unroll
         for (int k = 0; k < DK / 16; ++k) y[k] = *reinterpret_cast<const float4*>(&St[from][r][16 * k + 4 * g]);
 #pragma unroll
         for (int k = 0; k < DK / 16; ++k)
 #pragma unroll
-            for (int t = 0; t < TILES; ++t) s[t] = mfma4(now.m[t][k].x, now.m[t][k].y, now.m[t][k].z, now.m[t][k].w, y[k], s[t]);
+            for (int t = 0; t < TILES; ++t) {
+                part[t][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.m[t][k].x, y[k].x, part[t][0], 0, 0, 0);
+                part[t][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.m[t][k].y, y[k].y, part[t][1], 0, 0, 0);
+                part[t][2] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.m[t][k].z, y[k].z, part[t][2], 0, 0, 0);
+                part[t][3] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.m[t][k].w, y[k].w, part[t][3], 0, 0, 0);
+            }
+#pragma unroll
+        for (int t = 0; t < TILES; ++t)
+            s[t] = (part[t][0] + part[t][1]) + (part[t][2] + part[t][3]) + (f32x4){now.x[t].x, now.x[t].y, now.x[t].z, now.x[t].w};
 #pragma unroll
         for (int t = 0; t < TILES; ++t) {
             if (wave * TILES + t < ch_tiles) adds[place(c, t)] = old[t];
