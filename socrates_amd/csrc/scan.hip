@@ -121,9 +121,25 @@ __device__ __forceinline__ void scan_values(float* __restrict__ out, int H, int 
     constexpr int LS = DK + 4, PER = NW * 16 / DK, TILES = 2 / PER;      // PER: waves that share 16 channels
     if (NW == 8 || wave < 8) {
         const int I = wave / 2, p = wave % 2;
+        const float* row = X + (I * 16 + r) * SCAN_AS + 4 * g;
+        const float* col_v = Vs + 4 * g * SCAN_VS + p * 16 + r;
+        float v0 = col_v[16 * I * SCAN_VS], v1 = col_v[(16 * I + 1) * SCAN_VS], v2 = col_v[(16 * I + 2) * SCAN_VS], v3 = col_v[(16 * I + 3) * SCAN_VS];
+        f32x4 own = {0.f, 0.f, 0.f, 0.f};
+        // The tokens' own run: X is 0 above its diagonal, and 0 times a later token's value that is not finite is not 0. Such a
+        // run (any lane's four of the 16 x 16 values) is added up token by token, its products below are of zeros.
+        if (__any(!(v0 * 0.f + v1 * 0.f + v2 * 0.f + v3 * 0.f == 0.f))) {
+            for (int j = 0; j <= r; ++j) {
+                const float x = X[(I * 16 + r) * SCAN_AS + I * 16 + j];
+                const float* v = Vs + (I * 16 + j) * SCAN_VS + p * 16 + 4 * g;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) own[e] = fmaf(x, v[e], own[e]);
+            }
+            v0 = v1 = v2 = v3 = 0.f;
+        }
         f32x4 o = {0.f, 0.f, 0.f, 0.f};
-        for (int s = 0; s <= I; ++s)
-            o += mfma_col_row(Vs + (16 * s + 4 * g) * SCAN_VS + p * 16 + r, SCAN_VS, X + (I * 16 + r) * SCAN_AS + 16 * s + 4 * g, (f32x4){0.f, 0.f, 0.f, 0.f});
+        for (int s = 0; s < I; ++s) o += mfma_col_row(col_v + 16 * s * SCAN_VS, SCAN_VS, row + 16 * s, (f32x4){0.f, 0.f, 0.f, 0.f});
+        o += mfma4(v0, v1, v2, v3, *reinterpret_cast<const float4*>(row + 16 * I), (f32x4){0.f, 0.f, 0.f, 0.f});
+        o += own;
         const int t = I * 16 + r, col = col0 + p * 16 + 4 * g;
         if (t < nt) {
             float* to = out + ((size_t)(lo + t) * H + head) * Dv + col;
@@ -363,7 +379,10 @@ scan_chunks_kernel(ScanArgs a) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) f[e] = I == J ? dg[0][I][r][4 * g + e] : p * sfx[J * 16 + 4 * g + e];
         }
-        float4 s = make_float4(sc[x][0] * f[0], sc[x][1] * f[1], sc[x][2] * f[2], sc[x][3] * f[3]);
+        float y[4];                                  // (a later key that is not finite: its score is 0, not 0 times that)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[e] = I != J || 4 * g + e <= r ? sc[x][e] * f[e] : 0.f;
+        float4 s = make_float4(y[0], y[1], y[2], y[3]);
         if (MODE == SCAN_STEP && I == J) {
             if (r == 4 * g) s.x += skip;
             if (r == 4 * g + 1) s.y += skip;
@@ -635,6 +654,7 @@ delta_chunks_kernel(DeltaArgs a) {
     __shared__ __align__(16) float dg[4][16][16];
     __shared__ float sa[SCAN_C], sb[SCAN_C], from[SCAN_C], rest[SCAN_C];
     __shared__ double pin[SCAN_C], sfx[SCAN_C], tot[4];
+    __shared__ int broken;                           // the first token whose key, decay or step size is not finite
     const int head = blockIdx.x, c = blockIdx.y, seq = blockIdx.z, tid = threadIdx.x;
     const int lo = a.qstart[seq] + (a.first + c) * SCAN_C, hi = a.qstart[seq + 1];
     if (lo >= hi) return;
@@ -644,6 +664,7 @@ delta_chunks_kernel(DeltaArgs a) {
 
     const float* q = a.q + (size_t)(head / a.group) * a.hq + (size_t)lo * a.ldq;
     const float* k = a.k + (size_t)(head / a.group) * a.hq + (size_t)lo * a.ldq;
+    if (tid == 0) broken = SCAN_C;
     constexpr int ROUNDS = SCAN_C * Q4 / NT;
     float4 fq[ROUNDS], fk[ROUNDS];
 #pragma unroll
@@ -657,13 +678,25 @@ delta_chunks_kernel(DeltaArgs a) {
         sa[tid] = tid < nt ? gb.x : 1.f;
         sb[tid] = tid < nt ? gb.y : 0.f;
     }
+    lds_barrier();
+    if (tid < nt && !(sa[tid] * 0.f + sb[tid] * 0.f == 0.f)) atomicMin(&broken, tid);
 #pragma unroll
     for (int it = 0; it < ROUNDS; ++it) {
         const int e = it * NT + tid, t = e / Q4, i = e % Q4 * 4;
         *reinterpret_cast<float4*>(Qs + t * LS + i) = fq[it];
         *reinterpret_cast<float4*>(Ks + t * LS + i) = fk[it];
+        if (!(fk[it].x * 0.f + fk[it].y * 0.f + fk[it].z * 0.f + fk[it].w * 0.f == 0.f)) atomicMin(&broken, t);
     }
     __syncthreads();
+    // From such a token on nothing of the head is finite, neither results nor state; the tokens before it do not see it. The
+    // chunk is computed as if it ended there, and NaN put where the later results and the state are made (its queries' rows
+    // and the diagonal of its transition).
+    const int sound = broken;
+    if (sound < SCAN_C) {
+        for (int e = sound * LS + tid; e < SCAN_C * LS; e += NT) Qs[e] = Ks[e] = 0.f;
+        if (tid < SCAN_C && tid >= sound) { sa[tid] = 1.f; sb[tid] = 0.f; }
+        __syncthreads();
+    }
     if (tid < SCAN_C) {
         const int I = tid / 16, j = tid % 16;
         double p = 1.0;
@@ -786,6 +819,7 @@ delta_chunks_kernel(DeltaArgs a) {
             o += mfma4(-from[j] * col[0], -from[j + 1] * col[LS], -from[j + 2] * col[2 * LS], -from[j + 3] * col[3 * LS],
                        *reinterpret_cast<const float4*>(Ms + i * SCAN_AS + j), (f32x4){0.f, 0.f, 0.f, 0.f});
         }
+        if (i >= sound) o[0] = o[1] = o[2] = o[3] = NAN;
         *reinterpret_cast<float4*>(a.queries + (slot * SCAN_C + i) * DK + ct * 16 + 4 * g) = make_float4(o[0], o[1], o[2], o[3]);
         f32x4 w = {0.f, 0.f, 0.f, 0.f};
         for (int s = I; s < 4; ++s) {                // row I * 16 + r of T^T
@@ -810,7 +844,7 @@ delta_chunks_kernel(DeltaArgs a) {
     auto fetch = [&](int col) { return scan_quad(v + (size_t)vt * a.ldv + col, v, vt < nt ? a.Dv - col : 0, a.vec); };
     float4 next = fetch(vc);
     lds_barrier();
-    const float whole = (float)(tot[0] * tot[1] * tot[2] * tot[3]);
+    const float whole = sound < SCAN_C ? NAN : (float)(tot[0] * tot[1] * tot[2] * tot[3]);
 #pragma unroll
     for (int y0 = 0; y0 < DK / 16 / PER; y0 += 4 / PER) {
         f32x4 s[4 / PER];

@@ -332,3 +332,71 @@ def test_from_which_portion_on(kernel_sets):
     assert [delta([n]) for n in (1, 255, 256, 3000)] == [False, False, True, True] and not delta([3000], 129)
     assert [delta([n] * 2) for n in (256, 500, 1000)] == [False, True, True]             # side by side the walks cost little more
     assert not delta([500] * 3) and delta([1000] * 3) and not delta([1000] * 5) and delta([2000] + [1] * 20)
+
+
+# (token, what is not finite there): in the first and the last place of a run, in a run's middle, in the last token
+BROKEN = {"results": [(3, "v", float("inf")), (79, "v", float("nan")), (200, "q", float("nan"))],
+          "keys": [(37, "k", float("inf")), (95, "v", float("-inf")), (170, "k", float("nan"))],
+          "steps": [(64, "decay", float("nan")), (81, "k", float("nan")), (130, "decay", float("nan"))]}
+
+
+@pytest.mark.parametrize("dtype", list(DTYPES))
+@pytest.mark.parametrize("where", list(BROKEN))
+@pytest.mark.parametrize("kind", ["retention", "lightning", "gated", "prepared", "bonus", "step", "delta"])
+def test_what_is_not_finite_touches_no_earlier_token(kernel_sets, dtype, where, kind):
+    """Results and states that the walk leaves finite are finite in chunks too, and what they are without (the 16 sums of a run
+    with such a value are added up in another order: 16 roundings of 2^-24 of the largest)."""
+    ops, dt, ctx = kernel_sets[dtype], DTYPES[dtype], step_of([65, 16, 17, 200])
+    N, H, D = ctx.n_tokens, 2, {"delta": 36, "bonus": 20}.get(kind, 72)
+    f32 = torch.float32
+    if kind in ("bonus", "delta"):
+        q, k, v = (rnd((N, H * D), dt, i, 0.5) for i in range(3))
+        decay = decays_of((N, H * D) if kind == "bonus" else (N, H), 4)
+    elif kind == "step":
+        xbc, decay = rnd((N, H * 40 + 2 * D), dt, 1, 0.5), rnd((N, H), f32, 2)
+        v, k, q = xbc[:, :H * 40], xbc[:, H * 40:H * 40 + D], xbc[:, H * 40 + D:]
+    else:
+        x, decay = rnd((N, 3 * H * D), dt, 1, 0.5), rnd((N, H * D), f32, 3)
+        q, k, v = (x[:, i * H * D:(i + 1) * H * D] for i in range(3))
+    if kind == "prepared":
+        given = torch.stack([q.float(), k.float(), decays_of((N, H * D), 4)], 1).contiguous()
+        q, k, decay = given.unbind(1)
+    one, per_head = rnd((H,), f32, 6), torch.tensor([0.9, 0.5], device=DEV)
+    if kind == "delta":
+        qk = torch.zeros(N, 2, H, 64, device=DEV)
+        qk[..., :D] = torch.nn.functional.normalize(torch.stack([q, k], 1).float().view(N, 2, H, D), dim=-1)
+        gates = torch.stack([decay, torch.full_like(decay, 0.7)], -1).contiguous()
+        q, k, decay = qk[:, 0].view(N, -1), qk[:, 1].view(N, -1), gates.view(N, -1)
+    calls = {"retention": lambda s: ops.retention(x, (0, H * D, 2 * H * D), H, D, D, None, 0, 0.1, per_head, s, 0, ctx),
+             "lightning": lambda s: ops.linear_attention(x, (0, H * D, 2 * H * D), H, D, D, 0.1, True, per_head, None, None, 1.0, s, 0, ctx),
+             "gated": lambda s: ops.linear_attention(x, (0, H * D, 2 * H * D), H, D, D, 0.1, False, None, decay, torch.zeros(H * D, device=DEV), 4.0, s, 0, ctx),
+             "prepared": lambda s: ops.linear_attention(x, (0, 0, 2 * H * D), H, D, D + 1, 1.0, False, None, None, None, 1.0, s, 0, ctx, prepared=given, ones=1),
+             "bonus": lambda s: ops.wkv(q, k, v, decay, v, rnd((H, D), f32, 8), rnd((H * D,), f32, 8), 1e-5, H, s, 0, ctx),
+             "step": lambda s: ops.ssd(xbc, decay, one, one, one, H, 40, D, 1, s, 0, ctx),
+             "delta": lambda s: delta_rule(ops, ctx, qk, v, gates, H, H, D, D, s)}
+    values = {"prepared": D + 1, "step": 40}.get(kind, D)
+    kept = ops.gated_group_norm
+    ops.gated_group_norm = lambda raw, *a, **kw: raw
+
+    def run(least):
+        state = rnd((4, H * D * values), f32, 9)
+        ops.scan_from = least
+        return calls[kind](state), state
+    try:
+        sound = run(1)
+        spoiled = 0
+        for token, what, value in BROKEN[where]:
+            if what == "decay" and kind in ("retention", "lightning"):
+                continue                                       # a constant of the head
+            t = {"q": q, "k": k, "v": v, "decay": decay}[what]
+            t[token, token % t.shape[1]] = value
+            spoiled += 1
+        walk, chunks = run(0), run(1)
+    finally:
+        ops.gated_group_norm = kept
+        del ops.scan_from
+    for a, b, c in zip(walk, chunks, sound):
+        fine = a.isfinite()
+        assert (not spoiled or not fine.all()) and fine.any()
+        assert torch.equal(b.isfinite(), fine)
+        assert float((b[fine] - c[fine]).abs().max()) <= 16 * 2.0 ** -24 * float(c.abs().max())
