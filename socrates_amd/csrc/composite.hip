@@ -450,7 +450,7 @@ __global__ void __launch_bounds__(256)
 linear_attention_kernel(const T* __restrict__ x, int ld, int col_q, int col_k, int col_v, float q_scale, int act,
                         const float* __restrict__ decays, const float* __restrict__ z, const float* __restrict__ z_bias,
                         float inv_tau, int H, int D, int Dv, float* __restrict__ state, size_t stride, int offset,
-                        const int* __restrict__ seq_qstart, const int* __restrict__ seq_rows, const float* __restrict__ prep,
+                        const int* __restrict__ seq_qstart, const int* __restrict__ seq_rows, int below, const float* __restrict__ prep,
                         int ones, float* __restrict__ out) {
     constexpr int REC_TB = rec_batch(DK), PARTS = 256 / CW, KPT = DK / PARTS, STAGE = (REC_TB * DK + 255) / 256;
     __shared__ float sq[2][REC_TB][DK], sk[2][REC_TB][DK];
@@ -459,7 +459,7 @@ linear_attention_kernel(const T* __restrict__ x, int ld, int col_q, int col_k, i
     const int blocks = (Dv + CW - 1) / CW;
     const int head = blockIdx.x / blocks, seq = blockIdx.y, tid = threadIdx.x;
     const int lo = seq_qstart[seq], hi = seq_qstart[seq + 1];
-    if (lo >= hi) return;
+    if (lo >= hi || hi - lo >= below) return;
     const int col0 = (blockIdx.x % blocks) * CW;
     const int col = col0 + tid % CW, part = tid / CW, i0 = part * KPT;
     const bool live = col < Dv;
@@ -563,12 +563,12 @@ linear_attention_kernel(const T* __restrict__ x, int ld, int col_q, int col_k, i
 template <typename T, int DK>
 static void launch_linear_attention(const void* x, int ld, int col_q, int col_k, int col_v, float q_scale, int act,
                                     const float* decays, const float* z, const float* z_bias, float inv_tau, int H, int D, int Dv,
-                                    float* state, long long stride, int offset, const int* seq_qstart, const int* seq_rows,
+                                    float* state, long long stride, int offset, const int* seq_qstart, const int* seq_rows, int below,
                                     const float* prep, int prepared, int ones, float* out, int n_seqs, int cw, hipStream_t stream) {
 #define SOC_LA_LAUNCH(CW, CH)                                                                                                  \
     hipLaunchKernelGGL((linear_attention_kernel<T, DK, CW, CH>), dim3(H * ((Dv + CW - 1) / CW), n_seqs), dim3(256), 0, stream, \
                        (const T*)x, ld, col_q, col_k, col_v, q_scale, act, decays, z, z_bias, inv_tau, H, D, Dv, state,        \
-                       (size_t)stride, offset, seq_qstart, seq_rows, prep, ones, out)
+                       (size_t)stride, offset, seq_qstart, seq_rows, below, prep, ones, out)
     if (z || prepared) { if (cw == 16) SOC_LA_LAUNCH(16, true); else SOC_LA_LAUNCH(64, true); }
     else   { if (cw == 16) SOC_LA_LAUNCH(16, false); else SOC_LA_LAUNCH(64, false); }
 #undef SOC_LA_LAUNCH
@@ -593,22 +593,22 @@ SOC_EXPORT int soc_linear_prepare(const void* x, int ld, int col_q, int col_k, f
 
 SOC_EXPORT int soc_linear_attention(const void* x, int ld, int col_q, int col_k, int col_v, float q_scale, int act,
                                     const float* decays, const float* z, const float* z_bias, float tau, int H, int D, int Dv,
-                                    float* state, long long stride, int offset, const int* seq_qstart, const int* seq_rows,
-                                    float* prep, int prepared, int ones, int n_tokens, float* out, int n_seqs, int max_q_len,
+                                    float* state, long long stride, int offset, const int* seq_qstart, const int* seq_rows, int below,
+                                    float* prep, int prepared, int ready, int ones, int n_tokens, float* out, int n_seqs, int max_q_len,
                                     int dtype, hipStream_t stream) {
     if (n_seqs <= 0 || H <= 0) return 0;
     if (D < 1 || D > 256 || Dv < 1 || n_seqs > 65535 || ones < 0 || ones >= Dv) return (int)hipErrorInvalidValue;
     if (prepared ? (!prep || z || decays)
                  : ((z == nullptr) == (decays == nullptr) || (z && (!z_bias || !(tau > 0.f))))) return (int)hipErrorInvalidValue;
-    const int cw = columns_per_workgroup(H, Dv, n_seqs, max_q_len);
+    const int cw = columns_per_workgroup(H, Dv, n_seqs, max_q_len, below);
     const float inv_tau = z ? 1.f / tau : 0.f;
-    if (prep && !prepared) {                                            // scratch [n_tokens, 2 or 3, H * D]
+    if (prep && !prepared && !ready) {                                  // scratch [n_tokens, 2 or 3, H * D]; ready: filled
         if (n_tokens <= 0) return (int)hipErrorInvalidValue;
         const int err = soc_linear_prepare(x, ld, col_q, col_k, q_scale, act, z, z_bias, tau, H * D, prep, n_tokens, dtype, stream);
         if (err) return err;
     }
-#define SOC_LA_F32(DK) launch_linear_attention<float, DK>(x, ld, col_q, col_k, col_v, q_scale, act, decays, z, z_bias, inv_tau, H, D, Dv, state, stride, offset, seq_qstart, seq_rows, prep, prepared, ones, out, n_seqs, cw, stream)
-#define SOC_LA_BF16(DK) launch_linear_attention<bf16, DK>(x, ld, col_q, col_k, col_v, q_scale, act, decays, z, z_bias, inv_tau, H, D, Dv, state, stride, offset, seq_qstart, seq_rows, prep, prepared, ones, out, n_seqs, cw, stream)
+#define SOC_LA_F32(DK) launch_linear_attention<float, DK>(x, ld, col_q, col_k, col_v, q_scale, act, decays, z, z_bias, inv_tau, H, D, Dv, state, stride, offset, seq_qstart, seq_rows, below, prep, prepared, ones, out, n_seqs, cw, stream)
+#define SOC_LA_BF16(DK) launch_linear_attention<bf16, DK>(x, ld, col_q, col_k, col_v, q_scale, act, decays, z, z_bias, inv_tau, H, D, Dv, state, stride, offset, seq_qstart, seq_rows, below, prep, prepared, ones, out, n_seqs, cw, stream)
     if (dtype == 0) { SOC_BY_STATE_SIZE(D, SOC_LA_F32) } else { SOC_BY_STATE_SIZE(D, SOC_LA_BF16) }
     return soc_last_error();
 }

@@ -2,6 +2,8 @@
 // and the recurrence itself, S <- g S; u = beta (v - S^T k); S <- S + k u^T; o = S^T q per head.
 //
 // Everything behind the projections is float32; values alone are rounded to the compute dtype between the two kernels.
+#include <climits>
+
 #include "common.h"
 #include "recurrent.h"
 
@@ -188,7 +190,7 @@ template <typename T, int NJ>
 __global__ void __launch_bounds__(256)
 delta_walk_kernel(const float* __restrict__ qk, const T* __restrict__ v, const float* __restrict__ gates, int G, int H, int D, int Dv,
                   float* __restrict__ state, size_t stride, int offset, const int* __restrict__ seq_qstart,
-                  const int* __restrict__ seq_rows, float* __restrict__ out) {
+                  const int* __restrict__ seq_rows, int below, float* __restrict__ out) {
     constexpr int DK = 64 * NJ, TB = NJ <= 2 ? 16 : 8, CW = 16, PIECES = TB * 2 * DK / 4, STAGE = PIECES / 256;
     static_assert(PIECES % 256 == 0, "whole rounds of 16-byte pieces");
     __shared__ __attribute__((aligned(16))) float sqk[2][TB][2][DK];
@@ -197,7 +199,7 @@ delta_walk_kernel(const float* __restrict__ qk, const T* __restrict__ v, const f
     const int blocks = (Dv + CW - 1) / CW;
     const int head = blockIdx.x / blocks, seq = blockIdx.y, tid = threadIdx.x, kv = head / (H / G);
     const int lo = seq_qstart[seq], hi = seq_qstart[seq + 1];
-    if (lo >= hi) return;
+    if (lo >= hi || hi - lo >= below) return;         // (from `below` tokens on: taken in chunks, scan.hip)
     const int col0 = (blockIdx.x % blocks) * CW, cl = tid / 16, p = tid % 16, col = col0 + cl;
     const bool live = col < Dv, vec = D % 4 == 0;
     float* S = state + (size_t)seq_rows[seq] * stride + offset + ((size_t)head * Dv + (live ? col : 0)) * D;
@@ -297,19 +299,26 @@ delta_walk_kernel(const float* __restrict__ qk, const T* __restrict__ v, const f
     }
 }
 
-SOC_EXPORT int soc_delta_walk(const float* qk, const void* v, const float* gates, int G, int H, int D, int Dv, int Dp, float* state,
-                              long long stride, int offset, const int* seq_qstart, const int* seq_rows, float* out, int n_seqs, int dtype,
-                              hipStream_t stream) {
+// The sequences of fewer than `below` tokens.
+SOC_EXPORT int soc_delta_walk_below(const float* qk, const void* v, const float* gates, int G, int H, int D, int Dv, int Dp, float* state,
+                                    long long stride, int offset, const int* seq_qstart, const int* seq_rows, int below, float* out,
+                                    int n_seqs, int dtype, hipStream_t stream) {
     if (n_seqs <= 0) return 0;
     if (G < 1 || H < 1 || H % G || D < 1 || Dv < 1 || Dp != (D + 63) / 64 * 64 || Dp > 256 || n_seqs > 65535 ||
         (D % 4 == 0 && (stride % 4 || offset % 4)))
         return (int)hipErrorInvalidValue;
 #define SOC_DW(T, NJ)                                                                                                               \
     hipLaunchKernelGGL((delta_walk_kernel<T, NJ>), dim3(H * ((Dv + 15) / 16), n_seqs), dim3(256), 0, stream, qk, (const T*)v, gates, G, \
-                       H, D, Dv, state, (size_t)stride, offset, seq_qstart, seq_rows, out)
+                       H, D, Dv, state, (size_t)stride, offset, seq_qstart, seq_rows, below, out)
 #define SOC_DW_T(T) switch (Dp / 64) { case 1: SOC_DW(T, 1); break; case 2: SOC_DW(T, 2); break; case 3: SOC_DW(T, 3); break; default: SOC_DW(T, 4); }
     if (dtype == 0) { SOC_DW_T(float) } else { SOC_DW_T(bf16) }
 #undef SOC_DW_T
 #undef SOC_DW
     return soc_last_error();
+}
+
+SOC_EXPORT int soc_delta_walk(const float* qk, const void* v, const float* gates, int G, int H, int D, int Dv, int Dp, float* state,
+                              long long stride, int offset, const int* seq_qstart, const int* seq_rows, float* out, int n_seqs, int dtype,
+                              hipStream_t stream) {
+    return soc_delta_walk_below(qk, v, gates, G, H, D, Dv, Dp, state, stride, offset, seq_qstart, seq_rows, INT_MAX, out, n_seqs, dtype, stream);
 }

@@ -189,14 +189,14 @@ __global__ void __launch_bounds__(256)
 retention_kernel(const T* __restrict__ x, int ld, int col_q, int col_k, int col_v, const int* __restrict__ positions,
                  const float* __restrict__ inv_freq, int half, float k_scale, const float* __restrict__ decays, int H, int D,
                  int Dv, float* __restrict__ state, size_t stride, int offset, const int* __restrict__ seq_qstart,
-                 const int* __restrict__ seq_rows, const float* __restrict__ turned, float* __restrict__ out) {
+                 const int* __restrict__ seq_rows, int below, const float* __restrict__ turned, float* __restrict__ out) {
     constexpr int REC_TB = rec_batch(DK), PARTS = 256 / CW, KPT = DK / PARTS, STAGE = (REC_TB * DK + 255) / 256;
     __shared__ float sq[2][REC_TB][DK], sk[2][REC_TB][DK];
     __shared__ float red[REC_TB][PARTS][CW];
     const int blocks = (Dv + CW - 1) / CW;
     const int head = blockIdx.x / blocks, seq = blockIdx.y, tid = threadIdx.x;
     const int lo = seq_qstart[seq], hi = seq_qstart[seq + 1];
-    if (lo >= hi) return;
+    if (lo >= hi || hi - lo >= below) return;
     const int col0 = (blockIdx.x % blocks) * CW;
     const int col = col0 + tid % CW, part = tid / CW, i0 = part * KPT;
     const bool live = col < Dv;
@@ -291,12 +291,12 @@ retention_kernel(const T* __restrict__ x, int ld, int col_q, int col_k, int col_
 template <typename T, int DK>
 static void launch_retention(const void* x, int ld, int col_q, int col_k, int col_v, const int* positions, const float* inv_freq,
                              int half, float k_scale, const float* decays, int H, int D, int Dv, float* state, long long stride,
-                             int offset, const int* seq_qstart, const int* seq_rows, const float* turned, float* out, int n_seqs,
-                             int cw, hipStream_t stream) {
+                             int offset, const int* seq_qstart, const int* seq_rows, int below, const float* turned, float* out,
+                             int n_seqs, int cw, hipStream_t stream) {
 #define SOC_RET_LAUNCH(CW)                                                                                                     \
     hipLaunchKernelGGL((retention_kernel<T, DK, CW>), dim3(H * ((Dv + CW - 1) / CW), n_seqs), dim3(256), 0, stream,            \
                        (const T*)x, ld, col_q, col_k, col_v, positions, inv_freq, half, k_scale, decays, H, D, Dv, state,      \
-                       (size_t)stride, offset, seq_qstart, seq_rows, turned, out)
+                       (size_t)stride, offset, seq_qstart, seq_rows, below, turned, out)
     if (cw == 16) SOC_RET_LAUNCH(16); else SOC_RET_LAUNCH(64);
 #undef SOC_RET_LAUNCH
 }
@@ -317,19 +317,20 @@ SOC_EXPORT int soc_retention_turn(const void* x, int ld, int col_q, int col_k, c
     return soc_last_error();
 }
 
+// turned: null, or scratch as above, with `ready` filled by the caller.
 SOC_EXPORT int soc_retention(const void* x, int ld, int col_q, int col_k, int col_v, const int* positions, const float* inv_freq,
                              int half, float k_scale, const float* decays, int H, int D, int Dv, float* state, long long stride,
-                             int offset, const int* seq_qstart, const int* seq_rows, float* turned, int n_tokens, float* out,
-                             int n_seqs, int max_q_len, int dtype, hipStream_t stream) {
+                             int offset, const int* seq_qstart, const int* seq_rows, int below, float* turned, int ready, int n_tokens,
+                             float* out, int n_seqs, int max_q_len, int dtype, hipStream_t stream) {
     if (n_seqs <= 0 || H <= 0) return 0;
     if (D < 1 || D > 256 || Dv < 1 || n_seqs > 65535 || 2 * half > D) return (int)hipErrorInvalidValue;
-    if (turned) {                                          // scratch [n_tokens, 2, H * D]: turn q and k ahead of the walk
+    if (turned && !ready) {                                // turn q and k ahead of the walk
         const int err = soc_retention_turn(x, ld, col_q, col_k, positions, inv_freq, half, k_scale, H, D, turned, n_tokens, dtype, stream);
         if (err) return err;
     }
-    const int cw = columns_per_workgroup(H, Dv, n_seqs, max_q_len);
-#define SOC_RET_F32(DK) launch_retention<float, DK>(x, ld, col_q, col_k, col_v, positions, inv_freq, half, k_scale, decays, H, D, Dv, state, stride, offset, seq_qstart, seq_rows, turned, out, n_seqs, cw, stream)
-#define SOC_RET_BF16(DK) launch_retention<bf16, DK>(x, ld, col_q, col_k, col_v, positions, inv_freq, half, k_scale, decays, H, D, Dv, state, stride, offset, seq_qstart, seq_rows, turned, out, n_seqs, cw, stream)
+    const int cw = columns_per_workgroup(H, Dv, n_seqs, max_q_len, below);
+#define SOC_RET_F32(DK) launch_retention<float, DK>(x, ld, col_q, col_k, col_v, positions, inv_freq, half, k_scale, decays, H, D, Dv, state, stride, offset, seq_qstart, seq_rows, below, turned, out, n_seqs, cw, stream)
+#define SOC_RET_BF16(DK) launch_retention<bf16, DK>(x, ld, col_q, col_k, col_v, positions, inv_freq, half, k_scale, decays, H, D, Dv, state, stride, offset, seq_qstart, seq_rows, below, turned, out, n_seqs, cw, stream)
     if (dtype == 0) { SOC_BY_STATE_SIZE(D, SOC_RET_F32) } else { SOC_BY_STATE_SIZE(D, SOC_RET_BF16) }
     return soc_last_error();
 }

@@ -514,14 +514,14 @@ template <typename T, int DK, int CW>
 __global__ void __launch_bounds__(256)
 wkv_kernel(const T* __restrict__ r, const T* __restrict__ k, const T* __restrict__ v, const float* __restrict__ decay,
            const float* __restrict__ bonus, int H, int D, float* __restrict__ state, size_t stride, int offset,
-           const int* __restrict__ seq_qstart, const int* __restrict__ seq_rows, float* __restrict__ out) {
+           const int* __restrict__ seq_qstart, const int* __restrict__ seq_rows, int below, float* __restrict__ out) {
     constexpr int REC_TB = rec_batch(DK), PARTS = 256 / CW, KPT = DK / PARTS, STAGE = (REC_TB * DK + 255) / 256;
     __shared__ float sr[2][REC_TB][DK], sk[2][REC_TB][DK], sw[2][REC_TB][DK];
     __shared__ float red[REC_TB][PARTS][CW], su[DK];
     const int blocks = (D + CW - 1) / CW;
     const int head = blockIdx.x / blocks, seq = blockIdx.y, tid = threadIdx.x;
     const int lo = seq_qstart[seq], hi = seq_qstart[seq + 1];
-    if (lo >= hi) return;
+    if (lo >= hi || hi - lo >= below) return;
     const int col0 = (blockIdx.x % blocks) * CW;
     const int col = col0 + tid % CW, part = tid / CW, i0 = part * KPT;
     const bool live = col < D;
@@ -600,22 +600,22 @@ wkv_kernel(const T* __restrict__ r, const T* __restrict__ k, const T* __restrict
 
 template <typename T, int DK>
 static void launch_wkv(const void* r, const void* k, const void* v, const float* decay, const float* bonus, int H, int D,
-                       float* state, long long stride, int offset, const int* seq_qstart, const int* seq_rows, float* out,
+                       float* state, long long stride, int offset, const int* seq_qstart, const int* seq_rows, int below, float* out,
                        int n_seqs, int cw, hipStream_t stream) {
 #define SOC_WKV_LAUNCH(CW)                                                                                                  \
     hipLaunchKernelGGL((wkv_kernel<T, DK, CW>), dim3(H * ((D + CW - 1) / CW), n_seqs), dim3(256), 0, stream, (const T*)r, \
-                       (const T*)k, (const T*)v, decay, bonus, H, D, state, (size_t)stride, offset, seq_qstart, seq_rows, out)
+                       (const T*)k, (const T*)v, decay, bonus, H, D, state, (size_t)stride, offset, seq_qstart, seq_rows, below, out)
     if (cw == 16) SOC_WKV_LAUNCH(16); else SOC_WKV_LAUNCH(64);
 }
 
 SOC_EXPORT int soc_wkv(const void* r, const void* k, const void* v, const float* decay, const float* bonus, int H, int D,
-                       float* state, long long stride, int offset, const int* seq_qstart, const int* seq_rows, float* out,
+                       float* state, long long stride, int offset, const int* seq_qstart, const int* seq_rows, int below, float* out,
                        int n_seqs, int max_q_len, int dtype, hipStream_t stream) {
     if (n_seqs <= 0 || H <= 0) return 0;
     if (D < 1 || D > 256 || n_seqs > 65535) return (int)hipErrorInvalidValue;
-    const int cw = columns_per_workgroup(H, D, n_seqs, max_q_len);
-#define SOC_WKV_F32(DK) launch_wkv<float, DK>(r, k, v, decay, bonus, H, D, state, stride, offset, seq_qstart, seq_rows, out, n_seqs, cw, stream)
-#define SOC_WKV_BF16(DK) launch_wkv<bf16, DK>(r, k, v, decay, bonus, H, D, state, stride, offset, seq_qstart, seq_rows, out, n_seqs, cw, stream)
+    const int cw = columns_per_workgroup(H, D, n_seqs, max_q_len, below);
+#define SOC_WKV_F32(DK) launch_wkv<float, DK>(r, k, v, decay, bonus, H, D, state, stride, offset, seq_qstart, seq_rows, below, out, n_seqs, cw, stream)
+#define SOC_WKV_BF16(DK) launch_wkv<bf16, DK>(r, k, v, decay, bonus, H, D, state, stride, offset, seq_qstart, seq_rows, below, out, n_seqs, cw, stream)
     if (dtype == 0) { SOC_BY_STATE_SIZE(D, SOC_WKV_F32) } else { SOC_BY_STATE_SIZE(D, SOC_WKV_BF16) }
     return soc_last_error();
 }
@@ -627,14 +627,14 @@ __global__ void __launch_bounds__(256)
 ssd_kernel(const T* __restrict__ xbc, const float* __restrict__ dt_raw, const float* __restrict__ dt_bias,
            const float* __restrict__ a_log, const float* __restrict__ skip, int H, int P, int Ns, int G,
            float* __restrict__ state, size_t stride, int offset, const int* __restrict__ seq_qstart,
-           const int* __restrict__ seq_rows, float* __restrict__ out) {
+           const int* __restrict__ seq_rows, int below, float* __restrict__ out) {
     constexpr int REC_TB = rec_batch(NK), PARTS = 256 / CW, KPT = NK / PARTS, STAGE = (REC_TB * NK + 255) / 256;
     __shared__ float sb[2][REC_TB][NK], sc[2][REC_TB][NK], skeep[2][REC_TB], sdt[2][REC_TB];
     __shared__ float red[REC_TB][PARTS][CW];
     const int blocks = (P + CW - 1) / CW;
     const int head = blockIdx.x / blocks, seq = blockIdx.y, tid = threadIdx.x;
     const int lo = seq_qstart[seq], hi = seq_qstart[seq + 1];
-    if (lo >= hi) return;
+    if (lo >= hi || hi - lo >= below) return;
     const int col0 = (blockIdx.x % blocks) * CW;
     const int col = col0 + tid % CW, part = tid / CW, i0 = part * KPT;
     const bool live = col < P;
@@ -725,21 +725,21 @@ ssd_kernel(const T* __restrict__ xbc, const float* __restrict__ dt_raw, const fl
 template <typename T, int NK>
 static void launch_ssd(const void* xbc, const float* dt_raw, const float* dt_bias, const float* a_log, const float* skip,
                        int H, int P, int Ns, int G, float* state, long long stride, int offset, const int* seq_qstart,
-                       const int* seq_rows, float* out, int n_seqs, int cw, hipStream_t stream) {
+                       const int* seq_rows, int below, float* out, int n_seqs, int cw, hipStream_t stream) {
 #define SOC_SSD_LAUNCH(CW)                                                                                                   \
     hipLaunchKernelGGL((ssd_kernel<T, NK, CW>), dim3(H * ((P + CW - 1) / CW), n_seqs), dim3(256), 0, stream, (const T*)xbc, \
-                       dt_raw, dt_bias, a_log, skip, H, P, Ns, G, state, (size_t)stride, offset, seq_qstart, seq_rows, out)
+                       dt_raw, dt_bias, a_log, skip, H, P, Ns, G, state, (size_t)stride, offset, seq_qstart, seq_rows, below, out)
     if (cw == 16) SOC_SSD_LAUNCH(16); else SOC_SSD_LAUNCH(64);
 }
 
 SOC_EXPORT int soc_ssd(const void* xbc, const float* dt_raw, const float* dt_bias, const float* a_log, const float* skip,
                        int H, int P, int Ns, int G, float* state, long long stride, int offset, const int* seq_qstart,
-                       const int* seq_rows, float* out, int n_seqs, int max_q_len, int dtype, hipStream_t stream) {
+                       const int* seq_rows, int below, float* out, int n_seqs, int max_q_len, int dtype, hipStream_t stream) {
     if (n_seqs <= 0 || H <= 0) return 0;
     if (Ns < 1 || Ns > 256 || P < 1 || G < 1 || H % G || n_seqs > 65535) return (int)hipErrorInvalidValue;
-    const int cw = columns_per_workgroup(H, P, n_seqs, max_q_len);
-#define SOC_SSD_F32(NK) launch_ssd<float, NK>(xbc, dt_raw, dt_bias, a_log, skip, H, P, Ns, G, state, stride, offset, seq_qstart, seq_rows, out, n_seqs, cw, stream)
-#define SOC_SSD_BF16(NK) launch_ssd<bf16, NK>(xbc, dt_raw, dt_bias, a_log, skip, H, P, Ns, G, state, stride, offset, seq_qstart, seq_rows, out, n_seqs, cw, stream)
+    const int cw = columns_per_workgroup(H, P, n_seqs, max_q_len, below);
+#define SOC_SSD_F32(NK) launch_ssd<float, NK>(xbc, dt_raw, dt_bias, a_log, skip, H, P, Ns, G, state, stride, offset, seq_qstart, seq_rows, below, out, n_seqs, cw, stream)
+#define SOC_SSD_BF16(NK) launch_ssd<bf16, NK>(xbc, dt_raw, dt_bias, a_log, skip, H, P, Ns, G, state, stride, offset, seq_qstart, seq_rows, below, out, n_seqs, cw, stream)
     if (dtype == 0) { SOC_BY_STATE_SIZE(Ns, SOC_SSD_F32) } else { SOC_BY_STATE_SIZE(Ns, SOC_SSD_BF16) }
     return soc_last_error();
 }

@@ -25,9 +25,10 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
     }
 
 // Columns per workgroup: 64, or 16 where heads and sequences alone leave most compute units idle.
-// (A step with a prompt portion in it is as long as that portion's walk, whatever else is in the step.)
-static int columns_per_workgroup(int H, int cols, int n_seqs, int max_q_len) {
-    if (max_q_len > 64) return 16;
+// (A step with a prompt portion in it is as long as that portion's walk, whatever else is in the step.) The walks leave
+// sequences of `below` tokens and more alone: those are taken in chunks (scan.hip).
+static int columns_per_workgroup(int H, int cols, int n_seqs, int max_q_len, int below) {
+    if (max_q_len > 64 && below > 65) return 16;
     return (long long)H * ((cols + 63) / 64) * n_seqs >= 192 ? 64 : 16;
 }
 

@@ -56,6 +56,7 @@ struct ScanArgs {
     int hq, hk, hv, group;                 // elements from one head to the next; heads that share q and k
     int H, D, Dv, held, v_act, vec;        // held: value columns in v, the others read 1; vec: rows may be read by fours
     int first, count, compact;             // chunks of every sequence: first .. first + count - 1; how slots are numbered
+    int n_seqs, least;                     // sequences of fewer than `least` tokens are not these kernels'
     const int* qstart;
     const int* rows;
     float* state;
@@ -73,9 +74,39 @@ struct ScanArgs {
 __device__ __forceinline__ int scan_col(int p, int r) { return r / 4 * 8 + p * 4 + r % 4; }     // within 32 columns
 __host__ __device__ __forceinline__ int scan_tiles(int Dv) { return (Dv + 31) / 32 * 2; }
 
-// Scratch of a sequence's chunk: with one launch over all tokens the chunks lie one behind the other.
-__device__ __forceinline__ size_t scan_slot(const ScanArgs& a, int seq, int c) {
-    return a.compact ? (size_t)(a.qstart[seq] / SCAN_C + seq + c) : (size_t)seq * a.count + c;
+// Chunks are numbered for the grid and for scratch. With one launch over all tokens (compact) those of the l-th sequence of
+// `least` tokens and more begin at number qstart / 64 + l, so that they lie nearly one behind the other whatever the
+// lengths; else at l * count. A wave looks at 64 sequences at a time. A step's decoding rows are not among these sequences: each
+// would fill one token of a chunk, and a chunk costs the same however few of its tokens there are.
+struct ScanPlace { int seq, c, slot; };
+template <typename Args, typename Is>
+__device__ __forceinline__ bool scan_search(const Args& a, ScanPlace& at, Is is) {
+    const int lane = threadIdx.x % 64;
+    for (int seq0 = 0, found = 0; seq0 < a.n_seqs; seq0 += 64) {
+        const int seq = min(seq0 + lane, a.n_seqs - 1), start = a.qstart[seq], len = a.qstart[seq + 1] - start;
+        const unsigned long long own = __ballot(seq0 + lane < a.n_seqs && len >= a.least);
+        const int l = found + __popcll(own & ((1ull << lane) - 1));
+        const int slot = a.compact ? start / SCAN_C + l : l * a.count;
+        const unsigned long long hit = __ballot((own >> lane & 1) && is(l, slot, a.compact ? (len + SCAN_C - 1) / SCAN_C : a.count));
+        if (hit) {
+            const int src = __builtin_ctzll(hit);
+            at.seq = seq0 + src;
+            at.slot = __builtin_amdgcn_readlane(slot, src);
+            return true;
+        }
+        found += __popcll(own);
+    }
+    return false;
+}
+// the sequence and the chunk of number b; or, of the l-th such sequence, the first chunk's number
+template <typename Args> __device__ __forceinline__ bool scan_chunk(const Args& a, int b, ScanPlace& at) {
+    if (!scan_search(a, at, [&](int, int slot, int n) { return slot <= b && b < slot + n; })) return false;
+    at.c = b - at.slot;
+    at.slot = b;
+    return true;
+}
+template <typename Args> __device__ __forceinline__ bool scan_sequence(const Args& a, int which, ScanPlace& at) {
+    return scan_search(a, at, [&](int l, int, int) { return l == which; });
 }
 
 // Four elements of a row of which the first n exist (n <= 0: none; then p is not read where vec). With vec the load
@@ -191,12 +222,14 @@ scan_chunks_kernel(ScanArgs a) {
     float* As = Qs;
     float* Vs = V_IN_Q ? Qs + SCAN_C * SCAN_AS : Vx;
 
-    const int head = blockIdx.x, c = blockIdx.y, seq = blockIdx.z, tid = threadIdx.x;
-    const int lo = a.qstart[seq] + (a.first + c) * SCAN_C, hi = a.qstart[seq + 1];
+    const int head = blockIdx.x, tid = threadIdx.x;
+    ScanPlace at;
+    if (!scan_chunk(a, blockIdx.y, at)) return;
+    const int lo = a.qstart[at.seq] + (a.first + at.c) * SCAN_C, hi = a.qstart[at.seq + 1];
     if (lo >= hi) return;
     const int nt = min(SCAN_C, hi - lo);
     const int lane = tid % 64, wave = tid / 64, r = lane % 16, g = lane / 16;
-    const size_t slot = scan_slot(a, seq, c) * a.H + head;
+    const size_t slot = (size_t)at.slot * a.H + head;
     float skip = 0.f;
 
     if constexpr (!CH) {
@@ -447,7 +480,9 @@ scan_chunks_kernel(ScanArgs a) {
 template <bool CH>
 __global__ void __launch_bounds__(256)
 scan_states_kernel(ScanArgs a, int dk) {
-    const int head = blockIdx.y, seq = blockIdx.z, tiles = scan_tiles(a.Dv);
+    ScanPlace in;
+    if (!scan_sequence(a, blockIdx.z, in)) return;
+    const int head = blockIdx.y, seq = in.seq, tiles = scan_tiles(a.Dv);
     const int size = (a.D + 15) / 16 * tiles * 64, at = (int)blockIdx.x * 256 + (int)threadIdx.x;     // in pieces of four
     const int left = a.qstart[seq + 1] - a.qstart[seq] - a.first * SCAN_C;
     if (at >= size || left <= 0) return;
@@ -455,7 +490,7 @@ scan_states_kernel(ScanArgs a, int dk) {
     const int lane = at % 64, ct = at / 64 % tiles, ch = at / 64 / tiles * 16 + lane / 16 * 4;
     const int col = ct / 2 * 32 + scan_col(ct % 2, lane % 16);
     float* S = a.state + (size_t)a.rows[seq] * a.stride + a.offset + (size_t)head * a.D * a.Dv + (size_t)ch * a.Dv + col;
-    const size_t slot0 = scan_slot(a, seq, 0) * a.H + head;
+    const size_t slot0 = (size_t)in.slot * a.H + head;
     float4* add = reinterpret_cast<float4*>(a.adds) + slot0 * size + at;
     const float* f = a.factors + slot0 * dk + (CH ? ch : 0);
     const size_t step = (size_t)a.H * size, fstep = (size_t)a.H * dk;
@@ -503,12 +538,14 @@ scan_apply_kernel(ScanArgs a) {
     constexpr int LS = DK + 4, Q4 = DK / 4;
     __shared__ __align__(16) float Qs[SCAN_C * LS];
     const int blocks = (a.Dv + 32 * CG - 1) / (32 * CG);
-    const int head = blockIdx.x / blocks, c = blockIdx.y, seq = blockIdx.z, tid = threadIdx.x;
-    const int lo = a.qstart[seq] + (a.first + c) * SCAN_C, hi = a.qstart[seq + 1];
+    const int head = blockIdx.x / blocks, tid = threadIdx.x;
+    ScanPlace at;
+    if (!scan_chunk(a, blockIdx.y, at)) return;
+    const int lo = a.qstart[at.seq] + (a.first + at.c) * SCAN_C, hi = a.qstart[at.seq + 1];
     if (lo >= hi) return;
     const int nt = min(SCAN_C, hi - lo);
     const int lane = tid % 64, wave = tid / 64, r = lane % 16, g = lane / 16;
-    const size_t slot = scan_slot(a, seq, c) * a.H + head;
+    const size_t slot = (size_t)at.slot * a.H + head;
     const int col0 = (blockIdx.x % blocks) * 32 * CG + (wave % CG) * 32, row0 = (wave / CG) * 16 * CG;
     // two tiles of 16 columns; channels 16 s + 4 g .. + 3 in piece s (tiles beyond the last channel's: the last one, whose
     // queries are zeros; columns beyond the last tile's: read at a place that exists, not used)
@@ -578,39 +615,41 @@ scan_apply_kernel(ScanArgs a) {
 }
 
 template <int DK, int MODE, typename TQ, typename TV>
-static void launch_scan(const ScanArgs& a, int n_seqs, hipStream_t s) {
-    hipLaunchKernelGGL((scan_chunks_kernel<DK, MODE, TQ, TV>), dim3(a.H, a.count, n_seqs), dim3(64 * scan_waves(DK, MODE >= SCAN_CHANNEL)), 0, s, a);
+static void launch_scan(const ScanArgs& a, int n_long, int slots, hipStream_t s) {
+    hipLaunchKernelGGL((scan_chunks_kernel<DK, MODE, TQ, TV>), dim3(a.H, slots), dim3(64 * scan_waves(DK, MODE >= SCAN_CHANNEL)), 0, s, a);
     const int pieces = (a.D + 15) / 16 * scan_tiles(a.Dv) * 64;
     constexpr bool CH = MODE >= SCAN_CHANNEL;
-    hipLaunchKernelGGL(scan_states_kernel<CH>, dim3((pieces + 255) / 256, a.H, n_seqs), dim3(256), 0, s, a, DK);
-    if (a.Dv <= 32) hipLaunchKernelGGL((scan_apply_kernel<DK, 1, CH, TQ>), dim3(a.H, a.count, n_seqs), dim3(256), 0, s, a);
-    else if (a.Dv <= 64) hipLaunchKernelGGL((scan_apply_kernel<DK, 2, CH, TQ>), dim3(a.H, a.count, n_seqs), dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((scan_apply_kernel<DK, 4, CH, TQ>), dim3(a.H * ((a.Dv + 127) / 128), a.count, n_seqs), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(scan_states_kernel<CH>, dim3((pieces + 255) / 256, a.H, n_long), dim3(256), 0, s, a, DK);
+    if (a.Dv <= 32) hipLaunchKernelGGL((scan_apply_kernel<DK, 1, CH, TQ>), dim3(a.H, slots), dim3(256), 0, s, a);
+    else if (a.Dv <= 64) hipLaunchKernelGGL((scan_apply_kernel<DK, 2, CH, TQ>), dim3(a.H, slots), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((scan_apply_kernel<DK, 4, CH, TQ>), dim3(a.H * ((a.Dv + 127) / 128), slots), dim3(256), 0, s, a);
 }
 
-// One of the recurrences above over chunks first .. first + count - 1 of every sequence (64 tokens each; a sequence
-// may have fewer), from and into the rows' states. D <= 128. adds, queries and factors: scratch of `slots` chunks,
-// n_tokens / 64 + n_seqs of them with compact (first 0 and count for the longest sequence), n_seqs * count without.
+// One of the recurrences above over chunks first .. first + count - 1 (64 tokens each; a sequence may have fewer) of every
+// sequence of `least` tokens and more, of which there are at most n_long, from and into the rows' states. D <= 128. adds,
+// queries and factors: scratch of `slots` chunks, n_tokens / 64 + n_long of them with compact (first 0 and count for the
+// longest sequence), n_long * count without.
 // q and k are float32 with q_f32, else in dtype like v. dtype 0 float32, 1 bfloat16.
 SOC_EXPORT int soc_scan(int mode, const void* q, long long ldq, int hq, const void* k, long long ldk, int hk, int group, int q_f32,
                         const void* v, long long ldv, int hv, int v_act, int ones, const float* decay, long long lda,
                         const float* p1, const float* p2, const float* p3, int H, int D, int Dv, float* state, long long stride,
-                        int offset, const int* seq_qstart, const int* seq_rows, int n_seqs, int first, int count, int compact,
-                        float* out, float* adds, float* queries, float* factors, int dtype, hipStream_t stream) {
-    if (n_seqs <= 0 || H <= 0 || count <= 0) return 0;
-    if (D < 1 || D > 128 || Dv < 1 || ones < 0 || ones >= Dv || group < 1 || H % group || n_seqs > 65535 || count > 65535 || first < 0 ||
-        (compact && first) || !adds || !queries || !factors || !decay) return (int)hipErrorInvalidValue;
+                        int offset, const int* seq_qstart, const int* seq_rows, int n_seqs, int least, int n_long, int slots,
+                        int first, int count, int compact, float* out, float* adds, float* queries, float* factors, int dtype,
+                        hipStream_t stream) {
+    if (n_seqs <= 0 || n_long <= 0 || H <= 0 || count <= 0) return 0;
+    if (D < 1 || D > 128 || Dv < 1 || ones < 0 || ones >= Dv || group < 1 || H % group || n_long > 65535 || slots < n_long || slots > 65535 ||
+        least < 1 || first < 0 || (compact && first) || (!compact && slots != (long long)n_long * count) || !adds || !queries || !factors || !decay) return (int)hipErrorInvalidValue;
     ScanArgs a;
     a.q = q; a.k = k; a.v = v; a.decay = decay; a.p1 = p1; a.p2 = p2; a.p3 = p3;
     a.ldq = ldq; a.ldk = ldk; a.ldv = ldv; a.lda = lda; a.hq = hq; a.hk = hk; a.hv = hv; a.group = group;
     a.H = H; a.D = D; a.Dv = Dv; a.held = Dv - ones; a.v_act = v_act;
-    a.first = first; a.count = count; a.compact = compact; a.qstart = seq_qstart; a.rows = seq_rows;
+    a.first = first; a.count = count; a.compact = compact; a.n_seqs = n_seqs; a.least = least; a.qstart = seq_qstart; a.rows = seq_rows;
     a.state = state; a.stride = stride; a.offset = offset; a.out = out; a.adds = adds; a.queries = queries; a.factors = factors;
     const int qe = q_f32 || dtype == 0 ? 16 : 8, ve = dtype == 0 ? 16 : 8;       // bytes of four elements
     a.vec = D % 4 == 0 && a.held % 4 == 0 && ldq % 4 == 0 && ldk % 4 == 0 && ldv % 4 == 0 && lda % 4 == 0 && hq % 4 == 0 && hk % 4 == 0 && hv % 4 == 0 &&
             (uintptr_t)q % qe == 0 && (uintptr_t)k % qe == 0 && (uintptr_t)v % ve == 0 && (uintptr_t)decay % 16 == 0;
 #define SOC_SCAN(MODE_, TQ_, TV_) \
-    do { if (D <= 64) launch_scan<64, MODE_, TQ_, TV_>(a, n_seqs, stream); else launch_scan<128, MODE_, TQ_, TV_>(a, n_seqs, stream); } while (0)
+    do { if (D <= 64) launch_scan<64, MODE_, TQ_, TV_>(a, n_long, slots, stream); else launch_scan<128, MODE_, TQ_, TV_>(a, n_long, slots, stream); } while (0)
     if (mode == SCAN_HEAD && q_f32) { if (dtype == 0) SOC_SCAN(SCAN_HEAD, float, float); else SOC_SCAN(SCAN_HEAD, float, bf16); }
     else if (mode == SCAN_CHANNEL && q_f32) { if (dtype == 0) SOC_SCAN(SCAN_CHANNEL, float, float); else SOC_SCAN(SCAN_CHANNEL, float, bf16); }
     else if (mode == SCAN_STEP && !q_f32 && p1 && p2 && p3) { if (dtype == 0) SOC_SCAN(SCAN_STEP, float, float); else SOC_SCAN(SCAN_STEP, bf16, bf16); }
@@ -634,7 +673,7 @@ struct DeltaArgs {
     const float *q, *k, *gates;
     const void* v;
     long long ldq, ldv;
-    int hq, hv, group, H, D, Dv, vec, first, count, compact;
+    int hq, hv, group, H, D, Dv, vec, first, count, compact, n_seqs, least;
     const int* qstart;
     const int* rows;
     float* state;
@@ -655,12 +694,14 @@ delta_chunks_kernel(DeltaArgs a) {
     __shared__ float sa[SCAN_C], sb[SCAN_C], from[SCAN_C], rest[SCAN_C];
     __shared__ double pin[SCAN_C], sfx[SCAN_C], tot[4];
     __shared__ int broken;                           // the first token whose key, decay or step size is not finite
-    const int head = blockIdx.x, c = blockIdx.y, seq = blockIdx.z, tid = threadIdx.x;
-    const int lo = a.qstart[seq] + (a.first + c) * SCAN_C, hi = a.qstart[seq + 1];
+    const int head = blockIdx.x, tid = threadIdx.x;
+    ScanPlace at;
+    if (!scan_chunk(a, blockIdx.y, at)) return;
+    const int lo = a.qstart[at.seq] + (a.first + at.c) * SCAN_C, hi = a.qstart[at.seq + 1];
     if (lo >= hi) return;
     const int nt = min(SCAN_C, hi - lo);
     const int lane = tid % 64, wave = tid / 64, r = lane % 16, g = lane / 16;
-    const size_t slot = (a.compact ? (size_t)(a.qstart[seq] / SCAN_C + seq + c) : (size_t)seq * a.count + c) * a.H + head;
+    const size_t slot = (size_t)at.slot * a.H + head;
 
     const float* q = a.q + (size_t)(head / a.group) * a.hq + (size_t)lo * a.ldq;
     const float* k = a.k + (size_t)(head / a.group) * a.hq + (size_t)lo * a.ldq;
@@ -895,14 +936,16 @@ __global__ void __launch_bounds__(256)
 delta_states_kernel(DeltaArgs a, int blocks) {
     constexpr int LS = DK + 4, TILES = DK / 64;       // tiles of 16 channels per wave
     __shared__ __align__(16) float St[2][16][LS];
-    const int b = blockIdx.x, head = b / (8 * blocks) * 8 + b % 8, cb = b / 8 % blocks, seq = blockIdx.y, tid = threadIdx.x;
-    if (head >= a.H) return;
+    const int b = blockIdx.x, head = b / (8 * blocks) * 8 + b % 8, cb = b / 8 % blocks, tid = threadIdx.x;
+    ScanPlace at;
+    if (head >= a.H || !scan_sequence(a, blockIdx.y, at)) return;
+    const int seq = at.seq;
     const int left = a.qstart[seq + 1] - a.qstart[seq] - a.first * SCAN_C;
     if (left <= 0) return;
     const int n = min(a.count, (left + SCAN_C - 1) / SCAN_C);
     const int lane = tid % 64, wave = tid / 64, r = lane % 16, g = lane / 16;
     float* S = a.state + (size_t)a.rows[seq] * a.stride + a.offset + (size_t)head * a.Dv * a.D;
-    const size_t slot0 = (a.compact ? (size_t)(a.qstart[seq] / SCAN_C + seq) : (size_t)seq * a.count) * a.H + head;
+    const size_t slot0 = (size_t)at.slot * a.H + head;
     for (int e = tid; e < 16 * DK; e += 256) {
         const int cl = e / DK, ch = e % DK, col = cb / 2 * 32 + scan_col(cb % 2, cl);
         St[0][cl][ch] = col < a.Dv && ch < a.D ? S[(size_t)col * a.D + ch] : 0.f;
@@ -966,35 +1009,37 @@ delta_states_kernel(DeltaArgs a, int blocks) {
 }
 
 template <int DK>
-static void launch_delta(const DeltaArgs& a, int n_seqs, int dtype, hipStream_t s) {
-    if (dtype == 0) hipLaunchKernelGGL((delta_chunks_kernel<DK, float>), dim3(a.H, a.count, n_seqs), dim3(64 * scan_waves(DK, true)), 0, s, a);
-    else hipLaunchKernelGGL((delta_chunks_kernel<DK, bf16>), dim3(a.H, a.count, n_seqs), dim3(64 * scan_waves(DK, true)), 0, s, a);
+static void launch_delta(const DeltaArgs& a, int n_long, int slots, int dtype, hipStream_t s) {
+    if (dtype == 0) hipLaunchKernelGGL((delta_chunks_kernel<DK, float>), dim3(a.H, slots), dim3(64 * scan_waves(DK, true)), 0, s, a);
+    else hipLaunchKernelGGL((delta_chunks_kernel<DK, bf16>), dim3(a.H, slots), dim3(64 * scan_waves(DK, true)), 0, s, a);
     const int blocks = scan_tiles(a.Dv);
-    hipLaunchKernelGGL((delta_states_kernel<DK>), dim3((a.H + 7) / 8 * 8 * blocks, n_seqs), dim3(256), 0, s, a, blocks);
+    hipLaunchKernelGGL((delta_states_kernel<DK>), dim3((a.H + 7) / 8 * 8 * blocks, n_long), dim3(256), 0, s, a, blocks);
     ScanArgs b = {};
-    b.H = a.H; b.D = a.D; b.Dv = a.Dv; b.first = a.first; b.count = a.count; b.compact = a.compact; b.qstart = a.qstart;
+    b.H = a.H; b.D = a.D; b.Dv = a.Dv; b.first = a.first; b.count = a.count; b.compact = a.compact; b.n_seqs = a.n_seqs; b.least = a.least;
+    b.qstart = a.qstart;
     b.out = a.out; b.adds = a.adds; b.queries = a.queries;
-    if (a.Dv <= 32) hipLaunchKernelGGL((scan_apply_kernel<DK, 1, true, float>), dim3(a.H, a.count, n_seqs), dim3(256), 0, s, b);
-    else if (a.Dv <= 64) hipLaunchKernelGGL((scan_apply_kernel<DK, 2, true, float>), dim3(a.H, a.count, n_seqs), dim3(256), 0, s, b);
-    else hipLaunchKernelGGL((scan_apply_kernel<DK, 4, true, float>), dim3(a.H * ((a.Dv + 127) / 128), a.count, n_seqs), dim3(256), 0, s, b);
+    if (a.Dv <= 32) hipLaunchKernelGGL((scan_apply_kernel<DK, 1, true, float>), dim3(a.H, slots), dim3(256), 0, s, b);
+    else if (a.Dv <= 64) hipLaunchKernelGGL((scan_apply_kernel<DK, 2, true, float>), dim3(a.H, slots), dim3(256), 0, s, b);
+    else hipLaunchKernelGGL((scan_apply_kernel<DK, 4, true, float>), dim3(a.H * ((a.Dv + 127) / 128), slots), dim3(256), 0, s, b);
 }
 
-// The gated delta rule over chunks first .. first + count - 1 of every sequence, from and into the rows' states. qk float32
-// [N, 2, G, Dp] as soc_delta_prepare leaves it, Dp 64 or 128; v [N, H Dv] in dtype. Scratch as for soc_scan, queries
+// The gated delta rule over chunks first .. first + count - 1 of every sequence of `least` tokens and more, from and into the
+// rows' states. qk float32 [N, 2, G, Dp] as soc_delta_prepare leaves it, Dp 64 or 128; v [N, H Dv] in dtype. n_long and
+// scratch as for soc_scan, queries
 // [slots, H, 64, Dp], moves [slots, H, Dp, Dp].
 SOC_EXPORT int soc_delta_scan(const float* qk, const void* v, const float* gates, int G, int H, int D, int Dv, int Dp, float* state,
-                              long long stride, int offset, const int* seq_qstart, const int* seq_rows, int n_seqs, int first, int count,
-                              int compact, float* out, float* adds, float* queries, float* moves, int dtype, hipStream_t stream) {
-    if (n_seqs <= 0 || H <= 0 || count <= 0) return 0;
-    if (G < 1 || H % G || D < 1 || Dv < 1 || Dp != (D + 63) / 64 * 64 || Dp > 128 || n_seqs > 65535 || count > 65535 || first < 0 ||
-        (compact && first) || !adds || !queries || !moves)
+                              long long stride, int offset, const int* seq_qstart, const int* seq_rows, int n_seqs, int least, int n_long,
+                              int slots, int first, int count, int compact, float* out, float* adds, float* queries, float* moves, int dtype, hipStream_t stream) {
+    if (n_seqs <= 0 || n_long <= 0 || H <= 0 || count <= 0) return 0;
+    if (G < 1 || H % G || D < 1 || Dv < 1 || Dp != (D + 63) / 64 * 64 || Dp > 128 || n_long > 65535 || slots < n_long || slots > 65535 ||
+        least < 1 || first < 0 || (compact && first) || (!compact && slots != (long long)n_long * count) || !adds || !queries || !moves)
         return (int)hipErrorInvalidValue;
     DeltaArgs a;
     a.q = qk; a.k = qk + (size_t)G * Dp; a.gates = gates; a.v = v; a.ldq = 2ll * G * Dp; a.ldv = (long long)H * Dv;
     a.hq = Dp; a.hv = Dv; a.group = H / G; a.H = H; a.D = D; a.Dv = Dv;
     a.vec = Dv % 4 == 0 && (uintptr_t)v % (dtype == 0 ? 16 : 8) == 0;
-    a.first = first; a.count = count; a.compact = compact; a.qstart = seq_qstart; a.rows = seq_rows;
+    a.first = first; a.count = count; a.compact = compact; a.n_seqs = n_seqs; a.least = least; a.qstart = seq_qstart; a.rows = seq_rows;
     a.state = state; a.stride = stride; a.offset = offset; a.out = out; a.adds = adds; a.queries = queries; a.moves = moves;
-    if (Dp == 64) launch_delta<64>(a, n_seqs, dtype, stream); else launch_delta<128>(a, n_seqs, dtype, stream);
+    if (Dp == 64) launch_delta<64>(a, n_long, slots, dtype, stream); else launch_delta<128>(a, n_long, slots, dtype, stream);
     return soc_last_error();
 }

@@ -59,9 +59,9 @@ _MIXER_SIGNATURES = {
     "soc_glu_clamped": [P, P, I, I, I, F, F, I, P],
     "soc_token_shift": [P, P, I, P, L, I, P, P, P, I, I, I, I, I, P],
     "soc_wkv_decay": [P, P, P, P, I, I, I, I, P],
-    "soc_wkv": [P, P, P, P, P, I, I, P, L, I, P, P, P, I, I, I, P],
+    "soc_wkv": [P, P, P, P, P, I, I, P, L, I, P, P, I, P, I, I, I, P],
     "soc_causal_conv_silu": [P, I, I, I, P, P, I, P, L, I, P, P, P, I, I, I, P],
-    "soc_ssd": [P, P, P, P, P, I, I, I, I, P, L, I, P, P, P, I, I, I, P],
+    "soc_ssd": [P, P, P, P, P, I, I, I, I, P, L, I, P, P, I, P, I, I, I, P],
     "soc_gated_group_norm": [P, P, I, P, I, I, I, F, I, I, P, I, P],
     "soc_latent_query_turn": [P, I, I, I, I, I, I, I, P, I, P, P, I, P],
     "soc_latent_prepare": [P, I, I, P, P, I, I, P, I, I, P, F, P, I, P, P, P, I, P, I, I, I, I, I, I, P],
@@ -71,7 +71,7 @@ _MIXER_SIGNATURES = {
 _HYBRID_SIGNATURES = {
     "soc_attn_prepare": [P, I, I, I, I, P, I, P, P, P, P, P, I, P, P, P, P, P, I, I, I, I, I, I, I, I, F, I, P],
     "soc_head_gate": [P, P, I, P, I, I, I, I, I, P],
-    "soc_retention": [P, I, I, I, I, P, P, I, F, P, I, I, I, P, L, I, P, P, P, I, P, I, I, I, P],
+    "soc_retention": [P, I, I, I, I, P, P, I, F, P, I, I, I, P, L, I, P, P, I, P, I, I, P, I, I, I, P],
     "soc_retention_turn": [P, I, I, I, P, P, I, F, I, I, P, I, I, P],
     "soc_relu_squared": [P, P, L, I, P],
     "soc_moe_route": [P, I, P, P, I, I, I, I, I, F, I, I, F, I, P, P, P],
@@ -88,7 +88,7 @@ _COMPOSITE_SIGNATURES = {
     "soc_window_prepare": [P, I, I, I, I, P, P, P, P, P, I, P, P, P, P, I, F, P, I, F, P, I, I, I, I, I, I, I, I, P],
     "soc_pool_blocks": [P, P, P, I, P, P, P, I, P, P, P, I, I, I, I, I, I, I, P],
     "soc_turn_back": [P, P, P, P, I, I, I, I, I, P],
-    "soc_linear_attention": [P, I, I, I, I, F, I, P, P, P, F, I, I, I, P, L, I, P, P, P, I, I, I, P, I, I, I, P],
+    "soc_linear_attention": [P, I, I, I, I, F, I, P, P, P, F, I, I, I, P, L, I, P, P, I, P, I, I, I, I, P, I, I, I, P],
     "soc_linear_prepare": [P, I, I, I, F, I, P, P, F, I, P, I, I, P],
     "soc_scaled_sum": [P, I, F, P, I, F, P, P, I, I, I, P],
     "soc_glu_gelu": [P, P, I, I, I, I, P],
@@ -105,10 +105,11 @@ _STREAMS_SIGNATURES = {
 _DELTA_SIGNATURES = {
     "soc_delta_prepare": [P] + [I] * 7 + [P, I, F, F, P, P, P, P, L, I, P, P, P, P, P, I, I, I, P],
     "soc_delta_walk": [P, P, P, I, I, I, I, I, P, L, I, P, P, P, I, I, P],
+    "soc_delta_walk_below": [P, P, P, I, I, I, I, I, P, L, I, P, P, I, P, I, I, P],
 }
 _SCAN_SIGNATURES = {
-    "soc_scan": [I, P, L, I, P, L, I, I, I, P, L, I, I, I, P, L, P, P, P, I, I, I, P, L, I, P, P, I, I, I, I, P, P, P, P, I, P],
-    "soc_delta_scan": [P, P, P, I, I, I, I, I, P, L, I, P, P, I, I, I, I, P, P, P, P, I, P],
+    "soc_scan": [I, P, L, I, P, L, I, I, I, P, L, I, I, I, P, L, P, P, P, I, I, I, P, L, I, P, P, I, I, I, I, I, I, I, P, P, P, P, I, P],
+    "soc_delta_scan": [P, P, P, I, I, I, I, I, P, L, I, P, P, I, I, I, I, I, I, I, P, P, P, P, I, P],
 }
 _SAMPLING_SIGNATURES = {"soc_sample": [P, P, P, P, P, I, I, P], "soc_argmax": [P, P, P, I, I, I, P]}
 _ATTENTION_SIGNATURES = {

@@ -13,9 +13,9 @@ import torch
 
 from .build import load_library
 from .common import _COMPOSITE_SIGNATURES, KernelError, _check, _declare, _ptr
+from .scan import CHANNEL, HEAD, NO_LIMIT
 
 _NORMS = {None: 0, "head": 1, "whole": 2, "turned": 3}
-from .scan import CHANNEL, HEAD
 
 
 class Composite:
@@ -201,23 +201,26 @@ class Composite:
         # walk (each of a head's workgroups would take them again); single tokens and short portions where they
         # are staged
         prep = prepared
-        chunks = self._in_chunks(ctx, D)
-        if prepared is None and (chunks or (activate or z is not None) and ctx.max_q_len >= self.linear_prepare_ahead):
+        least = self._chunks_from(ctx, D, H * -(-Dv // 16))
+        if prepared is None and (least or (activate or z is not None) and ctx.max_q_len >= self.linear_prepare_ahead):
             prep = torch.empty((N, 3 if z is not None else 2, H * D), dtype=torch.float32, device=self.device)
-        if chunks:
+        if least:
             if prepared is None:
                 _check(self._composite().soc_linear_prepare(
                     _ptr(x), c_int(ld), c_int(col_q), c_int(col_k), c_float(q_scale), c_int(1 if activate else 0), _ptr(z), _ptr(z_bias),
                     c_float(tau), c_int(H * D), _ptr(prep), c_int(N), c_int(self.code), self._stream()), "linear_prepare")
             planes = prep.shape[1]
             q, k, a = (c_void_p(prep.data_ptr() + 4 * i * H * D) for i in range(3))
-            return self._scan(CHANNEL if planes == 3 else HEAD, q, planes * H * D, D, k, planes * H * D, D,
+            if not self._scan(CHANNEL if planes == 3 else HEAD, q, planes * H * D, D, k, planes * H * D, D,
                               c_void_p(x.data_ptr() + col_v * x.element_size()), ld, Dv - ones, a if planes == 3 else _ptr(decays), H, D,
-                              Dv, state, stride, offset, ctx, N, out, v_act=activate, ones=ones, lda=planes * H * D if planes == 3 else 0)
+                              Dv, state, stride, offset, ctx, N, out, least, v_act=activate, ones=ones,
+                              lda=planes * H * D if planes == 3 else 0):
+                return out
         _check(self._composite().soc_linear_attention(
             _ptr(x), c_int(ld), c_int(col_q), c_int(col_k), c_int(col_v), c_float(q_scale), c_int(1 if activate else 0),
             _ptr(decays), _ptr(z), _ptr(z_bias), c_float(tau), c_int(H), c_int(D), c_int(Dv), _ptr(state), stride, c_int(offset),
-            _ptr(ctx.seq_qstart), _ptr(ctx.seq_rows), _ptr(prep), c_int(1 if prepared is not None else 0), c_int(ones), c_int(N),
+            _ptr(ctx.seq_qstart), _ptr(ctx.seq_rows), c_int(least or NO_LIMIT), _ptr(prep), c_int(1 if prepared is not None else 0),
+            c_int(1 if least else 0), c_int(ones), c_int(N),
             _ptr(out), c_int(ctx.n_seqs), c_int(ctx.max_q_len), c_int(self.code), self._stream()), "linear_attention")
         return out
 

@@ -9,6 +9,7 @@ import torch
 
 from .build import load_library
 from .common import _DELTA_SIGNATURES, KernelError, _check, _declare, _ptr
+from .scan import NO_LIMIT
 
 
 class Delta:
@@ -52,9 +53,13 @@ class Delta:
             c_float(q_scale), c_float(unit_eps), _ptr(z), _ptr(a_log), _ptr(dt_bias), _ptr(state), stride, c_int(conv_offset),
             _ptr(ctx.seq_qstart), _ptr(ctx.seq_rows), _ptr(qk), _ptr(v), _ptr(gates), c_int(ctx.n_seqs),
             c_int(max(1, ctx.max_q_len)), c_int(self.code), self._stream()), "delta_prepare")
-        if self._delta_in_chunks(ctx, N, D, H, Dv):
-            return self._delta_scan(qk, v, gates, G, H, D, Dv, Dp, state, stride, offset, ctx, N, out)
-        _check(lib.soc_delta_walk(
+        least = self._delta_in_chunks(ctx, N, D, H, Dv)
+        if least:
+            self._delta_scan(qk, v, gates, G, H, D, Dv, Dp, state, stride, offset, ctx, N, out, least)
+            if not self._split(ctx, least)[1]:
+                return out
+        _check(lib.soc_delta_walk_below(
             _ptr(qk), _ptr(v), _ptr(gates), c_int(G), c_int(H), c_int(D), c_int(Dv), c_int(Dp), _ptr(state), stride, c_int(offset),
-            _ptr(ctx.seq_qstart), _ptr(ctx.seq_rows), _ptr(out), c_int(ctx.n_seqs), c_int(self.code), self._stream()), "delta_walk")
+            _ptr(ctx.seq_qstart), _ptr(ctx.seq_rows), c_int(least or NO_LIMIT), _ptr(out), c_int(ctx.n_seqs), c_int(self.code),
+            self._stream()), "delta_walk")
         return out

@@ -11,6 +11,7 @@ import torch
 
 from .build import load_library
 from .common import _HYBRID_SIGNATURES, KernelError, _check, _declare, _ptr
+from .scan import HEAD, NO_LIMIT
 
 MAX_EXPERTS = 256        # what the routing and sorting kernels hold per token and per workgroup
 EXPERT_TILE = 16         # places of one expert that a workgroup of the products per expert takes ...
@@ -18,7 +19,6 @@ EXPERT_TILE = 16         # places of one expert that a workgroup of the products
 # the two products at 32 experts of 2,432 and a width of 2,560, tiles of 16 / 128 / 256 places: 19 places per expert
 # 395 / 389 / 404, 37: 506 / 401 / 413, 125: 1,068 / 451 / 459, 260: 2,156 / 754 / 640, 375: 3,067 / 897 / 701.
 EXPERT_TILES_MANY = ((160, 256, 64), (48, 128, 8))
-from .scan import HEAD
 
 
 class ExpertRuns:
@@ -141,22 +141,23 @@ class Hybrid:
         # a step with a portion of some length: q and k are turned once, ahead of the walk (each of a head's
         # workgroups would turn them again); single tokens and short portions are turned where they are staged
         turned = None
-        chunks = self._in_chunks(ctx, D)
-        if chunks or half and ctx.max_q_len >= self.retention_turn_ahead:
+        least = self._chunks_from(ctx, D, H * -(-Dv // 16))
+        if least or half and ctx.max_q_len >= self.retention_turn_ahead:
             turned = torch.empty((N, 2, H * D), dtype=torch.float32, device=self.device)
-        if chunks:
+        if least:
             _check(self._hybrid().soc_retention_turn(
                 _ptr(x), c_int(ld), c_int(col_q), c_int(col_k), _ptr(ctx.positions), _ptr(inv_freq if half else None), c_int(half),
                 c_float(k_scale), c_int(H), c_int(D), _ptr(turned), c_int(N), c_int(self.code), self._stream()), "retention_turn")
             ahead = [turned.data_ptr(), turned.data_ptr() + 4 * H * D]
-            return self._scan(HEAD, c_void_p(ahead[0]), 2 * H * D, D, c_void_p(ahead[1]), 2 * H * D, D,
+            if not self._scan(HEAD, c_void_p(ahead[0]), 2 * H * D, D, c_void_p(ahead[1]), 2 * H * D, D,
                               c_void_p(x.data_ptr() + col_v * x.element_size()), ld, Dv, _ptr(decays), H, D, Dv, state, stride, offset,
-                              ctx, N, out)
+                              ctx, N, out, least):
+                return out
         _check(self._hybrid().soc_retention(
             _ptr(x), c_int(ld), c_int(col_q), c_int(col_k), c_int(col_v), _ptr(ctx.positions), _ptr(inv_freq if half else None),
             c_int(half), c_float(k_scale), _ptr(decays), c_int(H), c_int(D), c_int(Dv), _ptr(state), stride, c_int(offset),
-            _ptr(ctx.seq_qstart), _ptr(ctx.seq_rows), _ptr(turned), c_int(N), _ptr(out), c_int(ctx.n_seqs), c_int(ctx.max_q_len),
-            c_int(self.code), self._stream()), "retention")
+            _ptr(ctx.seq_qstart), _ptr(ctx.seq_rows), c_int(least or NO_LIMIT), _ptr(turned), c_int(1 if least else 0), c_int(N), _ptr(out),
+            c_int(ctx.n_seqs), c_int(ctx.max_q_len), c_int(self.code), self._stream()), "retention")
         return out
 
     # -- feed-forwards --------------------------------------------------------------------------------------------

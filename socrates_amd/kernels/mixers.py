@@ -11,7 +11,7 @@ import torch
 from .build import load_library
 from .common import _DTYPE_CODE, _MIXER_SIGNATURES, KernelError, _check, _declare, _ptr
 from .hybrid import ExpertSums
-from .scan import BONUS, STEP
+from .scan import BONUS, NO_LIMIT, STEP
 
 
 class Mixers:
@@ -161,13 +161,12 @@ class Mixers:
         self._want(gain, "gain", torch.float32, (C,))
         stride = self._state(state, offset, H * D * D, ctx)
         raw = torch.empty((N, C), dtype=torch.float32, device=self.device)
-        if self._in_chunks(ctx, D, self.scan_from * 8 // 5):
-            self._scan(BONUS, _ptr(r), C, D, _ptr(k), C, D, _ptr(v), C, D, _ptr(decay), H, D, D, state, stride, offset, ctx, N, raw,
-                       q_f32=False, lda=C, params=[_ptr(bonus)])
-            return self.gated_group_norm(raw, g, gain, H, eps, gate_first=False)
-        _check(self._mixers().soc_wkv(_ptr(r), _ptr(k), _ptr(v), _ptr(decay), _ptr(bonus), c_int(H), c_int(D), _ptr(state),
-                                      stride, c_int(offset), _ptr(ctx.seq_qstart), _ptr(ctx.seq_rows), _ptr(raw),
-                                      c_int(ctx.n_seqs), c_int(ctx.max_q_len), c_int(self.code), self._stream()), "wkv")
+        least = self._chunks_from(ctx, D, H * -(-D // 16), self.scan_from * 8 // 5)
+        if not least or self._scan(BONUS, _ptr(r), C, D, _ptr(k), C, D, _ptr(v), C, D, _ptr(decay), H, D, D, state, stride, offset, ctx,
+                                   N, raw, least, q_f32=False, lda=C, params=[_ptr(bonus)]):
+            _check(self._mixers().soc_wkv(_ptr(r), _ptr(k), _ptr(v), _ptr(decay), _ptr(bonus), c_int(H), c_int(D), _ptr(state),
+                                          stride, c_int(offset), _ptr(ctx.seq_qstart), _ptr(ctx.seq_rows), c_int(least or NO_LIMIT),
+                                          _ptr(raw), c_int(ctx.n_seqs), c_int(ctx.max_q_len), c_int(self.code), self._stream()), "wkv")
         # (a head's columns are spread over workgroups: its norm is a kernel of its own)
         return self.gated_group_norm(raw, g, gain, H, eps, gate_first=False)
 
@@ -202,14 +201,16 @@ class Mixers:
             raise KernelError(f"ssd: {H} heads in {G} groups, state {Ns}, head size {P}")
         stride = self._state(state, offset, H * Ns * P, ctx)
         out = torch.empty((N, H * P), dtype=torch.float32, device=self.device)
-        if self._in_chunks(ctx, Ns, self.scan_from * 8 // 5):
+        least = self._chunks_from(ctx, Ns, H * -(-P // 16), self.scan_from * 8 // 5)
+        if least:
             ld, item = H * P + 2 * G * Ns, xbc.element_size()
             b, c = (c_void_p(xbc.data_ptr() + (H * P + i * G * Ns) * item) for i in range(2))
-            return self._scan(STEP, c, ld, Ns, b, ld, Ns, _ptr(xbc), ld, P, _ptr(dt), H, Ns, P, state, stride, offset, ctx, N, out,
-                              group=H // G, q_f32=False, params=[_ptr(dt_bias), _ptr(a_log), _ptr(skip)])
+            if not self._scan(STEP, c, ld, Ns, b, ld, Ns, _ptr(xbc), ld, P, _ptr(dt), H, Ns, P, state, stride, offset, ctx, N, out, least,
+                              group=H // G, q_f32=False, params=[_ptr(dt_bias), _ptr(a_log), _ptr(skip)]):
+                return out
         _check(self._mixers().soc_ssd(_ptr(xbc), _ptr(dt), _ptr(dt_bias), _ptr(a_log), _ptr(skip), c_int(H), c_int(P), c_int(Ns),
                                       c_int(G), _ptr(state), stride, c_int(offset), _ptr(ctx.seq_qstart), _ptr(ctx.seq_rows),
-                                      _ptr(out), c_int(ctx.n_seqs), c_int(ctx.max_q_len), c_int(self.code), self._stream()), "ssd")
+                                      c_int(least or NO_LIMIT), _ptr(out), c_int(ctx.n_seqs), c_int(ctx.max_q_len), c_int(self.code), self._stream()), "ssd")
         return out
 
     def gated_group_norm(self, y, z, gain, groups, eps, gate_first=True, sigmoid=False):

@@ -6,6 +6,7 @@ from __future__ import annotations
 
 from ctypes import c_int, c_longlong, c_void_p
 
+import numpy as np
 import torch
 
 from .build import load_library
@@ -13,6 +14,7 @@ from .common import _SCAN_SIGNATURES, _check, _declare, _ptr
 
 CHUNK = 64
 HEAD, STEP, CHANNEL, BONUS = range(4)          # what the decays are: see csrc/scan.hip
+NO_LIMIT = (1 << 31) - 1                       # the walks' sequences: those of fewer tokens than this
 
 
 def _tiles(D, Dv):
@@ -41,29 +43,67 @@ class Scan:
         return lib
 
     def _in_chunks(self, ctx, D, least=None):
-        """Whether a step's recurrences with keys of ``D`` run in chunks: a portion of some length (single tokens and
-        short portions walk: a chunk costs the same however few of its tokens there are) and a state whose
-        queries, keys and decays of a chunk fit LDS. ``least``: tokens, in place of ``scan_from``."""
+        """Whether a step's longest portion is one for chunks: of some length, and with keys of ``D`` whose queries, keys
+        and decays of a chunk fit LDS. ``least``: tokens, in place of ``scan_from``."""
         return 0 < (self.scan_from if least is None else least) <= ctx.max_q_len and D <= 128
 
-    def _delta_in_chunks(self, ctx, N, D, H, Dv):
-        """Whether a step's gated delta rules run in chunks. The walk takes sequences side by side, its time goes with the
-        longest of them until their columns (16 to a workgroup) fill the chip; a chunk fills it alone, its time goes with
-        all tokens, behind a start worth 165 tokens of the walk. Measured in us, walk -> chunks, 20 heads of 128 x 128:
-        2 sequences of 300 tokens 96 -> 82, of 500 146 -> 128, of 1,000 271 -> 197; 3 of 300 101 -> 130, of 500
-        151 -> 151, of 1,000 280 -> 270; 5 of 300 139 -> 147, of 1,000 404 -> 455; 8 of 1,000 568 -> 682."""
-        return self._in_chunks(ctx, D, self.delta_scan_from) and N * H * -(-Dv // 16) < 600 * (ctx.max_q_len - 165)
+    def _chunks_from(self, ctx, D, cols, least=None, token=None, busy=7e-4, start=32.0, chunk=0.0145):
+        """Tokens from which on a sequence of the step is taken in chunks (0: all walk): of all such lines, the one whose estimate
+        is least. A chunk costs the same however few of its tokens there are, so decoding rows walk beside a portion in
+        chunks. With ``cols`` blocks of 16 columns in the states of all heads, in us:
+        a walk: 12 and the most of ``token`` for every token of its longest sequence, ``busy`` for every token and block,
+        its states' bytes; chunks: ``start`` and ``chunk`` for every chunk and block. Fitted to 20 heads of 128 x 128, 10 of
+        128 x 256, 40 of 64 x 64 and 80 of 128 x 64; measured, all walk -> all in chunks -> as this says: 160 tokens beside 50
+        decoding rows: retention 93 -> 152 -> 84, ssd 116 -> 324 -> 116 (below its least), 2,000 beside 60: 890 -> 294 -> 154,
+        1,149 -> 609 -> 286; 500 beside 60: wkv 158 -> 187 -> 90, linear attention 270 -> 263 -> 114.
+        A step that does not say its lengths on the host is taken in chunks whole."""
+        if not self._in_chunks(ctx, D, least):
+            return 0
+        lens = self._portion_lengths(ctx)
+        if lens is None:
+            return 1
+        lines = ctx.host.setdefault("chunks_from", {})
+        key = (D, cols, token, busy, start, chunk)
+        if key not in lines:
+            lens = np.sort(lens)[::-1]
+            longest, walking = np.append(lens, 0), np.arange(len(lens), -1, -1)               # with the i longest in chunks
+            tokens = lens.sum() - np.append(0, np.cumsum(lens))
+            cost = np.maximum((0.12 + 0.0028 * D if token is None else token) * longest, busy * cols * tokens)
+            cost = np.maximum(cost, cols * D * 128 / 4.8e6 * walking) + 12.0 * (walking > 0)
+            cost[1:] += start + chunk * cols * np.cumsum(-(-lens // CHUNK))
+            cost[1:-1][lens[:-1] == lens[1:]] = np.inf                                        # equals go together
+            best = int(np.argmin(cost))
+            lines[key] = int(lens[best - 1]) if best else 0
+        return lines[key]
 
-    def _scan_scratch(self, ctx, N, sizes):
+    def _delta_in_chunks(self, ctx, N, D, H, Dv):
+        """The same for the gated delta rule, whose chunk costs more and whose walk is faster. Measured in us, walk -> chunks, 20
+        heads of 128 x 128: 2 sequences of 300 tokens 96 -> 82, of 500 146 -> 128, of 1,000 271 -> 197; 3 of 300 101 -> 130,
+        of 500 148 -> 147, of 1,000 280 -> 270; 5 of 300 139 -> 147, of 1,000 395 -> 455; 8 of 1,000 568 -> 682; 300 beside 60
+        decoding rows 93 -> 116, 2,000 beside 60 492 -> 283."""
+        cols = H * -(-Dv // 16)
+        if self._portion_lengths(ctx) is None and N * cols >= 600 * (ctx.max_q_len - 165):
+            return 0
+        return self._chunks_from(ctx, D, cols, self.delta_scan_from, token=0.255, busy=5.5e-4, start=48.0, chunk=0.032)
+
+    def _split(self, ctx, least):
+        """(most sequences that go in chunks, whether others walk) of a step taken in chunks from ``least`` tokens on."""
+        lens = self._portion_lengths(ctx)
+        if lens is None or least <= 1:
+            return ctx.n_seqs, False
+        n_long = int((lens >= least).sum())
+        return n_long, n_long < ctx.n_seqs
+
+    def _scan_scratch(self, ctx, N, n_long, sizes):
         """(chunks of the longest portion, chunks of every sequence that one launch takes, whether those lie one behind the
-        other, the scratch of ``sizes`` floats per chunk slot, the addresses of its parts): all chunks at once where the scratch allows it, else rounds
-        over a few chunks of every sequence with the state in the row between them."""
+        other, slots, the scratch of ``sizes`` floats per slot, the addresses of its parts): all chunks at once where the scratch allows
+        it, else rounds over a few chunks of every sequence with the state in the row between them. ``n_long``: sequences."""
         chunks, per_slot = -(-ctx.max_q_len // CHUNK), 4 * sum(sizes)
-        slots, count = N // CHUNK + ctx.n_seqs, chunks
-        compact = slots * per_slot <= self.scan_scratch
+        slots, count = N // CHUNK + n_long, chunks
+        compact = slots * per_slot <= self.scan_scratch and slots <= 65535
         if not compact:
-            count = max(1, min(chunks, self.scan_scratch // (ctx.n_seqs * per_slot)))
-            slots = ctx.n_seqs * count
+            count = max(1, min(chunks, self.scan_scratch // (n_long * per_slot), 65535 // n_long))
+            slots = n_long * count
         # one allocation, each part on 16 bytes
         at, ends = 0, []
         for n in sizes:
@@ -71,15 +111,16 @@ class Scan:
             at += (slots * n + 3) & ~3
         scratch = torch.empty(at, dtype=torch.float32, device=self.device)
         base = scratch.data_ptr()
-        return chunks, count, compact, scratch, [c_void_p(base + 4 * e) for e in ends]
+        return chunks, count, compact, slots, scratch, [c_void_p(base + 4 * e) for e in ends]
 
-    def _scan(self, mode, q, ldq, hq, k, ldk, hk, v, ldv, hv, decay, H, D, Dv, state, stride, offset, ctx, N, out, group=1, q_f32=True,
-              v_act=False, ones=0, lda=0, params=()):
-        """``q``, ``k``, ``v``, ``decay`` and ``params`` are addresses (``c_void_p``), ld* elements from one token to
-        the next, h* from one head to the next."""
+    def _scan(self, mode, q, ldq, hq, k, ldk, hk, v, ldv, hv, decay, H, D, Dv, state, stride, offset, ctx, N, out, least, group=1,
+              q_f32=True, v_act=False, ones=0, lda=0, params=()):
+        """The sequences of ``least`` tokens and more; returns whether others are left to walk. ``q``, ``k``, ``v``, ``decay`` and
+        ``params`` are addresses (``c_void_p``), ld* elements from one token to the next, h* from one head to the next."""
         dk = 64 if D <= 64 else 128
         rows = CHUNK * dk if mode in (CHANNEL, BONUS) else CHUNK
-        chunks, count, compact, scratch, parts = self._scan_scratch(ctx, N, [H * _tiles(D, Dv), H * rows, H * dk])
+        n_long, others = self._split(ctx, least)
+        chunks, count, compact, slots, scratch, parts = self._scan_scratch(ctx, N, n_long, [H * _tiles(D, Dv), H * rows, H * dk])
         p = list(params) + [None] * (3 - len(params))
         self.forms["scan"] += 1
         for first in range(0, chunks, count):
@@ -87,17 +128,18 @@ class Scan:
                 c_int(mode), q, c_longlong(ldq), c_int(hq), k, c_longlong(ldk), c_int(hk), c_int(group), c_int(1 if q_f32 else 0),
                 v, c_longlong(ldv), c_int(hv), c_int(1 if v_act else 0), c_int(ones), decay, c_longlong(lda), *p, c_int(H), c_int(D),
                 c_int(Dv), _ptr(state), stride, c_int(offset), _ptr(ctx.seq_qstart), _ptr(ctx.seq_rows), c_int(ctx.n_seqs),
-                c_int(first), c_int(count), c_int(1 if compact else 0), _ptr(out),
+                c_int(least), c_int(n_long), c_int(slots), c_int(first), c_int(count), c_int(1 if compact else 0), _ptr(out),
                 *parts, c_int(self.code), self._stream()), "scan")
-        return out
+        return others
 
-    def _delta_scan(self, qk, v, gates, G, H, D, Dv, Dp, state, stride, offset, ctx, N, out):
-        """The gated delta rule in chunks, from what ``soc_delta_prepare`` leaves."""
-        chunks, count, compact, scratch, parts = self._scan_scratch(ctx, N, [H * _tiles(D, Dv), H * CHUNK * Dp, H * Dp * Dp])
+    def _delta_scan(self, qk, v, gates, G, H, D, Dv, Dp, state, stride, offset, ctx, N, out, least=1):
+        """The gated delta rule in chunks for the sequences of ``least`` tokens and more, from what ``soc_delta_prepare`` leaves."""
+        n_long, _ = self._split(ctx, least)
+        chunks, count, compact, slots, scratch, parts = self._scan_scratch(ctx, N, n_long, [H * _tiles(D, Dv), H * CHUNK * Dp, H * Dp * Dp])
         self.forms["scan"] += 1
         for first in range(0, chunks, count):
             _check(self._scan_lib().soc_delta_scan(
                 _ptr(qk), _ptr(v), _ptr(gates), c_int(G), c_int(H), c_int(D), c_int(Dv), c_int(Dp), _ptr(state), stride, c_int(offset),
-                _ptr(ctx.seq_qstart), _ptr(ctx.seq_rows), c_int(ctx.n_seqs), c_int(first), c_int(count), c_int(1 if compact else 0),
-                _ptr(out), *parts, c_int(self.code), self._stream()), "delta_scan")
+                _ptr(ctx.seq_qstart), _ptr(ctx.seq_rows), c_int(ctx.n_seqs), c_int(least), c_int(n_long), c_int(slots), c_int(first),
+                c_int(count), c_int(1 if compact else 0), _ptr(out), *parts, c_int(self.code), self._stream()), "delta_scan")
         return out

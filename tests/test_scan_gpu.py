@@ -334,24 +334,16 @@ def test_from_which_portion_on(kernel_sets):
     assert not delta([500] * 3) and delta([1000] * 3) and not delta([1000] * 5) and delta([2000] + [1] * 20)
 
 
-# (token, what is not finite there): in the first and the last place of a run, in a run's middle, in the last token
-BROKEN = {"results": [(3, "v", float("inf")), (79, "v", float("nan")), (200, "q", float("nan"))],
-          "keys": [(37, "k", float("inf")), (95, "v", float("-inf")), (170, "k", float("nan"))],
-          "steps": [(64, "decay", float("nan")), (81, "k", float("nan")), (130, "decay", float("nan"))]}
+KINDS = ["retention", "lightning", "gated", "prepared", "bonus", "step", "delta"]
 
 
-@pytest.mark.parametrize("dtype", list(DTYPES))
-@pytest.mark.parametrize("where", list(BROKEN))
-@pytest.mark.parametrize("kind", ["retention", "lightning", "gated", "prepared", "bonus", "step", "delta"])
-def test_what_is_not_finite_touches_no_earlier_token(kernel_sets, dtype, where, kind):
-    """Results and states that the walk leaves finite are finite in chunks too, and what they are without (the 16 sums of a run
-    with such a value are added up in another order: 16 roundings of 2^-24 of the largest)."""
-    ops, dt, ctx = kernel_sets[dtype], DTYPES[dtype], step_of([65, 16, 17, 200])
+def layer(ops, dt, kind, ctx):
+    """(call of one recurrence, its queries, keys, values and decays (views, None: a constant), elements of a row's state)."""
     N, H, D = ctx.n_tokens, 2, {"delta": 36, "bonus": 20}.get(kind, 72)
     f32 = torch.float32
     if kind in ("bonus", "delta"):
         q, k, v = (rnd((N, H * D), dt, i, 0.5) for i in range(3))
-        decay = decays_of((N, H * D) if kind == "bonus" else (N, H), 4)
+        decay = decays_of((N, H * D), 4)
     elif kind == "step":
         xbc, decay = rnd((N, H * 40 + 2 * D), dt, 1, 0.5), rnd((N, H), f32, 2)
         v, k, q = xbc[:, :H * 40], xbc[:, H * 40:H * 40 + D], xbc[:, H * 40 + D:]
@@ -363,40 +355,86 @@ def test_what_is_not_finite_touches_no_earlier_token(kernel_sets, dtype, where, 
         q, k, decay = given.unbind(1)
     one, per_head = rnd((H,), f32, 6), torch.tensor([0.9, 0.5], device=DEV)
     if kind == "delta":
-        qk = torch.zeros(N, 2, H, 64, device=DEV)
-        qk[..., :D] = torch.nn.functional.normalize(torch.stack([q, k], 1).float().view(N, 2, H, D), dim=-1)
-        gates = torch.stack([decay, torch.full_like(decay, 0.7)], -1).contiguous()
-        q, k, decay = qk[:, 0].view(N, -1), qk[:, 1].view(N, -1), gates.view(N, -1)
+        x, decay = torch.cat([q, k, v], 1), rnd((N, 2 * H), f32, 3)          # the second half: logits of the decays
+        q, k, v = (x[:, i * H * D:(i + 1) * H * D] for i in range(3))
+        taps = rnd((3 * H * D, 4), f32, 5)
     calls = {"retention": lambda s: ops.retention(x, (0, H * D, 2 * H * D), H, D, D, None, 0, 0.1, per_head, s, 0, ctx),
              "lightning": lambda s: ops.linear_attention(x, (0, H * D, 2 * H * D), H, D, D, 0.1, True, per_head, None, None, 1.0, s, 0, ctx),
              "gated": lambda s: ops.linear_attention(x, (0, H * D, 2 * H * D), H, D, D, 0.1, False, None, decay, torch.zeros(H * D, device=DEV), 4.0, s, 0, ctx),
              "prepared": lambda s: ops.linear_attention(x, (0, 0, 2 * H * D), H, D, D + 1, 1.0, False, None, None, None, 1.0, s, 0, ctx, prepared=given, ones=1),
              "bonus": lambda s: ops.wkv(q, k, v, decay, v, rnd((H, D), f32, 8), rnd((H * D,), f32, 8), 1e-5, H, s, 0, ctx),
              "step": lambda s: ops.ssd(xbc, decay, one, one, one, H, 40, D, 1, s, 0, ctx),
-             "delta": lambda s: delta_rule(ops, ctx, qk, v, gates, H, H, D, D, s)}
-    values = {"prepared": D + 1, "step": 40}.get(kind, D)
+             "delta": lambda s: ops.delta_rule(x, 0, H, H, D, D, taps, 1.0, 1e-6, decay, one, one, s, 0, 9 * H * D, ctx)}
+    parts = {"q": q, "k": k, "v": v, "decay": None if kind in ("retention", "lightning") else decay}
+    return calls[kind], parts, H * D * {"prepared": D + 1, "step": 40, "delta": D + 9}.get(kind, D)
+
+
+# (token, what is not finite there): in the first and the last place of a run, in a run's middle, in the last token
+BROKEN = {"results": [(3, "v", float("inf")), (79, "v", float("nan")), (200, "q", float("nan"))],
+          "keys": [(37, "k", float("inf")), (95, "v", float("-inf")), (170, "k", float("nan"))],
+          "steps": [(64, "decay", float("nan")), (81, "k", float("nan")), (130, "decay", float("nan"))]}
+
+
+@pytest.mark.parametrize("dtype", list(DTYPES))
+@pytest.mark.parametrize("where", list(BROKEN))
+@pytest.mark.parametrize("kind", KINDS)
+def test_what_is_not_finite_touches_no_earlier_token(kernel_sets, dtype, where, kind):
+    """Results and states that the walk leaves finite are finite in chunks too, and what they are without (the 16 sums of a run
+    with such a value are added up in another order: 16 roundings of 2^-24 of the largest)."""
+    ops, dt, ctx = kernel_sets[dtype], DTYPES[dtype], step_of([65, 16, 17, 200])
+    call, parts, size = layer(ops, dt, kind, ctx)
     kept = ops.gated_group_norm
     ops.gated_group_norm = lambda raw, *a, **kw: raw
 
     def run(least):
-        state = rnd((4, H * D * values), f32, 9)
-        ops.scan_from = least
-        return calls[kind](state), state
+        state = rnd((4, size), torch.float32, 9)
+        ops.scan_from = ops.delta_scan_from = least
+        return call(state), state
     try:
         sound = run(1)
         spoiled = 0
         for token, what, value in BROKEN[where]:
-            if what == "decay" and kind in ("retention", "lightning"):
-                continue                                       # a constant of the head
-            t = {"q": q, "k": k, "v": v, "decay": decay}[what]
-            t[token, token % t.shape[1]] = value
-            spoiled += 1
+            if parts[what] is not None:
+                parts[what][token, token % parts[what].shape[1]] = value
+                spoiled += 1
         walk, chunks = run(0), run(1)
     finally:
         ops.gated_group_norm = kept
-        del ops.scan_from
+        del ops.scan_from, ops.delta_scan_from
     for a, b, c in zip(walk, chunks, sound):
         fine = a.isfinite()
         assert (not spoiled or not fine.all()) and fine.any()
         assert torch.equal(b.isfinite(), fine)
         assert float((b[fine] - c[fine]).abs().max()) <= 16 * 2.0 ** -24 * float(c.abs().max())
+
+
+@pytest.mark.parametrize("dtype", list(DTYPES))
+@pytest.mark.parametrize("rounds", [False, True])
+@pytest.mark.parametrize("kind", KINDS)
+def test_short_sequences_walk_beside_long_ones(kernel_sets, dtype, rounds, kind):
+    """Decoding rows and short portions before, between and behind portions in chunks, more than a wave looks at in one go:
+    the short ones' results and states are the walk's bits, the long ones' those of a step that is in chunks whole."""
+    lengths = [1] * 40 + [300, 1, 9] + [1] * 30 + [129, 1, 17, 400] + [1] * 3
+    ops, dt, ctx = kernel_sets[dtype], DTYPES[dtype], step_of(lengths)
+    call, _, size = layer(ops, dt, kind, ctx)
+    kept, got = ops.gated_group_norm, {}
+    ops.gated_group_norm = lambda raw, *a, **kw: raw
+    if rounds:
+        ops.scan_scratch = 1
+    try:
+        for name, least in (("walk", 0), ("whole", 1), ("split", 1)):
+            ops.scan_from = ops.delta_scan_from = least
+            if name == "split":
+                ops._chunks_from = lambda *a, **kw: 100
+                ctx.host = {"seq_qstart": ctx.seq_qstart.cpu().numpy()}
+            state = rnd((len(lengths), size), torch.float32, 9)
+            got[name] = call(state), state
+    finally:
+        ops.gated_group_norm = kept
+        for n in ("scan_from", "delta_scan_from", "_chunks_from", "scan_scratch"):
+            vars(ops).pop(n, None)
+    starts, rows = ctx.seq_qstart.tolist(), ctx.seq_rows.tolist()
+    for i, n in enumerate(lengths):
+        like = got["whole" if n >= 100 else "walk"]
+        assert torch.equal(got["split"][0][starts[i]:starts[i + 1]], like[0][starts[i]:starts[i + 1]]), (i, n)
+        assert torch.equal(got["split"][1][rows[i]], like[1][rows[i]]), (i, n)
