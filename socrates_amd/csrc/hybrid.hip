@@ -790,7 +790,8 @@ __device__ __forceinline__ int ga_swap(int row) { return (row >> 1) & 7; }
 __device__ __forceinline__ void ga_load(const bf16* from, uint16_t* lds) {
     // (the wave's LDS address goes through m0; nothing comes back in registers)
     const uint32_t to = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t*)lds;
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(__builtin_amdgcn_readfirstlane(to)), "v"(from) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(__builtin_amdgcn_readfirstlane(to)), "v"(from)
+                 : "memory", "m0");
 }
 
 template <bool GLU, typename TO>
