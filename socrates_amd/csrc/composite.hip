@@ -654,7 +654,8 @@ __global__ void glu_gelu_kernel(const T* __restrict__ gate_up, T* __restrict__ o
 
 // The same for ff and ld in steps of 8 at addresses in steps of 16 bytes: eight consecutive elements to a lane, so one
 // division by ff and two or four wide loads for eight of them (2,048 rows, ff 9,728, bf16: 23 against 42 us; the 120 MB
-// go at the rate of a copy). Same arithmetic.
+// go at the rate of a copy). Same arithmetic. Eight tanhf behind each other are the longer way while they leave compute units
+// without a workgroup: 1 row 2.6 against 2.0 us, 16 2.7 / 2.2, 32 2.7 / 2.4, 64 (304 workgroups) 2.9 / 3.0, 128 3.5 / 4.4.
 template <typename T>
 __global__ void __launch_bounds__(256)
 glu_gelu_vec8_kernel(const T* __restrict__ gate_up, T* __restrict__ out, size_t groups, int ff, int ld) {
@@ -685,7 +686,7 @@ SOC_EXPORT int soc_glu_gelu(const void* gate_up, void* out, int N, int ff, int l
     const size_t total = (size_t)N * ff;
     if (!total) return 0;
     if (ff < 1 || 2 * ff > ld) return (int)hipErrorInvalidValue;
-    if (ff % 8 == 0 && ld % 8 == 0 && ((uintptr_t)gate_up | (uintptr_t)out) % 16 == 0 && total / 8 <= (size_t)0x7fffff00) {
+    if (ff % 8 == 0 && ld % 8 == 0 && ((uintptr_t)gate_up | (uintptr_t)out) % 16 == 0 && total / 8 >= 256 * 256 && total / 8 <= (size_t)0x7fffff00) {
         const size_t groups = total / 8;
         const dim3 grid((unsigned)((groups + 255) / 256));
         if (dtype == 0)

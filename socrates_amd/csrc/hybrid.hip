@@ -966,7 +966,8 @@ __global__ void moe_combine_kernel(const float* __restrict__ y, const int* __res
 
 // The same for d in steps of 4 at addresses in steps of 16 bytes (8 for two-byte types), top of them known to the
 // compiler: four elements to a lane and every expert's row on its way before the first is added, where the kernel above
-// waits for one after the other (2,048 tokens, d 2,560, 4 experts and a shared one: 22 against 43 us, the rate of its 115 MB).
+// waits for one after the other (2,048 tokens, d 2,560, 4 experts and a shared one: 22 against 43 us, the rate of its 115 MB;
+// 1 token 1.9 against 2.3, 16 2.1 / 2.4, 64 2.2 / 2.6, 512 3.8 / 7.4).
 // Same additions in the same order.
 template <typename T, int TOP>
 __global__ void __launch_bounds__(256)

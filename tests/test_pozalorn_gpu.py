@@ -498,3 +498,19 @@ def test_gelu_gate_in_runs_of_eight(kernel_sets, dtype, N, ff, ld):
     # 1 + tanh loses the low bits where tanh is near -1: steps of 2^-24 of g u, a few of them
     slack = 8 * 2.0 ** -24 * (g * u).abs() + (2.0 ** -8 if dt == torch.bfloat16 else 0.0) * want.abs()
     assert ((ops.glu_gelu(x, ff).double() - want).abs() <= slack + 1e-30).all()
+
+
+@pytest.mark.parametrize("dtype", list(DTYPES))
+@pytest.mark.parametrize("N,ff,ld", [(63, 8192, 16384), (64, 8192, 16384), (65, 8200, 16416), (64, 8192, 16388), (64, 8196, 16400)])
+def test_gelu_gate_of_many_rows(kernel_sets, dtype, N, ff, ld):
+    """Around the number of elements from which a lane takes eight, with rows that it may not read so; each row's bits are those
+    of the row alone, which a lane per element makes."""
+    ops = kernel_sets[dtype]
+    x = torch.randn((N, ld), generator=torch.Generator().manual_seed(N)).to(DTYPES[dtype]).to(DEV)
+    got = ops.glu_gelu(x, ff)
+    for n in (0, 1, N // 2, N - 1):
+        assert torch.equal(got[n], ops.glu_gelu(x[n:n + 1].contiguous(), ff)[0])
+    g, u = x[:, :ff].double(), x[:, ff:2 * ff].double()
+    want = torch.nn.functional.gelu(g, approximate="tanh") * u
+    slack = 8 * 2.0 ** -24 * (g * u).abs() + (2.0 ** -8 if dtype == "bfloat16" else 0.0) * want.abs()
+    assert ((got.double() - want).abs() <= slack + 1e-30).all()
