@@ -6,7 +6,6 @@ from __future__ import annotations
 
 from ctypes import c_int, c_longlong, c_void_p
 
-import numpy as np
 import torch
 
 from .build import load_library
@@ -24,14 +23,13 @@ def _tiles(D, Dv):
 
 class Scan:
     # Tokens of a step's longest portion from which it is taken in chunks (0: never). Measured in us, walk -> chunks, at
-    # the heads of a 4B-sized layer: 64 tokens: retention 34 -> 42, gated linear attention 34 -> 57, wkv 30 -> 48,
-    # ssd 33 -> 32; 100 tokens: 46 -> 40, 48 -> 58, 39 -> 45, 48 -> 33; 300: 149 -> 60, 162 -> 72, 85 -> 44, 175 -> 63.
-    # The gated delta rule, whose chunk costs more and whose walk is faster: 200 tokens 62 -> 73, 256: 76 -> 68, 300: 89 -> 75.
-    # (For the others chunks stay ahead with several sequences: 5 of 200 tokens: 122 -> 77, 137 -> 80, 144 -> 71, 248 -> 117.)
+    # the heads of a 4B-sized layer: 64 tokens: retention 30 -> 41, gated linear attention 33 -> 54, wkv 30 -> 41,
+    # ssd 33 -> 31; 100 tokens: 43 -> 41, 47 -> 54, 33 -> 41, 48 -> 33; 300: 142 -> 50, 158 -> 63, 80 -> 41, 127 -> 48.
+    # The gated delta rule, whose chunk costs more and whose walk is faster: 200 tokens 59 -> 69, 256: 73 -> 71, 300: 83 -> 72.
     # A step of so few tokens is bound by the host's launches, of which chunks have two more per layer, so the line lies
-    # where whole steps gain (us, walk -> chunks, one prompt unless two are named): linear attention, 8 layers, 140 tokens
-    # 2,290 -> 2,360, 2 x 162 2,700 -> 2,470, 200 2,680 -> 2,390; retention, 6 layers, 140 3,140 -> 3,080; wkv and ssd, 6
-    # layers, 2 x 162 2,230 -> 2,310, 200 2,190 -> 2,260, 300 2,360 -> 2,290, 500 2,990 -> 2,370: from 8 / 5 as many.
+    # where whole steps gain (us, walk -> chunks, one prompt): linear attention, 8 layers, 140 tokens 2,240 -> 2,360, 200
+    # 2,480 -> 2,370; retention, 6 layers, 200 3,300 -> 3,180; wkv and ssd, 6 layers, 200 2,030 -> 2,100, 256 2,020 -> 2,090,
+    # 300 2,140 -> 2,160, 500 2,760 -> 2,160: from twice as many; the delta rule, 4 layers, 256 2,500 -> 2,490, 300 2,850 -> 2,800.
     scan_from, delta_scan_from = 160, 256
     scan_scratch = 1 << 30           # bytes of scratch that one launch over all chunks may take; beyond, in rounds
 
@@ -54,45 +52,61 @@ class Scan:
         a walk: 12 and the most of ``token`` for every token of its longest sequence, ``busy`` for every token and block,
         its states' bytes; chunks: ``start`` and ``chunk`` for every chunk and block. Fitted to 20 heads of 128 x 128, 10 of
         128 x 256, 40 of 64 x 64 and 80 of 128 x 64; measured, all walk -> all in chunks -> as this says: 160 tokens beside 50
-        decoding rows: retention 93 -> 152 -> 84, ssd 116 -> 324 -> 116 (below its least), 2,000 beside 60: 890 -> 294 -> 154,
-        1,149 -> 609 -> 286; 500 beside 60: wkv 158 -> 187 -> 90, linear attention 270 -> 263 -> 114.
+        decoding rows: retention 93 -> 154 -> 83; 500 beside 60: wkv 158 -> 187 -> 89, linear attention 270 -> 263 -> 114;
+        2,000 beside 60: retention 890 -> 299 -> 156, ssd 1,149 -> 606 -> 286.
         A step that does not say its lengths on the host is taken in chunks whole."""
         if not self._in_chunks(ctx, D, least):
             return 0
-        lens = self._portion_lengths(ctx)
-        if lens is None:
+        step = self._lengths_and_lines(ctx)
+        if step is None:
             return 1
-        lines = ctx.host.setdefault("chunks_from", {})
+        lens, lines = step
         key = (D, cols, token, busy, start, chunk)
         if key not in lines:
-            lens = np.sort(lens)[::-1]
-            longest, walking = np.append(lens, 0), np.arange(len(lens), -1, -1)               # with the i longest in chunks
-            tokens = lens.sum() - np.append(0, np.cumsum(lens))
-            cost = np.maximum((0.12 + 0.0028 * D if token is None else token) * longest, busy * cols * tokens)
-            cost = np.maximum(cost, cols * D * 128 / 4.8e6 * walking) + 12.0 * (walking > 0)
-            cost[1:] += start + chunk * cols * np.cumsum(-(-lens // CHUNK))
-            cost[1:-1][lens[:-1] == lens[1:]] = np.inf                                        # equals go together
-            best = int(np.argmin(cost))
-            lines[key] = int(lens[best - 1]) if best else 0
+            token = 0.12 + 0.0028 * D if token is None else token
+            state, tokens, chunks, n = cols * D * 128 / 4.8e6, sum(lens), 0, len(lens)
+            best, lines[key] = 12.0 + max(token * lens[0], busy * cols * tokens, state * n), 0
+            for i, length in enumerate(lens, 1):
+                chunks, tokens = chunks - (-length // CHUNK), tokens - length
+                if i < n and lens[i] == length:
+                    continue                                      # equals go together
+                cost = start + chunk * cols * chunks
+                if i < n:
+                    cost += 12.0 + max(token * lens[i], busy * cols * tokens, state * (n - i))
+                if cost < best:
+                    best, lines[key] = cost, length
         return lines[key]
+
+    def _lengths_and_lines(self, ctx):
+        """(a step's lengths, the longest first, what was found out about them), kept with the step: every layer asks. None
+        if the step does not say its lengths."""
+        host = getattr(ctx, "host", None)
+        if host is None or "seq_qstart" not in host:
+            return None
+        if "chunks_from" not in host:
+            host["chunks_from"] = (sorted(self._portion_lengths(ctx).tolist(), reverse=True), {})
+        return host["chunks_from"]
 
     def _delta_in_chunks(self, ctx, N, D, H, Dv):
         """The same for the gated delta rule, whose chunk costs more and whose walk is faster. Measured in us, walk -> chunks, 20
-        heads of 128 x 128: 2 sequences of 300 tokens 96 -> 82, of 500 146 -> 128, of 1,000 271 -> 197; 3 of 300 101 -> 130,
-        of 500 148 -> 147, of 1,000 280 -> 270; 5 of 300 139 -> 147, of 1,000 395 -> 455; 8 of 1,000 568 -> 682; 300 beside 60
-        decoding rows 93 -> 116, 2,000 beside 60 492 -> 283."""
+        heads of 128 x 128: 2 sequences of 300 tokens 94 -> 84, of 500 144 -> 133, of 1,000 271 -> 208; 3 of 300 96 -> 135,
+        of 500 148 -> 157, of 1,000 278 -> 286; 5 of 1,000 394 -> 479; 8 of 1,000 549 -> 710; 300 beside 60 decoding rows that
+        walk 93 -> 116, 500 141 -> 126, 2,000 492 -> 281."""
         cols = H * -(-Dv // 16)
-        if self._portion_lengths(ctx) is None and N * cols >= 600 * (ctx.max_q_len - 165):
+        if self._lengths_and_lines(ctx) is None and N * cols >= 600 * (ctx.max_q_len - 165):
             return 0
         return self._chunks_from(ctx, D, cols, self.delta_scan_from, token=0.255, busy=5.5e-4, start=48.0, chunk=0.032)
 
     def _split(self, ctx, least):
         """(most sequences that go in chunks, whether others walk) of a step taken in chunks from ``least`` tokens on."""
-        lens = self._portion_lengths(ctx)
-        if lens is None or least <= 1:
+        step = None if least <= 1 else self._lengths_and_lines(ctx)
+        if step is None:
             return ctx.n_seqs, False
-        n_long = int((lens >= least).sum())
-        return n_long, n_long < ctx.n_seqs
+        lens, lines = step
+        if least not in lines:
+            n_long = sum(n >= least for n in lens)
+            lines[least] = n_long, n_long < ctx.n_seqs
+        return lines[least]
 
     def _scan_scratch(self, ctx, N, n_long, sizes):
         """(chunks of the longest portion, chunks of every sequence that one launch takes, whether those lie one behind the

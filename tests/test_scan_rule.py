@@ -24,7 +24,7 @@ def test_decoding_rows_are_not_in_chunks(lengths, least):
     """20 heads of 128 x 128: 160 blocks of 16 columns."""
     rule, ctx = Rule(), step(lengths)
     assert rule._chunks_from(ctx, 128, 160) == least
-    assert rule._split(ctx, least or 1 << 20) == (sum(n >= least for n in lengths) if least else 0, not least or min(lengths) < least)
+    assert rule._split(ctx, least or 1 << 20) == (sum(n >= (least or 1 << 20) for n in lengths), min(lengths) < (least or 1 << 20))
     assert not rule._chunks_from(ctx, 129, 160)
 
 
