@@ -543,7 +543,7 @@ moe_sort_kernel(const int* __restrict__ idx, int M, int E, int TM, int max_tiles
                 if (tile0[mid] <= t) lo = mid; else hi = mid - 1;
             }
             e = lo;
-            // (256 places: an expert's places in as many tiles, of nearly equal size in blocks of 16)
+            // (256 places: an expert's places in as few tiles as hold them, of nearly equal size in blocks of 16)
             const int n = tile0[e + 1] - tile0[e], rows = TM == 256 ? ((count[e] + n - 1) / n + 15) / 16 * 16 : TM;
             first = start[e] + (t - tile0[e]) * rows;
         }
@@ -778,12 +778,14 @@ grouped_mfma_kernel(const bf16* __restrict__ x, int ldx, const int* __restrict__
 // swapped among themselves instead, by a pattern over the rows that lets 16 rows of one k be read without bank
 // conflicts. The weights are the first operand: a lane ends up with four neighbouring outputs of one place.
 // An expert's places are cut into tiles of nearly equal size (moe_sort), because each tile reads the expert's weights
-// again. Workgroups go round-robin over the eight XCDs; each XCD gets a run of (tile, block of outputs) in order,
+// again and one with few places does little for it. A tile's products go by 64 places, though, so the even cut can multiply more
+// padding than full tiles and a rest: 292 places are 160 + 132, computed as 384 rows (256 + 36: 320), 333 are 176 + 157 (384
+// either way), 272 are 144 + 128 (320 either way). Workgroups go round-robin over the eight XCDs; each XCD gets a run of (tile, block of outputs) in order,
 // so that the tiles of an expert meet in one L2. Measured against the kernel above (tiles of 128) at 32 experts of 2,432
 // and a width of 2,560, us: 8,320 places gate / up 469 -> 388, down 285 -> 252; 12,000 places 550 -> 436 and 347 -> 265
-// (685 TFLOP/s; its weights alone take 166 us at a copy's rate). Bound by the LDS reads beside the products and,
-// with one workgroup per compute unit, by the last round of workgroups, which is seldom full. K is a multiple of 64; places and weight rows outside are read from
-// a row that exists and not written.
+// (685 TFLOP/s; its weights alone take 166 us at a copy's rate). Bound by the LDS reads beside the products, that padding and,
+// with one workgroup per compute unit, by the last round of workgroups, which is seldom full. K is a multiple of 64; places
+// and weight rows outside are read from a row that exists and not written.
 template <int N> struct ga_blocks { static constexpr int value = N; };
 __device__ __forceinline__ int ga_swap(int row) { return (row >> 1) & 7; }
 

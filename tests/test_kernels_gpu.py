@@ -563,6 +563,27 @@ def test_float32_products_on_the_matrix_cores(kernel_sets, M, N, K, a, w):
     assert not hip.forms
 
 
+@pytest.mark.parametrize("K,N", [(2560, 320), (9728, 192), (516, 1000)])
+@pytest.mark.parametrize("w", [torch.float32, torch.bfloat16])
+def test_float32_rows_in_steps_of_other_sizes(kernel_sets, K, N, w):
+    """How K is cut depends on the rows of the step, so the same row's sums are added up in another order beside other rows.
+    Each is within K roundings of 2^-24 of the sum of its products' sizes, in whatever order, so two differ by twice that at
+    most; what is seen is a few roundings of the result (rows alone against rows in steps of up to 300)."""
+    hip, _ = kernel_sets[torch.float32]
+    x, weight = rnd((300, K), torch.float32, 41), rnd((N, K), w, 42)
+    sizes = x.double().abs() @ weight.double().abs().T
+    want = x.double() @ weight.double().T
+    alone = torch.cat([hip.linear(x[i:i + 1].contiguous(), weight) for i in (0, 1, 7)])
+    for rows in (2, 8, 40, 131, 300):
+        got = hip.linear(x[:rows].contiguous(), weight)
+        some = [i for i in (0, 1, 7) if i < rows]
+        off = (got[some] - alone[:len(some)]).double().abs()
+        assert (off <= 2 * K * 2.0 ** -24 * sizes[some]).all()
+        assert float(off.norm() / want[some].norm()) <= 16 * 2.0 ** -24
+        again = hip.linear(x[:rows].contiguous(), weight)
+        assert torch.equal(got, again)
+
+
 def test_linear_float32_is_not_reduced_precision(kernel_sets):
     """Values that bfloat16 or a 19-bit matrix mode would round away survive."""
     hip, _ = kernel_sets[torch.float32]

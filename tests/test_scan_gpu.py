@@ -82,11 +82,14 @@ def check(ops, call, want, S0, S1, slack=2e-7):
 @pytest.mark.parametrize("lengths", LENGTHS)
 @pytest.mark.parametrize("H,D,Dv", [(2, 64, 64), (1, 128, 256), (3, 20, 33), (1, 100, 65)])
 @pytest.mark.parametrize("kind", ["head", "channel", "prepared"])
-def test_linear_attention_in_chunks(kernel_sets, dtype, lengths, H, D, Dv, kind):
+@pytest.mark.parametrize("lead", [5, 0])
+def test_linear_attention_in_chunks(kernel_sets, dtype, lengths, H, D, Dv, kind, lead):
+    """``lead``: columns of a row before the queries; with 5 nothing starts on four elements, with none (and rows in steps of
+    eight) everything may, up to an odd number of value columns beside one of ones."""
     ops, dt, ctx = kernel_sets[dtype], DTYPES[dtype], step_of(lengths)
     N = ctx.n_tokens
-    x = rnd((N, 5 + 2 * H * D + H * Dv), dt, 1, 0.5)
-    cols = (5, 5 + H * D, 5 + 2 * H * D)
+    x = rnd((N, lead + 2 * H * D + H * Dv + (0 if lead else -(2 * H * D + H * Dv) % 8)), dt, 1, 0.5)
+    cols = (lead, lead + H * D, lead + 2 * H * D)
     q, k = (x[:, c:c + H * D].double().view(N, H, D) for c in cols[:2])
     v = x[:, cols[2]:cols[2] + H * Dv].double().view(N, H, Dv)
     S0 = rnd((len(lengths), 3 + H * D * Dv), torch.float32, 2)
