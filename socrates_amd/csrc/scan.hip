@@ -99,13 +99,22 @@ __device__ __forceinline__ bool scan_search(const Args& a, ScanPlace& at, Is is)
     return false;
 }
 // the sequence and the chunk of number b; or, of the l-th such sequence, the first chunk's number
+// (one sequence alone is not searched for: its chunks' numbers are their own)
 template <typename Args> __device__ __forceinline__ bool scan_chunk(const Args& a, int b, ScanPlace& at) {
+    if (a.n_seqs == 1) {
+        at.seq = 0; at.c = at.slot = b;
+        return true;
+    }
     if (!scan_search(a, at, [&](int, int slot, int n) { return slot <= b && b < slot + n; })) return false;
     at.c = b - at.slot;
     at.slot = b;
     return true;
 }
 template <typename Args> __device__ __forceinline__ bool scan_sequence(const Args& a, int which, ScanPlace& at) {
+    if (a.n_seqs == 1) {
+        at.seq = at.slot = 0;
+        return true;
+    }
     return scan_search(a, at, [&](int l, int, int) { return l == which; });
 }
 

@@ -29,7 +29,7 @@ class Scan:
     # A step of so few tokens is bound by the host's launches, of which chunks have two more per layer, so the line lies
     # where whole steps gain (us, walk -> chunks, one prompt): linear attention, 8 layers, 140 tokens 2,240 -> 2,360, 200
     # 2,480 -> 2,370; retention, 6 layers, 200 3,300 -> 3,180; wkv and ssd, 6 layers, 200 2,030 -> 2,100, 256 2,020 -> 2,090,
-    # 300 2,140 -> 2,160, 500 2,760 -> 2,160: from twice as many; the delta rule, 4 layers, 256 2,500 -> 2,490, 300 2,850 -> 2,800.
+    # 300 2,110 -> 2,000 to 2,160, 500 2,740 -> 2,100: from 9 / 5 as many; the delta rule, 4 layers, 256 2,500 -> 2,490, 300 2,850 -> 2,800.
     scan_from, delta_scan_from = 160, 256
     scan_scratch = 1 << 30           # bytes of scratch that one launch over all chunks may take; beyond, in rounds
 
