@@ -45,12 +45,12 @@ class Scan:
         and decays of a chunk fit LDS. ``least``: tokens, in place of ``scan_from``."""
         return 0 < (self.scan_from if least is None else least) <= ctx.max_q_len and D <= 128
 
-    def _chunks_from(self, ctx, D, cols, least=None, token=None, busy=7e-4, start=32.0, chunk=0.0145):
+    def _chunks_from(self, ctx, D, cols, least=None, token=None, serial=0.0, busy=7e-4, start=32.0, chunk=0.0145):
         """Tokens from which on a sequence of the step is taken in chunks (0: all walk): of all such lines, the one whose estimate
         is least. A chunk costs the same however few of its tokens there are, so decoding rows walk beside a portion in
         chunks. With ``cols`` blocks of 16 columns in the states of all heads, in us:
-        a walk: 12 and the most of ``token`` for every token of its longest sequence, ``busy`` for every token and block,
-        its states' bytes; chunks: ``start`` and ``chunk`` for every chunk and block. Fitted to 20 heads of 128 x 128, 10 of
+        a walk: 12 and the most of ``token`` for every token of its longest sequence, ``serial`` for those and ``busy`` for every
+        token and block, its states' bytes; chunks: ``start`` and ``chunk`` for every chunk and block. Fitted to 20 heads of 128 x 128, 10 of
         128 x 256, 40 of 64 x 64 and 80 of 128 x 64; measured, all walk -> all in chunks -> as this says: 160 tokens beside 50
         decoding rows: retention 93 -> 154 -> 83; 500 beside 60: wkv 158 -> 187 -> 89, linear attention 270 -> 263 -> 114;
         2,000 beside 60: retention 890 -> 299 -> 156, ssd 1,149 -> 606 -> 286.
@@ -61,18 +61,18 @@ class Scan:
         if step is None:
             return 1
         lens, lines = step
-        key = (D, cols, token, busy, start, chunk)
+        key = (D, cols, token, serial, busy, start, chunk)
         if key not in lines:
             token = 0.12 + 0.0028 * D if token is None else token
             state, tokens, chunks, n = cols * D * 128 / 4.8e6, sum(lens), 0, len(lens)
-            best, lines[key] = 12.0 + max(token * lens[0], busy * cols * tokens, state * n), 0
+            best, lines[key] = 12.0 + max(token * lens[0], serial * lens[0] + busy * cols * tokens, state * n), 0
             for i, length in enumerate(lens, 1):
                 chunks, tokens = chunks - (-length // CHUNK), tokens - length
                 if i < n and lens[i] == length:
                     continue                                      # equals go together
                 cost = start + chunk * cols * chunks
                 if i < n:
-                    cost += 12.0 + max(token * lens[i], busy * cols * tokens, state * (n - i))
+                    cost += 12.0 + max(token * lens[i], serial * lens[i] + busy * cols * tokens, state * (n - i))
                 if cost < best:
                     best, lines[key] = cost, length
         return lines[key]
@@ -89,13 +89,17 @@ class Scan:
 
     def _delta_in_chunks(self, ctx, N, D, H, Dv):
         """The same for the gated delta rule, whose chunk costs more and whose walk is faster. Measured in us, walk -> chunks, 20
-        heads of 128 x 128: 2 sequences of 300 tokens 94 -> 84, of 500 144 -> 133, of 1,000 271 -> 208; 3 of 300 96 -> 135,
-        of 500 148 -> 157, of 1,000 278 -> 286; 5 of 1,000 394 -> 479; 8 of 1,000 549 -> 710; 300 beside 60 decoding rows that
-        walk 93 -> 116, 500 141 -> 126, 2,000 492 -> 281."""
+        heads of 128 x 128: 1,000 tokens 238 -> 133, 2 sequences of 500 149 -> 132, 3 of 500 148 -> 157, of 1,000 281 -> 286, 8 of
+        1,000 557 -> 707; 32 heads: 256 tokens 76 -> 69, 3 of 1,000 359 -> 412, 8 of 1,000 791 -> 1,068; 8 heads: 3 of 1,000
+        241 -> 142, 8 of 1,000 309 -> 287; 10 of 128 x 256: 3 of 1,000 284 -> 238, 8 of 1,000 561 -> 639; 40 of 64 x 64: 256
+        65 -> 44, 3 of 1,000 243 -> 237, 8 of 1,000 441 -> 627; 16 of 64 x 128: 8 of 1,000 310 -> 305. 20 heads, 300 tokens beside 60
+        decoding rows that walk 93 -> 116, 1,000 256 -> 187."""
         cols = H * -(-Dv // 16)
         if self._lengths_and_lines(ctx) is None and N * cols >= 600 * (ctx.max_q_len - 165):
             return 0
-        return self._chunks_from(ctx, D, cols, self.delta_scan_from, token=0.255, busy=5.5e-4, start=48.0, chunk=0.032)
+        wide = D / 128.0
+        return self._chunks_from(ctx, D, cols, self.delta_scan_from, token=0.171 + 0.058 * wide, serial=0.088 + 0.042 * wide,
+                                 busy=(2.2 + 1.04 * wide) * 1e-4, start=36.0, chunk=0.02 + 0.012 * wide)
 
     def _split(self, ctx, least):
         """(most sequences that go in chunks, whether others walk) of a step taken in chunks from ``least`` tokens on."""

@@ -34,7 +34,7 @@ def test_heads_that_fill_the_chip_side_by_side_are_not_walked_in_turns():
 
 
 @pytest.mark.parametrize("lengths,least", [
-    ([300], 300), ([200], 0), ([300] + [1] * 60, 0), ([2000] + [1] * 60, 2000), ([500] * 2, 500), ([500] * 3, 0), ([1000] * 5, 0)])
+    ([300], 300), ([200], 0), ([300] + [1] * 60, 0), ([2000] + [1] * 60, 2000), ([500] * 2, 500), ([500] * 3, 0), ([1000] * 5, 0), ([1000] * 8, 0)])
 def test_the_delta_rule_weighs_its_chunks(lengths, least):
     assert Rule()._delta_in_chunks(step(lengths), sum(lengths), 128, 20, 128) == least
 
