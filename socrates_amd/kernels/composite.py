@@ -201,7 +201,7 @@ class Composite:
         # walk (each of a head's workgroups would take them again); single tokens and short portions where they
         # are staged
         prep = prepared
-        least = self._chunks_from(ctx, D, H * -(-Dv // 16))
+        least = self._chunks_from(ctx, D, H * -(-Dv // 16), 23 / 20)
         if prepared is None and (least or (activate or z is not None) and ctx.max_q_len >= self.linear_prepare_ahead):
             prep = torch.empty((N, 3 if z is not None else 2, H * D), dtype=torch.float32, device=self.device)
         if least:

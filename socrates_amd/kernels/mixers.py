@@ -161,7 +161,7 @@ class Mixers:
         self._want(gain, "gain", torch.float32, (C,))
         stride = self._state(state, offset, H * D * D, ctx)
         raw = torch.empty((N, C), dtype=torch.float32, device=self.device)
-        least = self._chunks_from(ctx, D, H * -(-D // 16), self.scan_from * 9 // 5)
+        least = self._chunks_from(ctx, D, H * -(-D // 16), 9 / 5)
         if not least or self._scan(BONUS, _ptr(r), C, D, _ptr(k), C, D, _ptr(v), C, D, _ptr(decay), H, D, D, state, stride, offset, ctx,
                                    N, raw, least, q_f32=False, lda=C, params=[_ptr(bonus)]):
             _check(self._mixers().soc_wkv(_ptr(r), _ptr(k), _ptr(v), _ptr(decay), _ptr(bonus), c_int(H), c_int(D), _ptr(state),
@@ -201,7 +201,7 @@ class Mixers:
             raise KernelError(f"ssd: {H} heads in {G} groups, state {Ns}, head size {P}")
         stride = self._state(state, offset, H * Ns * P, ctx)
         out = torch.empty((N, H * P), dtype=torch.float32, device=self.device)
-        least = self._chunks_from(ctx, Ns, H * -(-P // 16), self.scan_from * 9 // 5)
+        least = self._chunks_from(ctx, Ns, H * -(-P // 16), 9 / 5)
         if least:
             ld, item = H * P + 2 * G * Ns, xbc.element_size()
             b, c = (c_void_p(xbc.data_ptr() + (H * P + i * G * Ns) * item) for i in range(2))

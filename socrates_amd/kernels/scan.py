@@ -22,14 +22,10 @@ def _tiles(D, Dv):
 
 
 class Scan:
-    # Tokens of a step's longest portion from which it is taken in chunks (0: never). Measured in us, walk -> chunks, at
+    # Tokens of a step's longest portion from which it may be taken in chunks (0: never). Measured in us, walk -> chunks, at
     # the heads of a 4B-sized layer: 64 tokens: retention 30 -> 41, gated linear attention 33 -> 54, wkv 30 -> 41,
     # ssd 33 -> 31; 100 tokens: 43 -> 41, 47 -> 54, 33 -> 41, 48 -> 33; 300: 142 -> 50, 158 -> 63, 80 -> 41, 127 -> 48.
     # The gated delta rule, whose chunk costs more and whose walk is faster: 200 tokens 59 -> 69, 256: 73 -> 71, 300: 83 -> 72.
-    # A step of so few tokens is bound by the host's launches, of which chunks have two more per layer, so the line lies
-    # where whole steps gain (us, walk -> chunks, one prompt): linear attention, 8 layers, 140 tokens 2,240 -> 2,360, 200
-    # 2,480 -> 2,370; retention, 6 layers, 200 3,300 -> 3,180; wkv and ssd, 6 layers, 200 2,030 -> 2,100, 256 2,020 -> 2,090,
-    # 300 2,110 -> 2,000 to 2,160, 500 2,740 -> 2,100: from 9 / 5 as many; the delta rule, 4 layers, 256 2,500 -> 2,490, 300 2,850 -> 2,800.
     scan_from, delta_scan_from = 160, 256
     scan_scratch = 1 << 30           # bytes of scratch that one launch over all chunks may take; beyond, in rounds
 
@@ -45,34 +41,47 @@ class Scan:
         and decays of a chunk fit LDS. ``least``: tokens, in place of ``scan_from``."""
         return 0 < (self.scan_from if least is None else least) <= ctx.max_q_len and D <= 128
 
-    def _chunks_from(self, ctx, D, cols, least=None, token=None, serial=0.0, busy=7e-4, start=32.0, chunk=0.0145):
+    def _chunks_from(self, ctx, D, cols, work=1.0, least=None, token=None, serial=0.0, busy=7e-4, start=32.0, chunk=0.0145):
         """Tokens from which on a sequence of the step is taken in chunks (0: all walk): of all such lines, the one whose estimate
         is least. A chunk costs the same however few of its tokens there are, so decoding rows walk beside a portion in
         chunks. With ``cols`` blocks of 16 columns in the states of all heads, in us:
         a walk: 12 and the most of ``token`` for every token of its longest sequence, ``serial`` for those and ``busy`` for every
-        token and block, its states' bytes; chunks: ``start`` and ``chunk`` for every chunk and block. Fitted to 20 heads of 128 x 128, 10 of
-        128 x 256, 40 of 64 x 64 and 80 of 128 x 64; measured, all walk -> all in chunks -> as this says: 160 tokens beside 50
-        decoding rows: retention 93 -> 154 -> 83; 500 beside 60: wkv 158 -> 187 -> 89, linear attention 270 -> 263 -> 114;
-        2,000 beside 60: retention 890 -> 299 -> 156, ssd 1,149 -> 606 -> 286.
+        token and block, its states' bytes; chunks: ``start`` and ``chunk`` for every chunk and block; 15 for the launch of a walk
+        beside them. Fitted to 20 heads of 128 x 128, 10 of 128 x 256, 40 of 64 x 64 and 80 of 128 x 64; measured, all walk -> all
+        in chunks -> walks beside chunks: 160 tokens beside 50 decoding rows: retention 93 -> 154 -> 83; 500 beside 60: wkv
+        158 -> 187 -> 89, linear attention 270 -> 263 -> 114; 2,000 beside 60: retention 890 -> 299 -> 156, ssd 1,149 -> 606 -> 286.
+
+        A step of few tokens is bound by the host's launches, of which chunks have two more per layer and a walk beside them
+        another, so there the kernels' gain is none of the step's: the mean of the longest sequence and of all tokens
+        in chunks has to reach ``work`` times ``scan_from``, beside a walk 5 / 4 of that. Whole steps, us, walk -> chunks
+        throughout (-> beside a walk): wkv and ssd (9 / 5), 6 layers: 256 tokens 1,977 -> 1,989, 300 2,115 -> 2,014, 2 x 162 1,951
+        -> 2,022, 2 x 200 2,103 -> 2,042, 260 to 78 in five 2,854 -> 2,610, 300 beside 30 decoding rows 2,940 -> 3,002 -> 3,040,
+        500 beside 7 2,887 -> 2,383 -> 2,442; linear attention (23 / 20), 8 layers: 162 2,214 -> 2,375, 200 2,480 -> 2,348, 2 x 162 2,622 -> 2,423, 250
+        beside 7 2,926 -> 2,709 -> 2,816; retention (1), 6 layers: 162 2,894 -> 2,819, 162 beside 60 3,864 -> 3,999 -> 3,925, 250 beside 60
+        4,410 -> 4,533 -> 4,323.
         A step that does not say its lengths on the host is taken in chunks whole."""
         if not self._in_chunks(ctx, D, least):
             return 0
+        enough = 2 * work * (self.scan_from if least is None else least)
         step = self._lengths_and_lines(ctx)
         if step is None:
-            return 1
+            return int(2 * ctx.max_q_len >= enough)
         lens, lines = step
-        key = (D, cols, token, serial, busy, start, chunk)
+        key = (D, cols, work, token, serial, busy, start, chunk)
         if key not in lines:
             token = 0.12 + 0.0028 * D if token is None else token
-            state, tokens, chunks, n = cols * D * 128 / 4.8e6, sum(lens), 0, len(lens)
-            best, lines[key] = 12.0 + max(token * lens[0], serial * lens[0] + busy * cols * tokens, state * n), 0
+
+            def walk(longest, tokens, n):
+                return 12.0 + max(token * longest, serial * longest + busy * cols * tokens, cols * D * 128 / 4.8e6 * n)
+            left, chunks, n = sum(lens), 0, len(lens)
+            total, best, lines[key] = left, walk(lens[0], left, n), 0
             for i, length in enumerate(lens, 1):
-                chunks, tokens = chunks - (-length // CHUNK), tokens - length
+                chunks, left = chunks - (-length // CHUNK), left - length
                 if i < n and lens[i] == length:
                     continue                                      # equals go together
-                cost = start + chunk * cols * chunks
-                if i < n:
-                    cost += 12.0 + max(token * lens[i], serial * lens[i] + busy * cols * tokens, state * (n - i))
+                if 4 * (lens[0] + total - left) < (5 if i < n else 4) * enough:
+                    continue
+                cost = start + chunk * cols * chunks + (15.0 + walk(lens[i], left, n - i) if i < n else 0.0)
                 if cost < best:
                     best, lines[key] = cost, length
         return lines[key]
@@ -98,7 +107,7 @@ class Scan:
         if self._lengths_and_lines(ctx) is None and N * cols >= 600 * (ctx.max_q_len - 165):
             return 0
         wide = D / 128.0
-        return self._chunks_from(ctx, D, cols, self.delta_scan_from, token=0.171 + 0.058 * wide, serial=0.088 + 0.042 * wide,
+        return self._chunks_from(ctx, D, cols, least=self.delta_scan_from, token=0.171 + 0.058 * wide, serial=0.088 + 0.042 * wide,
                                  busy=(2.2 + 1.04 * wide) * 1e-4, start=36.0, chunk=0.02 + 0.012 * wide)
 
     def _split(self, ctx, least):

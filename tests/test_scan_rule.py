@@ -18,7 +18,7 @@ def step(lengths):
 
 
 @pytest.mark.parametrize("lengths,least", [
-    ([200], 200), ([100], 0), ([1] * 50 + [160], 160), ([200] + [1] * 60, 200), ([2000] + [1] * 60, 2000), ([200] * 5, 200),
+    ([200], 200), ([100], 0), ([1] * 50 + [160], 0), ([1] * 7 + [160], 1), ([200] + [1] * 60, 200), ([2000] + [1] * 60, 2000), ([200] * 5, 200),
     ([1100, 698, 330], 330), ([1, 500, 300, 1, 7], 1), ([1] * 20 + [500, 300, 7], 300), ([260] + [64] * 30, 64), ([1] * 64, 0)])
 def test_decoding_rows_are_not_in_chunks(lengths, least):
     """20 heads of 128 x 128: 160 blocks of 16 columns."""
@@ -37,6 +37,18 @@ def test_heads_that_fill_the_chip_side_by_side_are_not_walked_in_turns():
     ([300], 300), ([200], 0), ([300] + [1] * 60, 0), ([2000] + [1] * 60, 2000), ([500] * 2, 500), ([500] * 3, 0), ([1000] * 5, 0), ([1000] * 8, 0)])
 def test_the_delta_rule_weighs_its_chunks(lengths, least):
     assert Rule()._delta_in_chunks(step(lengths), sum(lengths), 128, 20, 128) == least
+
+
+@pytest.mark.parametrize("work,lengths,least", [
+    (9 / 5, [287], 0), (9 / 5, [288], 288), (9 / 5, [162] * 2, 0), (9 / 5, [200] * 2, 200), (9 / 5, [260, 215, 169, 124, 78], 78),
+    (9 / 5, [150] * 8, 0), (9 / 5, [300] + [1] * 30, 0), (9 / 5, [400] + [1] * 30, 400), (9 / 5, [300] + [1] * 7, 1),
+    (23 / 20, [183], 0), (23 / 20, [184], 184), (23 / 20, [162] * 2, 162), (23 / 20, [200] + [1] * 60, 0), (23 / 20, [250] + [1] * 60, 250)])
+def test_steps_that_wait_for_the_host_walk(work, lengths, least):
+    """Where a step of few tokens is no faster for its kernels, the launches decide: by the longest sequence and all tokens."""
+    rule = Rule()
+    assert rule._chunks_from(step(lengths), 64, 160, work) == least
+    rule.scan_from = 0
+    assert not rule._chunks_from(step(lengths), 64, 160, work)
 
 
 def test_a_step_that_does_not_say_its_lengths_is_in_chunks_whole():
