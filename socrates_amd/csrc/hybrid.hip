@@ -9,6 +9,7 @@
 // whatever the compute dtype; a value is rounded once, where it is stored in the compute dtype.
 #include "common.h"
 #include "recurrent.h"
+#include "wide.h"
 
 __device__ __forceinline__ float hyb_sigmoid(float x) { return 1.f / (1.f + expf(-x)); }
 
@@ -505,6 +506,12 @@ SOC_EXPORT int soc_moe_route(const float* z, int ldz, const float* bias, const f
 // = (expert, first place), expert -1 behind the last tile, and behind those the number of tiles. max_tiles >= M / TM + E.
 // Tiles hold TM places and an expert's last one the rest; with TM = 256 an expert's tiles hold nearly the same number. A
 // pair whose expert is E or more (an identity expert: nothing to compute) gets no place: -1.
+__device__ __forceinline__ int moe_wide_tiles(int count) { return (count + 255) / 256; }
+__device__ __forceinline__ int moe_wide_rows(int count) {
+    const int n = moe_wide_tiles(count);
+    return ((count + n - 1) / n + 31) / 32 * 32;             // (at most 256, so that no tile but an expert's last is short)
+}
+
 __global__ void __launch_bounds__(1024)
 moe_sort_kernel(const int* __restrict__ idx, int M, int E, int TM, int max_tiles, int* __restrict__ offsets,
                 int* __restrict__ place, int* __restrict__ pair_at, int* __restrict__ tiles) {
@@ -543,9 +550,8 @@ moe_sort_kernel(const int* __restrict__ idx, int M, int E, int TM, int max_tiles
                 if (tile0[mid] <= t) lo = mid; else hi = mid - 1;
             }
             e = lo;
-            // (256 places: an expert's places in as few tiles as hold them, of nearly equal size in blocks of 16)
-            const int n = tile0[e + 1] - tile0[e], rows = TM == 256 ? ((count[e] + n - 1) / n + 15) / 16 * 16 : TM;
-            first = start[e] + (t - tile0[e]) * rows;
+            // (256 places: an expert's places in as few tiles as hold them, of nearly equal size in blocks of 32)
+            first = start[e] + (t - tile0[e]) * (TM == 256 ? moe_wide_rows(count[e]) : TM);
         }
         tiles[2 * t] = e;
         tiles[2 * t + 1] = first;
@@ -770,135 +776,62 @@ grouped_mfma_kernel(const bf16* __restrict__ x, int ldx, const int* __restrict__
         }
 }
 
-// The same for many places per expert: up to 256 places x 256 weight rows by eight waves (2 x 4; blocks of 16 places take
-// turns between the two, 64 weight rows each), 64 k at a time in two LDS buffers that global_load_lds fills while the
-// other is multiplied: no registers, no LDS writes, one barrier per 64 k. A wave's products of 128 x 64 read LDS for
-// three quarters of their own time; at 64 x 64 a wave the reads take longer than the products. Such a load
-// puts a wave's 64 pieces of 16 bytes one behind the other, so rows cannot be padded apart: a row's eight pieces are
-// swapped among themselves instead, by a pattern over the rows that lets 16 rows of one k be read without bank
-// conflicts. The weights are the first operand: a lane ends up with four neighbouring outputs of one place.
-// An expert's places are cut into tiles of nearly equal size (moe_sort), because each tile reads the expert's weights
-// again and one with few places does little for it. A tile's products go by 64 places, though, so the even cut can multiply more
-// padding than full tiles and a rest: 292 places are 160 + 132, computed as 384 rows (256 + 36: 320), 333 are 176 + 157 (384
-// either way), 272 are 144 + 128 (320 either way). Workgroups go round-robin over the eight XCDs; each XCD gets a run of (tile, block of outputs) in order,
-// so that the tiles of an expert meet in one L2. Measured against the kernel above (tiles of 128) at 32 experts of 2,432
-// and a width of 2,560, us: 8,320 places gate / up 469 -> 388, down 285 -> 252; 12,000 places 550 -> 436 and 347 -> 265
-// (685 TFLOP/s; its weights alone take 166 us at a copy's rate). Bound by the LDS reads beside the products, that padding and,
-// with one workgroup per compute unit, by the last round of workgroups, which is seldom full. K is a multiple of 64; places
-// and weight rows outside are read from a row that exists and not written.
-template <int N> struct ga_blocks { static constexpr int value = N; };
-__device__ __forceinline__ int ga_swap(int row) { return (row >> 1) & 7; }
-
-__device__ __forceinline__ void ga_load(const bf16* from, uint16_t* lds) {
-    // (the wave's LDS address goes through m0; nothing comes back in registers)
-    const uint32_t to = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t*)lds;
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(__builtin_amdgcn_readfirstlane(to)), "v"(from)
-                 : "memory", "m0");
-}
-
-template <bool GLU, typename TO>
-__global__ void __launch_bounds__(512)
-grouped_wide_kernel(const bf16* __restrict__ x, int ldx, const int* __restrict__ pair_at, int top, const bf16* __restrict__ w,
-                    const int* __restrict__ offsets, const int* __restrict__ tiles, int max_tiles, int blocks, TO* __restrict__ out, int n_out,
-                    int K, int ff, float limit, float slope, float shift, int squared) {
-    constexpr int BM = 256, BN = 256, BK = 64, COLS = GLU ? BN / 2 : BN;
-    __shared__ __attribute__((aligned(1024))) uint16_t As[2][BM * BK], Ws[2][BN * BK];
-    const int n_tiles = tiles[2 * max_tiles], total = n_tiles * blocks, chunk = (total + 7) / 8;
-    const int item = (int)(blockIdx.x % 8) * chunk + (int)(blockIdx.x / 8);
-    if ((int)(blockIdx.x / 8) >= chunk || item >= total) return;
-    const int tile = item / blocks, o0 = item % blocks * COLS;
-    const int e = tiles[2 * tile], p0 = tiles[2 * tile + 1];
-    const int pend = tile + 1 < n_tiles && tiles[2 * tile + 2] == e ? tiles[2 * tile + 3] : offsets[e + 1];
-    const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64), li = lane % 16, g = lane / 16;
-    const int wm = wave / 4, wn = wave % 4;
-    const bf16* we = w + (size_t)e * (GLU ? 2 * ff : n_out) * K;
-    const bf16* a_src[4];                                    // a wave fills 32 rows of each, eight per load
-    const bf16* w_src[4];
+// The same for many places per expert: up to 256 places x 256 weight rows by the loop of wide.h. A tile of places is computed
+// in blocks of 32, as many as it has (64 at least): 292 places are 160 + 132 and cost 320 rows.
+// Workgroups go round-robin over the eight XCDs; each XCD gets a run of (expert, block of outputs, tile), so that the tiles of an
+// expert read a block's weights at the same time and from one L2. Measured at 32 experts of 2,432 and a width of 2,560, us,
+// against eight waves of 128 x 64 that drained their loads at every step and computed whole blocks of 64: 8,320 places gate / up
+// 325 -> 251, down 200 -> 163; 9,356 places 374 -> 275 and 193 -> 162; 12,000 places 398 -> 309 and 214 -> 179 (970 TFLOP/s).
+// Bound by the products (1.3 to 1.5 PFLOP/s inside a tile), the last round of workgroups and, below some 100 places per expert,
+// the weights (1.2 GB at 4.6 TB/s).
+// K is a multiple of 64; places and weight rows outside are read from a row that exists and not written.
+template <int MI, int ACT, typename TO>
+__device__ __forceinline__ void grouped_wide_tile(uint16_t* lds, const bf16* x, int ldx, const int* pair_at, int top, const bf16* we, int p0,
+                                                  int pend, int o0, TO* out, int n_out, int K, WideGate gate) {
+    const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    uint32_t xo[MI], wo[8];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int row = (wave * 4 + i) * 8 + lane / 8, piece = ((lane % 8) ^ ga_swap(row)) * 8, p = min(p0 + row, pend - 1);
-        a_src[i] = x + (size_t)(pair_at ? pair_at[p] / top : p) * ldx + piece;
-        int at;
-        if (GLU) at = min(o0 + row / 64 * 32 + row % 64 / 32 * 16 + row % 16, ff - 1) + (row / 16 % 2 ? ff : 0);     // gate and up tiles alternate
-        else at = min(o0 + row, n_out - 1);
-        w_src[i] = we + (size_t)at * K + piece;
+    for (int i = 0; i < MI; ++i) {
+        const int row = (wave * MI + i) * 8 + lane / 8, p = min(p0 + row, pend - 1);
+        xo[i] = ((uint32_t)(pair_at ? pair_at[p] / top : p - p0) * (uint32_t)ldx + ((lane % 8) ^ wide_swap(row)) * 8) * 2;
     }
-    const int rows = pend - p0, steps = K / BK;
-    auto issue = [&](int k0, int buf) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) ga_load(w_src[i] + k0, &Ws[buf][(wave * 4 + i) * 512]);
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            if ((wave * 4 + i) * 8 < rows) ga_load(a_src[i] + k0, &As[buf][(wave * 4 + i) * 512]);      // the same in all lanes
-    };
-    hyb_f32x4 acc[8][4];
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = (hyb_f32x4){0.f, 0.f, 0.f, 0.f};
-    issue(0, 0);
-    // NB: blocks of 16 places per wave (a branch per block would stand between every read and its products)
-    auto walk = [&](auto blocks_of_16) {
-        constexpr int NB = decltype(blocks_of_16)::value;
-        for (int s = 0; s < steps; ++s) {
-            // this step's pieces have landed, and every wave has read the other buffer
-            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            if (s + 1 < steps) issue((s + 1) * BK, (s + 1) % 2);
-            const uint16_t* a = As[s % 2];
-            const uint16_t* b = Ws[s % 2];
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                hyb_bf16x8 wf[4];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int row = wn * 64 + j * 16 + li;
-                    wf[j] = *reinterpret_cast<const hyb_bf16x8*>(&b[row * BK + ((4 * h + g) ^ ga_swap(row)) * 8]);
-                }
-#pragma unroll
-                for (int i = 0; i < NB; ++i) {
-                    const int row = (2 * i + wm) * 16 + li;
-                    const hyb_bf16x8 af = *reinterpret_cast<const hyb_bf16x8*>(&a[row * BK + ((4 * h + g) ^ ga_swap(row)) * 8]);
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], af, acc[i][j], 0, 0, 0);
-                }
-            }
-        }
-    };
-    if (rows > 192) walk(ga_blocks<8>{});
-    else if (rows > 128) walk(ga_blocks<6>{});
-    else if (rows > 64) walk(ga_blocks<4>{});
-    else walk(ga_blocks<2>{});
-    // acc[i][j][r] belongs to place lane % 16 of block i and weight row 4 g + r of tile j
+    if (!pair_at) x += (size_t)p0 * ldx;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        const int p = p0 + (2 * i + wm) * 16 + li;
-        if (p >= pend) continue;
-        constexpr int STEP = GLU ? 2 : 1;
-#pragma unroll
-        for (int j = 0; j < 4; j += STEP) {
-            const int col = o0 + (GLU ? wn * 32 + j / 2 * 16 : wn * 64 + j * 16) + 4 * g;
-            float y[4];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                if constexpr (GLU) {
-                    const float gt = fminf(to_float(from_float<bf16>(acc[i][j][r])), limit);
-                    const float up = fminf(fmaxf(to_float(from_float<bf16>(acc[i][j + 1][r])), -limit), limit);
-                    y[r] = gt * hyb_sigmoid(slope * gt) * (up + shift);
-                } else {
-                    y[r] = acc[i][j][r];
-                    if (squared) { y[r] = fmaxf(y[r], 0.f); y[r] *= y[r]; }
-                }
-            }
-            TO* to = out + (size_t)p * n_out + col;
-            if (n_out % 4 == 0 && col + 4 <= n_out) {
-                if constexpr (sizeof(TO) == 4) *reinterpret_cast<float4*>(to) = make_float4(y[0], y[1], y[2], y[3]);
-                else *reinterpret_cast<uint2*>(to) = make_uint2(pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3]));
-            } else {
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    if (col + r < n_out) to[r] = from_float<TO>(y[r]);
-            }
-        }
+        const int row = (wave * 8 + i) * 8 + lane / 8;
+        const int at = wide_pairs(ACT) ? min(o0 + row / 32 * 16 + row % 16, n_out - 1) + (row / 16 % 2 ? n_out : 0) : min(o0 + row, n_out - 1);
+        wo[i] = ((uint32_t)at * (uint32_t)K + ((lane % 8) ^ wide_swap(row)) * 8) * 2;
+    }
+    f32x4_t acc[MI][8];
+    wide_walk<MI, 8>(reinterpret_cast<const char*>(x), reinterpret_cast<const char*>(we), xo, wo, K / 64, lds, acc);
+    wide_results<MI, 8, ACT, TO>(acc, out, p0, pend, o0, n_out, gate, n_out % 8 != 0);
+}
+
+template <int ACT, typename TO>
+__global__ void __launch_bounds__(256, 1)
+grouped_wide_kernel(const bf16* __restrict__ x, int ldx, const int* __restrict__ pair_at, int top, const bf16* __restrict__ w,
+                    const int* __restrict__ offsets, const int* __restrict__ tiles, int max_tiles, int blocks, TO* __restrict__ out, int n_out,
+                    int K, WideGate gate) {
+    __shared__ __attribute__((aligned(1024))) uint16_t lds[40 * 2048];
+    const int total = tiles[2 * max_tiles] * blocks, chunk = (total + 7) / 8;
+    const int item = (int)(blockIdx.x % 8) * chunk + (int)(blockIdx.x / 8);
+    if ((int)(blockIdx.x / 8) >= chunk || item >= total) return;
+    const int tile = item / blocks, e = tiles[2 * tile], start = offsets[e], end = offsets[e + 1];
+    // the tiles of this tile's expert, and which of them and of its blocks of outputs this workgroup takes
+    const int n = moe_wide_tiles(end - start), rows = moe_wide_rows(end - start), first = tile - (tiles[2 * tile + 1] - start) / rows;
+    const int at = item - first * blocks, o0 = at / n * (wide_pairs(ACT) ? 128 : 256), p0 = start + at % n * rows, pend = min(p0 + rows, end);
+    const bf16* we = w + (size_t)e * (wide_pairs(ACT) ? 2 : 1) * n_out * K;
+    auto run = [&](auto blocks_of_32) {
+        grouped_wide_tile<decltype(blocks_of_32)::value, ACT, TO>(lds, x, ldx, pair_at, top, we, p0, pend, o0, out, n_out, K, gate);
+    };
+    switch ((pend - p0 + 31) / 32) {
+        case 8: run(WideHalf<8>{}); break;
+        case 7: run(WideHalf<7>{}); break;
+        case 6: run(WideHalf<6>{}); break;
+        case 5: run(WideHalf<5>{}); break;
+        case 4: run(WideHalf<4>{}); break;
+        case 3: run(WideHalf<3>{}); break;
+        default: run(WideHalf<2>{}); break;
     }
 }
 
@@ -917,15 +850,18 @@ SOC_EXPORT int soc_grouped_linear(const void* x, int ldx, const int* pair_at, in
     hipLaunchKernelGGL((grouped_mfma_kernel<WM, WN, MI, NI, GLU, TO>), dim3((n_out + (GLU ? 63 : 127)) / (GLU ? 64 : 128), max_tiles), \
                        dim3(256), 0, stream, (const bf16*)x, ldx, pair_at, top, (const bf16*)w, offsets, tiles, (TO*)out, n_out, \
                        K, ff, limit, slope, shift, squared)
-#define SOC_GA(GLU, TO)                                                                                                          \
+#define SOC_GA(ACT, TO)                                                                                                          \
     do {                                                                                                                         \
-        const int blocks = (n_out + (GLU ? 127 : 255)) / (GLU ? 128 : 256);                                                      \
-        hipLaunchKernelGGL((grouped_wide_kernel<GLU, TO>), dim3((blocks * max_tiles + 7) / 8 * 8), dim3(512), 0, stream, (const bf16*)x, ldx, \
-                           pair_at, top, (const bf16*)w, offsets, tiles, max_tiles, blocks, (TO*)out, n_out, K, ff, limit, slope, shift, squared); \
+        const int blocks = (n_out + (wide_pairs(ACT) ? 127 : 255)) / (wide_pairs(ACT) ? 128 : 256);                              \
+        hipLaunchKernelGGL((grouped_wide_kernel<ACT, TO>), dim3((blocks * max_tiles + 7) / 8 * 8), dim3(256), 0, stream, (const bf16*)x, ldx, \
+                           pair_at, top, (const bf16*)w, offsets, tiles, max_tiles, blocks, (TO*)out, n_out, K, WideGate{limit, slope, shift}); \
     } while (0)
         if (tile == 256) {
             if (K % 64 || (uintptr_t)x % 16 || (uintptr_t)w % 16) return (int)hipErrorInvalidValue;
-            if (ff > 0) SOC_GA(true, bf16); else if (out_f32) SOC_GA(false, float); else SOC_GA(false, bf16);
+            if (ff > 0) SOC_GA(WIDE_GATED, bf16);
+            else if (squared) { if (out_f32) SOC_GA(WIDE_SQUARED, float); else SOC_GA(WIDE_SQUARED, bf16); }
+            else if (out_f32) SOC_GA(WIDE_PLAIN, float);
+            else SOC_GA(WIDE_PLAIN, bf16);
 #undef SOC_GA
         } else if (tile == 128) {
             if (ff > 0) SOC_GM(2, 2, 4, 4, true, bf16); else if (out_f32) SOC_GM(2, 2, 4, 4, false, float); else SOC_GM(2, 2, 4, 4, false, bf16);

@@ -15,10 +15,12 @@ from .scan import HEAD, NO_LIMIT
 
 MAX_EXPERTS = 256        # what the routing and sorting kernels hold per token and per workgroup
 EXPERT_TILE = 16         # places of one expert that a workgroup of the products per expert takes ...
-# ... or, in bfloat16, (places per expert on average from which, places, what both sums' lengths are multiples of). Us for
-# the two products at 32 experts of 2,432 and a width of 2,560, tiles of 16 / 128 / 256 places: 19 places per expert
-# 395 / 389 / 404, 37: 506 / 401 / 413, 125: 1,068 / 451 / 459, 260: 2,156 / 754 / 640, 375: 3,067 / 897 / 701.
-EXPERT_TILES_MANY = ((160, 256, 64), (48, 128, 8))
+# ... or, in bfloat16, (places per expert on average from which, places, what both sums' lengths are multiples of, the least of
+# both lengths). Us for the two products at 32 experts of 2,432 and a width of 2,560, tiles of 16 / 128 / 256 places: 12 places
+# per expert 218 / 271 / 243, 19: 301 / 275 / 247, 38: 447 / 287 / 253, 100: 771 / 326 / 288, 160: 1,191 / 470 / 333. With
+# short sums a tile of 256 does not get past its beginning and end: width 512 and experts of 512, 14 places 19.3 / 25.2 / 18.8,
+# 48: 26.5 / 30.8 / 20.5; 256 and 256, 48 places 12.8 / 21.0 / 14.1, 150: 19.6 / 23.6 / 26.4.
+EXPERT_TILES_MANY = ((160, 256, 64, 0), (14, 256, 64, 512), (48, 128, 8, 0))
 
 
 class ExpertRuns:
@@ -207,7 +209,7 @@ class Hybrid:
         self._want(idx, "experts", torch.int32)
         if not 1 <= E <= MAX_EXPERTS:
             raise KernelError(f"{E} experts (at most {MAX_EXPERTS})")
-        if tile not in (EXPERT_TILE,) + tuple(t for _, t, _ in EXPERT_TILES_MANY):
+        if tile not in (EXPERT_TILE,) + tuple(t for _, t, _, _ in EXPERT_TILES_MANY):
             raise KernelError(f"tiles of {tile} places")
         M = N * top
         max_tiles = (M + tile - 1) // tile + min(E, M)
@@ -241,6 +243,8 @@ class Hybrid:
         out_dtype = out_dtype or self.dtype
         if out_dtype not in (self.dtype, torch.float32) or (glu is not None and out_dtype != self.dtype):
             raise KernelError(f"products per expert: a result in {out_dtype}")
+        if runs.tile == 256 and max(x.shape[0] * x.stride(0) if by_token else 0, rows * K) >= 1 << 31:
+            raise KernelError("products per expert: tiles of 256 places address x and an expert's weights by 32 bits of bytes")
         out = torch.empty((M, n_out), dtype=out_dtype, device=self.device)
         limit, slope, shift = (tuple(glu) + (1.0,))[:3] if glu is not None else (0.0, 0.0, 1.0)
         _check(self._hybrid().soc_grouped_linear(
@@ -284,9 +288,11 @@ class Hybrid:
         # many tokens per expert, in bfloat16 with rows that start on 16 bytes: the larger tiles of the matrix cores
         # (a weight row then comes from memory once per 128 or 256 tokens of its expert)
         if self.dtype == torch.bfloat16 and x.stride(0) % 8 == 0:
-            aligned = all(t.data_ptr() % 16 == 0 for t in (x,) + weights)
-            return next((t for least, t, of in EXPERT_TILES_MANY
-                         if M >= least * E and d % of == 0 and ff % of == 0 and (t < 256 or aligned)), EXPERT_TILE)
+            # (the largest tiles address x and one expert's weights by 32 bits of bytes)
+            aligned = all(t.data_ptr() % 16 == 0 for t in (x,) + weights) and max(x.shape[0] * x.stride(0), 2 * d * ff) < 1 << 31
+            return next((t for least, t, of, length in EXPERT_TILES_MANY
+                         if M >= least * E and d % of == 0 and ff % of == 0 and min(d, ff) >= length and (t < 256 or aligned)),
+                        EXPERT_TILE)
         return EXPERT_TILE
 
     def moe_experts(self, x, idx, weight, w_gate_up, w_down, limit, slope, extra=None, shift=1.0, extra_gate=None, whole=True,
