@@ -22,6 +22,7 @@ recurrences with a matrix state in chunks of a prompt portion,
 from __future__ import annotations
 
 import collections
+import functools
 from ctypes import c_float, c_int, c_longlong, c_void_p
 
 import torch
@@ -34,8 +35,8 @@ from .latent import Latent
 from .memory import Memory
 from .mixers import Mixers
 from .build import KernelBuildError, build_all, compile_library, load_library
-from .common import (_ATTENTION_SIGNATURES, _ATTENTION_UP_TO_256, _DTYPE_CODE, _EW_SIGNATURES, _GEMM_SIGNATURES, _SAMPLING_SIGNATURES, KernelError,
-                     NormOwed, RowsByTile, _check, _declare, _ptr)
+from .common import (_ATTENTION_SIGNATURES, _ATTENTION_UP_TO_256, _DTYPE_CODE, _EW_SIGNATURES, _GEMM_SIGNATURES, _SAMPLING_SIGNATURES, _WIDE_SIGNATURES,
+                     KernelError, NormOwed, RowsByTile, _check, _declare, _ptr)
 from .planning import MAX_KEY_SPLITS, plan_key_splits
 from .products import Products
 from .scan import Scan
@@ -57,10 +58,12 @@ class HipKernels(Products, Attention, Latent, Mixers, Hybrid, Composite, Memory,
         self._ew = load_library("elementwise")
         self._gemm = load_library("gemm")
         self._sampling = load_library("sampling")
+        self._wide = load_library("wide")
         self._attn = {}
         _declare(self._ew, _EW_SIGNATURES)
         _declare(self._gemm, _GEMM_SIGNATURES)
         _declare(self._sampling, _SAMPLING_SIGNATURES)
+        _declare(self._wide, _WIDE_SIGNATURES)
         self.attention_splits = None        # (split_len, n_splits) override, for tests and capture
         self.attention_row_tiles = None     # row tiles per wave of the MFMA kernel, override
         self.last_attention_kernel = None   # (kernel, row tiles) the last bfloat16 call went to
@@ -85,10 +88,21 @@ class HipKernels(Products, Attention, Latent, Mixers, Hybrid, Composite, Memory,
         self.latent_splits = self.latent_row_waves = None
         self.latent_target, self.latent_min_keys = 256, 256
         self.latent_mfma = True
-        # bfloat16 products with more than 16 rows go to the library (hipBLASLt through
-        # torch.mm), as the reference's all do (nn.Linear); False keeps them on this
-        # package's tiled MFMA kernel
+        # False keeps every bfloat16 product with more than 16 rows on this package's tiled MFMA kernel; True leaves
+        # those that no other kernel here takes to the library (hipBLASLt through torch.mm), as the reference's all do
+        # (nn.Linear)
         self.library_gemm = True
+        # bfloat16 products of more than ``wide_rows`` rows and at least ``wide_min_outputs`` outputs: tiles of up to 256 x 256
+        # (csrc/wide.hip). Partial sums always, an activation over gate and up from ``wide_min_pairs`` operations on, whole
+        # sums from ``wide_min_whole`` operations or terms of a sum on; the rest goes to the library. Us inside replayed
+        # graphs, weights from memory, own / library (which has an activation's 3 to 23 us besides): partial sums 2,560 x
+        # 2,560 9.1 / 13.3 at 65 rows, 23.4 / 23.3 at 1,100; 2,560 x 9,728 16.5 / 25.9 and 60 / 73. Gate and up of 9,728 x
+        # 2,560 36 / 33 at 80 rows, 36 / 42 at 130, 50 / 55 at 512, 172 / 211 at 2,048. Whole sums 2,560 x 2,560 17.5 / 14.9
+        # at 200, 27.6 / 23.3 at 1,100, 32.4 / 35.6 at 2,048; 5,120 x 2,560 27.0 / 28.4 at 500; 2,560 x 9,728 21.4 / 25.9 at
+        # 65 and 64 / 73 at 1,100; 640 x 2,560 11.2 / 8.7 at 65, 21.4 / 18.5 at 3,000. 0 rows: never.
+        self.wide_rows, self.wide_min_outputs = 64, 256
+        self.wide_min_pairs, self.wide_min_whole = 8e9, (15e9, 4096)
+        self._wide_form = functools.lru_cache(maxsize=4096)(self._wide_plan)
         self.swiglu_waves = 8           # waves of the fused gate+up product (measured: 4, 8, 16 within 5 %)
         # The sweep form of the skinny product (one workgroup per compute unit keeps its slices
         # of x in registers and walks over the weight tiles): from this many rows of x on, for

@@ -52,6 +52,10 @@ _GEMM_SIGNATURES = {
     "soc_gemm_bf16_stream": [P, P, P, I, I, I, I, I, I, I, I, P],
     "soc_gemm_stream_plan": [I, I, I, I, P, P],
 }
+_WIDE_SIGNATURES = {
+    "soc_wide_plan": [I, I, I, I, I, P, P, P, P],
+    "soc_wide_linear": [P, P, P, P] + [I] * 9 + [F, F, F, I, P],
+}
 L = c_longlong
 _MIXER_SIGNATURES = {
     "soc_gated_norm_add": [P, P, I, P, P, I, P, P, F, F, P, F, P, I, I, I, P],

@@ -1,6 +1,6 @@
 """Matrix products of the kernel set: the forms a product can take (a workgroup per weight
 tile, a sweep over tiles with x in registers, parts of K over sweeping workgroups, K outermost,
-the library), the epilogues folded into them (activation, residual sum, norm) and the rule or
+wide tiles for many rows, the library), the epilogues folded into them (activation, residual sum, norm) and the rule or
 the measurement that chooses among them. A mixin of ``HipKernels``."""
 
 from __future__ import annotations
@@ -97,6 +97,13 @@ class Products:
                     out = self._swiglu_out(M, N, by_tile)
                     self._k_outermost(plan, x, w_gate_up, out, True, what="linear_swiglu")
                     return out
+        if owed is None and w_gate_up.dim() == 2 and K == w_gate_up.shape[1] and (interleave == 16 or not interleave and N % 32 == 0):
+            self._want(x, "x")
+            self._want(w_gate_up, "weight")
+            out = self._wide_or_none(x, w_gate_up, torch.bfloat16, act=self.WIDE_SILU, halves=not interleave,
+                                     by_library=lambda: self.swiglu(torch.mm(x, w_gate_up.t()), interleave))
+            if out is not None:
+                return out
         return self.swiglu(self.linear(owed if owed is not None else x, w_gate_up), interleave)
 
     _SK_SWIGLU, _SK_SCALED = 1, 2
@@ -411,8 +418,8 @@ class Products:
     def linear(self, x, w, out_dtype=None, allow_partial=False, row_tiles=0, n_waves=0, k_splits=0):
         """x [M, K] times w [N, K] transposed. float32 operands (either) take the
         float32 kernels. bfloat16 pairs: up to 16 rows the skinny MFMA kernel (it streams
-        the weights faster than the library does there); more rows the library product,
-        or this package's tiled MFMA kernel if ``library_gemm`` is off. ``allow_partial``: the consumer
+        the weights faster than the library does there); more than 64 rows wide tiles where they are
+        faster, else the library product, or this package's tiled MFMA kernel if ``library_gemm`` is off. ``allow_partial``: the consumer
         (the residual-add + norm kernel) accepts float32 split-K partial sums [S, M, N]; the
         skinny kernel then spreads a narrow output over more workgroups, and a product of 17 to
         ``parts_rows`` rows is swept with K split over workgroups instead of going to the library."""
@@ -529,10 +536,13 @@ class Products:
                    f"linear [{M}x{K}] x [{N}x{K}]^T")
             return out
         if both_bf16 and self.library_gemm:
+            def by_library():
+                return torch.mm(x, w.t()) if out_dtype == torch.bfloat16 else torch.mm(x, w.t(), out_dtype=out_dtype)
+            out = self._wide_or_none(x, w, out_dtype, bool(allow_partial), by_library=by_library)
+            if out is not None:
+                return out
             self.forms["library"] += 1
-            if out_dtype == torch.bfloat16:
-                return torch.mm(x, w.t())
-            return torch.mm(x, w.t(), out_dtype=out_dtype)
+            return by_library()
         if not both_bf16:
             out = self._linear_f32(x, w, out_dtype, allow_partial)
             if out is not None:
@@ -546,6 +556,50 @@ class Products:
                                               c_int(_DTYPE_CODE[out_dtype]), self._stream())
         _check(err, f"linear [{M}x{K}] x [{N}x{K}]^T")
         return out
+
+    WIDE_PLAIN, WIDE_SILU, WIDE_GATED, WIDE_GELU, WIDE_SQUARED = range(5)
+
+    def _wide_plan(self, M, N, K, act=0, partial=False):
+        """(blocks of 32 rows, of 32 outputs, last tiles halved, parts of K) of a product of many rows, or None."""
+        form = [c_int(0) for _ in range(4)]
+        if M <= self.wide_rows or not self.wide_rows or N < self.wide_min_outputs or not self._wide.soc_wide_plan(
+                c_int(M), c_int(N), c_int(K), c_int(act), c_int(1 if partial else 0), *map(ctypes.byref, form)):
+            return None
+        operations = 2.0 * M * N * K
+        if act in (self.WIDE_SILU, self.WIDE_GATED, self.WIDE_GELU):
+            enough = operations >= self.wide_min_pairs
+        else:
+            enough = form[3].value > 1 and partial or operations >= self.wide_min_whole[0] or K >= self.wide_min_whole[1]
+        return tuple(f.value for f in form) if enough else None
+
+    def _wide_product(self, form, x, w, out_dtype, partial=False, act=0, halves=False, gate=(0.0, 1.0, 0.0)):
+        """x [M, K] times w [N, K] transposed by ``form``; with an activation over pairs [M, N / 2] (``halves``: w holds gate rows
+        and then up rows, else they alternate by 16). ``partial``: parts of K come back as they are, float32 [parts, M, N]."""
+        (M, K), N = x.shape, w.shape[0]
+        mi, nj, tail, parts = form
+        pairs = act in (self.WIDE_SILU, self.WIDE_GATED, self.WIDE_GELU)
+        sums = torch.empty((parts, M, N), dtype=torch.float32, device=self.device) if parts > 1 else None
+        out = None if partial and parts > 1 else torch.empty((M, N // 2 if pairs else N), dtype=out_dtype, device=self.device)
+        self.forms["wide"] += 1
+        _check(self._wide.soc_wide_linear(
+            _ptr(x), _ptr(w), _ptr(out), _ptr(sums), c_int(M), c_int(N), c_int(K), c_int(mi), c_int(nj), c_int(tail), c_int(parts),
+            c_int(act), c_int(N // 2 if halves else 0), c_float(gate[0]), c_float(gate[1]), c_float(gate[2]),
+            c_int(1 if out_dtype == torch.float32 else 0), self._stream()), f"linear [{M}x{K}] x [{N}x{K}]^T")
+        return sums if out is None else out
+
+    def _wide_or_none(self, x, w, out_dtype, partial=False, act=0, by_library=None, **kw):
+        """The product through ``_wide_product`` where it applies and a tuning pass has not found the library faster."""
+        (M, K), N = x.shape, w.shape[0]
+        if (not self.library_gemm or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or x.data_ptr() % 16 or w.data_ptr() % 16):
+            return None
+        form = self._wide_form(M, N, K, act, partial)
+        if form is None:
+            return None
+        key = (M, N, K, f"act {act}" if act else out_dtype, partial)
+        choice = self.product_choice.get(key)
+        if choice is None and self._tuning and not torch.cuda.is_current_stream_capturing():
+            choice = self.product_choice[key] = self._faster(lambda: self._wide_product(form, x, w, out_dtype, partial, act, **kw), by_library)
+        return None if choice == "library" else self._wide_product(form, x, w, out_dtype, partial, act, **kw)
 
     def _linear_f32(self, x, w, out_dtype, allow_partial, tiles=0, splits=0):
         """A product with a float32 operand on the matrix cores, in float32 throughout; None where

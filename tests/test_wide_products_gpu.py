@@ -44,3 +44,77 @@ def test_short_sums_keep_smaller_tiles(ops):
     x = rnd((64, 512), 1)
     for d, ff, m, tile in ((512, 512, 13, 16), (512, 512, 14, 256), (512, 448, 47, 16), (512, 448, 48, 128), (512, 448, 160, 256)):
         assert ops._expert_tile(x, m * 4, 4, d, ff, rnd((4, 2 * ff, d), 2)) == tile
+
+
+FORMS = [(8, 8, 0), (8, 8, 1), (6, 8, 0), (6, 8, 1), (5, 8, 0), (4, 8, 0), (4, 8, 1), (3, 8, 0), (2, 8, 0), (8, 4, 0), (8, 6, 0), (6, 6, 0),
+         (8, 5, 0), (4, 6, 0), (5, 5, 0), (4, 5, 0), (4, 4, 0), (3, 5, 0)]
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("M,N,K", [(65, 264, 64), (257, 1096, 320), (700, 3080, 448)])
+def test_whole_and_partial_sums(ops, form, M, N, K):
+    """Tiles with one row or a few columns, more tiles than an XCD has in a round, fewer and more steps than the rings hold, parts
+    of unequal length. K roundings of float32 at the sum of sizes, and the result's own, are the bound."""
+    x, w = rnd((M, K), 1), rnd((N, K), 2, 0.3)
+    want, slack = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T * K * 2.0 ** -24 + 1e-6
+    for parts in (1, 2, 3):
+        if parts > K // 64:
+            continue
+        got = ops._wide_product(form + (parts,), x, w, torch.float32)
+        assert ((got.double() - want).abs() <= slack).all()
+        rounded = ops._wide_product(form + (parts,), x, w, torch.bfloat16)
+        assert torch.equal(rounded, got.bfloat16())
+        if parts > 1:
+            sums = ops._wide_product(form + (parts,), x, w, torch.bfloat16, partial=True)
+            assert sums.shape == (parts, M, N) and torch.equal(sum(sums[1:], sums[0]), got)
+
+
+@pytest.mark.parametrize("form", [f for f in FORMS if f[1] % 4 == 0])
+@pytest.mark.parametrize("M,ff,K", [(65, 144, 64), (300, 1552, 320)])
+def test_activations_in_the_epilogue(ops, form, M, ff, K):
+    """Gate and up rows that alternate by 16 or lie in halves; both products are rounded to bfloat16 (a step either way where a
+    float32 sum lies near the middle), the activation's own error is below the result's rounding."""
+    x, gate, up = rnd((M, K), 1), rnd((ff, K), 2, K ** -0.5), rnd((ff, K), 3, K ** -0.5)
+    g, u = (x.double() @ t.double().T for t in (gate, up))
+    apart = torch.cat([gate, up]).contiguous()
+    mixed = torch.stack([gate.view(ff // 16, 16, K), up.view(ff // 16, 16, K)], 1).reshape(2 * ff, K).contiguous()
+    gg, uu = (t.float().bfloat16().double() for t in (g, u))
+    size = 2.0 ** -7 * (gg.abs() + 1) * (uu.abs() + 2)
+    limit = 0.7
+    want = {ops.WIDE_SILU: torch.nn.functional.silu(gg) * uu,
+            ops.WIDE_GATED: gg.clamp(max=limit) * torch.sigmoid(1.702 * gg.clamp(max=limit)) * (uu.clamp(-limit, limit) + 1),
+            ops.WIDE_GELU: torch.nn.functional.gelu(gg, approximate="tanh") * uu}
+    for act, y in want.items():
+        a = ops._wide_product(form + (1,), x, mixed, torch.bfloat16, act=act, gate=(limit, 1.702, 1.0))
+        b = ops._wide_product(form + (1,), x, apart, torch.bfloat16, act=act, halves=True, gate=(limit, 1.702, 1.0))
+        assert torch.equal(a, b) and ((a.double() - y).abs() <= size + 2.0 ** -8 * y.abs()).all(), act
+    y = ops._wide_product(form + (1,), x, apart, torch.bfloat16, act=ops.WIDE_SQUARED)
+    both = torch.cat([gg, uu], 1)
+    assert ((y.double() - both.clamp(min=0) ** 2).abs() <= 2.0 ** -6 * both ** 2 + 1e-4).all()
+
+
+def test_what_is_not_finite_stays_where_it_was(ops):
+    """Infinities and NaN in a gate or an up row come out as the activation of plain rows has them."""
+    M, ff, K = 70, 64, 64
+    x, w = rnd((M, K), 1), rnd((2 * ff, K), 2, 0.1)
+    x[3, 5], x[4, 6], x[5, 7] = float("inf"), float("nan"), -float("inf")
+    both = torch.mm(x.float(), w.float().T).bfloat16()
+    got = ops._wide_product((2, 8, 0, 1), x, w, torch.bfloat16, act=ops.WIDE_SILU, halves=True)
+    want = ops.swiglu(both)
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    got = ops._wide_product((2, 8, 0, 1), x, w, torch.bfloat16, act=ops.WIDE_GELU, halves=True)
+    assert torch.equal(got.isnan(), ops.glu_gelu(both, ff).isnan())
+
+
+def test_which_products_are_wide(ops):
+    """Rows, outputs, operations and alignment decide; what the kernel does not take goes the way it went."""
+    form = ops._wide_form
+    assert form(64, 2560, 9728) is None and form(65, 2560, 9728) is not None and form(65, 248, 9728) is None
+    assert form(1100, 2560, 2560) is None and form(2048, 2560, 2560) is not None and form(65, 2560, 2560, 0, True)[3] > 1
+    assert form(2048, 2560, 2592) is None and form(2048, 2564, 2560) is None and form(65, 19456, 2560, ops.WIDE_SILU) is None
+    x, w = rnd((70, 4096), 1), rnd((264, 4096), 2, 0.02)
+    shifted = torch.empty(w.numel() + 1, dtype=w.dtype, device=DEV)[1:].view_as(w).copy_(w)
+    for weight, name in ((w, "wide"), (shifted, "library")):
+        ops.forms.clear()
+        y = ops.linear(x, weight)
+        assert ops.forms[name] == 1 and torch.allclose(y.double(), x.double() @ w.double().T, atol=2e-2, rtol=2e-2)
