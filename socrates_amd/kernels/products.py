@@ -601,6 +601,19 @@ class Products:
             choice = self.product_choice[key] = self._faster(lambda: self._wide_product(form, x, w, out_dtype, partial, act, **kw), by_library)
         return None if choice == "library" else self._wide_product(form, x, w, out_dtype, partial, act, **kw)
 
+    def linear_activated(self, x, w, kind, limit=0.0, slope=1.0):
+        """The activation of x w^T on the product's own sums, for many rows: "gated" (``glu_clamped``) and "gelu" (``glu_gelu``)
+        over [gate | up] rows of w, "squared" (``relu_squared``) over all. None where the caller's product and activation
+        are two kernels."""
+        self._want(x, "x")
+        self._want(w, "weight")
+        if x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1]:
+            raise KernelError(f"linear: x {tuple(x.shape)} does not fit weight {tuple(w.shape)}")
+        act = {"gated": self.WIDE_GATED, "gelu": self.WIDE_GELU, "squared": self.WIDE_SQUARED}[kind]
+        if self.dtype != torch.bfloat16 or self._tuning:
+            return None
+        return self._wide_or_none(x, w, torch.bfloat16, act=act, halves=kind != "squared", gate=(limit, slope, 1.0))
+
     def _linear_f32(self, x, w, out_dtype, allow_partial, tiles=0, splits=0):
         """A product with a float32 operand on the matrix cores, in float32 throughout; None where
         that kernel does not apply (K no multiple of four, an operand that is not aligned to four

@@ -51,6 +51,12 @@ class SwiGLU:
         return self.ops.linear(act, self.w_down, allow_partial=True)
 
 
+def _activated(ops, x, w, kind, *constants):
+    """The activation of x w^T where the kernel set has it in one kernel, else None."""
+    fused = getattr(ops, "linear_activated", None)
+    return None if fused is None else fused(x, w, kind, *constants)
+
+
 class ClampedGLU:
     """y = Wd(g * sigmoid(slope * g) * (u + 1)), g = min(Wg x, limit), u = clamp(Wu x, +-limit)."""
 
@@ -76,6 +82,10 @@ class ClampedGLU:
 
     def forward(self, x, ctx=None):
         ff = self.spec.intermediate
+        act = _activated(self.ops, x, self.w_gate_up[:2 * ff], "gated", self.spec.limit, self.spec.slope)
+        if act is not None:
+            y = self.ops.linear(act, self.w_down)
+            return (y, self.ops.linear(x, self.w_gate_up[2 * ff:])) if self.adopted else y
         both = self.ops.linear(x, self.w_gate_up)
         act = self.ops.glu_clamped(both, self.spec.limit, self.spec.slope, ff)
         y = self.ops.linear(act, self.w_down)
@@ -94,7 +104,10 @@ class ReluSquared:
         self.w_up, self.w_down = tensors["up"], tensors["down"]
 
     def forward(self, x, ctx=None):
-        return self.ops.linear(self.ops.relu_squared(self.ops.linear(x, self.w_up)), self.w_down)
+        act = _activated(self.ops, x, self.w_up, "squared")
+        if act is None:
+            act = self.ops.relu_squared(self.ops.linear(x, self.w_up))
+        return self.ops.linear(act, self.w_down)
 
 
 class GeluGLU:
@@ -111,7 +124,9 @@ class GeluGLU:
         self.w_down = tensors["down"]
 
     def forward(self, x, ctx=None):
-        act = self.ops.glu_gelu(self.ops.linear(x, self.w_gate_up), self.spec.intermediate)
+        act = _activated(self.ops, x, self.w_gate_up, "gelu")
+        if act is None:
+            act = self.ops.glu_gelu(self.ops.linear(x, self.w_gate_up), self.spec.intermediate)
         return self.ops.linear(act, self.w_down)
 
 

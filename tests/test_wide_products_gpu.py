@@ -118,3 +118,17 @@ def test_which_products_are_wide(ops):
         ops.forms.clear()
         y = ops.linear(x, weight)
         assert ops.forms[name] == 1 and torch.allclose(y.double(), x.double() @ w.double().T, atol=2e-2, rtol=2e-2)
+
+
+@pytest.mark.parametrize("kind,rows", [("gated", 1024), ("gelu", 1024), ("squared", 512)])
+def test_activated_products_where_they_are_long_enough(ops, kind, rows):
+    x, w = rnd((4100, 1024), 1), rnd((rows, 1024), 2, 1024 ** -0.5)
+    both = ops.linear(x, w)
+    want = {"gated": lambda: ops.glu_clamped(both, 0.7, 1.702), "gelu": lambda: ops.glu_gelu(both, 512), "squared": lambda: ops.relu_squared(both)}[kind]()
+    got = ops.linear_activated(x, w, kind, 0.7, 1.702)
+    if kind == "squared":
+        assert got is None                               # 4.3 of the 15 billion operations from which whole sums are wide
+        got = ops._wide_product((8, 8, 1, 1), x, w, torch.bfloat16, act=ops.WIDE_SQUARED)
+    # a product whose float32 sum lies between two bfloat16 values may round to either: a step of gate and of up
+    torch.testing.assert_close(got.float(), want.float(), atol=2e-2, rtol=2e-2)
+    assert ops.linear_activated(x[:70].contiguous(), w, kind) is None
