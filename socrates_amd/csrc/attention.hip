@@ -1188,28 +1188,13 @@ __device__ __forceinline__ int pf_k_row(int k) {    // LDS row of key k of a til
     return 16 * ((k >> 2) & 1) + 4 * (k >> 3) + (k & 3);
 }
 
-// LDS row of key k of a tile for the 32-row products: bits 2 and 3 of k change places, so that
-// the 16 scores a lane gets from one 32 x 32 product are two runs of eight neighbouring keys,
-// which is what the second product wants from it as operand B.
-__device__ __forceinline__ int pf_k_row32(int k) { return (k & ~12) | ((k & 4) << 1) | ((k & 8) >> 1); }
-
-typedef __attribute__((ext_vector_type(16))) float f32x16_t;
-
 // Entry e of a row's pages of means walks through the prompt kernel as the key PF_MEAN + e (a multiple of every
 // page size, so a key's place in its page is the entry's).
 constexpr int PF_MEAN = -(1 << 30);
 
 // PAIR: pages hold an even, power-of-two number of keys, so a thread's two keys share a page.
-// M32: a wave owns 32 rows and multiplies with the 32 x 32 x 16 instruction (RT = 1; head
-// sizes that are multiples of 32): per row, half the loads, LDS reads, stores and barriers
-// of RT = 1, as RT = 2 has with the 16 x 16 products; the two are equally fast.
-// KS = 2 (with M32): eight waves; waves 0-3 walk the first half of the block's key tiles and
-// waves 4-7, with the same rows, the second half, each four with tiles of their own in LDS;
-// at the end the two partial results are combined through LDS. Twice the waves for the same
-// number of workgroups: for launches whose workgroups are too few, or too uneven (a prompt
-// from its start: the last block sees all keys, the first none), to fill the GPU otherwise.
-template <int RT, bool PAIR, bool M32, int KS, bool CAP = false>
-__global__ void __launch_bounds__(256 * KS)
+template <int RT, bool PAIR, bool CAP = false>
+__global__ void __launch_bounds__(256)
 paged_attn_prefill_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k_pool,
                           const bf16* __restrict__ v_pool, const int* __restrict__ block_table,
                           int table_width, const int* __restrict__ token_rows,
@@ -1219,13 +1204,10 @@ paged_attn_prefill_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k
                           const bf16* __restrict__ mean_k, const bf16* __restrict__ mean_v,
                           const int* __restrict__ mean_table, int mean_table_width, int pool, float softcap) {
     static_assert(D <= 128, "one key pair per thread");
-    static_assert(KS == 1 || (KS == 2 && M32), "key halves come with the 32-row products");
     constexpr int PF_TILE_ELEMS = PF_K_ELEMS + PF_V_ELEMS;          // one K tile and one V^T tile
-    __shared__ __attribute__((aligned(16))) uint16_t tiles_lds[KS * 2 * PF_TILE_ELEMS];
-    const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x / SOC_WAVE), lane = threadIdx.x % SOC_WAVE;
-    const int half = wave_all / 4, wave = wave_all % 4;             // which keys, which rows
-    const int tid = threadIdx.x % 256;                              // among the four waves that share tiles
-    uint16_t* const k_lds[2] = {tiles_lds + (half * 2) * PF_TILE_ELEMS, tiles_lds + (half * 2 + 1) * PF_TILE_ELEMS};
+    __shared__ __attribute__((aligned(16))) uint16_t tiles_lds[2 * PF_TILE_ELEMS];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / SOC_WAVE), lane = threadIdx.x % SOC_WAVE, tid = threadIdx.x;
+    uint16_t* const k_lds[2] = {tiles_lds, tiles_lds + PF_TILE_ELEMS};
     uint16_t* const v_lds[2] = {k_lds[0] + PF_K_ELEMS, k_lds[1] + PF_K_ELEMS};
     const int li = lane % 16, kb = lane / 16;
     const int G = Hq / Hkv, Gp = 1 << group_pad_log2;
@@ -1236,7 +1218,7 @@ paged_attn_prefill_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k
     const int tok0 = row_blocks ? row_blocks[2 * blk] : blk, ntok = row_blocks ? row_blocks[2 * blk + 1] : 1;
     const int pos0 = positions[tok0];
     const int* table = block_table + (size_t)token_rows[tok0] * table_width;
-    const int tokens_per_wave = ((M32 ? 32 : 16 * RT)) >> group_pad_log2;
+    const int tokens_per_wave = (16 * RT) >> group_pad_log2;
 
     const int khi = pos0 + ntok;                                    // keys any row of the block sees
     int kmin = first_seen(pos0, window);
@@ -1258,16 +1240,7 @@ paged_attn_prefill_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k
     const int first_real = klo;                                     // virtual keys from here on are real ones
     const int pre_shift = klo - n_pre * PF_KEYS;                    // a virtual key before that is the real key minus this
     const int pre_base = (pool > 0 ? PF_MEAN : 0) - pre_shift;      // (or the entry of the pages of means, as PF_MEAN + entry)
-    if (KS == 1) klo = pre_shift;
-    // kend: where this half's walk over the tiles ends. Both halves take the same number of
-    // steps (they share the barriers); the second may run past khi, where keys are stand-ins
-    // that no row sees.
-    int kend = khi;
-    if constexpr (KS == 2) {
-        const int per_half = ((khi - klo + PF_KEYS - 1) / PF_KEYS + 1) / 2 * PF_KEYS;
-        klo += half * per_half;
-        kend = klo + per_half;
-    }
+    klo = pre_shift;
     // this wave's rows
     const int wtok0 = wave * tokens_per_wave;                       // first token of the wave in the block
     const int wave_lo_pos = pos0 + wtok0;                           // its first and last positions
@@ -1305,32 +1278,6 @@ paged_attn_prefill_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k
 #pragma unroll
         for (int j = 0; j < DV; ++j) o[rt][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
     }
-    // 32-row products: the lane's row is lane % 32, its half of every 16-wide k step lane / 32
-    constexpr int DQ32 = D / 16, DB32 = D / 32;
-    const int c32 = lane % 32, g32 = lane / 32;
-    int row_pos32 = -1, row_first32 = 0, mean_end32 = PF_MEAN;
-    float sink32_l2 = 0.f;
-    size_t row_q32 = 0;
-    uint4 qf32[M32 ? DQ32 : 1];                           // the lane's slices of its query row
-    f32x16_t o32[M32 ? DB32 : 1];
-    float m32 = -INFINITY, l32 = 0.f;
-    if constexpr (M32) {
-        const int tt = wtok0 + (c32 >> group_pad_log2), gh = chunk * 16 + (c32 & (Gp - 1));
-        const bool ok = tt < ntok && gh < G;
-        row_pos32 = ok ? pos0 + tt : -1;
-        row_first32 = first_seen(ok ? pos0 + tt : pos0, window);
-        row_q32 = ((size_t)(tok0 + (ok ? tt : 0)) * Hq + (size_t)kvh * G + (ok ? gh : 0)) * D;
-        if (pool > 0 && ok) mean_end32 = PF_MEAN + blocks_before(pos0 + tt);
-        if (sink == 2 && ok) sink32_l2 = sinks[kvh * G + gh] * 1.44269504088896340736f;
-#pragma unroll
-        for (int t = 0; t < DQ32; ++t)
-            qf32[t] = ok ? *reinterpret_cast<const uint4*>(q + row_q32 + 16 * t + 8 * g32) : make_uint4(0u, 0u, 0u, 0u);
-#pragma unroll
-        for (int b = 0; b < DB32; ++b)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) o32[b][i] = 0.f;
-    }
-
     // Cooperative tile loads: a thread owns two neighbouring keys (2 kp, 2 kp + 1) and one
     // 16-byte part of them, of K and of V. Keys that no row of the block sees are never read;
     // zeros stand in for them.
@@ -1398,7 +1345,7 @@ paged_attn_prefill_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k
             if ((key < kmin && key >= kept) || key >= khi) { k0 = make_uint4(0u, 0u, 0u, 0u); v0 = k0; }
             if ((key + 1 < kmin && key + 1 >= kept) || key + 1 >= khi) { k1 = make_uint4(0u, 0u, 0u, 0u); v1 = k1; }
         }
-        const int r0 = M32 ? pf_k_row32(2 * kp) : pf_k_row(2 * kp), r1 = M32 ? pf_k_row32(2 * kp + 1) : pf_k_row(2 * kp + 1);
+        const int r0 = pf_k_row(2 * kp), r1 = pf_k_row(2 * kp + 1);
         *reinterpret_cast<uint4*>(&k_lds[buf][r0 * PF_K_STRIDE + part * 8]) = k0;
         *reinterpret_cast<uint4*>(&k_lds[buf][r1 * PF_K_STRIDE + part * 8]) = k1;
         const uint32_t a[4] = {v0.x, v0.y, v0.z, v0.w};
@@ -1497,85 +1444,6 @@ paged_attn_prefill_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k
                     o[rt][j], 0, 0, 0);
     };
 
-    // The same with 32 rows per wave: S^T [32 keys x 32 rows] from D / 16 products, a row's
-    // scores in two lanes (16 each), O^T [32 d x 32 rows] per 32-wide block of d.
-    auto scores32 = [&](int key0, int buf, auto masked_tag, uint4 (&pf)[2], float& alpha, bool& rescale) {
-        constexpr bool MASKED = decltype(masked_tag)::value;
-        const uint16_t* kt = k_lds[buf];
-        f32x16_t sc;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) sc[i] = 0.f;
-#pragma unroll
-        for (int t = 0; t < DQ32; ++t) {
-            const uint4 ka = *reinterpret_cast<const uint4*>(kt + c32 * PF_K_STRIDE + 16 * t + 8 * g32);
-            sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8_t*>(&ka),
-                                                         *reinterpret_cast<const bf16x8_t*>(&qf32[t]), sc, 0, 0, 0);
-        }
-        const int last_seen = key0 < 0 ? mean_end32 - 1 : row_pos32;
-        const int first_seen_key = key0 < 0 ? key0 : row_first32, kept_seen = key0 < 0 ? key0 : keep_first;
-        float mx = -INFINITY;                               // of the raw scores: the scale is positive
-        if constexpr (CAP) {                                // (a form of its own: a layer without a cap pays nothing)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) sc[i] = capped(sc[i]);
-        }
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            if constexpr (MASKED) {
-                const int key = key0 + 16 * (i / 8) + 8 * g32 + i % 8;       // (no branch, see the per-wave kernel)
-                const bool seen = (key <= last_seen) & ((key >= first_seen_key) | (key < kept_seen));
-                sc[i] = seen ? sc[i] : -INFINITY;
-            }
-            mx = fmaxf(mx, sc[i]);
-        }
-        mx = max_xor32(mx) * c2;
-        // m32 is the row's reference for the exponentials, not its maximum: it moves only when
-        // a tile's maximum lies more than LAZY_MAX above it, so the accumulators are rescaled a
-        // few times per row instead of in most tiles; weights stay below 2^LAZY_MAX
-        rescale = mx > m32 + LAZY_MAX;
-        const float mn = rescale ? mx : m32;
-        const float ms = mn == -INFINITY ? 0.f : mn;
-        alpha = rescale ? __builtin_amdgcn_exp2f(m32 - ms) : 1.f;
-        float p[16];
-        float psum = 0.f;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            p[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[i], c2, -ms));
-            psum += p[i];
-        }
-        l32 = l32 * alpha + psum;
-        m32 = mn;
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-            pf[h] = make_uint4(pack_bf16x2(p[8 * h], p[8 * h + 1]), pack_bf16x2(p[8 * h + 2], p[8 * h + 3]),
-                               pack_bf16x2(p[8 * h + 4], p[8 * h + 5]), pack_bf16x2(p[8 * h + 6], p[8 * h + 7]));
-    };
-    auto weighted32 = [&](int buf, const uint4 (&pf)[2], float alpha, bool rescale) {
-        const uint16_t* vt = v_lds[buf];
-        if (__any(rescale)) {                               // rare; in place (see scale_in_place)
-            scale_fence();
-#pragma unroll
-            for (int b = 0; b < DB32; ++b)
-#pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    float v = o32[b][i];
-                    scale_in_place(v, alpha);
-                    o32[b][i] = v;
-                }
-            scale_fence();
-        }
-#pragma unroll
-        for (int b = 0; b < DB32; ++b) {
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const uint2* src = reinterpret_cast<const uint2*>(vt + (32 * b + c32) * PF_V_STRIDE + 16 * h + 8 * g32);
-                const uint2 lo = src[0], hi = src[1];
-                const uint4 va = make_uint4(lo.x, lo.y, hi.x, hi.y);
-                o32[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8_t*>(&va),
-                                                                  *reinterpret_cast<const bf16x8_t*>(&pf[h]), o32[b], 0, 0, 0);
-            }
-        }
-    };
-
     // Two tiles of global loads are in flight while one is computed: at the top of the
     // iteration of tile t, tile t sits in LDS buffer t % 2, the loads of tile t + 1 are on
     // their way into one pair of staging registers, and the pages of tile t + 2 were asked
@@ -1593,21 +1461,12 @@ paged_attn_prefill_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k
             // the window of its last one (of means: all its entries are seen by the wave's first row)
             const bool whole = of_means ? key0 - PF_MEAN + PF_KEYS <= means_lo
                                         : key0 + PF_KEYS - 1 <= wave_lo_pos && key0 >= wave_first;
-            if constexpr (M32) {
-                uint4 pf[2];
-                float alpha;
-                bool rescale;
-                if (whole) scores32(key0, buf, std::false_type{}, pf, alpha, rescale);
-                else scores32(key0, buf, std::true_type{}, pf, alpha, rescale);
-                weighted32(buf, pf, alpha, rescale);
-            } else {
-                uint4 pf[RT];
-                float alpha[RT];
-                bool any_rescale;
-                if (whole) scores(key0, buf, std::false_type{}, pf, alpha, any_rescale);
-                else scores(key0, buf, std::true_type{}, pf, alpha, any_rescale);
-                weighted(buf, pf, alpha, any_rescale);
-            }
+            uint4 pf[RT];
+            float alpha[RT];
+            bool any_rescale;
+            if (whole) scores(key0, buf, std::false_type{}, pf, alpha, any_rescale);
+            else scores(key0, buf, std::true_type{}, pf, alpha, any_rescale);
+            weighted(buf, pf, alpha, any_rescale);
         }
     };
     int pg0[2], pg1[2];
@@ -1618,11 +1477,11 @@ paged_attn_prefill_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k
     lookup(real(klo + PF_KEYS), pg1);
     fetch(real(klo), pg0, kr0, vr0);
     lookup(real(klo + 2 * PF_KEYS), pg0);
-    if (klo + PF_KEYS < kend) fetch(real(klo + PF_KEYS), pg1, kr1, vr1);
+    if (klo + PF_KEYS < khi) fetch(real(klo + PF_KEYS), pg1, kr1, vr1);
     stash(0, real(klo), kr0, vr0);
     __syncthreads();
     int key0 = klo;
-    for (; key0 + 3 * PF_KEYS < kend; key0 += 2 * PF_KEYS) {
+    for (; key0 + 3 * PF_KEYS < khi; key0 += 2 * PF_KEYS) {
         lookup(real(key0 + 3 * PF_KEYS), pg1);
         fetch(real(key0 + 2 * PF_KEYS), pg0, kr0, vr0);
         tile(real(key0), 0);
@@ -1634,7 +1493,7 @@ paged_attn_prefill_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k
         stash(0, real(key0 + 2 * PF_KEYS), kr0, vr0);
         __syncthreads();
     }
-    const bool has1 = key0 + PF_KEYS < kend, has2 = key0 + 2 * PF_KEYS < kend;    // the same in all threads
+    const bool has1 = key0 + PF_KEYS < khi, has2 = key0 + 2 * PF_KEYS < khi;    // the same in all threads
     if (has2) fetch(real(key0 + 2 * PF_KEYS), pg0, kr0, vr0);
     tile(real(key0), 0);
     if (has1) {
@@ -1648,50 +1507,6 @@ paged_attn_prefill_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k
         }
     }
 
-    if constexpr (M32) {
-        float L = sum_xor32(l32);
-        float m_ref = m32 == -INFINITY ? 0.f : m32;          // what the weights in L are relative to
-        if constexpr (KS == 2) {
-            // the second half hands its result over: [wave][value][lane] floats where the tiles were
-            static_assert(KS * 2 * PF_TILE_ELEMS * 2 >= 4 * 64 * (16 * DB32 + 2) * 4, "the tiles' space holds the exchange");
-            float* xch = reinterpret_cast<float*>(tiles_lds) + (size_t)wave * (16 * DB32 + 2) * 64 + lane;
-            __syncthreads();                                 // every wave is done with the tiles
-            if (half == 1) {
-#pragma unroll
-                for (int b = 0; b < DB32; ++b)
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) xch[(16 * b + i) * 64] = o32[b][i];
-                xch[(16 * DB32) * 64] = m32;
-                xch[(16 * DB32 + 1) * 64] = L;
-            }
-            __syncthreads();
-            if (half == 1) return;
-            const float m_b = xch[(16 * DB32) * 64], l_b = xch[(16 * DB32 + 1) * 64];
-            const float mn = fmaxf(m32, m_b);
-            const float ms = mn == -INFINITY ? 0.f : mn;
-            const float wa = __builtin_amdgcn_exp2f(m32 - ms), wb = __builtin_amdgcn_exp2f(m_b - ms);
-            L = L * wa + l_b * wb;
-            m_ref = ms;
-#pragma unroll
-            for (int b = 0; b < DB32; ++b)
-#pragma unroll
-                for (int i = 0; i < 16; ++i) o32[b][i] = o32[b][i] * wa + xch[(16 * b + i) * 64] * wb;
-        }
-        if (sink) L += __builtin_amdgcn_exp2f(sink32_l2 - m_ref);   // one more weight (of score 0, or the head's own), no value
-        if (row_pos32 >= 0) {
-            const float inv = L > 0.f ? 1.0f / L : 0.f;
-#pragma unroll
-            for (int b = 0; b < DB32; ++b)
-#pragma unroll
-                for (int a = 0; a < 4; ++a) {                 // o32[b][4a + j] is d = 32 b + 8 a + 4 g32 + j
-                    uint2 pk;
-                    pk.x = pack_bf16x2(o32[b][4 * a] * inv, o32[b][4 * a + 1] * inv);
-                    pk.y = pack_bf16x2(o32[b][4 * a + 2] * inv, o32[b][4 * a + 3] * inv);
-                    *reinterpret_cast<uint2*>(out + row_q32 + 32 * b + 8 * a + 4 * g32) = pk;
-                }
-        }
-        return;
-    }
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
         float L = l[rt];
@@ -1708,6 +1523,321 @@ paged_attn_prefill_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k
         }
     }
 }
+
+// The same with 32 rows per wave through the 32 x 32 x 16 products (head sizes in steps of 32): tiles of 64 keys, which
+// global_load_lds brings to LDS as they lie in their pages, 16 bytes per lane, while the tile before is computed: no staging
+// registers, no LDS writes, and V is read transposed, the next 16 keys' while 16 are multiplied. LDS row r of 32 holds key
+// pm_key(r), in that order because a lane then gets two runs of eight neighbouring keys out of a product with K, which is what
+// the second product wants as operand B; the 16-byte pieces of a row are swapped among themselves so that neither read meets
+// bank conflicts. Two tiles of 32 scores side by side in a wave are two independent chains of products.
+// KS = 2: eight waves; waves 0-3 walk the first half of the block's key tiles and waves 4-7, with the same rows, the second half,
+// each four with tiles of their own in LDS; at the end the two partial results are combined through LDS. Twice the waves for the
+// same number of workgroups: for launches whose workgroups are too few, or too uneven (a prompt from its start: the last block
+// sees all keys, the first none), to fill the GPU otherwise.
+// Against tiles of 32 keys staged through registers, one chain of scores, 8 kv heads of 4 x 128, us, KS 2 / KS 1: 512 tokens from
+// 0 20.8 / 23.5, now 18.0 / 20.7; 2,048 from 0 67.8 / 80.4, now 57.3 / 70.6; 8,192 from 0 780 / 689, now 672 / 636 (0.87
+// PFLOP/s); 1,981 behind 750 96.8 / 102, now 84.6 / 90.9; 1,024 behind 3,072 101 / 137, now 83.0 / 115. What bounds it: a tile
+// costs a wave some 1,500 cycles of vector instructions (32 exponentials a lane, 16 cycles each, are a third) beside 1,024 of
+// products, and the two waves of a SIMD hardly overlap them. Taken back: the halves one phase apart behind two barriers a tile
+// (65.9 / 799 for 2,048 and 8,192 tokens: a phase without its own neighbour waits for LDS), the next tile's scores between
+// this one's exponentials (spills), a wave priority around the products (no change).
+#if SOC_HEAD_DIM % 32 == 0 && SOC_HEAD_DIM <= 128
+constexpr int PM_KEYS = 64;
+constexpr int PM_TILE = PM_KEYS * D;                 // elements of a tile of K or of V
+
+__device__ __forceinline__ int pm_key(int r) { return (r & ~12) | ((r & 4) << 1) | ((r & 8) >> 1); }   // its own inverse
+__device__ __forceinline__ int pm_swap_k(int r) { return D % 128 == 0 ? r & 15 : D % 64 == 0 ? (r >> 1) & 7 : (r >> 2) & 3; }
+__device__ __forceinline__ int pm_swap_v(int r) { return D % 128 == 0 ? (r & 3) << 2 : D % 64 == 0 ? ((r >> 1) & 1) << 2 : 0; }
+
+typedef __attribute__((ext_vector_type(16))) float f32x16_t;
+
+__device__ __forceinline__ void pm_load(uint32_t lds, const bf16* from) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(from) : "m0");
+}
+
+// SHIFT: pages hold a power of two of keys.
+template <int KS, bool SHIFT, bool CAP>
+__global__ void __launch_bounds__(256 * KS, 2)
+paged_attn_prompt_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k_pool, const bf16* __restrict__ v_pool,
+                         const int* __restrict__ block_table, int table_width, const int* __restrict__ token_rows,
+                         const int* __restrict__ positions, const int* __restrict__ row_blocks, bf16* __restrict__ out, int Hq,
+                         int Hkv, int BS, int bs_shift, float scale, int window, int group_pad_log2, int keep_first, int sink,
+                         const float* __restrict__ sinks, const bf16* __restrict__ mean_k, const bf16* __restrict__ mean_v,
+                         const int* __restrict__ mean_table, int mean_table_width, int pool, float softcap) {
+    constexpr int DQ = D / 16, DB = D / 32, PARTS = D / 8, NI = D / 32;      // NI: loads of a wave per tile of K, and of V
+    __shared__ __attribute__((aligned(1024))) uint16_t tiles[KS * 4 * PM_TILE];
+    const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x / SOC_WAVE), lane = threadIdx.x % SOC_WAVE;
+    const int half = wave_all / 4, wave = wave_all % 4;             // which keys, which rows
+    uint16_t* const mine = tiles + half * 4 * PM_TILE;              // [buffer][K, V]
+    const uint32_t mine_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t*)mine;
+    const int G = Hq / Hkv, Gp = 1 << group_pad_log2, chunks = (G + 15) / 16;
+    // late row blocks see the most keys: they go first, so that the short ones fill the end
+    const int blk = (int)(gridDim.x / (Hkv * chunks)) - 1 - (int)(blockIdx.x / (Hkv * chunks));
+    const int kvh = (blockIdx.x / chunks) % Hkv, chunk = blockIdx.x % chunks;
+    const int tok0 = row_blocks ? row_blocks[2 * blk] : blk, ntok = row_blocks ? row_blocks[2 * blk + 1] : 1;
+    const int pos0 = positions[tok0];
+    const int* table = block_table + (size_t)token_rows[tok0] * table_width;
+    const int tokens_per_wave = 32 >> group_pad_log2;
+
+    // the walk over kept first keys or means and then the window's keys: see the kernel above
+    const int khi = pos0 + ntok;                                    // keys any row of the block sees
+    int kmin = first_seen(pos0, window);
+    int kept = window > 0 ? min(keep_first, kmin) : 0, n_pre = (kept + PM_KEYS - 1) / PM_KEYS;
+    if (n_pre * PM_KEYS > (kmin & ~(PM_KEYS - 1))) { kmin = 0; kept = 0; n_pre = 0; }
+    auto blocks_before = [&](int pos) { const int d = pos - window + 1; return d > 0 ? d / pool : 0; };
+    const int n_means = pool > 0 ? blocks_before(khi - 1) : 0;      // entries any row of the block sees
+    if (pool > 0) n_pre = (n_means + PM_KEYS - 1) / PM_KEYS;
+    const int* mtable = pool > 0 ? mean_table + (size_t)token_rows[tok0] * mean_table_width : table;
+    int klo = kmin & ~(PM_KEYS - 1);
+    const int first_real = klo;                                     // virtual keys from here on are real ones
+    const int pre_shift = klo - n_pre * PM_KEYS;                    // a virtual key before that is the real key minus this
+    const int pre_base = (pool > 0 ? PF_MEAN : 0) - pre_shift;      // (or the entry of the pages of means, as PF_MEAN + entry)
+    if (KS == 1) klo = pre_shift;
+    // kend: where this half's walk over the tiles ends. Both halves take the same number of steps (they share the
+    // barriers); the second may run past khi, where keys are stand-ins that no row sees.
+    int kend = khi;
+    if constexpr (KS == 2) {
+        const int per_half = ((khi - klo + PM_KEYS - 1) / PM_KEYS + 1) / 2 * PM_KEYS;
+        klo += half * per_half;
+        kend = klo + per_half;
+    }
+    // this wave's rows, and this lane's: row lane % 32, half lane / 32 of every 16-wide step of the head
+    const int wtok0 = wave * tokens_per_wave;                       // first token of the wave in the block
+    const int wave_lo_pos = pos0 + wtok0;                           // its first and last positions
+    const int wave_hi_pos = min(khi, wave_lo_pos + tokens_per_wave) - 1;
+    const bool wave_has_rows = wtok0 < ntok;
+    const int wave_first = first_seen(wave_hi_pos, window);         // the first key that all of the wave's rows see
+    const float c2 = scale * 1.44269504088896340736f;               // to base 2
+    const SoftCap capped(scale, softcap);
+    const int means_lo = pool > 0 ? blocks_before(wave_lo_pos) : 0; // entries that all / any of the wave's rows see
+    const int means_hi = pool > 0 ? blocks_before(wave_hi_pos) : 0;
+    const int c32 = lane % 32, g32 = lane / 32;
+    const int tt = wtok0 + (c32 >> group_pad_log2), gh = chunk * 16 + (c32 & (Gp - 1));
+    const bool ok = tt < ntok && gh < G;
+    const int row_pos = ok ? pos0 + tt : -1, row_first = first_seen(ok ? pos0 + tt : pos0, window);
+    const size_t row_q = ((size_t)(tok0 + (ok ? tt : 0)) * Hq + (size_t)kvh * G + (ok ? gh : 0)) * D;
+    const int mean_end = pool > 0 && ok ? PF_MEAN + blocks_before(pos0 + tt) : PF_MEAN;   // the first entry the row does not see
+    const float sink_l2 = sink == 2 && ok ? sinks[kvh * G + gh] * 1.44269504088896340736f : 0.f;
+    uint4 qf[DQ];
+#pragma unroll
+    for (int t = 0; t < DQ; ++t) qf[t] = ok ? *reinterpret_cast<const uint4*>(q + row_q + 16 * t + 8 * g32) : make_uint4(0u, 0u, 0u, 0u);
+    f32x16_t o[DB];
+    float m = -INFINITY, l = 0.f;
+#pragma unroll
+    for (int b = 0; b < DB; ++b)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[b][i] = 0.f;
+
+    // This lane's pieces of a tile: piece s of (wave NI + i) 64 + lane lies in row s / PARTS. A key outside the range is
+    // redirected to the nearest one inside, which lies in the same tile (behind the last one: in the last tile that has
+    // keys): its weight is 0, and a value that is not finite reaches no row that its own tile would not have reached.
+    const size_t page_stride = (size_t)Hkv * BS * D, head = (size_t)kvh * BS * D;
+    int row_key[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) row_key[i] = pm_key(((wave * NI + i) * 64 + lane) / PARTS);
+    // (everything is read before it is chosen from: the compiler turns a choice between two captured variables into one between
+    // their addresses, and they end up in scratch memory)
+    auto key_of = [&](int key0, int i) {                     // key0 < 0: a tile of means, PF_MEAN + entry
+        const int first = key0 < 0 ? key0 - PF_MEAN : key0, last_mean = n_means - 1, last_kept = kept - 1, last = khi - 1, lowest = kmin;
+        const bool front = key0 < first_real;                // means or kept keys
+        const int low = front ? 0 : lowest, high = front ? (key0 < 0 ? last_mean : last_kept) : last;
+        return min(max(first + row_key[i], low), high);
+    };
+    auto lookup = [&](int key0, int (&pg)[NI]) {
+        const int *of_tokens = table, *of_means = mtable, *tb = key0 < 0 ? of_means : of_tokens;      // uniform
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const int key = key_of(key0, i);
+            pg[i] = tb[SHIFT ? key >> bs_shift : key / BS];
+        }
+    };
+    auto fetch = [&](int key0, const int (&pg)[NI], int buf) {
+        const bf16 *k0 = k_pool, *k1 = mean_k, *v0 = v_pool, *v1 = mean_v;
+        const bf16* kp = (key0 < 0 ? k1 : k0) + head;
+        const bf16* vp = (key0 < 0 ? v1 : v0) + head;
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const int key = key_of(key0, i), s = (wave * NI + i) * 64 + lane, r = s / PARTS, part = s % PARTS;
+            const size_t off = (size_t)pg[i] * page_stride + (size_t)((SHIFT ? key & (BS - 1) : key % BS) * D);
+            const uint32_t to = __builtin_amdgcn_readfirstlane(mine_lds + (buf * 2 * PM_TILE + (wave * NI + i) * 512) * 2);
+            pm_load(to, kp + off + (part ^ pm_swap_k(r)) * 8);
+            pm_load(to + PM_TILE * 2, vp + off + (part ^ pm_swap_v(r)) * 8);
+        }
+    };
+
+    // V^T of 16 keys of a tile. A transposed read: 16 lanes name the 8-byte pieces of a block of 4 keys x 16 elements and each
+    // receives one element of the 4 keys; keys 4 to 7 of a lane's eight lie eight rows further on (pm_key).
+    auto values = [&](int buf, int h, uint4 (&va)[DB]) {
+        const int li = lane % 16, r0 = 4 * g32 + li / 4, piece = lane / 16 % 2 * 2 + li % 4 / 2;
+        const uint16_t* vt = mine + buf * 2 * PM_TILE + PM_TILE + (r0 + h * 16) * D + li % 2 * 4;
+#pragma unroll
+        for (int b = 0; b < DB; ++b) {
+            const uint16_t* at = vt + ((4 * b + piece) ^ pm_swap_v(r0)) * 8;
+            const s16x4_t v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)at);
+            const s16x4_t v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)(at + 8 * D));
+            const uint2 lo = *reinterpret_cast<const uint2*>(&v0), hi = *reinterpret_cast<const uint2*>(&v1);
+            va[b] = make_uint4(lo.x, lo.y, hi.x, hi.y);
+        }
+    };
+    // Scores and softmax weights (packed as operand B of the second product); MASKED: some key of the tile is hidden from
+    // some row. The second half is one piece of code behind both variants, so that the accumulators have one home.
+    auto scores = [&](int key0, int buf, auto masked_tag, uint4 (&pf)[4], uint4 (&va)[DB], float& alpha, bool& rescale) {
+        constexpr bool MASKED = decltype(masked_tag)::value;
+        const uint16_t* kt = mine + buf * 2 * PM_TILE + c32 * D;
+        f32x16_t sc[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) sc[u][i] = 0.f;
+#pragma unroll
+        for (int t = 0; t < DQ; ++t)
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const uint4 ka = *reinterpret_cast<const uint4*>(kt + u * 32 * D + ((2 * t + g32) ^ pm_swap_k(c32)) * 8);
+                sc[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8_t*>(&ka),
+                                                                *reinterpret_cast<const bf16x8_t*>(&qf[t]), sc[u], 0, 0, 0);
+            }
+        values(buf, 0, va);                                  // (on their way under the softmax)
+        __builtin_amdgcn_sched_barrier(0);
+        const int last_seen = key0 < 0 ? mean_end - 1 : row_pos;
+        const int first_seen_key = key0 < 0 ? key0 : row_first, kept_seen = key0 < 0 ? key0 : keep_first;
+        float mx[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};      // of the raw scores: the scale is positive
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                if constexpr (CAP) sc[u][i] = capped(sc[u][i]);          // (a form of its own: a layer without a cap pays nothing)
+                if constexpr (MASKED) {
+                    const int key = key0 + 32 * u + 16 * (i / 8) + 8 * g32 + i % 8;      // (no branch, see the per-wave kernel)
+                    const bool seen = (key <= last_seen) & ((key >= first_seen_key) | (key < kept_seen));
+                    sc[u][i] = seen ? sc[u][i] : -INFINITY;
+                }
+                mx[i % 4] = fmaxf(mx[i % 4], sc[u][i]);
+            }
+        const float top = max_xor32(fmaxf(fmaxf(mx[0], mx[1]), fmaxf(mx[2], mx[3]))) * c2;
+        // m is the row's reference for the exponentials, not its maximum: it moves only when a tile's maximum lies more
+        // than LAZY_MAX above it, so the accumulators are rescaled a few times per row instead of in most tiles; weights
+        // stay below 2^LAZY_MAX
+        rescale = top > m + LAZY_MAX;
+        const float mn = rescale ? top : m;
+        const float ms = mn == -INFINITY ? 0.f : mn;
+        alpha = rescale ? __builtin_amdgcn_exp2f(m - ms) : 1.f;
+        float psum[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                float p[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    p[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[u][8 * h + i], c2, -ms));
+                    psum[i % 4] += p[i];
+                }
+                pf[2 * u + h] = make_uint4(pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3]), pack_bf16x2(p[4], p[5]), pack_bf16x2(p[6], p[7]));
+            }
+        l = l * alpha + ((psum[0] + psum[1]) + (psum[2] + psum[3]));
+        m = mn;
+    };
+    auto weighted = [&](int buf, const uint4 (&pf)[4], uint4 (&va)[2][DB], float alpha, bool rescale) {
+        if (__any(rescale)) {                               // rare; in place (see scale_in_place)
+            scale_fence();
+#pragma unroll
+            for (int b = 0; b < DB; ++b)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    float v = o[b][i];
+                    scale_in_place(v, alpha);
+                    o[b][i] = v;
+                }
+            scale_fence();
+        }
+        // O^T += V^T P^T, 16 keys at a time, those of the next 16 read meanwhile
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+            if (h < 3) values(buf, h + 1, va[(h + 1) % 2]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int b = 0; b < DB; ++b)
+                o[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8_t*>(&va[h % 2][b]),
+                                                               *reinterpret_cast<const bf16x8_t*>(&pf[h]), o[b], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    auto tile = [&](int key0, int buf) {
+        const bool of_means = key0 < 0;                      // uniform
+        if (wave_has_rows && (of_means ? key0 - PF_MEAN < means_hi : key0 <= wave_hi_pos)) {
+            // whole: every key of the tile is at or before the wave's first position and inside the window of its last
+            // one (of means: all its entries are seen by the wave's first row)
+            const bool whole = of_means ? key0 - PF_MEAN + PM_KEYS <= means_lo : key0 + PM_KEYS - 1 <= wave_lo_pos && key0 >= wave_first;
+            uint4 pf[4], va[2][DB];
+            float alpha;
+            bool rescale;
+            if (whole) scores(key0, buf, std::false_type{}, pf, va[0], alpha, rescale);
+            else scores(key0, buf, std::true_type{}, pf, va[0], alpha, rescale);
+            weighted(buf, pf, va, alpha, rescale);
+        }
+    };
+    // A tile's loads have the whole tile before it to land, and its pages are looked up one more tile ahead.
+    auto real = [&](int v) { return v < first_real ? v + pre_base : v; };      // (the walk is over virtual keys)
+    int pg[NI];
+    lookup(real(klo), pg);
+    fetch(real(klo), pg, 0);
+    if (klo + PM_KEYS < kend) lookup(real(klo + PM_KEYS), pg);
+    int buf = 0;
+    for (int key0 = klo; key0 < kend; key0 += PM_KEYS, buf ^= 1) {
+        // this wave's pieces of the tile have landed and it has read the other buffer; behind the barrier so have all
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (key0 + PM_KEYS < kend) {
+            fetch(real(key0 + PM_KEYS), pg, buf ^ 1);
+            if (key0 + 2 * PM_KEYS < kend) lookup(real(key0 + 2 * PM_KEYS), pg);
+        }
+        tile(real(key0), buf);
+    }
+
+    float L = sum_xor32(l);
+    float m_ref = m == -INFINITY ? 0.f : m;                  // what the weights in L are relative to
+    if constexpr (KS == 2) {
+        // the second half hands its result over: [wave][value][lane] floats where the tiles were
+        static_assert(KS * 4 * PM_TILE * 2 >= 4 * 64 * (16 * DB + 2) * 4, "the tiles' space holds the exchange");
+        float* xch = reinterpret_cast<float*>(tiles) + (size_t)wave * (16 * DB + 2) * 64 + lane;
+        __syncthreads();                                     // every wave is done with the tiles
+        if (half == 1) {
+#pragma unroll
+            for (int b = 0; b < DB; ++b)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) xch[(16 * b + i) * 64] = o[b][i];
+            xch[(16 * DB) * 64] = m;
+            xch[(16 * DB + 1) * 64] = L;
+        }
+        __syncthreads();
+        if (half == 1) return;
+        const float m_b = xch[(16 * DB) * 64], l_b = xch[(16 * DB + 1) * 64];
+        const float mn = fmaxf(m, m_b);
+        const float ms = mn == -INFINITY ? 0.f : mn;
+        const float wa = __builtin_amdgcn_exp2f(m - ms), wb = __builtin_amdgcn_exp2f(m_b - ms);
+        L = L * wa + l_b * wb;
+        m_ref = ms;
+#pragma unroll
+        for (int b = 0; b < DB; ++b)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) o[b][i] = o[b][i] * wa + xch[(16 * b + i) * 64] * wb;
+    }
+    if (sink) L += __builtin_amdgcn_exp2f(sink_l2 - m_ref);  // one more weight (of score 0, or the head's own), no value
+    if (row_pos >= 0) {
+        const float inv = L > 0.f ? 1.0f / L : 0.f;
+#pragma unroll
+        for (int b = 0; b < DB; ++b)
+#pragma unroll
+            for (int a = 0; a < 4; ++a) {                    // o[b][4a + j] is d = 32 b + 8 a + 4 g32 + j
+                uint2 pk;
+                pk.x = pack_bf16x2(o[b][4 * a] * inv, o[b][4 * a + 1] * inv);
+                pk.y = pack_bf16x2(o[b][4 * a + 2] * inv, o[b][4 * a + 3] * inv);
+                *reinterpret_cast<uint2*>(out + row_q + 32 * b + 8 * a + 4 * g32) = pk;
+            }
+    }
+}
+
+#endif  // head sizes in steps of 32 up to 128
 
 // bfloat16 only, head sizes up to 128, no key splits. row_blocks [n_row_blocks, 2] = (first
 // token, tokens) of each block of at most 4 * ((16 * row_tiles) >> group_pad_log2) tokens of
@@ -1746,22 +1876,33 @@ SOC_EXPORT int soc_paged_attention_prefill(const void* q, const void* k_pool, co
         token_rows, positions, row_blocks, (bf16*)out, Hq, Hkv, BS, bs_shift, scale, window, group_pad_log2, \
         keep_first, sink, sinks, (const bf16*)mean_k, (const bf16*)mean_v, mean_table, mean_table_width, pool, softcap
         const bool pair = bs_shift >= 1;
-#define SOC_PF_LAUNCH(RT_, M32_, KS_)                                                                            \
+#define SOC_PF_LAUNCH(RT_)                                                                                        \
     do {                                                                                                    \
         if (softcap > 0.f) {                                                                                \
-            if (pair) hipLaunchKernelGGL((paged_attn_prefill_kernel<RT_, true, M32_, KS_, true>), dim3((unsigned)groups), dim3(256 * KS_), 0, stream, SOC_PF_ARGS); \
-            else hipLaunchKernelGGL((paged_attn_prefill_kernel<RT_, false, M32_, KS_, true>), dim3((unsigned)groups), dim3(256 * KS_), 0, stream, SOC_PF_ARGS);     \
-        } else if (pair) hipLaunchKernelGGL((paged_attn_prefill_kernel<RT_, true, M32_, KS_>), dim3((unsigned)groups), dim3(256 * KS_), 0, stream, SOC_PF_ARGS); \
-        else hipLaunchKernelGGL((paged_attn_prefill_kernel<RT_, false, M32_, KS_>), dim3((unsigned)groups), dim3(256 * KS_), 0, stream, SOC_PF_ARGS);     \
+            if (pair) hipLaunchKernelGGL((paged_attn_prefill_kernel<RT_, true, true>), dim3((unsigned)groups), dim3(256), 0, stream, SOC_PF_ARGS); \
+            else hipLaunchKernelGGL((paged_attn_prefill_kernel<RT_, false, true>), dim3((unsigned)groups), dim3(256), 0, stream, SOC_PF_ARGS);     \
+        } else if (pair) hipLaunchKernelGGL((paged_attn_prefill_kernel<RT_, true>), dim3((unsigned)groups), dim3(256), 0, stream, SOC_PF_ARGS); \
+        else hipLaunchKernelGGL((paged_attn_prefill_kernel<RT_, false>), dim3((unsigned)groups), dim3(256), 0, stream, SOC_PF_ARGS);     \
     } while (0)
-        if (row_tiles == 1) SOC_PF_LAUNCH(1, false, 1);
-        else if (row_tiles == 2) SOC_PF_LAUNCH(2, false, 1);
+#define SOC_PM_LAUNCH(KS_)                                                                                        \
+    do {                                                                                                    \
+        if (softcap > 0.f) {                                                                                \
+            if (bs_shift >= 0) hipLaunchKernelGGL((paged_attn_prompt_kernel<KS_, true, true>), dim3((unsigned)groups), dim3(256 * KS_), 0, stream, SOC_PF_ARGS); \
+            else hipLaunchKernelGGL((paged_attn_prompt_kernel<KS_, false, true>), dim3((unsigned)groups), dim3(256 * KS_), 0, stream, SOC_PF_ARGS); \
+        } else if (bs_shift >= 0) hipLaunchKernelGGL((paged_attn_prompt_kernel<KS_, true, false>), dim3((unsigned)groups), dim3(256 * KS_), 0, stream, SOC_PF_ARGS); \
+        else hipLaunchKernelGGL((paged_attn_prompt_kernel<KS_, false, false>), dim3((unsigned)groups), dim3(256 * KS_), 0, stream, SOC_PF_ARGS); \
+    } while (0)
+        if (row_tiles == 1) SOC_PF_LAUNCH(1);
+        else if (row_tiles == 2) SOC_PF_LAUNCH(2);
         else if (row_tiles == 32 || row_tiles == 64) {       // 32 rows per wave through the 32 x 32 products
-            if constexpr (D % 32 == 0) {
-                if (row_tiles == 32) SOC_PF_LAUNCH(1, true, 1);
-                else SOC_PF_LAUNCH(1, true, 2);              // and the keys of a block in two halves
-            } else return (int)hipErrorInvalidValue;
+#if SOC_HEAD_DIM % 32 == 0 && SOC_HEAD_DIM <= 128
+            if (row_tiles == 32) SOC_PM_LAUNCH(1);
+            else SOC_PM_LAUNCH(2);                           // and the keys of a block in two halves
+#else
+            return (int)hipErrorInvalidValue;
+#endif
         } else return (int)hipErrorInvalidValue;
+#undef SOC_PM_LAUNCH
 #undef SOC_PF_LAUNCH
 #undef SOC_PF_ARGS
         return soc_last_error();
