@@ -6,6 +6,7 @@
 // the weighted sum over depth are float32 whatever the compute dtype; a value is rounded once, where it
 // is stored in the compute dtype.
 #include "common.h"
+#include "prepare.h"
 #include "recurrent.h"
 
 __device__ __forceinline__ float cmp_sigmoid(float x) { return 1.f / (1.f + expf(-x)); }
@@ -297,6 +298,15 @@ SOC_EXPORT int soc_window_prepare(const void* x, int ld, int col_q, int col_k, i
     if ((norm == 1 || norm == 2) && (!q_gain || !k_gain)) return (int)hipErrorInvalidValue;
     if (half && !inv_freq) return (int)hipErrorInvalidValue;
     if (value_freq && Dv % 2) return (int)hipErrorInvalidValue;
+    if (dtype == 1) {
+        const PrepareArgs a{(const bf16*)x, ld, col_q, col_k, col_v, bias, nullptr, 0, nullptr, (bf16*)q_out, (bf16*)k_pool, (bf16*)v_pool, table,
+                            table_width, token_rows, positions, q_gain, k_gain, norm, eps, inv_freq, half, magnitude, value_freq, Hq, Hkv, BS};
+        if (heads_prepare_fits(a, N, D, Dv, P, true)) {
+            if (D == 128) hipLaunchKernelGGL((heads_prepare_kernel<128, true>), dim3(N), dim3(256), 0, stream, a);
+            else hipLaunchKernelGGL((heads_prepare_kernel<64, true>), dim3(N), dim3(256), 0, stream, a);
+            return soc_last_error();
+        }
+    }
     // A token's heads go to as many workgroups as give the step about two per compute unit (a decode step has few
     // tokens: one workgroup per token left the GPU idle), at most one per head.
     int groups = (512 + N - 1) / N;
@@ -399,11 +409,39 @@ __global__ void turn_back_kernel(const T* __restrict__ o, T* __restrict__ out, c
     }
 }
 
+// The same eight elements at a time (P and Dv multiples of 8, rows on 16 bytes), bfloat16, a workgroup per token that takes
+// its angles once: 2,048 tokens of 32 heads of 128 24 -> 7 us.
+__global__ void __launch_bounds__(256)
+turn_back_vec8_kernel(const bf16* __restrict__ o, bf16* __restrict__ out, const int* __restrict__ positions,
+                      const float* __restrict__ value_freq, int H, int P, int Dv) {
+    __shared__ float cs[256], sn[256];
+    const size_t n = blockIdx.x;
+    for (int m = threadIdx.x; m < Dv / 2; m += 256) sincosf((float)positions[n] * value_freq[m], &sn[m], &cs[m]);
+    __syncthreads();
+    const int per = Dv / 8;
+    for (int i = threadIdx.x; i < H * per; i += 256) {
+        const int h = i / per, j = i % per * 8;
+        float v[8], y[8];
+        VecLoad<bf16, 8>::load(o + (n * H + h) * P + j, v);
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) {
+            const float c = cs[(j + e) / 2], s = sn[(j + e) / 2];
+            y[e] = v[e] * c + v[e + 1] * s;
+            y[e + 1] = v[e + 1] * c - v[e] * s;
+        }
+        *reinterpret_cast<uint4*>(out + (n * H + h) * Dv + j) = make_uint4(pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3]), pack_bf16x2(y[4], y[5]), pack_bf16x2(y[6], y[7]));
+    }
+}
+
 SOC_EXPORT int soc_turn_back(const void* o, void* out, const int* positions, const float* value_freq, int N, int H, int P, int Dv,
                              int dtype, hipStream_t stream) {
     const size_t total = (size_t)N * H * Dv;
     if (!total) return 0;
     if (Dv > P || (value_freq && Dv % 2)) return (int)hipErrorInvalidValue;
+    if (dtype == 1 && value_freq && P % 8 == 0 && Dv % 8 == 0 && Dv <= 512 && ((uintptr_t)o | (uintptr_t)out) % 16 == 0) {
+        hipLaunchKernelGGL(turn_back_vec8_kernel, dim3(N), dim3(256), 0, stream, (const bf16*)o, (bf16*)out, positions, value_freq, H, P, Dv);
+        return soc_last_error();
+    }
     const int blocks = (int)((total + 255) / 256 < 8192 ? (total + 255) / 256 : 8192);
     if (dtype == 0)
         hipLaunchKernelGGL(turn_back_kernel<float>, dim3(blocks), dim3(256), 0, stream, (const float*)o, (float*)out, positions,

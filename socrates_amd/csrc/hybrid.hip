@@ -8,6 +8,7 @@
 // Statistics, angles, routers, the recurrence and its state and the residual sum are float32
 // whatever the compute dtype; a value is rounded once, where it is stored in the compute dtype.
 #include "common.h"
+#include "prepare.h"
 #include "recurrent.h"
 #include "wide.h"
 
@@ -108,6 +109,16 @@ SOC_EXPORT int soc_attn_prepare(const void* x, int ld, int col_q, int col_k, int
                                 float eps, int dtype, hipStream_t stream) {
     if (N <= 0) return 0;
     if (D < 1 || Dv < 1 || D > P || Dv > P || P > 256 || 2 * half > D || BS < 1) return (int)hipErrorInvalidValue;
+    if (dtype == 1 && !q_gain == !k_gain) {
+        const PrepareArgs a{(const bf16*)x, ld, col_q, col_k, col_v, nullptr, (const bf16*)first, first ? ldf : 0, lam, (bf16*)q_out, (bf16*)k_pool,
+                            (bf16*)v_pool, table, table_width, token_rows, positions, q_gain, k_gain, q_gain ? 1 : 0, eps, inv_freq, half, 1.f,
+                            nullptr, Hq, Hkv, BS};
+        if (heads_prepare_fits(a, N, D, Dv, P, false)) {
+            if (D == 128) hipLaunchKernelGGL((heads_prepare_kernel<128, false>), dim3(N), dim3(256), 0, stream, a);
+            else hipLaunchKernelGGL((heads_prepare_kernel<64, false>), dim3(N), dim3(256), 0, stream, a);
+            return soc_last_error();
+        }
+    }
     const long long items = (long long)N * (Hq + 2 * Hkv);
     const dim3 grid((unsigned)((items + 3) / 4));
 #define SOC_PREP(T)                                                                                                           \
@@ -134,10 +145,31 @@ __global__ void head_gate_kernel(const T* __restrict__ o, const T* __restrict__ 
     }
 }
 
+// The same eight elements at a time (P and Dv multiples of 8, rows on 16 bytes), bfloat16: 2,339 tokens of 32 heads of 128
+// 25 -> 8.4 us.
+__global__ void __launch_bounds__(256)
+head_gate_vec8_kernel(const bf16* __restrict__ o, const bf16* __restrict__ g, int ldg, bf16* __restrict__ out, unsigned groups, int H,
+                      int P, int Dv) {
+    const unsigned i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= groups) return;
+    const unsigned per = Dv / 8, nh = i / per, j = i % per * 8;
+    float v[8];
+    VecLoad<bf16, 8>::load(o + (size_t)nh * P + j, v);
+    const float open = g ? hyb_sigmoid(to_float(g[(size_t)(nh / H) * ldg + nh % H])) : 1.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] *= open;
+    *reinterpret_cast<uint4*>(out + (size_t)i * 8) = make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7]));
+}
+
 SOC_EXPORT int soc_head_gate(const void* o, const void* g, int ldg, void* out, int N, int H, int P, int Dv, int dtype,
                              hipStream_t stream) {
     const size_t total = (size_t)N * H * Dv;
     if (!total) return 0;
+    if (dtype == 1 && P % 8 == 0 && Dv % 8 == 0 && ((uintptr_t)o | (uintptr_t)out) % 16 == 0 && total / 8 < 1u << 31) {
+        hipLaunchKernelGGL(head_gate_vec8_kernel, dim3((unsigned)((total / 8 + 255) / 256)), dim3(256), 0, stream, (const bf16*)o, (const bf16*)g,
+                           ldg, (bf16*)out, (unsigned)(total / 8), H, P, Dv);
+        return soc_last_error();
+    }
     const int blocks = (int)((total + 255) / 256 < 4096 ? (total + 255) / 256 : 4096);
     if (dtype == 0)
         hipLaunchKernelGGL(head_gate_kernel<float>, dim3(blocks), dim3(256), 0, stream, (const float*)o, (const float*)g, ldg,
