@@ -228,6 +228,115 @@ gemm_f32_mfma_kernel(const TA* __restrict__ A, const TW* __restrict__ W, float* 
     }
 }
 
+// The same for two float32 operands and K in steps of 64: a workgroup owns 16 MT x 16 NT outputs and its four waves share K,
+// 16 k at a time in turn. A wave holds all the tile's sums, so it loads every operand once, straight into registers, one chunk of
+// 16 k ahead, and nothing is staged, shared or waited for until the waves' sums meet in LDS at the end, a quarter of the tile
+// each. The kernel above reads LDS four times for three products, stops at a barrier per 32 k, and with three blocks of rows
+// reads the weights three times; 131 rows ran at half of the matrix instruction's rate. Us cold, above -> here:
+// 131 rows x 2,560 -> 19,456 182 -> 116, -> 6,144 54 -> 48, 9,728 -> 2,560 83 -> 66, 4,096 -> 2,560 39 -> 32; 200 rows x 2,560 ->
+// 19,456 241 -> 177; 40 rows 67 -> 60. The error against 64 bits is the kernel's above or less: four shorter chains.
+// Bound by the matrix cores (45 products of 16 x 16 x 4 a chunk and k take 96 us at the first shape), where one workgroup per
+// compute unit fills the card; a row past M or N is read from the last one and not written.
+__device__ __forceinline__ void f32_product(f32x4& c, float a, float b) {
+    // (through the builtin the compiler moves accumulators about; it does not look into this one: f32_fence before they are read)
+    asm volatile("v_mfma_f32_16x16x4_f32 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+}
+
+template <int MT, int NT>
+__global__ void __launch_bounds__(256, 1)
+gemm_f32_own_k_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C, bf16* __restrict__ Cb, int M, int N,
+                      int K, int m_blocks, int n_blocks, int k_part) {
+    constexpr int NB = MT * NT;
+    __shared__ __align__(16) float4 meet[3][NB][64];
+    const int xcd = blockIdx.x % 8, idx = blockIdx.x / 8;    // (as above: the row blocks of one run of weights on one XCD)
+    const int nb = idx / m_blocks * 8 + xcd, mb = idx % m_blocks;
+    if (nb >= n_blocks) return;
+    const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), r = lane % 16, g = lane / 16;
+    const int m0 = mb * 16 * MT, n0 = nb * 16 * NT;
+    const int k_lo = blockIdx.y * k_part, steps = (min(K, k_lo + k_part) - k_lo) / 64;
+    const float *a[MT], *w[NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) a[i] = A + (size_t)min(m0 + 16 * i + r, M - 1) * K + k_lo + 16 * wave + 4 * g;
+#pragma unroll
+    for (int j = 0; j < NT; ++j) w[j] = W + (size_t)min(n0 + 16 * j + r, N - 1) * K + k_lo + 16 * wave + 4 * g;
+    f32x4 acc[NT][MT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int i = 0; i < MT; ++i) acc[j][i] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    struct Chunk { float4 x[MT], y[NT]; };
+    auto load = [&](int s, Chunk& c) {                       // (past the end the last chunk again)
+        const int at = min(s, steps - 1) * 64;
+#pragma unroll
+        for (int j = 0; j < NT; ++j) c.y[j] = *reinterpret_cast<const float4*>(w[j] + at);
+#pragma unroll
+        for (int i = 0; i < MT; ++i) c.x[i] = *reinterpret_cast<const float4*>(a[i] + at);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto products = [&](const Chunk& c, auto part) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int i = 0; i < MT; ++i) f32_product(acc[j][i], part(c.y[j]), part(c.x[i]));
+    };
+    auto multiply = [&](const Chunk& c) {
+        products(c, [](const float4& v) { return v.x; });
+        products(c, [](const float4& v) { return v.y; });
+        products(c, [](const float4& v) { return v.z; });
+        products(c, [](const float4& v) { return v.w; });
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    Chunk c0, c1;
+    load(0, c0);
+    int s = 0;
+    for (; s + 2 <= steps; s += 2) {
+        load(s + 1, c1);
+        multiply(c0);
+        load(s + 2, c0);
+        multiply(c1);
+    }
+    if (s < steps) multiply(c0);
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int i = 0; i < MT; ++i) asm volatile("" : "+a"(acc[j][i]));
+    // block b belongs to wave b % 4; the others hand theirs over, each in a place of its own
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+        if (b % 4 != wave) {
+            const f32x4& v = acc[b / MT][b % MT];
+            meet[(wave + 3 - b % 4) % 4][b][lane] = make_float4(v[0], v[1], v[2], v[3]);
+        }
+    __syncthreads();
+    if (C) C += (size_t)blockIdx.y * M * N;
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+        if (b % 4 == wave) {
+            const f32x4& v = acc[b / MT][b % MT];
+            float y[4] = {v[0], v[1], v[2], v[3]};
+#pragma unroll
+            for (int o = 0; o < 3; ++o) {
+                const float4 t = meet[o][b][lane];
+                y[0] += t.x; y[1] += t.y; y[2] += t.z; y[3] += t.w;
+            }
+            const int m = m0 + b % MT * 16 + r, n = n0 + b / MT * 16 + 4 * g;
+            const size_t at = (size_t)m * N + n;
+            if (m >= M) continue;
+            if (n + 4 <= N && N % 4 == 0) {
+                if (C) *reinterpret_cast<float4*>(C + at) = make_float4(y[0], y[1], y[2], y[3]);
+                else *reinterpret_cast<uint2*>(Cb + at) = make_uint2(pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3]));
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (n + e < N) {
+                        if (C) C[at + e] = y[e];
+                        else Cb[at + e] = from_float<bf16>(y[e]);
+                    }
+            }
+        }
+}
+
 // out[i] = the sum of parts[s][i] over s, in order; n is a multiple of four.
 template <typename TC>
 __global__ void __launch_bounds__(256)
@@ -245,8 +354,8 @@ sum_parts_kernel(const float* __restrict__ parts, TC* __restrict__ out, size_t n
 
 // Form of such a product, the cheapest by a count of cycles whose constants were fitted to a sweep of all forms over the
 // shapes above (the choice is within 10 % of the sweep's best at each): `tiles` of 16 rows per wave (1 to 4, four waves along N; 5: 128 x 128 by two times two
-// waves) and how many workgroups share K.
-SOC_EXPORT int soc_gemm_f32_plan(int M, int N, int K, int partial_ok, int* tiles, int* splits) {
+// waves; from 100 on 100 MT + NT of the kernel whose waves share K, for two float32 operands) and how many workgroups share K.
+SOC_EXPORT int soc_gemm_f32_plan(int M, int N, int K, int partial_ok, int both_f32, int* tiles, int* splits) {
     if (M < 1 || N < 1 || K < 4 || K % 4) return 0;
     double best = 0.0;
     *tiles = 0;
@@ -270,7 +379,44 @@ SOC_EXPORT int soc_gemm_f32_plan(int M, int N, int K, int partial_ok, int* tiles
             if (*tiles == 0 || us < best) { best = us; *tiles = t; *splits = s; }
         }
     }
+    if (!both_f32 || K % 64) return *tiles != 0;
+    // Waves that share K: a product of 16 x 16 x 4 takes a SIMD 32 cycles, 5 % more as measured, and a round of workgroups 12 us
+    // beside its products (the first chunk's way, the sums' meeting), the launch 5. (131 rows x 2,560 -> 19,456: 118 by this,
+    // 116 measured; x 9,728 -> 2,560 in eight parts 65 and 65; 2,560 -> 6,144 51 and 49.)
+    static const int forms[] = {205, 305, 405, 505, 605, 705, 805, 905, 308, 408, 508};
+    for (const int f : forms) {
+        const int mt = f / 100, nt = f % 100, steps = K / 64;
+        const long blocks = (long)((M + 16 * mt - 1) / (16 * mt)) * ((N + 16 * nt - 1) / (16 * nt));
+        for (int s = 1; s <= 16; ++s) {
+            const int part = (steps + s - 1) / s;
+            if (s > 1 && (part < 4 || part * (s - 1) >= steps || N % 4)) continue;
+            double us = 5.0 + (double)((blocks * s + 255) / 256) * (0.056 * mt * nt * part + 12.0);
+            const double stream = (double)N * K * 4 / 4.5e6;
+            if (us < stream) us = stream;
+            if (s > 1) us += (double)s * M * N * 4 * 2 / 4e6 + (partial_ok ? 0.0 : 4.0);
+            if (us < best) { best = us; *tiles = f; *splits = s; }
+        }
+    }
     return *tiles != 0;
+}
+
+// tiles: 100 MT + NT
+static int launch_f32_own_k(const float* A, const float* W, float* C, bf16* Cb, int M, int N, int K, int tiles, int splits, hipStream_t s) {
+    const int bm = 16 * (tiles / 100), bn = 16 * (tiles % 100);
+    if (K % 64 || bm < 16 || bn < 16) return (int)hipErrorInvalidValue;
+    const int mb = (M + bm - 1) / bm, nb = (N + bn - 1) / bn, part = ((K / 64 + splits - 1) / splits) * 64;
+    const long blocks = (long)((nb + 7) / 8) * 8 * mb;
+    if (blocks > 0x7fffffffL || (long)part * (splits - 1) >= K) return (int)hipErrorInvalidValue;
+    const dim3 grid((unsigned)blocks, splits);
+#define SOC_F32K(MT_, NT_) \
+    case 100 * MT_ + NT_: hipLaunchKernelGGL((gemm_f32_own_k_kernel<MT_, NT_>), grid, dim3(256), 0, s, A, W, C, Cb, M, N, K, mb, nb, part); break;
+    switch (tiles) {
+        SOC_F32K(2, 5) SOC_F32K(3, 5) SOC_F32K(4, 5) SOC_F32K(5, 5) SOC_F32K(6, 5) SOC_F32K(7, 5) SOC_F32K(8, 5) SOC_F32K(9, 5)
+        SOC_F32K(3, 8) SOC_F32K(4, 8) SOC_F32K(5, 8)
+        default: return (int)hipErrorInvalidValue;
+    }
+#undef SOC_F32K
+    return soc_last_error();
 }
 
 template <typename TA, typename TW>
@@ -307,7 +453,10 @@ SOC_EXPORT int soc_gemm_f32_mfma(const void* A, const void* W, void* C, float* p
     float* out = splits > 1 ? parts : c_dtype == 0 ? (float*)C : nullptr;
     bf16* out_b = out ? nullptr : (bf16*)C;
     int err;
-    if (a_dtype == 0 && w_dtype == 0) err = launch_f32_mfma<float, float>(A, W, out, out_b, M, N, K, tiles, splits, stream);
+    if (tiles >= 100) {
+        if (a_dtype || w_dtype) return (int)hipErrorInvalidValue;
+        err = launch_f32_own_k((const float*)A, (const float*)W, out, out_b, M, N, K, tiles, splits, stream);
+    } else if (a_dtype == 0 && w_dtype == 0) err = launch_f32_mfma<float, float>(A, W, out, out_b, M, N, K, tiles, splits, stream);
     else if (a_dtype == 0 && w_dtype == 1) err = launch_f32_mfma<float, bf16>(A, W, out, out_b, M, N, K, tiles, splits, stream);
     else if (a_dtype == 1 && w_dtype == 0) err = launch_f32_mfma<bf16, float>(A, W, out, out_b, M, N, K, tiles, splits, stream);
     else return (int)hipErrorInvalidValue;

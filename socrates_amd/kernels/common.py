@@ -39,7 +39,7 @@ _EW_SIGNATURES = {
 _GEMM_SIGNATURES = {
     "soc_gemm_generic": [P, P, P, I, I, I, I, I, I, P],
     "soc_gemm_f32_mfma": [P, P, P, P, I, I, I, I, I, I, I, I, P],
-    "soc_gemm_f32_plan": [I, I, I, I, P, P],
+    "soc_gemm_f32_plan": [I, I, I, I, I, P, P],
     "soc_gemm_bf16_mfma": [P, P, P, I, I, I, I, P],
     "soc_gemm_bf16_skinny": [P, P, P, P, I, I, I, I, I, I, I, I, P],
     "soc_gemm_skinny_plan": [I, I, I, I, P, P, P],

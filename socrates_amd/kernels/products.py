@@ -623,7 +623,7 @@ class Products:
             return None
         t, s = c_int(0), c_int(0)
         if not self._gemm.soc_gemm_f32_plan(c_int(M), c_int(N), c_int(K), c_int(1 if allow_partial else 0),
-                                            ctypes.byref(t), ctypes.byref(s)):
+                                            c_int(1 if x.dtype == w.dtype == torch.float32 else 0), ctypes.byref(t), ctypes.byref(s)):
             return None
         tiles, splits = tiles or t.value, splits or s.value
         parts = torch.empty((splits, M, N), dtype=torch.float32, device=self.device) if splits > 1 else None

@@ -132,3 +132,21 @@ def test_activated_products_where_they_are_long_enough(ops, kind, rows):
     # a product whose float32 sum lies between two bfloat16 values may round to either: a step of gate and of up
     torch.testing.assert_close(got.float(), want.float(), atol=2e-2, rtol=2e-2)
     assert ops.linear_activated(x[:70].contiguous(), w, kind) is None
+
+
+@pytest.mark.parametrize("tiles", [205, 305, 405, 505, 605, 705, 805, 905, 308, 408, 508])
+@pytest.mark.parametrize("M,N,K", [(1, 4, 64), (33, 81, 128), (145, 644, 192), (70, 1000, 832)])
+def test_float32_products_whose_waves_share_k(ops, tiles, M, N, K):
+    """One chunk per wave and several, an even and an odd number of them, a tile's first row or column alone, parts of K. K roundings
+    of float32 at the sum of sizes are the bound."""
+    x, w = (torch.randn(s, generator=torch.Generator().manual_seed(s[0])).to(DEV) for s in ((M, K), (N, K)))
+    want, slack = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T * K * 2.0 ** -24 + 1e-12
+    for splits in (1, 2, 3):
+        if splits > 1 and (N % 4 or -(-(K // 64) // splits) * (splits - 1) >= K // 64):
+            continue
+        got = ops._linear_f32(x, w, torch.float32, False, tiles, splits)
+        assert ((got.double() - want).abs() <= slack).all()
+        assert torch.equal(ops._linear_f32(x, w, torch.bfloat16, False, tiles, splits), got.bfloat16())
+        if splits > 1:
+            parts = ops._linear_f32(x, w, torch.float32, True, tiles, splits)
+            assert parts.shape == (splits, M, N) and torch.equal(sum(parts[1:], parts[0]), got)
