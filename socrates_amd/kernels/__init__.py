@@ -22,7 +22,6 @@ recurrences with a matrix state in chunks of a prompt portion,
 from __future__ import annotations
 
 import collections
-import functools
 from ctypes import c_float, c_int, c_longlong, c_void_p
 
 import torch
@@ -38,7 +37,7 @@ from .build import KernelBuildError, build_all, compile_library, load_library
 from .common import (_ATTENTION_SIGNATURES, _ATTENTION_UP_TO_256, _DTYPE_CODE, _EW_SIGNATURES, _GEMM_SIGNATURES, _SAMPLING_SIGNATURES, _WIDE_SIGNATURES,
                      KernelError, NormOwed, RowsByTile, _check, _declare, _ptr)
 from .planning import MAX_KEY_SPLITS, plan_key_splits
-from .products import Products
+from .products import Products, wide_planner
 from .scan import Scan
 from .streams import Streams
 
@@ -102,7 +101,7 @@ class HipKernels(Products, Attention, Latent, Mixers, Hybrid, Composite, Memory,
         # 65 and 64 / 73 at 1,100; 640 x 2,560 11.2 / 8.7 at 65, 21.4 / 18.5 at 3,000. 0 rows: never.
         self.wide_rows, self.wide_min_outputs = 64, 256
         self.wide_min_pairs, self.wide_min_whole = 8e9, (15e9, 4096)
-        self._wide_form = functools.lru_cache(maxsize=4096)(self._wide_plan)
+        self._wide_plan = wide_planner(self._wide)
         self.swiglu_waves = 8           # waves of the fused gate+up product (measured: 4, 8, 16 within 5 %)
         # The sweep form of the skinny product (one workgroup per compute unit keeps its slices
         # of x in registers and walks over the weight tiles): from this many rows of x on, for

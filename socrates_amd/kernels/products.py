@@ -6,11 +6,23 @@ the measurement that chooses among them. A mixin of ``HipKernels``."""
 from __future__ import annotations
 
 import ctypes
+import functools
 from ctypes import c_float, c_int
 
 import torch
 
 from .common import _DTYPE_CODE, KernelError, NormOwed, RowsByTile, _check, _ptr
+
+
+def wide_planner(lib):
+    """The form of a product of many rows by its sizes (``soc_wide_plan``, some 200 estimates), those of the last 4,096 kept: a step
+    asks for the same few of every layer. Holds nothing but the library."""
+    @functools.lru_cache(maxsize=4096)
+    def plan(M, N, K, act, partial):
+        form = [c_int(0) for _ in range(4)]
+        found = lib.soc_wide_plan(c_int(M), c_int(N), c_int(K), c_int(act), c_int(1 if partial else 0), *map(ctypes.byref, form))
+        return tuple(f.value for f in form) if found else None
+    return plan
 
 
 class Products:
@@ -559,18 +571,19 @@ class Products:
 
     WIDE_PLAIN, WIDE_SILU, WIDE_GATED, WIDE_GELU, WIDE_SQUARED = range(5)
 
-    def _wide_plan(self, M, N, K, act=0, partial=False):
+    def _wide_form(self, M, N, K, act=0, partial=False):
         """(blocks of 32 rows, of 32 outputs, last tiles halved, parts of K) of a product of many rows, or None."""
-        form = [c_int(0) for _ in range(4)]
-        if M <= self.wide_rows or not self.wide_rows or N < self.wide_min_outputs or not self._wide.soc_wide_plan(
-                c_int(M), c_int(N), c_int(K), c_int(act), c_int(1 if partial else 0), *map(ctypes.byref, form)):
+        if M <= self.wide_rows or not self.wide_rows or N < self.wide_min_outputs:
+            return None
+        form = self._wide_plan(M, N, K, act, bool(partial))
+        if form is None:
             return None
         operations = 2.0 * M * N * K
         if act in (self.WIDE_SILU, self.WIDE_GATED, self.WIDE_GELU):
             enough = operations >= self.wide_min_pairs
         else:
-            enough = form[3].value > 1 and partial or operations >= self.wide_min_whole[0] or K >= self.wide_min_whole[1]
-        return tuple(f.value for f in form) if enough else None
+            enough = form[3] > 1 and partial or operations >= self.wide_min_whole[0] or K >= self.wide_min_whole[1]
+        return form if enough else None
 
     def _wide_product(self, form, x, w, out_dtype, partial=False, act=0, halves=False, gate=(0.0, 1.0, 0.0)):
         """x [M, K] times w [N, K] transposed by ``form``; with an activation over pairs [M, N / 2] (``halves``: w holds gate rows
