@@ -45,6 +45,9 @@ __all__ = ["HipKernels", "KernelBuildError", "KernelError", "MAX_KEY_SPLITS", "N
            "compile_library", "load_library", "plan_key_splits"]
 
 
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (lambda index: torch.cuda.current_stream(index).cuda_stream)
+
+
 class HipKernels(Products, Attention, Latent, Mixers, Hybrid, Composite, Memory, Streams, Delta, Scan):
     def __init__(self, dtype=torch.bfloat16, device="cuda:0"):
         if dtype not in _DTYPE_CODE:
@@ -92,15 +95,19 @@ class HipKernels(Products, Attention, Latent, Mixers, Hybrid, Composite, Memory,
         # (nn.Linear)
         self.library_gemm = True
         # bfloat16 products of more than ``wide_rows`` rows and at least ``wide_min_outputs`` outputs: tiles of up to 256 x 256
-        # (csrc/wide.hip). Partial sums always, an activation over gate and up from ``wide_min_pairs`` operations on, whole
-        # sums from ``wide_min_whole`` operations or terms of a sum on; the rest goes to the library. Us inside replayed
-        # graphs, weights from memory, own / library (which has an activation's 3 to 23 us besides): partial sums 2,560 x
-        # 2,560 9.1 / 13.3 at 65 rows, 23.4 / 23.3 at 1,100; 2,560 x 9,728 16.5 / 25.9 and 60 / 73. Gate and up of 9,728 x
+        # (csrc/wide.hip). Partial sums always, an activation over gate and up from ``wide_min_pairs`` operations on. Whole sums
+        # from ``wide_min_whole`` operations on, but for ``wide_not_whole`` (from, to) operations with sums of fewer than
+        # ``wide_long_sums`` terms. The rest goes to the library.
+        # Us inside replayed graphs, weights from memory, own / library (which has an activation's 3 to 23 us besides): partial sums
+        # 2,560 x 2,560 9.1 / 13.3 at 65 rows, 23.4 / 23.3 at 1,100; 2,560 x 9,728 16.5 / 25.9 and 60 / 73. Gate and up of 9,728 x
         # 2,560 36 / 33 at 80 rows, 36 / 42 at 130, 50 / 55 at 512, 172 / 211 at 2,048. Whole sums 2,560 x 2,560 17.5 / 14.9
-        # at 200, 27.6 / 23.3 at 1,100, 32.4 / 35.6 at 2,048; 5,120 x 2,560 27.0 / 28.4 at 500; 2,560 x 9,728 21.4 / 25.9 at
-        # 65 and 64 / 73 at 1,100; 640 x 2,560 11.2 / 8.7 at 65, 21.4 / 18.5 at 3,000. 0 rows: never.
+        # at 200, 22 / 19 at 500, 27.6 / 23.3 at 1,100, 32.4 / 35.6 at 2,048; 5,120 x 2,560 27.0 / 28.4 at 500; 2,560 x 9,728 21.4 /
+        # 25.9 at 65 and 64 / 73 at 1,100. Short ones stay here all the same: a step of some hundred rows waits for the host's
+        # launches, and the library's take it 25 us against 12 (whole prompt steps, library / own: Qwen3-4B, 12 layers, 70 tokens
+        # 1,915 / 1,590, 150 tokens 1,650 / 1,576, 300 tokens 1,890 / 1,920; Mitisun, 6 layers, 100 tokens 1,884 / 1,645, 500 tokens
+        # 2,023 / 1,910). 0 rows: never.
         self.wide_rows, self.wide_min_outputs = 64, 256
-        self.wide_min_pairs, self.wide_min_whole = 8e9, (15e9, 4096)
+        self.wide_min_pairs, self.wide_min_whole, self.wide_not_whole, self.wide_long_sums = 8e9, 1e9, (7e9, 15e9), 4096
         self._wide_plan = wide_planner(self._wide)
         self.swiglu_waves = 8           # waves of the fused gate+up product (measured: 4, 8, 16 within 5 %)
         # The sweep form of the skinny product (one workgroup per compute unit keeps its slices
@@ -167,16 +174,20 @@ class HipKernels(Products, Attention, Latent, Mixers, Hybrid, Composite, Memory,
 
     # -- helpers -----------------------------------------------------------------------------
     def _stream(self):
-        return c_void_p(torch.cuda.current_stream(self.device).cuda_stream)
+        """The current stream of the kernel set's device, as the number that the entry points' declared pointers take. (Through
+        ``torch.cuda.current_stream`` it costs 4 to 5 us a launch, a quarter of what a launch costs the host: steps of a
+        few dozen tokens, 90 launches for 12 layers, are bound by that.)"""
+        index = self.device.index
+        return _raw_stream(torch.cuda.current_device() if index is None else index)
 
     def _want(self, t, name, dtype=None, shape=None):
-        if t.device.type != "cuda":
+        if not t.is_cuda:
             raise KernelError(f"{name} is on {t.device}, the kernels need it on the GPU")
         if not t.is_contiguous():
             raise KernelError(f"{name} is not contiguous")
         if dtype is not None and t.dtype != dtype:
             raise KernelError(f"{name} has dtype {t.dtype}, expected {dtype}")
-        if shape is not None and tuple(t.shape) != tuple(shape):
+        if shape is not None and t.shape != shape and tuple(t.shape) != tuple(shape):
             raise KernelError(f"{name} has shape {tuple(t.shape)}, expected {tuple(shape)}")
         return t
 

@@ -15,7 +15,8 @@ class KernelError(RuntimeError):
 
 
 def _ptr(t):
-    return None if t is None else c_void_p(t.data_ptr())
+    """What a declared pointer argument takes (every entry point's arguments are declared: ``_declare``)."""
+    return None if t is None else t.data_ptr()
 
 
 def _check(err, what):

@@ -582,7 +582,9 @@ class Products:
         if act in (self.WIDE_SILU, self.WIDE_GATED, self.WIDE_GELU):
             enough = operations >= self.wide_min_pairs
         else:
-            enough = form[3] > 1 and partial or operations >= self.wide_min_whole[0] or K >= self.wide_min_whole[1]
+            low, high = self.wide_not_whole
+            enough = (form[3] > 1 and partial or K >= self.wide_long_sums
+                      or operations >= self.wide_min_whole and not low <= operations < high)
         return form if enough else None
 
     def _wide_product(self, form, x, w, out_dtype, partial=False, act=0, halves=False, gate=(0.0, 1.0, 0.0)):
