@@ -85,10 +85,6 @@ __device__ __forceinline__ void wide_walk(const char* x, const char* w, const ui
         if (of_x) a[h][n] = *reinterpret_cast<const bf16x8_t*>(&xs[(2 * n + wm) * 1024 + at[h]]);
         else b[h][n] = *reinterpret_cast<const bf16x8_t*>(&ws[(wn * NJ + n) * 1024 + at[h]]);
     };
-#pragma unroll
-    for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
     // one half: its products, the reads of the next half and one operand's loads of a later step
     auto half = [&](auto second, const uint16_t* xs, const uint16_t* ws, int s, int slot) {
         constexpr int H = decltype(second)::value, T = MI * NJ, R = MI + NJ, L = H ? MI : NJ;
@@ -123,6 +119,15 @@ __device__ __forceinline__ void wide_walk(const char* x, const char* w, const ui
             for (int i = 0; i < MI; ++i) load_x(s + RX, s + RX, i);
         }
     }
+    __builtin_amdgcn_sched_barrier(0);                       // (while they are on their way)
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) asm volatile("" : "+a"(acc[i][j]));
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(Rings::NEWER + MI) : "memory");
 #pragma unroll
     for (int r = 0; r < MI + NJ; ++r) read(0, lds, wlds, r);

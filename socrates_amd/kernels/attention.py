@@ -357,10 +357,10 @@ class Attention:
             # block's keys. Chosen by the number of 32-row workgroups the long portions give
             # (measured at 8 kv heads of 4 x 128 and 4 x 64, in us for 16 / 2 x 16 / 32 rows /
             # 32 rows in two key halves; 512 slots of four waves on the GPU):
-            #   256 tokens from 0 (64 workgroups): 11 / 14 / 13 / 14;  512 (128): 17 / 21 / 20 / 19
-            #   1,024 from 0 (256): 32 / 36 / 34 / 29;  2,048 (512): 82 / 74 / 69 / 62
-            #   3,072 from 0 (768): 163 / 112 / 107 / 123;  8,192 (2,048): 941 / 650 / 633 / 695
-            #   1,024 behind 3,072 (256): 117 / 122 / 111 / 89;  2,048 behind 6,144 (512): 488 / 305 / 296 / 297
+            #   256 tokens from 0 (64 workgroups): 13 / 15 / 14 / 13;  512 (128): 21 / 22 / 21 / 18
+            #   1,024 from 0 (256): 38 / 39 / 35 / 28;  2,048 (512): 86 / 78 / 71 / 57
+            #   3,072 from 0 (768): 154 / 112 / 110 / 115;  8,192 (2,048): 960 / 650 / 636 / 672
+            #   1,024 behind 3,072 (256): 130 / 122 / 115 / 83;  2,048 behind 6,144 (512): 581 / 305 / 295 / 302
             # at head size 64 the eight-wave form stays ahead or level up to 8,192 tokens.
             th = self.prompt_form_thresholds
             wg_rt = 1
