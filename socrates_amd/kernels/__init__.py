@@ -76,12 +76,14 @@ class HipKernels(Products, Attention, Latent, Mixers, Hybrid, Composite, Memory,
         self.attention_mfma = True          # bfloat16 takes the MFMA kernels
         self.attention_workgroup = True     # prompt portions take the kernel that shares K/V through LDS
         # Which form of the prompt-portion attention a step takes, by the number of workgroups
-        # its long portions give (of 32 rows x 4 waves for the first three, of the chosen form
-        # for the last). Measured on an MI355X (256 compute units) at 8 kv heads of 4 x 128 and
+        # its long portions give (of the chosen form for the first, of 32 rows x 4 waves for the others
+        # but the last). Measured on an MI355X (256 compute units) at 8 kv heads of 4 x 128 and
         # 4 x 64; another head layout or another GPU may want other values: set them here.
         self.prompt_form_thresholds = {
             "workgroup_kernel": 256,          # below: the per-wave kernel with key splits
-            "eight_waves": 256,               # from here: 32 rows per wave, keys in two halves
+            "eight_waves": 128,               # from here (head sizes over 64): 32 rows per wave, keys in two halves
+            "eight_waves_small_heads": 256,   # the same for head sizes up to 64
+            "four_waves_with_kept_keys": 256, # with kept first keys or means, from here: four waves of 32 rows
             "four_waves_of_32_rows": 768,     # from here (head sizes over 64): four waves of 32 rows
             "two_tiles_of_16_rows": 512,      # head sizes that are no multiple of 32, up to 64
         }

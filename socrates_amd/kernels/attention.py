@@ -363,6 +363,7 @@ class Attention:
             #   1,024 behind 3,072 (256): 130 / 122 / 115 / 83;  2,048 behind 6,144 (512): 581 / 305 / 295 / 302
             # at head size 64 the eight-wave form stays ahead or level up to 8,192 tokens.
             th = self.prompt_form_thresholds
+            eight = th["eight_waves" if D > 64 else "eight_waves_small_heads"]
             wg_rt = 1
             if self.attention_row_tiles in (1, 2, 32, 64):
                 wg_rt = self.attention_row_tiles
@@ -372,8 +373,10 @@ class Attention:
                 n32 = (n_long // (4 * max(1, 32 >> gpl))) * Hkv * ((G + 15) // 16)
                 if n32 >= th["four_waves_of_32_rows"] and D > 64:
                     wg_rt = 32
-                elif n32 >= th["eight_waves"]:
-                    wg_rt = 64 if not (keep_first or pool) else 32      # (no kept keys or means with the keys in two halves)
+                elif n32 >= eight and not (keep_first or pool):      # (no kept keys or means with the keys in two halves)
+                    wg_rt = 64
+                elif n32 >= th["four_waves_with_kept_keys"]:
+                    wg_rt = 32
             elif D <= 64 and (n_long // (4 * max(1, 32 >> gpl))) * Hkv * ((G + 15) // 16) >= th["two_tiles_of_16_rows"]:
                 wg_rt = 2
             wg_tokens = 4 * max(1, (32 if wg_rt >= 32 else 16 * wg_rt) >> gpl)
@@ -383,7 +386,9 @@ class Attention:
             # shorter portion behind a long context is better served by the per-wave kernel
             # with key splits (128 tokens behind 8 k: 95 us against 196 us). An override of
             # the row tiles (tests) forces the choice.
-            enough = ((n_long // wg_tokens) * Hkv * ((G + 15) // 16) >= th["workgroup_kernel"]
+            # The eight-wave form is enough with half as many: 512 tokens from 0 17.5 us against 20.4 of 16 rows a wave, behind 750
+            # 31 against 41, behind 3,072 71 against 107, behind 6,144 127 against 193.
+            enough = ((n_long // wg_tokens) * Hkv * ((G + 15) // 16) >= (eight if wg_rt == 64 else th["workgroup_kernel"])
                       or self.attention_row_tiles is not None)
             if (keep_first or pool) and wg_rt == 64:
                 wg_rt = 32

@@ -65,3 +65,29 @@ def test_tiles_of_64_keys(ops, D, BS, start, T, window, keep, cap):
             _ptr(out), c_int(T), c_int(Hq), c_int(Hkv), c_int(BS), c_float(D ** -0.5), c_int(window), c_int(form), c_int(2),
             c_int(keep), c_int(0), None, None, None, None, c_int(0), c_int(0), c_float(cap), ops._stream())
         assert err == 0 and ((out.double() - want).abs() <= slack).all(), (form, float(((out.double() - want).abs() - slack).max()))
+
+
+def test_which_form_a_portion_takes(ops):
+    """512 tokens of eight kv heads are 128 workgroups of 32 rows a wave: keys in two halves; fewer take 16 rows a wave or key
+    splits, kept first keys four waves from 256 workgroups on."""
+    from types import SimpleNamespace
+
+    import numpy as np
+    Hkv, G, D, BS = 8, 4, 128, 16
+    for T, want in ((511, None), (512, ("workgroup", 64)), (3071, ("workgroup", 64)), (3072, ("workgroup", 32))):
+        pages = -(-T // BS)
+        q = torch.randn((T, Hkv * G, D), generator=torch.Generator().manual_seed(1)).bfloat16().to(DEV)
+        k, v = (torch.randn((pages, Hkv, BS, D), generator=torch.Generator().manual_seed(s)).bfloat16().to(DEV) for s in (2, 3))
+        table = torch.arange(pages, dtype=torch.int32, device=DEV)[None]
+        slot = SimpleNamespace(k=k, v=v, block_table=table, block_size=BS)
+        starts = torch.tensor([0, T], dtype=torch.int32)
+        ctx = SimpleNamespace(token_rows=torch.zeros(T, dtype=torch.int32, device=DEV), positions=torch.arange(T, dtype=torch.int32, device=DEV),
+                              max_ctx_len=T, max_q_len=T, n_seqs=1, seq_qstart=starts.to(DEV),
+                              host={"seq_qstart": np.array([0, T], dtype=np.int32)})
+        out = ops.paged_attention(q, slot, ctx, D ** -0.5)
+        assert (ops.last_attention_kernel == want) if want else ops.last_attention_kernel != ("workgroup", 64), (T, ops.last_attention_kernel)
+        i = torch.tensor([0, 1, T // 2, T - 1], device=DEV)
+        kk, vv = (t.permute(1, 0, 2, 3).reshape(Hkv, -1, D)[:, :T].double().repeat_interleave(G, 0) for t in (k, v))
+        s = (torch.einsum("thd,hjd->htj", q[i].double(), kk) * D ** -0.5).masked_fill(torch.arange(T, device=DEV)[None] > i[:, None], -math.inf)
+        expect = (torch.softmax(s, -1) @ vv).transpose(0, 1)
+        torch.testing.assert_close(out.view(T, -1, D)[i].double(), expect, atol=2e-2, rtol=2e-2)
